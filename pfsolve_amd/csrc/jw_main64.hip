@@ -44,15 +44,24 @@ __device__ __forceinline__ int swz(int c)
 __device__ __forceinline__ void compiler_fence() { asm volatile("" ::: "memory"); }
 __host__ __device__ __forceinline__ int64_t max_i64(int64_t a, int64_t b) { return a > b ? a : b; }
 
+// A chunk (rows 2c, 2c + 1) at any 8-byte aligned address: gfx950 takes a 16-byte global
+// access at dword alignment, so systems of odd stride or offset move by the same
+// instructions as 16-byte aligned ones (LDS DMA does not: those paths stay aligned).
+typedef double jw_d2u __attribute__((ext_vector_type(2), aligned(8)));
+__device__ __forceinline__ double2 load_chunk(const double* p)
+{
+    const jw_d2u t = *reinterpret_cast<const jw_d2u*>(p);
+    return make_double2(t.x, t.y);
+}
+
 // store of a result chunk: written once and not read back by the step, so it is
 // marked nontemporal (streamed to memory without allocating in the caches)
-__device__ __forceinline__ void store_stream(double2* p, double2 v)
+__device__ __forceinline__ void store_stream(double* p, double2 v)
 {
-    typedef double d2v __attribute__((ext_vector_type(2)));
-    d2v t;
+    jw_d2u t;
     t.x = v.x;
     t.y = v.y;
-    __builtin_nontemporal_store(t, reinterpret_cast<d2v*>(p));
+    __builtin_nontemporal_store(t, reinterpret_cast<jw_d2u*>(p));
 }
 
 // keeps the scheduler from hoisting one phase's table loads into the previous
@@ -496,12 +505,11 @@ __device__ __forceinline__ void store_pair(const double2* stg, int lane, const j
 #pragma unroll
     for (int s = 0; s < 2; s++) {
         if (s == 1 && !ok1) continue;
-        // the host only selects this kernel when sys*stride + offSol is even and rhs is 16-byte aligned
-        double2* dst2 = reinterpret_cast<double2*>(g.rhs) + (((sys0 + s) * g.stride + g.offSol) >> 1);
+        double* dst = g.rhs + (sys0 + s) * g.stride + g.offSol;
 #pragma unroll
         for (int k = 0; k < H; k++) {
             const int c = 64 * k + lane;
-            if (c >= g.ocl && c < g.och) store_stream(dst2 + c, v[s][k]);
+            if (c >= g.ocl && c < g.och) store_stream(dst + 2 * c, v[s][k]);
         }
     }
     if (g.out_edge_lo || g.out_edge_hi) {
@@ -614,7 +622,7 @@ __device__ __forceinline__ void jw_groups64(const double* tab, double2* stg, int
         const int m = c & (LG - 1);
         const double2 v = stg[c];
         if (sys < sys_end && m >= g.ocl && m < g.och)
-            store_stream(reinterpret_cast<double2*>(g.rhs + sys * g.stride + g.offSol) + m, v);
+            store_stream(g.rhs + sys * g.stride + g.offSol + 2 * m, v);
     }
 #pragma unroll
     for (int e = 0; e < 2; e++) {
@@ -1187,11 +1195,11 @@ __device__ __forceinline__ void jw_single64(__amdgpu_buffer_rsrc_t tab, double2*
     for (int k = 0; k < H; k++) v[k] = stg[swz<H>(64 * k + lane)];
 #pragma unroll
     for (int k = 0; k < H; k++) asm volatile("" : "+v"(v[k].x), "+v"(v[k].y));
-    double2* dst2 = reinterpret_cast<double2*>(g.rhs) + ((sys * g.stride + g.offSol) >> 1);
+    double* dst = g.rhs + sys * g.stride + g.offSol;
 #pragma unroll
     for (int k = 0; k < H; k++) {
         const int c = 64 * k + lane;
-        if (c >= g.ocl && c < g.och) store_stream(dst2 + c, v[k]);
+        if (c >= g.ocl && c < g.och) store_stream(dst + 2 * c, v[k]);
     }
 #pragma unroll
     for (int e = 0; e < 2; e++) {
@@ -1244,15 +1252,15 @@ __device__ __forceinline__ void load_pair_direct(double2 (&pf)[2][R / 2], int la
 {
     constexpr int H = R / 2;
     const bool ok1 = sys0 + 1 < g.nsys;
-    const double2* src0 = reinterpret_cast<const double2*>(g.rhs) + ((sys0 * g.stride + g.offSol) >> 1);
+    const double* src0 = g.rhs + sys0 * g.stride + g.offSol;
 #pragma unroll
     for (int s = 0; s < 2; s++) {
-        const double2* src = src0 + s * (g.stride >> 1);
+        const double* src = src0 + s * g.stride;
 #pragma unroll
         for (int m = 0; m < H; m++) {
             const int c = lane * H + m;
             double2 v = make_double2(0.0, 0.0);
-            if (c >= g.icl && c < g.ich && (s == 0 || ok1)) v = src[c];
+            if (c >= g.icl && c < g.ich && (s == 0 || ok1)) v = load_chunk(src + 2 * c);
             pf[s][m] = v;
         }
     }
@@ -1369,7 +1377,7 @@ __device__ __forceinline__ void store_pair_packed(const double2* stg, int lane, 
             a += prev[k].x;
             b += prev[k].y;
         }
-        store_stream(dst + r, make_double2(a, b));
+        store_stream(reinterpret_cast<double*>(dst + r), make_double2(a, b));
     }
 }
 

@@ -662,9 +662,13 @@ static PfSolveResult append_impl(PfSolveApplication* app, const PfSolveLaunchPar
         if (p->long_only) return append_long(app, &src, &run, s, table);
         const uintptr_t base = (uintptr_t)run.rhs;
         run.vec2 = p->precision == JW_PREC_F64 && (base % 16) == 0 && (run.stride % 2) == 0 && (run.offSol % 2) == 0;
-        if (p->R64 && run.vec2 && cfg->kernelVariant != 1) {
+        if (p->R64 && (run.vec2 || (p->split64 && base % 8 == 0)) && cfg->kernelVariant != 1) {
             /* wave-per-system kernel: table format 2, built by a prologue launch or,
-             * in the compute / store split kernel, by every workgroup in LDS */
+             * in the compute / store split kernel, by every workgroup in LDS.  The split
+             * kernel loads and stores global memory from registers and takes systems at any
+             * 8-byte address (30000 systems of 333 rows, packed: 41.4 us a step, 61.8 us on
+             * the general kernel and its table launch); the others stage by LDS DMA, 16-byte
+             * aligned */
             if (nsys <= 0) return PFSOLVE_SUCCESS;
             if (!p->split64 && jwdev_prologue(&src, cfg->buffer[0], table, 64, p->R64, p->precision, 2, s) != 0)
                 return PFSOLVE_ERROR_FAILED_TO_LAUNCH_KERNEL;
