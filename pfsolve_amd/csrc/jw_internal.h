@@ -68,14 +68,13 @@ typedef struct jw_source_desc {
     int64_t alt_N;
 } jw_source_desc;
 
-/* Tables of a chained step (numConsecutiveJWIterations = K <= JW_CHAIN_MAX), built by one
- * launch with one workgroup per iteration; passed by value (no device copy of the jobs). */
+/* Matrices of a chained step (numConsecutiveJWIterations = K <= JW_CHAIN_MAX), passed to the
+ * kernels by value (no device copy). */
 #define JW_CHAIN_MAX 16
 typedef struct jw_chain_jobs {
     jw_source_desc src[JW_CHAIN_MAX];
     const void* matrices[JW_CHAIN_MAX];
-    void* table;              /* iteration k's format-2 table at table + k * tab_stride bytes */
-    int64_t tab_stride;
+    void* table;              /* the K tables, back to back, when they do not fit in LDS */
     int32_t K, R;
 } jw_chain_jobs;
 
@@ -233,11 +232,11 @@ int jwdev_main(const jw_run_desc* r, int L, int R, int precision, int waves, int
 int64_t jwdev_dd64_table_elems(int R);
 int jwdev_dd64_occupancy(int R, int waves);
 int jwdev_dd64(const jw_run_desc* r, int R, int waves, int grid, void* stream);
-/* chained steps: the K tables (one launch), then the kernel that keeps each pair of systems
- * in registers through the K iterations (FP64, 16-byte aligned pairs, R in {2,4,8,16}) */
-int jwdev_prologue_chain(const jw_chain_jobs* jobs, void* stream);
-int jwdev_chain64_occupancy(int R);
-int jwdev_chain64(const jw_run_desc* r, const void* tables, int64_t tab_elems, int K, int R, int grid, void* stream);
+/* chained steps, one launch when the K iterations' tables fit in LDS: wavefronts per
+ * workgroup (returns workgroups per CU, 0: not available), the step.  up: the upper
+ * matvec and lower solve (upperBanded 1), else the lower matvec and upper solve */
+int jwdev_chain64_shape(int R, int K, int* waves);
+int jwdev_chain64(const jw_run_desc* r, const jw_chain_jobs* jobs, int up, int grid, void* stream);
 /* long systems: rows per lane of a chunk, chunks per table build, the table of every
  * chunk (one workgroup per build of `nsub` chunks; pivots handed from build to build),
  * the chunk kernel in one of the JW_LONG_* modes, the reduced solve */

@@ -1014,48 +1014,6 @@ __global__ __launch_bounds__(max_threads<kLong64R>()) void jw_long64_front_kerne
 }
 
 // ---------------------------------------------------------------------------
-// Chained steps (numConsecutiveJWIterations = K): a wavefront owns a pair of systems
-// through all K iterations, whose right-hand sides stay in its registers in between (one
-// read and one write of HBM per K-step instead of K).  Iteration k applies its own
-// format-2 table; the K tables stay in global memory (every wavefront reads them, so they
-// are served from L2); LDS holds each wavefront's staging.  The input keep-range applies
-// to the first iteration's rows, the output keep-range to the last one's.
-// ---------------------------------------------------------------------------
-template <int R>
-constexpr int chain_waves() { return 4; }
-
-template <int R, bool ALL3>
-__global__ __launch_bounds__(256) void jw_chain64_kernel(jw_run_desc d, const double* tables, int64_t tab_elems,
-                                                         int K)
-{
-    extern __shared__ __align__(16) unsigned char smem[];
-    const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int nwaves = blockDim.x >> 6;
-    double2* stg = reinterpret_cast<double2*>(smem) + (size_t)wave * 64 * R;
-    zero_staging<R>(stg, lane);
-    __builtin_amdgcn_s_waitcnt(0xC07F);   // lgkmcnt(0): zeros written before any DMA lands
-    compiler_fence();
-    const int64_t npass = (d.nsys + 1) >> 1;
-    for (int64_t q = (int64_t)blockIdx.x * nwaves + wave; q < npass; q += (int64_t)gridDim.x * nwaves) {
-        const jw_pass64 g = make_pass64(reinterpret_cast<double*>(d.rhs), d.nsys, d.stride, d.offSol,
-                                        (int)d.in_lo, (int)d.in_hi, (int)d.out_lo, (int)d.out_hi, d.kl, d.ku,
-                                        d.fwd, d.b1, d.b2, d.apply_scale, d.scale_hi, lane);
-        dma_pair<R>(stg, lane, g, 2 * q);
-        __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0): the DMA writes have landed in LDS
-        compiler_fence();
-        double x0[R], x1[R];
-        read_pair<R>(stg, lane, g, 2 * q, x0, x1);
-        for (int k = 0; k < K; k++) compute_pair<R, ALL3>(tables + (int64_t)k * tab_elems, lane, g, x0, x1);
-        write_blocked<R>(stg, lane, x0, x1);
-        store_pair<R>(stg, lane, g, 2 * q);
-        rezero_input<R>(stg, lane, g);
-        __builtin_amdgcn_s_waitcnt(0xC07F);   // lgkmcnt(0): LDS traffic done before the next DMA lands
-        compiler_fence();
-    }
-}
-
-// ---------------------------------------------------------------------------
 // Long systems (R = 32 rows per lane, N <= 2048): one system per wavefront pass.
 // The 140 KiB table stays in global memory (every wavefront of the grid reads
 // it, so it is served from L2) and coefficients are streamed row by row instead
@@ -1279,6 +1237,247 @@ __device__ __forceinline__ void unpack_pair(const double2 (&pf)[2][R / 2], int l
         x1[2 * m + 1] = pf[1][m].y;
     }
     read_edges<R>(lane, g, sys0, x0, x1);
+}
+
+// ---------------------------------------------------------------------------
+// Chained steps (numConsecutiveJWIterations = K): a wavefront owns a pair of systems
+// through all K iterations, whose right-hand sides stay in its registers in between (one
+// read and one write of HBM per K-step instead of K).  The input keep-range applies to the
+// first iteration's rows, the output keep-range to the last one's.
+//
+// An iteration is a bidiagonal matvec and a unit-bidiagonal solve: per row the diagonal,
+// one off-diagonal and the solve's off-diagonal, and the 7 scan multipliers of its one
+// recurrence.  As a table of its own (JW_CHAIN_TAB, 15.5 KiB at R = 8 against the 44 KiB of
+// format 2) the K tables fit in LDS, where every workgroup builds them from the matrices
+// (no pivots: the build is the loads and one product scan), so the step is one launch and
+// the loop touches HBM for right-hand sides only.  Bound: HBM.  65536 systems, N = 512 ->
+// 509, K = 4: 114 us per step; 240 us when a launch of its own wrote format-2 tables
+// and every pass read 24 KiB of them per iteration through the L2.
+// A chain whose tables leave no room for 4 wavefronts' stagings (N = 512: K >= 10; N = 1024:
+// K >= 5) keeps the first ones in LDS and reads the others, written by
+// jw_chain_tables_kernel, through the L2.
+// ---------------------------------------------------------------------------
+// doubles of one iteration's table: (v0, voff) of row-in-lane i, lane t at (64 i + t) 2, the
+// solve's off-diagonal at 128 R + 64 i + t, multiplier k at 192 R + 64 k + t
+__host__ __device__ constexpr int chain_tab_elems(int R) { return (3 * R + 7) * 64; }
+
+// rows of iteration k's table: 64 R rows from thread `tid` in steps of nthr
+template <int R, bool UP>
+__device__ __forceinline__ void chain_rows(const jw_source_desc& d, const double* mat, double* tab, int tid, int nthr)
+{
+    const int64_t N = d.N, ncols = d.Ncols > 0 ? d.Ncols : N;
+    const bool band = d.band_kind != JW_BAND_NONE, solve = d.solve_kind != JW_SOLVE_NONE;
+    const int64_t offA = UP ? d.udA : d.ldA, offS = UP ? d.ldS : d.udS;
+    for (int r = tid; r < 64 * R; r += nthr) {
+        const bool in = r < N;
+        const int64_t P = source_pos(d, in ? r : 0, N);
+        // entries of the matvec and the solve inside the matrix; the others are read at an
+        // in-bounds position and dropped by the selects
+        const double v0 = !band || d.unit_diag ? 1.0 : mat[d.mdA + P];
+        const double vo = band ? mat[offA + P] : 0.0;
+        const double so = solve ? mat[offS + P] : 0.0;
+        const bool vin = UP ? r + 1 < ncols : r >= 1 && r - 1 < ncols;
+        const bool sin = UP ? r >= 1 : r + 1 < N;
+        const int i = r % R, t = r / R;
+        *reinterpret_cast<double2*>(tab + (64 * i + t) * 2) = make_double2(in ? v0 : 0.0, in && vin ? vo : 0.0);
+        tab[128 * R + 64 * i + t] = in && sin ? so : 0.0;
+    }
+}
+
+// the scan multipliers of one table by one wavefront, once its rows are written: as the
+// format-2 build's (jw_prologue.h), for the forward (UP: the upper matvec's lower solve) or
+// the backward recurrence
+template <int R, bool UP>
+__device__ __forceinline__ void chain_multipliers(double* tab, int t)
+{
+    double v = 1.0;
+#pragma unroll
+    for (int i = 0; i < R; i++) v *= -tab[128 * R + 64 * i + t];
+    double* m = tab + 192 * R;
+    const int tr = t & 15, rw = t >> 4;
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        const int s = 1 << k;
+        m[64 * k + t] = v;
+        const bool from = UP ? tr >= s : tr + s <= 15;
+        const double w = lane_fetch(v, from ? (UP ? t - s : t + s) : t);
+        if (from) v *= w;
+    }
+    if (UP) {
+        const double pre47 = lane_fetch(v, 47);
+        m[64 * 4 + t] = v;
+        m[64 * 5 + t] = rw == 2 ? v : (rw == 3 ? pre47 * v : 0.0);
+        m[64 * 6 + t] = 0.0;
+    } else {
+        const double P1 = lane_fetch(v, 16), P2 = lane_fetch(v, 32);
+        m[64 * 4 + t] = rw == 0 ? v : 0.0;
+        m[64 * 5 + t] = rw == 0 ? v * P1 : (rw == 1 ? v : 0.0);
+        m[64 * 6 + t] = rw == 0 ? v * P1 * P2 : (rw == 1 ? v * P2 : (rw == 2 ? v : 0.0));
+    }
+}
+
+// one iteration on a pair in registers (the steps of compute_pair for these operators)
+template <int R, bool UP>
+__device__ __forceinline__ void chain_pair(const double* tab, int lane, bool band, bool solve, bool apply_scale,
+                                           double row0_scale, double (&x0)[R], double (&x1)[R])
+{
+    if (band) {
+        double na = UP ? dpp_d<DPP_WAVE_SHL1>(x0[0]) : dpp_d<DPP_WAVE_SHR1>(x0[R - 1]);
+        double nb = UP ? dpp_d<DPP_WAVE_SHL1>(x1[0]) : dpp_d<DPP_WAVE_SHR1>(x1[R - 1]);
+#pragma unroll
+        for (int k = 0; k < R; k++) {
+            const int i = UP ? R - 1 - k : k;   // from the end whose neighbour came from the next lane
+            const double2 v = *reinterpret_cast<const double2*>(tab + (64 * i + lane) * 2);
+            const double xa = x0[i], xb = x1[i];
+            x0[i] = __builtin_fma(v.y, na, v.x * xa);
+            x1[i] = __builtin_fma(v.y, nb, v.x * xb);
+            na = xa;
+            nb = xb;
+        }
+    }
+    if (!solve) return;
+    double s[R];
+#pragma unroll
+    for (int i = 0; i < R; i++) s[i] = tab[128 * R + 64 * i + lane];
+    const double* m = tab + 192 * R + lane;
+    // row order of the recurrence: forward (UP) or backward
+    double a = x0[UP ? 0 : R - 1], b = x1[UP ? 0 : R - 1];
+#pragma unroll
+    for (int k = 1; k < R; k++) {
+        const int i = UP ? k : R - 1 - k;
+        a = __builtin_fma(-s[i], a, x0[i]);
+        b = __builtin_fma(-s[i], b, x1[i]);
+    }
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        const double f = m[64 * k];
+        double sa, sb;
+        switch (k) {
+        case 0: sa = dpp_d<UP ? DPP_ROW_SHR(1) : DPP_ROW_SHL(1)>(a); sb = dpp_d<UP ? DPP_ROW_SHR(1) : DPP_ROW_SHL(1)>(b); break;
+        case 1: sa = dpp_d<UP ? DPP_ROW_SHR(2) : DPP_ROW_SHL(2)>(a); sb = dpp_d<UP ? DPP_ROW_SHR(2) : DPP_ROW_SHL(2)>(b); break;
+        case 2: sa = dpp_d<UP ? DPP_ROW_SHR(4) : DPP_ROW_SHL(4)>(a); sb = dpp_d<UP ? DPP_ROW_SHR(4) : DPP_ROW_SHL(4)>(b); break;
+        default: sa = dpp_d<UP ? DPP_ROW_SHR(8) : DPP_ROW_SHL(8)>(a); sb = dpp_d<UP ? DPP_ROW_SHR(8) : DPP_ROW_SHL(8)>(b); break;
+        }
+        a = __builtin_fma(f, sa, a);
+        b = __builtin_fma(f, sb, b);
+    }
+    if (UP) {
+        const double f4 = m[64 * 4], f5 = m[64 * 5];
+        const double sa = dpp_rm<DPP_ROW_BCAST15, 0xa>(a), sb = dpp_rm<DPP_ROW_BCAST15, 0xa>(b);
+        a = __builtin_fma(f4, sa, a);
+        b = __builtin_fma(f4, sb, b);
+        const double ta = dpp_rm<DPP_ROW_BCAST31, 0xc>(a), tb = dpp_rm<DPP_ROW_BCAST31, 0xc>(b);
+        a = __builtin_fma(f5, ta, a);
+        b = __builtin_fma(f5, tb, b);
+    } else {
+        const double a1 = readlane_d(a, 16), a2 = readlane_d(a, 32), a3 = readlane_d(a, 48);
+        const double b1 = readlane_d(b, 16), b2 = readlane_d(b, 32), b3 = readlane_d(b, 48);
+        const double c1 = m[64 * 4], c2 = m[64 * 5], c3 = m[64 * 6];
+        a = __builtin_fma(c1, a1, a);
+        b = __builtin_fma(c1, b1, b);
+        a = __builtin_fma(c2, a2, a);
+        b = __builtin_fma(c2, b2, b);
+        a = __builtin_fma(c3, a3, a);
+        b = __builtin_fma(c3, b3, b);
+    }
+    double wa = UP ? dpp_d<DPP_WAVE_SHR1>(a) : dpp_d<DPP_WAVE_SHL1>(a);
+    double wb = UP ? dpp_d<DPP_WAVE_SHR1>(b) : dpp_d<DPP_WAVE_SHL1>(b);
+#pragma unroll
+    for (int k = 0; k < R; k++) {
+        const int i = UP ? k : R - 1 - k;
+        wa = __builtin_fma(-s[i], wa, x0[i]);
+        wb = __builtin_fma(-s[i], wb, x1[i]);
+        x0[i] = wa;
+        x1[i] = wb;
+    }
+    if (apply_scale) {
+        x0[0] *= row0_scale;
+        x1[0] *= row0_scale;
+    }
+}
+
+// one system's results through a staging of 32 R chunks to contiguous 16-byte stores of
+// the output keep-range; odd range ends by their owning lanes
+template <int R>
+__device__ __forceinline__ void store_system(double2* stg, int lane, const jw_pass64& g, int64_t sys,
+                                             const double (&x)[R])
+{
+    constexpr int H = R / 2;
+    compiler_fence();   // the staging's previous reads are issued (LDS keeps their order)
+#pragma unroll
+    for (int m = 0; m < H; m++) stg[swz<H>(lane * H + m)] = make_double2(x[2 * m], x[2 * m + 1]);
+    compiler_fence();
+    double2 v[H];
+#pragma unroll
+    for (int k = 0; k < H; k++) v[k] = stg[swz<H>(64 * k + lane)];
+#pragma unroll
+    for (int k = 0; k < H; k++) asm volatile("" : "+v"(v[k].x), "+v"(v[k].y));
+    double* dst = g.rhs + sys * g.stride + g.offSol;
+#pragma unroll
+    for (int k = 0; k < H; k++) {
+        const int c = 64 * k + lane;
+        if (c >= g.ocl && c < g.och) store_stream(dst + 2 * c, v[k]);
+    }
+    if (g.out_edge_lo && lane == g.out_lo / R) dst[g.out_lo] = pick_row<R>(x, g.out_lo % R);
+    if (g.out_edge_hi && lane == (g.out_hi - 1) / R) dst[g.out_hi - 1] = pick_row<R>(x, (g.out_hi - 1) % R);
+}
+
+__host__ __device__ constexpr int chain_max_waves(int R) { return R <= 8 ? 16 : 8; }
+
+// LDS: the first kl tables, then one system's staging per wavefront; the tables of
+// iterations kl .. K-1 (if any) are in global memory
+template <int R, bool UP>
+__global__ __launch_bounds__(64 * chain_max_waves(R)) void jw_chain64_kernel(jw_run_desc d, jw_chain_jobs jobs, int kl)
+{
+    constexpr int TE = chain_tab_elems(R);
+    extern __shared__ __align__(16) unsigned char smem[];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int nwaves = blockDim.x >> 6;
+    const int K = jobs.K;
+    const double* gtab = reinterpret_cast<const double*>(jobs.table);
+    double* ltab = reinterpret_cast<double*>(smem);
+    double2* stg = reinterpret_cast<double2*>(smem + (size_t)kl * TE * 8) + (size_t)wave * 32 * R;
+    const int64_t npass = (d.nsys + 1) >> 1, step = (int64_t)gridDim.x * nwaves;
+    int64_t q = (int64_t)blockIdx.x * nwaves + wave;
+    const jw_pass64 g = make_pass64(reinterpret_cast<double*>(d.rhs), d.nsys, d.stride, d.offSol, (int)d.in_lo,
+                                    (int)d.in_hi, (int)d.out_lo, (int)d.out_hi, 0, 0, false, false, false,
+                                    d.apply_scale, d.scale_hi, lane);
+    const bool solve = d.fwd || d.b1;
+    // the first pair's loads overlap the table build
+    double2 pf[2][R / 2];
+    if (q < npass) load_pair_direct<R>(pf, lane, g, 2 * q);
+    for (int k = 0; k < kl; k++)
+        chain_rows<R, UP>(jobs.src[k], reinterpret_cast<const double*>(jobs.matrices[k]), ltab + k * TE, threadIdx.x,
+                          blockDim.x);
+    __syncthreads();
+    if (solve)
+        for (int k = wave; k < kl; k += nwaves) chain_multipliers<R, UP>(ltab + k * TE, lane);
+    __syncthreads();
+    while (q < npass) {
+        double x0[R], x1[R];
+        unpack_pair<R>(pf, lane, g, 2 * q, x0, x1);
+        const int64_t qn = q + step;
+        if (qn < npass) load_pair_direct<R>(pf, lane, g, 2 * qn);
+        for (int k = 0; k < kl; k++)
+            chain_pair<R, UP>(ltab + k * TE, lane, d.band, solve, g.apply_scale, g.row0_scale, x0, x1);
+        for (int k = kl; k < K; k++)
+            chain_pair<R, UP>(gtab + (int64_t)k * TE, lane, d.band, solve, g.apply_scale, g.row0_scale, x0, x1);
+        store_system<R>(stg, lane, g, 2 * q, x0);
+        if (2 * q + 1 < d.nsys) store_system<R>(stg, lane, g, 2 * q + 1, x1);
+        q = qn;
+    }
+}
+
+// the tables of the iterations from kl on, one workgroup each
+template <int R, bool UP>
+__global__ __launch_bounds__(256) void jw_chain_tables_kernel(jw_chain_jobs jobs, int kl)
+{
+    const int k = kl + blockIdx.x;
+    double* tab = reinterpret_cast<double*>(jobs.table) + (int64_t)k * chain_tab_elems(R);
+    chain_rows<R, UP>(jobs.src[k], reinterpret_cast<const double*>(jobs.matrices[k]), tab, threadIdx.x, blockDim.x);
+    __syncthreads();   // the rows are visible to the workgroup
+    if (jobs.src[k].solve_kind != JW_SOLVE_NONE && threadIdx.x < 64) chain_multipliers<R, UP>(tab, threadIdx.x);
 }
 
 // Fused block operators (compute / store split kernel, IOMODE 1 and 2): the pair
@@ -2131,51 +2330,94 @@ int jwdev_main64(const jw_run_desc* r, int R, int waves, int grid, void* stream)
     return e == hipSuccess ? 0 : -3;
 }
 
-static const void* pick_chain(int R, bool all3)
+}  // extern "C"
+
+namespace {
+template <int R, bool UP>
+const void* chain_ptr(bool tables)
+{
+    return tables ? reinterpret_cast<const void*>(&jw_chain_tables_kernel<R, UP>)
+                  : reinterpret_cast<const void*>(&jw_chain64_kernel<R, UP>);
+}
+
+// the chain kernel, or the build of its global tables
+const void* pick_chain(int R, bool up, bool tables)
 {
     switch (R) {
-    case 2: return all3 ? reinterpret_cast<const void*>(&jw_chain64_kernel<2, true>)
-                        : reinterpret_cast<const void*>(&jw_chain64_kernel<2, false>);
-    case 4: return all3 ? reinterpret_cast<const void*>(&jw_chain64_kernel<4, true>)
-                        : reinterpret_cast<const void*>(&jw_chain64_kernel<4, false>);
-    case 8: return all3 ? reinterpret_cast<const void*>(&jw_chain64_kernel<8, true>)
-                        : reinterpret_cast<const void*>(&jw_chain64_kernel<8, false>);
-    case 16: return all3 ? reinterpret_cast<const void*>(&jw_chain64_kernel<16, true>)
-                         : reinterpret_cast<const void*>(&jw_chain64_kernel<16, false>);
+    case 2: return up ? chain_ptr<2, true>(tables) : chain_ptr<2, false>(tables);
+    case 4: return up ? chain_ptr<4, true>(tables) : chain_ptr<4, false>(tables);
+    case 8: return up ? chain_ptr<8, true>(tables) : chain_ptr<8, false>(tables);
+    case 16: return up ? chain_ptr<16, true>(tables) : chain_ptr<16, false>(tables);
     default: return nullptr;
     }
 }
 
-static int64_t chain_lds_bytes(int R) { return 2LL * 64 * R * 8 * 4; }   /* 4 wavefronts' stagings */
+int64_t chain_stage_bytes(int R) { return 64LL * R * 8; }   // one system per wavefront
 
-/* workgroups (of 4 wavefronts) per CU of the chained-step kernel */
-int jwdev_chain64_occupancy(int R)
+// Tables in LDS and wavefronts per workgroup: every table with at least 4 stagings after
+// them (one wavefront per SIMD), else as many tables as leave room for 8 stagings (6 at
+// R = 16): N = 1000, K = 8, 16384 systems: 161 us with 4 of the 8 tables in LDS, 195 us with none.
+void chain_split(int R, int K, int* kl, int* waves)
 {
+    const int64_t tab = (int64_t)chain_tab_elems(R) * 8;
+    int64_t w = (kLdsBytesMax - K * tab) / chain_stage_bytes(R);
+    *kl = K;
+    if (w < 4) {
+        w = R == 16 ? 6 : 8;
+        *kl = (int)((kLdsBytesMax - w * chain_stage_bytes(R)) / tab);
+    }
+    *waves = w > chain_max_waves(R) ? chain_max_waves(R) : (int)w;
+}
+
+size_t chain_lds(int R, int kl, int waves)
+{
+    return (size_t)(kl * (int64_t)chain_tab_elems(R) * 8 + waves * chain_stage_bytes(R));
+}
+}  // namespace
+
+extern "C" {
+
+/* wavefronts per workgroup, workgroups per CU of a chained step (0: not available) */
+int jwdev_chain64_shape(int R, int K, int* waves)
+{
+    if (!pick_chain(R, true, false) || K < 1) return 0;
+    int kl = 0;
+    chain_split(R, K, &kl, waves);
+    const int lds = (int)chain_lds(R, kl, *waves);
     int best = -1;
-    for (int v = 0; v < 2; v++) {
-        const void* f = pick_chain(R, v == 0);
-        if (!f) return 0;
-        const int lds = (int)chain_lds_bytes(R);
+    for (int up = 0; up < 2; up++) {
+        const void* f = pick_chain(R, up, false);
         if (hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess) return 0;
         int nb = 0;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, f, 256, lds) != hipSuccess) return 0;
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, f, 64 * *waves, lds) != hipSuccess) return 0;
         if (best < 0 || nb < best) best = nb;
     }
     return best;
 }
 
-int jwdev_chain64(const jw_run_desc* r, const void* tables, int64_t tab_elems, int K, int R, int grid, void* stream)
+int jwdev_chain64(const jw_run_desc* r, const jw_chain_jobs* jobs, int up, int grid, void* stream)
 {
-    if (!r->rhs || !tables) { snprintf(g_err64, sizeof(g_err64), "chain64: no rhs or tables"); return -1; }
-    const void* f = pick_chain(R, r->fwd && r->b1 && r->b2);
-    if (!f || K < 1) { snprintf(g_err64, sizeof(g_err64), "no chained-step kernel for R=%d", R); return -1; }
-    const size_t lds = (size_t)chain_lds_bytes(R);
+    if (!r->rhs || jobs->K < 1 || jobs->K > JW_CHAIN_MAX || grid < 1 || !pick_chain(jobs->R, up, false)) {
+        snprintf(g_err64, sizeof(g_err64), "chain64: no rhs, or a bad chain");
+        return -1;
+    }
+    int kl = 0, waves = 0;
+    chain_split(jobs->R, jobs->K, &kl, &waves);
+    if (kl < jobs->K && !jobs->table) { snprintf(g_err64, sizeof(g_err64), "chain64: no tables"); return -1; }
+    hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+    jw_run_desc rr = *r;
+    jw_chain_jobs jj = *jobs;
+    if (kl < jobs->K) {
+        void* args[] = {&jj, &kl};
+        if (hipLaunchKernel(pick_chain(jobs->R, up, true), dim3(jobs->K - kl), dim3(256), args, 0, s) != hipSuccess)
+            return -3;
+    }
+    const void* f = pick_chain(jobs->R, up, false);
+    const size_t lds = chain_lds(jobs->R, kl, waves);
     hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) return -2;
-    jw_run_desc rr = *r;
-    const double* t = static_cast<const double*>(tables);
-    void* args[] = {&rr, &t, &tab_elems, &K};
-    e = hipLaunchKernel(f, dim3(grid), dim3(256), args, lds, reinterpret_cast<hipStream_t>(stream));
+    void* args[] = {&rr, &jj, &kl};
+    e = hipLaunchKernel(f, dim3(grid), dim3(64 * waves), args, lds, s);
     return e == hipSuccess ? 0 : -3;
 }
 

@@ -36,8 +36,9 @@ struct pfsolve_plan {
      * lane (0 = not used), waves per workgroup, workgroups per CU */
     int dd64_R, dd64_waves, dd64_occ;
     /* chained steps: iterations (1 = none), rows per lane of the chained kernel, its
-     * workgroups per CU; a slot's table area holds K format-2 tables of chain_tab bytes */
-    int chain_K, chain_R, chain_occ;
+     * workgroups per CU and wavefronts per workgroup; a slot's area has chain_tab bytes per
+     * iteration for the tables of a chain too long for LDS */
+    int chain_K, chain_R, chain_occ, chain_waves;
     size_t chain_tab;
     /* ALT variant: two parity subsystems, one format-1 table of alt_tab bytes each */
     int alt;

@@ -180,15 +180,16 @@ static PfSolveResult plan_setup(PfSolveApplication* app, struct pfsolve_plan* p)
                  cfg->jw_type, (long long)cfg->jw_control_bitmask, (unsigned long long)cfg->Msplit[0],
                  cfg->numConsecutiveJWIterations, cfg->useMultipleInputBuffers);
         if (cfg->numConsecutiveJWIterations > 1) {
-            /* chained steps: K format-2 tables (one per iteration) per stream slot and the
-             * chained kernel, R rows per lane for the largest iteration */
+            /* chained steps: the chained kernel, R rows per lane for the largest iteration; the
+             * slot's area holds the K tables of a chain too long for LDS (sized as K format-2
+             * tables, which hold them) */
             const int K = cfg->numConsecutiveJWIterations;
             const int64_t nmax = cfg->upperBanded ? p->N : p->N + K - 1;
             int r64 = 2;
             while (r64 * 64 < nmax) r64 *= 2;
             p->chain_K = K;
             p->chain_R = r64;
-            p->chain_occ = jwdev_chain64_occupancy(r64);
+            p->chain_occ = jwdev_chain64_shape(r64, K, &p->chain_waves);
             if (p->chain_occ < 1) return PFSOLVE_ERROR_FAILED_TO_SET_DYNAMIC_SHARED_MEMORY;
             p->chain_tab = (size_t)jwdev_table64_elems(r64) * 8;
             p->L = 64;
@@ -405,10 +406,11 @@ static PfSolveResult append_fused_blocks(PfSolveApplication* app, const PfSolveL
     return PFSOLVE_SUCCESS;
 }
 
-/* Chained steps (numConsecutiveJWIterations = K > 1): the K iterations' tables in one
- * launch, then one launch of the chained kernel that keeps each pair of systems in
- * registers through the K iterations (pfSolve_JonesWorland.h:95-374).  Iteration i reads its
- * matrices from buffer[i] with useMultipleInputBuffers, from buffer[0] otherwise
+/* Chained steps (numConsecutiveJWIterations = K > 1): one launch of the chained kernel,
+ * which builds the K iterations' tables and keeps each pair of systems in registers through
+ * the K iterations (pfSolve_JonesWorland.h:95-374); the tables a long chain has no LDS for
+ * are built by a launch before it.  Iteration i reads its matrices from buffer[i] with
+ * useMultipleInputBuffers, from buffer[0] otherwise
  * (pfSolve_DispatchPlan.h:231-235); with useMultipleInputBuffers a declared bufferSize holds
  * one size per buffer. */
 static PfSolveResult append_chain(PfSolveApplication* app, const PfSolveLaunchParams* lp, jw_run_desc* run,
@@ -450,17 +452,15 @@ static PfSolveResult append_chain(PfSolveApplication* app, const PfSolveLaunchPa
     const int64_t nsys = run->nsys;
     if (nsys <= 0) return PFSOLVE_SUCCESS;
     jobs.table = table;
-    jobs.tab_stride = (int64_t)p->chain_tab;
     jobs.K = K;
     jobs.R = p->chain_R;
-    if (jwdev_prologue_chain(&jobs, s) != 0) return PFSOLVE_ERROR_FAILED_TO_LAUNCH_KERNEL;
     const int64_t npass = (nsys + 1) / 2;
-    int64_t need = (npass + 3) / 4;
+    int64_t need = (npass + p->chain_waves - 1) / p->chain_waves;
     int64_t grid = (int64_t)p->cu_count * p->chain_occ;
     if (grid > need) grid = need;
     if (grid < 1) grid = 1;
     if (p->ev_start && hipEventRecord(p->ev_start, s) != hipSuccess) return PFSOLVE_ERROR_FAILED_TO_EVENT_RECORD;
-    if (jwdev_chain64(run, table, (int64_t)(p->chain_tab / 8), K, p->chain_R, (int)grid, s) != 0)
+    if (jwdev_chain64(run, &jobs, cfg->upperBanded != 0, (int)grid, s) != 0)
         return PFSOLVE_ERROR_FAILED_TO_LAUNCH_KERNEL;
     if (p->ev_stop && hipEventRecord(p->ev_stop, s) != hipSuccess) return PFSOLVE_ERROR_FAILED_TO_EVENT_RECORD;
     return PFSOLVE_SUCCESS;
