@@ -628,7 +628,7 @@ PfSolveResult pfsolve_batch_run_plain(pfsolve_batch* b, hipStream_t stream)
         const int64_t npass = R == 32 ? st->nsys : (st->nsys + 1) / 2;
         int64_t grid = (npass + waves - 1) / waves;
         if (grid > (int64_t)b->cu_count * occ) grid = (int64_t)b->cu_count * occ;
-        if (jwdev_main64(&run, R, waves, (int)grid, stream) != 0) return PFSOLVE_ERROR_FAILED_TO_LAUNCH_KERNEL;
+        if (jwdev_main64(&run, NULL, NULL, R, waves, (int)grid, stream) != 0) return PFSOLVE_ERROR_FAILED_TO_LAUNCH_KERNEL;
     }
     return PFSOLVE_SUCCESS;
 }

@@ -190,7 +190,10 @@ int64_t jwdev_table64_elems(int R);
 int jwdev_main64_waves(int R);
 int64_t jwdev_main64_lds_bytes(int R, int waves);
 int jwdev_main64_occupancy(int R, int waves);
-int jwdev_main64(const jw_run_desc* r, int R, int waves, int grid, void* stream);
+/* with a source the kernel builds its table in LDS (jwdev_main64_builds), else it reads r->table */
+int jwdev_main64_builds(int R);
+int jwdev_main64(const jw_run_desc* r, const jw_source_desc* src, const void* matrices, int R, int waves, int grid,
+                 void* stream);
 /* the same with compute / store split (R <= 8): compute wavefronts never store,
  * storer wavefronts write their results; *d_err is raised if a bounded wait ran out */
 int jwdev_main64s_shape(int R, int* ncomp, int* nstore);

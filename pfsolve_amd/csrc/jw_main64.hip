@@ -25,6 +25,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 #include <stdio.h>
+#include <string.h>
 
 #include "jw_common.h"
 #include "jw_prologue.h"
@@ -90,8 +91,18 @@ constexpr int waves_per_eu()
 template <int R>
 constexpr int max_threads()
 {
-    return R <= 4 ? 1024 : (R == 8 ? 768 : 320);
+    return R <= 4 ? 1024 : (R == 8 ? 768 : 512);
 }
+
+// How the pair kernels (plain, batch queue kernels 1 and 4) move right-hand sides.  R = 16:
+// contiguous loads into registers one pass ahead and a staging of one system (8 KiB), so
+// that 8 wavefronts fit beside the 76 KiB table and no wavefront waits for its own loads;
+// 16384 systems of 1000 rows: 64 us per step, 74.5 us when R = 16 staged pairs by LDS DMA
+// (16 KiB each: 5 wavefronts, which waited for their loads) behind a table build launch.
+// Smaller R: LDS DMA into a staging of two systems at the pass's start, where 12 and more
+// wavefronts hide it (512 sets of 512 to 257 rows, solve: 51.5 us, 54.3 us one pass ahead).
+__host__ __device__ constexpr bool pair_ahead(int R) { return R == 16; }
+__host__ __device__ constexpr int64_t pair_stage_bytes(int R) { return (pair_ahead(R) ? 1LL : 2LL) * 64 * R * 8; }
 
 // value of row r (which lane `lane` owns when r / R == lane) from the lane's registers
 template <int R>
@@ -564,7 +575,6 @@ __device__ __forceinline__ void jw_pair64(const double* tab, double2* stg, int l
     compiler_fence();
 }
 
-// A set's table (NTAB doubles, whole 1 KiB blocks) from global memory into LDS at `smem`
 // One pass of sub-wavefront groups (R = 2): the 2G consecutive systems sys0 .. sys0+2G-1
 // (those below sys_end) in one wavefront, group gi solving systems sys0 + 2 gi and
 // sys0 + 2 gi + 1.  Staging: system slot k (system sys0 + k) is chunks [k LG, (k+1) LG)
@@ -637,6 +647,142 @@ __device__ __forceinline__ void jw_groups64(const double* tab, double2* stg, int
     compiler_fence();
 }
 
+// Direct blocked loads (kernels that load one pass ahead): lane t fetches its own R
+// rows, 16-byte chunks t H .. t H + H-1, of both systems, straight into the
+// registers the recurrences use.  One instruction's 64 accesses are spread over
+// a 64 x 16H-byte span that its H sibling instructions complete, so every line
+// is fetched from memory once and the other accesses hit the cache; no LDS
+// transposition is needed.
+template <int R>
+__device__ __forceinline__ void load_pair_direct(double2 (&pf)[2][R / 2], int lane, const jw_pass64& g, int64_t sys0)
+{
+    constexpr int H = R / 2;
+    const bool ok1 = sys0 + 1 < g.nsys;
+    const double* src0 = g.rhs + sys0 * g.stride + g.offSol;
+#pragma unroll
+    for (int s = 0; s < 2; s++) {
+        const double* src = src0 + s * g.stride;
+#pragma unroll
+        for (int m = 0; m < H; m++) {
+            const int c = lane * H + m;
+            double2 v = make_double2(0.0, 0.0);
+            if (c >= g.icl && c < g.ich && (s == 0 || ok1)) v = load_chunk(src + 2 * c);
+            pf[s][m] = v;
+        }
+    }
+}
+
+// the directly loaded chunks as rows, the odd keep-range ends from global memory
+template <int R>
+__device__ __forceinline__ void unpack_pair(const double2 (&pf)[2][R / 2], int lane, const jw_pass64& g, int64_t sys0,
+                                            double (&x0)[R], double (&x1)[R])
+{
+#pragma unroll
+    for (int m = 0; m < R / 2; m++) {
+        x0[2 * m] = pf[0][m].x;
+        x0[2 * m + 1] = pf[0][m].y;
+        x1[2 * m] = pf[1][m].x;
+        x1[2 * m + 1] = pf[1][m].y;
+    }
+    read_edges<R>(lane, g, sys0, x0, x1);
+}
+
+// Contiguous loads one pass ahead: lane l takes chunk 64 k + l of instruction k (one KiB per
+// instruction); unpack_ahead turns them into a lane's own rows through the staging of one
+// system.  For R = 16, where load_pair_direct's lanes stand 128 bytes apart: each of a
+// line's 8 sibling loads misses the L1 once the wavefronts' rows exceed it, and the line
+// comes from the L2 8 times (1024 sets of 1024 to 513 rows, solve: 251 us direct, 187 us
+// contiguous; chained steps of 1000 rows, K = 4: 76 and 67 us).  At R <= 8 the chained steps
+// measured the same or up to 4 % faster direct.
+template <int R>
+__device__ __forceinline__ void load_pair_ahead(double2 (&pf)[2][R / 2], int lane, const jw_pass64& g, int64_t sys0)
+{
+    constexpr int H = R / 2;
+    const bool ok1 = sys0 + 1 < g.nsys;
+    const double* src0 = g.rhs + sys0 * g.stride + g.offSol;
+#pragma unroll
+    for (int s = 0; s < 2; s++) {
+        const double* src = src0 + s * g.stride;
+#pragma unroll
+        for (int k = 0; k < H; k++) {
+            const int c = 64 * k + lane;
+            double2 v = make_double2(0.0, 0.0);
+            if (c >= g.icl && c < g.ich && (s == 0 || ok1)) v = load_chunk(src + 2 * c);
+            pf[s][k] = v;
+        }
+    }
+}
+
+template <int R>
+__device__ __forceinline__ void unpack_ahead(const double2 (&pf)[2][R / 2], double2* stg, int lane, const jw_pass64& g,
+                                             int64_t sys0, double (&x0)[R], double (&x1)[R])
+{
+    constexpr int H = R / 2;
+#pragma unroll
+    for (int s = 0; s < 2; s++) {
+        double(&x)[R] = s == 0 ? x0 : x1;
+        compiler_fence();   // LDS keeps a wavefront's order: the previous reads come first
+#pragma unroll
+        for (int k = 0; k < H; k++) stg[swz<H>(64 * k + lane)] = pf[s][k];
+        compiler_fence();
+#pragma unroll
+        for (int m = 0; m < H; m++) {
+            const double2 v = stg[swz<H>(lane * H + m)];
+            x[2 * m] = v.x;
+            x[2 * m + 1] = v.y;
+        }
+    }
+    read_edges<R>(lane, g, sys0, x0, x1);
+}
+
+// one system's results through a staging of 32 R chunks to contiguous 16-byte stores of
+// the output keep-range; odd range ends by their owning lanes
+template <int R>
+__device__ __forceinline__ void store_system(double2* stg, int lane, const jw_pass64& g, int64_t sys,
+                                             const double (&x)[R])
+{
+    constexpr int H = R / 2;
+    compiler_fence();   // the staging's previous reads are issued (LDS keeps their order)
+#pragma unroll
+    for (int m = 0; m < H; m++) stg[swz<H>(lane * H + m)] = make_double2(x[2 * m], x[2 * m + 1]);
+    compiler_fence();
+    double2 v[H];
+#pragma unroll
+    for (int k = 0; k < H; k++) v[k] = stg[swz<H>(64 * k + lane)];
+#pragma unroll
+    for (int k = 0; k < H; k++) asm volatile("" : "+v"(v[k].x), "+v"(v[k].y));
+    double* dst = g.rhs + sys * g.stride + g.offSol;
+#pragma unroll
+    for (int k = 0; k < H; k++) {
+        const int c = 64 * k + lane;
+        if (c >= g.ocl && c < g.och) store_stream(dst + 2 * c, v[k]);
+    }
+    if (g.out_edge_lo && lane == g.out_lo / R) dst[g.out_lo] = pick_row<R>(x, g.out_lo % R);
+    if (g.out_edge_hi && lane == (g.out_hi - 1) / R) dst[g.out_hi - 1] = pick_row<R>(x, (g.out_hi - 1) % R);
+}
+
+// Pairs q, q + step, ... below q1 through one wavefront: each pair's rows were loaded into
+// registers a pass ahead (pf holds the first pair's on entry), results leave through a
+// staging of one system.  geo() gives the pass geometry, rebuilt every pass from the kernel
+// arguments, so that nothing derived from them stays live in registers across the loop.
+template <int R, bool ALL3, class Geo>
+__device__ __forceinline__ void stream_pairs(const double* tab, double2* stg, int lane, const Geo& geo, int64_t q,
+                                             int64_t q1, int64_t step, double2 (&pf)[2][R / 2])
+{
+    while (q < q1) {
+        const jw_pass64 g = geo();
+        double x0[R], x1[R];
+        unpack_ahead<R>(pf, stg, lane, g, 2 * q, x0, x1);
+        const int64_t qn = q + step;
+        if (qn < q1) load_pair_ahead<R>(pf, lane, g, 2 * qn);
+        compute_pair<R, ALL3>(tab, lane, g, x0, x1);
+        store_system<R>(stg, lane, g, 2 * q, x0);
+        if (2 * q + 1 < g.nsys) store_system<R>(stg, lane, g, 2 * q + 1, x1);
+        q = qn;
+    }
+}
+
+// A set's table (NTAB doubles, whole 1 KiB blocks) from global memory into LDS at `smem`
 template <int NTAB>
 __device__ __forceinline__ void copy_table_lds(unsigned char* smem, const void* table, int wave, int nwaves, int lane)
 {
@@ -644,8 +790,10 @@ __device__ __forceinline__ void copy_table_lds(unsigned char* smem, const void* 
     copy_to_lds(smem, table, NTAB * 8, wave, nwaves, lane);
 }
 
-template <int R, bool ALL3>
-__global__ __launch_bounds__(max_threads<R>()) void jw_main64_kernel(jw_run_desc d)
+// BUILD: the table is built in LDS from the caller's matrices (the stagings as scratch);
+// otherwise it is copied from global memory.
+template <int R, bool ALL3, bool BUILD>
+__global__ __launch_bounds__(max_threads<R>()) void jw_main64_kernel(jw_run_desc d, jw_source_desc src, const void* mat)
 {
     constexpr int NTAB = JW_TAB64_ELEMS(R);
     extern __shared__ __align__(16) unsigned char smem[];
@@ -653,18 +801,33 @@ __global__ __launch_bounds__(max_threads<R>()) void jw_main64_kernel(jw_run_desc
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int nwaves = blockDim.x >> 6;
-    copy_table_lds<NTAB>(smem, d.table, wave, nwaves, lane);
-    double2* stg = reinterpret_cast<double2*>(smem + NTAB * 8) + (size_t)wave * 64 * R;
-    zero_staging<R>(stg, lane);
-    __syncthreads();
-    const int64_t npass = (d.nsys + 1) >> 1;
-    for (int64_t q = (int64_t)blockIdx.x * nwaves + wave; q < npass; q += (int64_t)gridDim.x * nwaves) {
-        // rebuilt every pass from the kernel arguments, so that nothing derived from
-        // them stays live in registers across the loop
-        const jw_pass64 g = make_pass64(reinterpret_cast<double*>(d.rhs), d.nsys, d.stride, d.offSol,
-                                        (int)d.in_lo, (int)d.in_hi, (int)d.out_lo, (int)d.out_hi, d.kl, d.ku,
-                                        d.fwd, d.b1, d.b2, d.apply_scale, d.scale_hi, lane);
-        jw_pair64<R, ALL3>(tab, stg, lane, g, 2 * q);
+    double2* stg = reinterpret_cast<double2*>(smem + NTAB * 8 + wave * pair_stage_bytes(R));
+    const int64_t npass = (d.nsys + 1) >> 1, step = (int64_t)gridDim.x * nwaves;
+    int64_t q = (int64_t)blockIdx.x * nwaves + wave;
+    // rebuilt every pass from the kernel arguments, so that nothing derived from
+    // them stays live in registers across the loop
+    auto geo = [&] {
+        return make_pass64(reinterpret_cast<double*>(d.rhs), d.nsys, d.stride, d.offSol, (int)d.in_lo, (int)d.in_hi,
+                           (int)d.out_lo, (int)d.out_hi, d.kl, d.ku, d.fwd, d.b1, d.b2, d.apply_scale, d.scale_hi,
+                           lane);
+    };
+    if constexpr (pair_ahead(R)) {
+        // the first pair's loads overlap the table build
+        double2 pf[2][R / 2];
+        if (q < npass) load_pair_ahead<R>(pf, lane, geo(), 2 * q);
+        if constexpr (BUILD)
+            prologue_body<double, NoPivotHooks, true, 64 * R / max_threads<R>(), pro_rows(64 * R)>(
+                src, mat, reinterpret_cast<double*>(smem), 64, R, 2, smem + NTAB * 8);
+        else
+            copy_table_lds<NTAB>(smem, d.table, wave, nwaves, lane);
+        __syncthreads();
+        stream_pairs<R, ALL3>(tab, stg, lane, geo, q, npass, step, pf);
+    } else {
+        static_assert(!BUILD, "the build in the kernel: pair_ahead only");
+        copy_table_lds<NTAB>(smem, d.table, wave, nwaves, lane);
+        zero_staging<R>(stg, lane);
+        __syncthreads();
+        for (; q < npass; q += step) jw_pair64<R, ALL3>(tab, stg, lane, geo(), 2 * q);
     }
 }
 
@@ -1199,46 +1362,6 @@ __global__ __launch_bounds__(256) void jw_main64g_kernel(jw_run_desc d)
     }
 }
 
-// Direct blocked loads (compute / store split kernel): lane t fetches its own R
-// rows, 16-byte chunks t H .. t H + H-1, of both systems, straight into the
-// registers the recurrences use.  One instruction's 64 accesses are spread over
-// a 64 x 16H-byte span that its H sibling instructions complete, so every line
-// is fetched from memory once and the other accesses hit the cache; no LDS
-// transposition is needed.
-template <int R>
-__device__ __forceinline__ void load_pair_direct(double2 (&pf)[2][R / 2], int lane, const jw_pass64& g, int64_t sys0)
-{
-    constexpr int H = R / 2;
-    const bool ok1 = sys0 + 1 < g.nsys;
-    const double* src0 = g.rhs + sys0 * g.stride + g.offSol;
-#pragma unroll
-    for (int s = 0; s < 2; s++) {
-        const double* src = src0 + s * g.stride;
-#pragma unroll
-        for (int m = 0; m < H; m++) {
-            const int c = lane * H + m;
-            double2 v = make_double2(0.0, 0.0);
-            if (c >= g.icl && c < g.ich && (s == 0 || ok1)) v = load_chunk(src + 2 * c);
-            pf[s][m] = v;
-        }
-    }
-}
-
-// the directly loaded chunks as rows, the odd keep-range ends from global memory
-template <int R>
-__device__ __forceinline__ void unpack_pair(const double2 (&pf)[2][R / 2], int lane, const jw_pass64& g, int64_t sys0,
-                                            double (&x0)[R], double (&x1)[R])
-{
-#pragma unroll
-    for (int m = 0; m < R / 2; m++) {
-        x0[2 * m] = pf[0][m].x;
-        x0[2 * m + 1] = pf[0][m].y;
-        x1[2 * m] = pf[1][m].x;
-        x1[2 * m + 1] = pf[1][m].y;
-    }
-    read_edges<R>(lane, g, sys0, x0, x1);
-}
-
 // ---------------------------------------------------------------------------
 // Chained steps (numConsecutiveJWIterations = K): a wavefront owns a pair of systems
 // through all K iterations, whose right-hand sides stay in its registers in between (one
@@ -1396,32 +1519,6 @@ __device__ __forceinline__ void chain_pair(const double* tab, int lane, bool ban
     }
 }
 
-// one system's results through a staging of 32 R chunks to contiguous 16-byte stores of
-// the output keep-range; odd range ends by their owning lanes
-template <int R>
-__device__ __forceinline__ void store_system(double2* stg, int lane, const jw_pass64& g, int64_t sys,
-                                             const double (&x)[R])
-{
-    constexpr int H = R / 2;
-    compiler_fence();   // the staging's previous reads are issued (LDS keeps their order)
-#pragma unroll
-    for (int m = 0; m < H; m++) stg[swz<H>(lane * H + m)] = make_double2(x[2 * m], x[2 * m + 1]);
-    compiler_fence();
-    double2 v[H];
-#pragma unroll
-    for (int k = 0; k < H; k++) v[k] = stg[swz<H>(64 * k + lane)];
-#pragma unroll
-    for (int k = 0; k < H; k++) asm volatile("" : "+v"(v[k].x), "+v"(v[k].y));
-    double* dst = g.rhs + sys * g.stride + g.offSol;
-#pragma unroll
-    for (int k = 0; k < H; k++) {
-        const int c = 64 * k + lane;
-        if (c >= g.ocl && c < g.och) store_stream(dst + 2 * c, v[k]);
-    }
-    if (g.out_edge_lo && lane == g.out_lo / R) dst[g.out_lo] = pick_row<R>(x, g.out_lo % R);
-    if (g.out_edge_hi && lane == (g.out_hi - 1) / R) dst[g.out_hi - 1] = pick_row<R>(x, (g.out_hi - 1) % R);
-}
-
 __host__ __device__ constexpr int chain_max_waves(int R) { return R <= 8 ? 16 : 8; }
 
 // LDS: the first kl tables, then one system's staging per wavefront; the tables of
@@ -1446,7 +1543,12 @@ __global__ __launch_bounds__(64 * chain_max_waves(R)) void jw_chain64_kernel(jw_
     const bool solve = d.fwd || d.b1;
     // the first pair's loads overlap the table build
     double2 pf[2][R / 2];
-    if (q < npass) load_pair_direct<R>(pf, lane, g, 2 * q);
+    // (a lane's own rows, but contiguous chunks at R = 16: load_pair_ahead)
+    auto load = [&](int64_t p) {
+        if constexpr (pair_ahead(R)) load_pair_ahead<R>(pf, lane, g, 2 * p);
+        else load_pair_direct<R>(pf, lane, g, 2 * p);
+    };
+    if (q < npass) load(q);
     for (int k = 0; k < kl; k++)
         chain_rows<R, UP>(jobs.src[k], reinterpret_cast<const double*>(jobs.matrices[k]), ltab + k * TE, threadIdx.x,
                           blockDim.x);
@@ -1456,9 +1558,10 @@ __global__ __launch_bounds__(64 * chain_max_waves(R)) void jw_chain64_kernel(jw_
     __syncthreads();
     while (q < npass) {
         double x0[R], x1[R];
-        unpack_pair<R>(pf, lane, g, 2 * q, x0, x1);
+        if constexpr (pair_ahead(R)) unpack_ahead<R>(pf, stg, lane, g, 2 * q, x0, x1);
+        else unpack_pair<R>(pf, lane, g, 2 * q, x0, x1);
         const int64_t qn = q + step;
-        if (qn < npass) load_pair_direct<R>(pf, lane, g, 2 * qn);
+        if (qn < npass) load(qn);
         for (int k = 0; k < kl; k++)
             chain_pair<R, UP>(ltab + k * TE, lane, d.band, solve, g.apply_scale, g.row0_scale, x0, x1);
         for (int k = kl; k < K; k++)
@@ -1770,7 +1873,7 @@ __global__ __launch_bounds__(max_threads<R>()) void jw_batch64_kernel(const jw_b
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int nwaves = blockDim.x >> 6;
-    double2* stg = reinterpret_cast<double2*>(smem + NTAB * 8) + (size_t)wave * 64 * R;
+    double2* stg = reinterpret_cast<double2*>(smem + NTAB * 8 + wave * pair_stage_bytes(R));
     int cur = -1;
     for (;;) {
         __syncthreads();   // the previous unit is finished: s_unit and the table may change
@@ -1780,6 +1883,23 @@ __global__ __launch_bounds__(max_threads<R>()) void jw_batch64_kernel(const jw_b
         if (u >= nunits) break;
         const jw_batch_unit un = units[u];
         const jw_batch_item& it = items[un.item];
+        if constexpr (pair_ahead(R)) {
+            auto geo = [&] {
+                return make_pass64(reinterpret_cast<double*>(it.rhs), it.nsys, it.stride, it.offSol, 0, it.N, 0, it.N,
+                                   it.kl, it.ku, true, true, true, it.apply_scale != 0, it.scale, lane);
+            };
+            // the unit's first pairs are loaded before the table copy
+            double2 pf[2][R / 2];
+            const int64_t q = un.pair0 + wave;
+            if (q < un.pair1) load_pair_ahead<R>(pf, lane, geo(), 2 * q);
+            if (un.item != cur) {
+                copy_table_lds<NTAB>(smem, it.table, wave, nwaves, lane);
+                __syncthreads();
+                cur = un.item;
+            }
+            stream_pairs<R, true>(tab, stg, lane, geo, q, un.pair1, nwaves, pf);
+            continue;
+        }
         if (un.item != cur) {
             copy_table_lds<NTAB>(smem, it.table, wave, nwaves, lane);
             zero_staging<R>(stg, lane);   // the new set's keep-range may be narrower
@@ -1816,9 +1936,8 @@ __global__ __launch_bounds__(max_threads<R>()) void jw_batch64_kernel(const jw_b
 // also hold the table build's scratch while a set's table is built
 __host__ __device__ constexpr int64_t batch64b_lds_bytes(int R, int waves)
 {
-    return (int64_t)JW_TAB64_ELEMS(R) * 8 +
-           ((int64_t)2 * 64 * R * 8 * waves > (int64_t)(5 * 64 * R) * 8 ? (int64_t)2 * 64 * R * 8 * waves
-                                                                         : (int64_t)(5 * 64 * R) * 8);
+    const int64_t stagings = pair_stage_bytes(R) * waves, scratch = (int64_t)(5 * 64 * R) * 8;
+    return (int64_t)JW_TAB64_ELEMS(R) * 8 + (stagings > scratch ? stagings : scratch);
 }
 
 // one set's format-2 table built into LDS (the stagings after it as scratch); kept out of
@@ -1851,7 +1970,7 @@ __global__ __launch_bounds__(max_threads<R>()) void jw_batch64b_kernel(const jw_
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int nwaves = blockDim.x >> 6;
-    double2* stg = reinterpret_cast<double2*>(smem + NTAB * 8) + (size_t)wave * 64 * R;
+    double2* stg = reinterpret_cast<double2*>(smem + NTAB * 8 + wave * pair_stage_bytes(R));
     int cur = -1;
     for (;;) {
         __syncthreads();   // the previous unit is finished: s_unit, the table and the staging may change
@@ -1861,6 +1980,22 @@ __global__ __launch_bounds__(max_threads<R>()) void jw_batch64b_kernel(const jw_
         if (u >= nunits) break;
         const jw_batch_unit un = units[u];
         const jw_batch_item& it = items[un.item];
+        if constexpr (pair_ahead(R)) {
+            if (un.item != cur) {
+                build_table_lds<R>(jobs + un.item);
+                __syncthreads();   // the build's scratch (the stagings) is free again
+                cur = un.item;
+            }
+            auto geo = [&] {
+                return make_pass64(reinterpret_cast<double*>(it.rhs), it.nsys, it.stride, it.offSol, 0, it.N, 0, it.N,
+                                   it.kl, it.ku, true, true, true, it.apply_scale != 0, it.scale, lane);
+            };
+            double2 pf[2][R / 2];
+            const int64_t q = un.pair0 + wave;
+            if (q < un.pair1) load_pair_ahead<R>(pf, lane, geo(), 2 * q);
+            stream_pairs<R, true>(tab, stg, lane, geo, q, un.pair1, nwaves, pf);
+            continue;
+        }
         if (un.item != cur) {
             build_table_lds<R>(jobs + un.item);
             __syncthreads();   // the build's scratch (the stagings) is free again
@@ -2135,15 +2270,16 @@ __global__ __launch_bounds__(bsplit_threads<R>()) void jw_batch64s_kernel(const 
     queue_leave(counter);
 }
 
-template <int R>
+template <int R, bool BUILD = false>
 const void* kernel_ptr(bool all3)
 {
-    return all3 ? reinterpret_cast<const void*>(&jw_main64_kernel<R, true>)
-                : reinterpret_cast<const void*>(&jw_main64_kernel<R, false>);
+    return all3 ? reinterpret_cast<const void*>(&jw_main64_kernel<R, true, BUILD>)
+                : reinterpret_cast<const void*>(&jw_main64_kernel<R, false, BUILD>);
 }
 
-const void* pick64(int R, bool all3 = true)
+const void* pick64(int R, bool all3 = true, bool build = false)
 {
+    if (build) return R == 16 ? kernel_ptr<16, true>(all3) : nullptr;
     switch (R) {
     case 32: return all3 ? reinterpret_cast<const void*>(&jw_main64g_kernel<32, true>)
                          : reinterpret_cast<const void*>(&jw_main64g_kernel<32, false>);
@@ -2269,7 +2405,7 @@ bool split_shape(int R, int* ncomp, int* nstore)
     return true;
 }
 
-int max_waves64(int R) { return R <= 4 ? 16 : (R == 8 ? 12 : (R == 16 ? 5 : 4)); }
+int max_waves64(int R) { return R <= 4 ? 16 : R == 8 ? 12 : (R == 16 ? 8 : 4); }
 
 thread_local char g_err64[256];
 
@@ -2289,8 +2425,7 @@ int jwdev_main64_waves(int R)
     if (!pick64(R)) return 0;
     if (R == 32) return 4;
     const int64_t table = table_lds_bytes(R);
-    const int64_t per_wave = 2LL * 64 * R * 8;
-    int w = (int)((kLdsBytesMax - table) / per_wave);
+    int w = (int)((kLdsBytesMax - table) / pair_stage_bytes(R));
     if (w > max_waves64(R)) w = max_waves64(R);
     return w < 1 ? 0 : w;
 }
@@ -2298,15 +2433,18 @@ int jwdev_main64_waves(int R)
 int64_t jwdev_main64_lds_bytes(int R, int waves)
 {
     if (R == 32) return 64LL * R * 8 * waves;   /* one system per wavefront */
-    return table_lds_bytes(R) + 2LL * 64 * R * 8 * waves;
+    return table_lds_bytes(R) + pair_stage_bytes(R) * waves;
 }
 
-/* workgroups per CU, the smaller of the two variants (all recurrences / some) */
+/* 1 when the kernel of R rows per lane can build its table in LDS (jwdev_main64 with a source) */
+int jwdev_main64_builds(int R) { return pick64(R, true, true) != NULL; }
+
+/* workgroups per CU, the smallest of the variants (all recurrences or some, table built or copied) */
 int jwdev_main64_occupancy(int R, int waves)
 {
     int best = -1;
-    for (int v = 0; v < 2; v++) {
-        const void* f = pick64(R, v == 0);
+    for (int v = 0; v < (jwdev_main64_builds(R) ? 4 : 2); v++) {
+        const void* f = pick64(R, v % 2 == 0, v >= 2);
         if (!f) return 0;
         const int lds = (int)jwdev_main64_lds_bytes(R, waves);
         if (hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess) return 0;
@@ -2317,15 +2455,21 @@ int jwdev_main64_occupancy(int R, int waves)
     return best;
 }
 
-int jwdev_main64(const jw_run_desc* r, int R, int waves, int grid, void* stream)
+int jwdev_main64(const jw_run_desc* r, const jw_source_desc* src, const void* matrices, int R, int waves, int grid,
+                 void* stream)
 {
-    if (!r->rhs || !r->table) { snprintf(g_err64, sizeof(g_err64), "main64: no rhs or table"); return -1; }
-    const void* f = pick64(R, r->fwd && r->b1 && r->b2);
+    if (!r->rhs || (src ? !matrices : !r->table)) { snprintf(g_err64, sizeof(g_err64), "main64: no rhs or table"); return -1; }
+    /* the build's partition: 2 rows per thread of a full workgroup, its scratch in the stagings */
+    if (src && waves != jwdev_main64_waves(R)) { snprintf(g_err64, sizeof(g_err64), "main64: bad build shape"); return -1; }
+    const void* f = pick64(R, r->fwd && r->b1 && r->b2, src != NULL);
     if (!f) { snprintf(g_err64, sizeof(g_err64), "no 64-lane kernel for R=%d", R); return -1; }
     const size_t lds = (size_t)jwdev_main64_lds_bytes(R, waves);
     hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) return -2;
-    void* args[] = {const_cast<jw_run_desc*>(r)};
+    /* R = 32 takes the descriptor alone (a launch reads the arguments its kernel has) */
+    jw_source_desc none;
+    if (!src) memset(&none, 0, sizeof(none));
+    void* args[] = {const_cast<jw_run_desc*>(r), src ? const_cast<jw_source_desc*>(src) : &none, &matrices};
     e = hipLaunchKernel(f, dim3(grid), dim3(64 * waves), args, lds, reinterpret_cast<hipStream_t>(stream));
     return e == hipSuccess ? 0 : -3;
 }

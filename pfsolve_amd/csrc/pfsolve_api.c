@@ -662,15 +662,15 @@ static PfSolveResult append_impl(PfSolveApplication* app, const PfSolveLaunchPar
         if (p->long_only) return append_long(app, &src, &run, s, table);
         const uintptr_t base = (uintptr_t)run.rhs;
         run.vec2 = p->precision == JW_PREC_F64 && (base % 16) == 0 && (run.stride % 2) == 0 && (run.offSol % 2) == 0;
-        if (p->R64 && (run.vec2 || (p->split64 && base % 8 == 0)) && cfg->kernelVariant != 1) {
-            /* wave-per-system kernel: table format 2, built by a prologue launch or,
-             * in the compute / store split kernel, by every workgroup in LDS.  The split
-             * kernel loads and stores global memory from registers and takes systems at any
-             * 8-byte address (30000 systems of 333 rows, packed: 41.4 us a step, 61.8 us on
-             * the general kernel and its table launch); the others stage by LDS DMA, 16-byte
-             * aligned */
+        const int in_lds = p->split64 || jwdev_main64_builds(p->R64);
+        if (p->R64 && (run.vec2 || (in_lds && base % 8 == 0)) && cfg->kernelVariant != 1) {
+            /* wave-per-system kernel: table format 2, built by every workgroup in LDS (N <=
+             * 1024) or by a launch before.  The kernels that build in LDS load and store
+             * global memory from registers and take systems at any 8-byte address (30000
+             * systems of 333 rows, packed: 41.4 us a step, 61.8 us on the general kernel and
+             * its table launch); the other stages by LDS DMA, 16-byte aligned */
             if (nsys <= 0) return PFSOLVE_SUCCESS;
-            if (!p->split64 && jwdev_prologue(&src, cfg->buffer[0], table, 64, p->R64, p->precision, 2, s) != 0)
+            if (!in_lds && jwdev_prologue(&src, cfg->buffer[0], table, 64, p->R64, p->precision, 2, s) != 0)
                 return PFSOLVE_ERROR_FAILED_TO_LAUNCH_KERNEL;
             /* wavefront passes: pairs of systems, single systems for R = 32 */
             const int64_t npass = p->R64 == 32 ? nsys : (nsys + 1) / 2;
@@ -684,7 +684,8 @@ static PfSolveResult append_impl(PfSolveApplication* app, const PfSolveLaunchPar
                 run.wait_polls = p->wait_polls;
                 if (jwdev_main64s(&run, &src, cfg->buffer[0], p->R64, (int)grid, p->d_err, s) != 0)
                     return PFSOLVE_ERROR_FAILED_TO_LAUNCH_KERNEL;
-            } else if (jwdev_main64(&run, p->R64, p->waves64, (int)grid, s) != 0) {
+            } else if (jwdev_main64(&run, in_lds ? &src : NULL, in_lds ? cfg->buffer[0] : NULL, p->R64, p->waves64,
+                                    (int)grid, s) != 0) {
                 return PFSOLVE_ERROR_FAILED_TO_LAUNCH_KERNEL;
             }
             if (p->ev_stop && hipEventRecord(p->ev_stop, s) != hipSuccess) return PFSOLVE_ERROR_FAILED_TO_EVENT_RECORD;
