@@ -395,9 +395,7 @@ static PfSolveResult upload_queue(pfsolve_batch* b)
         source_of(&b->sets[s], &jobs[s].src);
         jobs[s].matrices = b->sets[s].matrices;
         jobs[s].table = (char*)b->tables + b->table_off[s];
-        jobs[s].L = 64;
         jobs[s].R = 2 << eff_group(b, s);
-        jobs[s].format = 2;
         if (b->group_kernel[eff_group(b, s)] == 4) continue;
         gjobs[b->n_gjobs++] = jobs[s];
         if (64 * jobs[s].R > b->max_RL) b->max_RL = 64 * jobs[s].R;
@@ -545,8 +543,7 @@ PfSolveResult pfsolve_batch_set_tuning(pfsolve_batch* b, const pfsolve_batch_tun
 static int run_prologue(pfsolve_batch* b, hipStream_t stream)
 {
     if (b->n_gjobs > 0)
-        return jwdev_prologue_batch(b->d_gjobs, (int)b->n_gjobs, b->max_RL, JW_PREC_F64, b->d_counters, 2 * NCLS,
-                                    stream);
+        return jwdev_prologue_batch(b->d_gjobs, (int)b->n_gjobs, b->max_RL, b->d_counters, 2 * NCLS, stream);
     return 0;
 }
 
@@ -628,7 +625,7 @@ PfSolveResult pfsolve_batch_run_plain(pfsolve_batch* b, hipStream_t stream)
         const int64_t npass = R == 32 ? st->nsys : (st->nsys + 1) / 2;
         int64_t grid = (npass + waves - 1) / waves;
         if (grid > (int64_t)b->cu_count * occ) grid = (int64_t)b->cu_count * occ;
-        if (jwdev_main64(&run, NULL, NULL, R, waves, (int)grid, stream) != 0) return PFSOLVE_ERROR_FAILED_TO_LAUNCH_KERNEL;
+        if (jwdev_main64(&run, R, waves, (int)grid, stream) != 0) return PFSOLVE_ERROR_FAILED_TO_LAUNCH_KERNEL;
     }
     return PFSOLVE_SUCCESS;
 }

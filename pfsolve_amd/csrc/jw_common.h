@@ -164,6 +164,13 @@ template <> struct Ar<dd> {
     __device__ static __forceinline__ dd sel(bool c, dd a, dd b) { return c ? a : b; }
 };
 
+// Global memory, stated at the access.  A pointer read from memory (a batch's items and
+// jobs) is generic to the compiler, which then uses flat instructions: they count as LDS
+// accesses too, so every wait for LDS data also waits for the loads in flight (1024 degrees,
+// N = 1024..513, solve: 186 us with flat loads one pass ahead, 174 us without).
+#define JW_GLOBAL __attribute__((address_space(1)))
+template <typename P> __device__ __forceinline__ JW_GLOBAL P* as_global(P* p) { return (JW_GLOBAL P*)p; }
+
 // element access of caller memory: T storage, or FP64 storage promoted to T
 template <typename T> __device__ __forceinline__ T mem_load(const void* base, int64_t idx, int mem_f64)
 {
@@ -176,7 +183,7 @@ template <typename T> __device__ __forceinline__ T mem_load(const void* base, in
 // it before the join).
 template <> __device__ __forceinline__ dd mem_load<dd>(const void* base, int64_t idx, int mem_f64)
 {
-    const double* p = reinterpret_cast<const double*>(base);
+    const JW_GLOBAL double* p = as_global(reinterpret_cast<const double*>(base));
     const int64_t i = mem_f64 ? idx : 2 * idx;
     const double h = p[i];
     const double l = p[mem_f64 ? i : i + 1];
@@ -184,7 +191,7 @@ template <> __device__ __forceinline__ dd mem_load<dd>(const void* base, int64_t
 }
 template <> __device__ __forceinline__ double mem_load<double>(const void* base, int64_t idx, int)
 {
-    return reinterpret_cast<const double*>(base)[idx];
+    return as_global(reinterpret_cast<const double*>(base))[idx];
 }
 template <typename T> __device__ __forceinline__ void mem_store(void* base, int64_t idx, T v, int mem_f64)
 {
@@ -222,21 +229,21 @@ __device__ __forceinline__ int64_t reorder_pos(int64_t i, int64_t N, int64_t Nal
     }
     // rows per thread of the register layout: from Nalign (the largest system of a
     // chained step) or the block size, the split of the stored rows over them: from N
-    uint32_t ws = ((NA + 1023u) / 1024u) * 64u;
-    if (NA < 512u) ws = 64u;
-    uint32_t R = (NA + ws - 1u) / ws;
+    uint32_t R;
+    if (NA <= 1024u) {
+        R = (NA + 63u) >> 6;   // 64 lanes
+    } else {
+        const uint32_t ws = ((NA + 1023u) >> 10) << 6;
+        R = (NA + ws - 1u) / ws;
+    }
     if ((R & 1u) == 0u) R++;
     const uint32_t base = blk == uN ? 0u : (ui / blk) * blk;
     const uint32_t n = base + blk > uN ? uN - base : blk;
     const uint32_t li = ui - base;
-    const uint32_t ceilq = (n + R - 1u) / R;
+    // register k holds nq + (k < rem) rows
     const uint32_t q = li / R, k = li - q * R;
     const uint32_t nq = n / R, rem = n - nq * R;
-    uint32_t ret = q;
-    if (k < rem)
-        ret += k * ceilq;
-    else
-        ret += rem * ceilq + (k - rem) * nq;
+    const uint32_t ret = q + k * nq + (k < rem ? k : rem);
     return (int64_t)(base + ret);
 }
 

@@ -44,23 +44,24 @@ __global__ __launch_bounds__(kPrologueThreads) void jw_prologue_kernel(jw_source
                                                                        int L, int R, int format)
 {
     extern __shared__ __align__(16) unsigned char pro_smem[];
-    if constexpr (SMALL)
-        prologue_body<T, NoPivotHooks, false, 1, 2>(d, mat, table, L, R, format, pro_smem);
-    else
-        prologue_body<T>(d, mat, table, L, R, format, pro_smem);
+    constexpr int J = SMALL ? 1 : kProRows, RT = SMALL ? 2 : kMaxRT;
+    if (format == 2) prologue_body<T, 2, NoPivotHooks, J, RT>(d, mat, table, L, R, pro_smem);
+    else prologue_body<T, 1, NoPivotHooks, J, RT>(d, mat, table, L, R, pro_smem);
 }
 
-// batched: one workgroup per matrix set; workgroup 0 also clears the work-queue counters.
-// NT = 256 when every set has at most 1024 rows: four such workgroups share a CU
-// (LDS and registers), so 1024 sets need one round instead of two.
-template <typename T, int NT>
-__global__ __launch_bounds__(NT) void jw_prologue_batch_kernel(const jw_prologue_job* jobs, int L_unused,
-                                                                             int* counters, int ncounters)
+// batched (FP64, format 2): one workgroup per matrix set; workgroup 0 also clears the
+// work-queue counters.  NT = 256 when every set has at most 1024 rows (4 per thread in the
+// row phases and the scan): four such workgroups share a CU (LDS and registers), so 1024 sets
+// need one round instead of two.
+template <int NT>
+__global__ __launch_bounds__(NT, NT == 256 ? 4 : 2) void jw_prologue_batch_kernel(const jw_prologue_job* jobs,
+                                                                                 int* counters, int ncounters)
 {
     extern __shared__ __align__(16) unsigned char pro_smem[];
     if (blockIdx.x == 0 && counters && (int)threadIdx.x < ncounters) counters[threadIdx.x] = 0;
     const jw_prologue_job& j = jobs[blockIdx.x];
-    prologue_body<T>(j.src, j.matrices, reinterpret_cast<T*>(j.table), j.L, j.R, j.format, pro_smem);
+    prologue_body<double, 2, NoPivotHooks, kProRows, NT == 256 ? 4 : kMaxRT>(
+        j.src, j.matrices, as_global(reinterpret_cast<double*>(j.table)), 64, j.R, pro_smem);
 }
 
 // ------------------------------------------------------------------------
@@ -551,11 +552,10 @@ int jwdev_prologue(const jw_source_desc* d, const void* matrices, void* table, i
     return 0;
 }
 
-int jwdev_prologue_batch(const jw_prologue_job* d_jobs, int njobs, int max_RL, int precision, int* d_counters,
-                         int ncounters, void* stream)
+int jwdev_prologue_batch(const jw_prologue_job* d_jobs, int njobs, int max_RL, int* d_counters, int ncounters,
+                         void* stream)
 {
-    const size_t elt = precision == JW_PREC_F64 ? 8 : 16;
-    const size_t lds = prologue_lds_bytes(max_RL, elt);
+    const size_t lds = prologue_lds_bytes(max_RL, 8);
     if (lds > 160 * 1024 || max_RL > kProRows * kPrologueThreads) {
         snprintf(g_err, sizeof(g_err), "prologue: too many rows");
         return -1;
@@ -564,20 +564,12 @@ int jwdev_prologue_batch(const jw_prologue_job* d_jobs, int njobs, int max_RL, i
     const bool narrow = max_RL <= kProRows * 256;
     const int nt = narrow ? 256 : kPrologueThreads;
     if (ncounters > nt) { snprintf(g_err, sizeof(g_err), "too many counters"); return -1; }
-    hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-    const void* fn;
-    if (precision == JW_PREC_F64)
-        fn = narrow ? reinterpret_cast<const void*>(&jw_prologue_batch_kernel<double, 256>)
-                    : reinterpret_cast<const void*>(&jw_prologue_batch_kernel<double, kPrologueThreads>);
-    else
-        fn = narrow ? reinterpret_cast<const void*>(&jw_prologue_batch_kernel<dd, 256>)
-                    : reinterpret_cast<const void*>(&jw_prologue_batch_kernel<dd, kPrologueThreads>);
+    const void* fn = narrow ? reinterpret_cast<const void*>(&jw_prologue_batch_kernel<256>)
+                            : reinterpret_cast<const void*>(&jw_prologue_batch_kernel<kPrologueThreads>);
     hipError_t ea = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (ea != hipSuccess) { set_err("hipFuncSetAttribute(prologue batch)", ea); return -2; }
-    const jw_prologue_job* jobs = d_jobs;
-    int zero = 0;
-    void* args[] = {const_cast<jw_prologue_job**>(&jobs), &zero, &d_counters, &ncounters};
-    hipError_t el = hipLaunchKernel(fn, dim3(njobs), dim3(nt), args, lds, s);
+    void* args[] = {const_cast<jw_prologue_job**>(&d_jobs), &d_counters, &ncounters};
+    hipError_t el = hipLaunchKernel(fn, dim3(njobs), dim3(nt), args, lds, reinterpret_cast<hipStream_t>(stream));
     if (el != hipSuccess) { set_err("prologue batch launch", el); return -1; }
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) { set_err("prologue batch launch", e); return -1; }

@@ -135,12 +135,12 @@ typedef struct jw_long_desc {
     int32_t nchunks, mode;
 } jw_long_desc;
 
-/* One matrix set for the batched prologue (one workgroup each). */
+/* One matrix set for the batched prologue (FP64, table format 2; one workgroup each). */
 typedef struct jw_prologue_job {
     jw_source_desc src;
     const void* matrices;
     void* table;
-    int32_t L, R, format, pad;
+    int32_t R, pad;
 } jw_prologue_job;
 
 /* Uneven-size batch: one item per matrix set, and work units (a range of
@@ -183,17 +183,18 @@ int64_t jwdev_table_elems(int L, int R);
 int64_t jwdev_lds_bytes(int L, int R, int precision);
 int jwdev_prologue(const jw_source_desc* d, const void* matrices, void* table, int L, int R,
                    int precision, int format, void* stream);
-int jwdev_prologue_batch(const jw_prologue_job* d_jobs, int njobs, int max_RL, int precision, int* d_counters,
-                         int ncounters, void* stream);
+int jwdev_prologue_batch(const jw_prologue_job* d_jobs, int njobs, int max_RL, int* d_counters, int ncounters,
+                         void* stream);
 /* wave-per-system FP64 kernel (table format 2, 64 lanes, R in {2,4,8,16}) */
 int64_t jwdev_table64_elems(int R);
 int jwdev_main64_waves(int R);
 int64_t jwdev_main64_lds_bytes(int R, int waves);
 int jwdev_main64_occupancy(int R, int waves);
-/* with a source the kernel builds its table in LDS (jwdev_main64_builds), else it reads r->table */
-int jwdev_main64_builds(int R);
-int jwdev_main64(const jw_run_desc* r, const jw_source_desc* src, const void* matrices, int R, int waves, int grid,
-                 void* stream);
+int jwdev_main64(const jw_run_desc* r, int R, int waves, int grid, void* stream);
+/* the same with the table built in each workgroup's LDS (R <= 16; systems at any 8-byte address) */
+int jwdev_main64b_waves(int R);
+int jwdev_main64b_occupancy(int R);
+int jwdev_main64b(const jw_run_desc* r, const jw_source_desc* src, const void* matrices, int R, int grid, void* stream);
 /* the same with compute / store split (R <= 8): compute wavefronts never store,
  * storer wavefronts write their results; *d_err is raised if a bounded wait ran out */
 int jwdev_main64s_shape(int R, int* ncomp, int* nstore);

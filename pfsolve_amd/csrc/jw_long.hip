@@ -74,16 +74,15 @@ constexpr int64_t long_tab_elems()
 template <typename T>
 __global__ __launch_bounds__(kPrologueThreads) void jw_long_prologue_kernel(jw_source_desc d, const void* mat,
                                                                           T* table, int chained, int* sync, T* gval,
-                                                                          int* err, int format)
+                                                                          int* err)
 {
     extern __shared__ __align__(16) unsigned char pro_smem[];
     __shared__ int s_build;
     constexpr int R = LongGeom<T>::R;
     constexpr int NSUB = LongGeom<T>::NSUB;
     constexpr int SR = NSUB * R * kLongL;
-    // format 1 for the chunk kernel here, format 2 (FP64) for the pair kernel's chunks
-    const int64_t TE = format == 2 ? (int64_t)JW_TAB64_ELEMS(R) : long_tab_elems<T>();
-    // the pivot carry follows the build's five row arrays
+    const int64_t TE = long_tab_elems<T>();
+    // the pivot carry follows the build's row arrays
     T* carry = reinterpret_cast<T*>(pro_smem + prologue_lds_bytes(SR, sizeof(T)));
     int64_t build = blockIdx.x;
     if (chained) {
@@ -97,8 +96,8 @@ __global__ __launch_bounds__(kPrologueThreads) void jw_long_prologue_kernel(jw_s
     if (chained && threadIdx.x == 0)
         carry[1] = rb > 0 ? mem_load<T>(mat, d.udS + source_pos(d, rb - 1, d.N), d.mem_f64) : Ar<T>::zero();
     const ChainHooks<T> hooks{carry, sync + 1, gval, err, build, chained};
-    prologue_body<T, ChainHooks<T>>(d, mat, table + build * NSUB * TE, kLongL, R, format, pro_smem, rb,
-                                    chained ? carry : nullptr, NSUB, hooks);
+    prologue_body<T, 1, ChainHooks<T>>(d, mat, table + build * NSUB * TE, kLongL, R, pro_smem, rb,
+                                       chained ? carry : nullptr, NSUB, hooks);
 }
 
 __global__ void jw_long_clear_kernel(int* p, int n)
@@ -583,12 +582,7 @@ int jwdev_long_prologue(const jw_source_desc* src, const void* matrices, void* t
 {
     if (!matrices || !table) return fail("long prologue: no matrices or table");
     const bool f64 = precision == JW_PREC_F64;
-    // the table size names the format: format 1 (the chunk kernel), or FP64 format 2 (the
-    // pair kernel's chunks, jw_long64_kernel)
-    int format = 1;
-    if (f64 && tab_elems == (int64_t)JW_TAB64_ELEMS(LongGeom<double>::R))
-        format = 2;
-    else if (tab_elems != (f64 ? long_tab_elems<double>() : long_tab_elems<dd>()))
+    if (tab_elems != (f64 ? long_tab_elems<double>() : long_tab_elems<dd>()))
         return fail("long prologue: table size mismatch");
     const int SR = f64 ? LongGeom<double>::NSUB * LongGeom<double>::R * kLongL
                        : LongGeom<dd>::NSUB * LongGeom<dd>::R * kLongL;
@@ -613,11 +607,10 @@ int jwdev_long_prologue(const jw_source_desc* src, const void* matrices, void* t
     const dim3 grid((unsigned)nit);
     if (f64)
         hipLaunchKernelGGL(jw_long_prologue_kernel<double>, grid, dim3(kPrologueThreads), lds, s, *src, matrices,
-                           reinterpret_cast<double*>(table), chained, sync, reinterpret_cast<double*>(gval), err,
-                           format);
+                           reinterpret_cast<double*>(table), chained, sync, reinterpret_cast<double*>(gval), err);
     else
         hipLaunchKernelGGL(jw_long_prologue_kernel<dd>, grid, dim3(kPrologueThreads), lds, s, *src, matrices,
-                           reinterpret_cast<dd*>(table), chained, sync, reinterpret_cast<dd*>(gval), err, format);
+                           reinterpret_cast<dd*>(table), chained, sync, reinterpret_cast<dd*>(gval), err);
     e = hipGetLastError();
     if (e != hipSuccess) return fail("long prologue launch", e);
     return 0;

@@ -51,7 +51,7 @@ __host__ __device__ __forceinline__ int64_t max_i64(int64_t a, int64_t b) { retu
 typedef double jw_d2u __attribute__((ext_vector_type(2), aligned(8)));
 __device__ __forceinline__ double2 load_chunk(const double* p)
 {
-    const jw_d2u t = *reinterpret_cast<const jw_d2u*>(p);
+    const jw_d2u t = *(const JW_GLOBAL jw_d2u*)p;
     return make_double2(t.x, t.y);
 }
 
@@ -62,7 +62,7 @@ __device__ __forceinline__ void store_stream(double* p, double2 v)
     jw_d2u t;
     t.x = v.x;
     t.y = v.y;
-    __builtin_nontemporal_store(t, reinterpret_cast<jw_d2u*>(p));
+    __builtin_nontemporal_store(t, (JW_GLOBAL jw_d2u*)p);
 }
 
 // keeps the scheduler from hoisting one phase's table loads into the previous
@@ -236,7 +236,7 @@ template <int R>
 __device__ __forceinline__ void read_edges(int lane, const jw_pass64& g, int64_t sys0, double (&x0)[R], double (&x1)[R])
 {
     const bool ok1 = sys0 + 1 < g.nsys;
-    const double* src0 = g.rhs + sys0 * g.stride + g.offSol;
+    const JW_GLOBAL double* src0 = as_global(g.rhs) + sys0 * g.stride + g.offSol;
     if (g.in_edge_lo || g.in_edge_hi) {
 #pragma unroll
         for (int e = 0; e < 2; e++) {
@@ -529,7 +529,7 @@ __device__ __forceinline__ void store_pair(const double2* stg, int lane, const j
             const bool on = e == 0 ? g.out_edge_lo : g.out_edge_hi;
             const int r = e == 0 ? g.out_lo : g.out_hi - 1;
             if (on && lane == 0) {
-                double* dst = g.rhs + sys0 * g.stride + g.offSol + r;
+                JW_GLOBAL double* dst = as_global(g.rhs) + sys0 * g.stride + g.offSol + r;
 #pragma unroll
                 for (int s = 0; s < 2; s++) {
                     if (s == 1 && !ok1) continue;
@@ -614,8 +614,8 @@ __device__ __forceinline__ void jw_groups64(const double* tab, double2* stg, int
         const bool on = e == 0 ? g.in_edge_lo : g.in_edge_hi;
         const int r = e == 0 ? g.in_lo : g.in_hi - 1;
         if (on && tl == r / 2) {
-            const double v0 = s0 < sys_end ? g.rhs[s0 * g.stride + g.offSol + r] : 0.0;
-            const double v1 = s1 < sys_end ? g.rhs[s1 * g.stride + g.offSol + r] : 0.0;
+            const double v0 = s0 < sys_end ? as_global(g.rhs)[s0 * g.stride + g.offSol + r] : 0.0;
+            const double v1 = s1 < sys_end ? as_global(g.rhs)[s1 * g.stride + g.offSol + r] : 0.0;
             if (r & 1) { x0[1] = v0; x1[1] = v1; } else { x0[0] = v0; x1[0] = v1; }
         }
     }
@@ -639,8 +639,8 @@ __device__ __forceinline__ void jw_groups64(const double* tab, double2* stg, int
         const bool on = e == 0 ? g.out_edge_lo : g.out_edge_hi;
         const int r = e == 0 ? g.out_lo : g.out_hi - 1;
         if (on && tl == r / 2) {
-            if (s0 < sys_end) g.rhs[s0 * g.stride + g.offSol + r] = (r & 1) ? x0[1] : x0[0];
-            if (s1 < sys_end) g.rhs[s1 * g.stride + g.offSol + r] = (r & 1) ? x1[1] : x1[0];
+            if (s0 < sys_end) as_global(g.rhs)[s0 * g.stride + g.offSol + r] = (r & 1) ? x0[1] : x0[0];
+            if (s1 < sys_end) as_global(g.rhs)[s1 * g.stride + g.offSol + r] = (r & 1) ? x1[1] : x1[0];
         }
     }
     __builtin_amdgcn_s_waitcnt(0xC07F);   // lgkmcnt(0): the staging is read before the next pass writes it
@@ -757,8 +757,8 @@ __device__ __forceinline__ void store_system(double2* stg, int lane, const jw_pa
         const int c = 64 * k + lane;
         if (c >= g.ocl && c < g.och) store_stream(dst + 2 * c, v[k]);
     }
-    if (g.out_edge_lo && lane == g.out_lo / R) dst[g.out_lo] = pick_row<R>(x, g.out_lo % R);
-    if (g.out_edge_hi && lane == (g.out_hi - 1) / R) dst[g.out_hi - 1] = pick_row<R>(x, (g.out_hi - 1) % R);
+    if (g.out_edge_lo && lane == g.out_lo / R) as_global(dst)[g.out_lo] = pick_row<R>(x, g.out_lo % R);
+    if (g.out_edge_hi && lane == (g.out_hi - 1) / R) as_global(dst)[g.out_hi - 1] = pick_row<R>(x, (g.out_hi - 1) % R);
 }
 
 // Pairs q, q + step, ... below q1 through one wavefront: each pair's rows were loaded into
@@ -790,8 +790,8 @@ __device__ __forceinline__ void copy_table_lds(unsigned char* smem, const void* 
     copy_to_lds(smem, table, NTAB * 8, wave, nwaves, lane);
 }
 
-// BUILD: the table is built in LDS from the caller's matrices (the stagings as scratch);
-// otherwise it is copied from global memory.
+// BUILD: the table is built in LDS from the caller's matrices (the stagings as scratch)
+// and pairs are loaded ahead at every R; otherwise it is copied from global memory.
 template <int R, bool ALL3, bool BUILD>
 __global__ __launch_bounds__(max_threads<R>()) void jw_main64_kernel(jw_run_desc d, jw_source_desc src, const void* mat)
 {
@@ -801,7 +801,7 @@ __global__ __launch_bounds__(max_threads<R>()) void jw_main64_kernel(jw_run_desc
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int nwaves = blockDim.x >> 6;
-    double2* stg = reinterpret_cast<double2*>(smem + NTAB * 8 + wave * pair_stage_bytes(R));
+    double2* stg = reinterpret_cast<double2*>(smem + NTAB * 8 + wave * (BUILD ? 512LL * R : pair_stage_bytes(R)));
     const int64_t npass = (d.nsys + 1) >> 1, step = (int64_t)gridDim.x * nwaves;
     int64_t q = (int64_t)blockIdx.x * nwaves + wave;
     // rebuilt every pass from the kernel arguments, so that nothing derived from
@@ -811,19 +811,20 @@ __global__ __launch_bounds__(max_threads<R>()) void jw_main64_kernel(jw_run_desc
                            (int)d.out_lo, (int)d.out_hi, d.kl, d.ku, d.fwd, d.b1, d.b2, d.apply_scale, d.scale_hi,
                            lane);
     };
-    if constexpr (pair_ahead(R)) {
-        // the first pair's loads overlap the table build
+    if constexpr (BUILD || pair_ahead(R)) {
+        // the first pair's loads go out behind the build's (or before the table copy)
         double2 pf[2][R / 2];
-        if (q < npass) load_pair_ahead<R>(pf, lane, geo(), 2 * q);
-        if constexpr (BUILD)
-            prologue_body<double, NoPivotHooks, true, 64 * R / max_threads<R>(), pro_rows(64 * R)>(
-                src, mat, reinterpret_cast<double*>(smem), 64, R, 2, smem + NTAB * 8);
-        else
+        auto first = [&] { if (q < npass) load_pair_ahead<R>(pf, lane, geo(), 2 * q); };
+        if constexpr (BUILD) {
+            prologue_body<double, 2, NoPivotHooks, R <= 8 ? 1 : 2, pro_rows(64 * R)>(
+                src, mat, reinterpret_cast<double*>(smem), 64, R, smem + NTAB * 8, 0, nullptr, 1, NoPivotHooks(), first);
+        } else {
+            first();
             copy_table_lds<NTAB>(smem, d.table, wave, nwaves, lane);
+        }
         __syncthreads();
         stream_pairs<R, ALL3>(tab, stg, lane, geo, q, npass, step, pf);
     } else {
-        static_assert(!BUILD, "the build in the kernel: pair_ahead only");
         copy_table_lds<NTAB>(smem, d.table, wave, nwaves, lane);
         zero_staging<R>(stg, lane);
         __syncthreads();
@@ -1058,10 +1059,10 @@ struct SlotHooks {
         }
         carry[0] = __longlong_as_double((long long)v);
     }
-    __device__ void publish(int tid, const double* sg, int RL) const
+    __device__ void publish(int tid, const double* gl) const
     {
         if (!chained || tid != 0) return;
-        const double g = sg[RL - 1];
+        const double g = *gl;
         const unsigned long long v = g != g ? 0x7FF8000000000000ull : (unsigned long long)__double_as_longlong(g);
         __hip_atomic_store(&slots[build], v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
@@ -1102,15 +1103,15 @@ __global__ __launch_bounds__(max_threads<kLong64R>()) void jw_long64_front_kerne
     const int tk = s_id;
     if (tk < nbuild) {
         const int64_t rb = (int64_t)tk * SR;
-        // the pivot carry follows the build's five row arrays; thread 0 reads the raw
+        // the pivot carry follows the build's row arrays; thread 0 reads the raw
         // super-diagonal entry of the row before the build (the build's first barrier
         // publishes it)
         double* carry = reinterpret_cast<double*>(smem + prologue_lds_bytes(SR, sizeof(double)));
         if (chained && threadIdx.x == 0)
             carry[1] = rb > 0 ? mem_load<double>(mat, src.udS + source_pos(src, rb - 1, src.N), src.mem_f64) : 0.0;
         const SlotHooks hooks{carry, slots, err, tk, chained};
-        prologue_body<double, SlotHooks>(src, mat, table + (int64_t)tk * kLong64Nsub * NTAB, 64, R, 2, smem, rb,
-                                         chained ? carry : nullptr, kLong64Nsub, hooks);
+        prologue_body<double, 2, SlotHooks>(src, mat, table + (int64_t)tk * kLong64Nsub * NTAB, 64, R, smem, rb,
+                                            chained ? carry : nullptr, kLong64Nsub, hooks);
         // every wavefront waits for its own table stores (written into the L2), then one
         // agent-scope release by thread 0 writes the L2 back and sets the flag (one L2
         // writeback per build: a fence in every wavefront measured 3x longer under the
@@ -1300,7 +1301,7 @@ __device__ __forceinline__ void jw_single64(__amdgpu_buffer_rsrc_t tab, double2*
         const bool on = e == 0 ? g.in_edge_lo : g.in_edge_hi;
         const int r = e == 0 ? g.in_lo : g.in_hi - 1;
         if (on && lane == r / R) {
-            const double v = src[r];
+            const double v = as_global(src)[r];
 #pragma unroll
             for (int k = 0; k < R; k++)
                 if (k == r % R) x[k] = v;
@@ -1328,7 +1329,7 @@ __device__ __forceinline__ void jw_single64(__amdgpu_buffer_rsrc_t tab, double2*
         const int r = e == 0 ? g.out_lo : g.out_hi - 1;
         if (on && lane == 0) {
             const double2 w = stg[swz<H>(r >> 1)];
-            g.rhs[sys * g.stride + g.offSol + r] = (r & 1) ? w.y : w.x;
+            as_global(g.rhs)[sys * g.stride + g.offSol + r] = (r & 1) ? w.y : w.x;
         }
     }
 #pragma unroll
@@ -1727,7 +1728,8 @@ constexpr int split_threads()
 }
 
 template <int R, bool ALL3, int IOMODE>
-__global__ __launch_bounds__(split_threads<R>()) void jw_main64s_kernel(jw_run_desc d, int ncomp, int* err,
+__global__ __launch_bounds__(split_threads<R>())
+__attribute__((amdgpu_waves_per_eu(split_threads<R>() / 256, split_threads<R>() / 256))) void jw_main64s_kernel(jw_run_desc d, int ncomp, int* err,
                                                                         jw_source_desc src, const void* mat)
 {
     constexpr int NTAB = JW_TAB64_ELEMS(R);
@@ -1743,10 +1745,14 @@ __global__ __launch_bounds__(split_threads<R>()) void jw_main64s_kernel(jw_run_d
     const int64_t step = (int64_t)gridDim.x * ncomp;
     const int polls = d.wait_polls > 0 ? d.wait_polls : (d.wait_polls < 0 ? 0 : kSpinLimit);
     int64_t q = (int64_t)blockIdx.x * ncomp + wave;
-    // a compute wavefront's first pair is loaded into registers before the table
-    // build, so its latency overlaps the build
+    // every workgroup builds the coefficient table in its own LDS from the
+    // caller's matrices (no separate prologue launch); the staging area, unused
+    // until the barrier below, is the build's scratch.  A compute wavefront's first pair
+    // is loaded into registers behind the build's loads, so its latency overlaps the build
+    // (before them, the build would wait for every wavefront's first pair)
     double2 pf[2][R / 2];
-    if (wave < ncomp && q < npass) {
+    auto first = [&] {
+        if (wave >= ncomp || q >= npass) return;
         if (IOMODE != 0) {
             load_pair_packed<R>(pf, lane, d, q);
         } else {
@@ -1755,13 +1761,9 @@ __global__ __launch_bounds__(split_threads<R>()) void jw_main64s_kernel(jw_run_d
                                             d.fwd, d.b1, d.b2, d.apply_scale, d.scale_hi, lane);
             load_pair_direct<R>(pf, lane, g, 2 * q);
         }
-    }
-    // every workgroup builds the coefficient table in its own LDS from the
-    // caller's matrices (no separate prologue launch); the staging area, unused
-    // until the barrier below, is the build's scratch
-    // (the default per-thread array bounds: smaller ones, 125 instead of 143 VGPRs at R = 8,
-    // measured 3-5 % slower on the whole kernel)
-    prologue_body<double, NoPivotHooks, true>(src, mat, reinterpret_cast<double*>(smem), 64, R, 2, smem + NTAB * 8);
+    };
+    prologue_body<double, 2, NoPivotHooks, 1, pro_rows(64 * R)>(src, mat, reinterpret_cast<double*>(smem), 64, R,
+                                                               smem + NTAB * 8, 0, nullptr, 1, NoPivotHooks(), first);
     // block operator factors past the staging and the build's scratch
     double* fin = reinterpret_cast<double*>(
         smem + NTAB * 8 + max_i64(2LL * 64 * R * 8 * ncomp, (int64_t)prologue_lds_bytes(64 * R, 8)));
@@ -1936,19 +1938,8 @@ __global__ __launch_bounds__(max_threads<R>()) void jw_batch64_kernel(const jw_b
 // also hold the table build's scratch while a set's table is built
 __host__ __device__ constexpr int64_t batch64b_lds_bytes(int R, int waves)
 {
-    const int64_t stagings = pair_stage_bytes(R) * waves, scratch = (int64_t)(5 * 64 * R) * 8;
+    const int64_t stagings = pair_stage_bytes(R) * waves, scratch = (int64_t)prologue_lds_bytes(64 * R, 8);
     return (int64_t)JW_TAB64_ELEMS(R) * 8 + (stagings > scratch ? stagings : scratch);
-}
-
-// one set's format-2 table built into LDS (the stagings after it as scratch); kept out of
-// line so that the build's registers do not add to the solve loop's
-// (the dynamic LDS is named here, not passed in, so the build addresses it as LDS)
-template <int R>
-__device__ __noinline__ void build_table_lds(const jw_prologue_job* job)
-{
-    extern __shared__ __align__(16) unsigned char smem_build[];
-    prologue_body<double, NoPivotHooks, false, pro_rows(64 * R), pro_rows(64 * R)>(
-        job->src, job->matrices, reinterpret_cast<double*>(smem_build), 64, R, 2, smem_build + JW_TAB64_ELEMS(R) * 8);
 }
 
 // The batch queue with the table built in LDS: as jw_batch64_kernel, but a workgroup
@@ -1958,13 +1949,37 @@ __device__ __noinline__ void build_table_lds(const jw_prologue_job* job)
 // table written and read back through HBM; the build's latency is paid per set change
 // by the workgroup, while the other workgroups keep HBM busy.  Needs at least 256
 // threads and 4 threads per 16 rows (prologue_body's partition).
-template <int R>
+// FULL: a full workgroup, whose threads take one or two rows each of a build.
+// (R = 16: the build out of line, before the unit's first loads; in line, its registers
+// spill the solve loop's: 266 us per step of the 1024-degree batch, 196 us out of line)
+template <int R, int MAXJ>
+__device__ __noinline__ void build_table_lds(const jw_prologue_job* job)
+{
+    extern __shared__ __align__(16) unsigned char smem_build[];   // named here: addressed as LDS
+    // the argument is the same in every lane, which the callee cannot know: the job through
+    // scalar loads (a descriptor in vector registers would make every branch on it divergent)
+    typedef const __attribute__((address_space(4))) uint32_t const_word;
+    const uint64_t p = reinterpret_cast<uint64_t>(job);
+    const_word* w = (const_word*)((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)p) |
+                                  ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(p >> 32)) << 32));
+    union {
+        jw_prologue_job j;
+        uint32_t u[sizeof(jw_prologue_job) / 4];
+    } x;
+#pragma unroll
+    for (size_t i = 0; i < sizeof(jw_prologue_job) / 4; i++) x.u[i] = w[i];
+    prologue_body<double, 2, NoPivotHooks, MAXJ, pro_rows(64 * R)>(
+        x.j.src, x.j.matrices, reinterpret_cast<double*>(smem_build), 64, R, smem_build + JW_TAB64_ELEMS(R) * 8);
+}
+
+template <int R, bool FULL>
 __global__ __launch_bounds__(max_threads<R>()) void jw_batch64b_kernel(const jw_batch_item* items,
                                                                        const jw_batch_unit* units, int nunits,
                                                                        int* counter, const jw_prologue_job* jobs)
 {
     extern __shared__ __align__(16) unsigned char smem[];
     constexpr int NTAB = JW_TAB64_ELEMS(R);
+    constexpr int MAXJ = FULL ? (R <= 8 ? 1 : 2) : pro_rows(64 * R);
     __shared__ int s_unit;
     const double* tab = reinterpret_cast<const double*>(smem);
     const int lane = threadIdx.x & 63;
@@ -1980,34 +1995,31 @@ __global__ __launch_bounds__(max_threads<R>()) void jw_batch64b_kernel(const jw_
         if (u >= nunits) break;
         const jw_batch_unit un = units[u];
         const jw_batch_item& it = items[un.item];
-        if constexpr (pair_ahead(R)) {
-            if (un.item != cur) {
-                build_table_lds<R>(jobs + un.item);
+        const int64_t q = un.pair0 + wave;
+        auto geo = [&] {
+            return make_pass64(reinterpret_cast<double*>(it.rhs), it.nsys, it.stride, it.offSol, 0, it.N, 0, it.N,
+                               it.kl, it.ku, true, true, true, it.apply_scale != 0, it.scale, lane);
+        };
+        if (un.item != cur) {
+            cur = un.item;
+            if constexpr (pair_ahead(R)) {
+                build_table_lds<R, MAXJ>(jobs + cur);
                 __syncthreads();   // the build's scratch (the stagings) is free again
-                cur = un.item;
+            } else {
+                const jw_prologue_job& job = jobs[cur];
+                prologue_body<double, 2, NoPivotHooks, MAXJ, pro_rows(64 * R)>(
+                    job.src, job.matrices, reinterpret_cast<double*>(smem), 64, R, smem + NTAB * 8);
+                __syncthreads();
+                zero_staging<R>(stg, lane);
+                __syncthreads();
             }
-            auto geo = [&] {
-                return make_pass64(reinterpret_cast<double*>(it.rhs), it.nsys, it.stride, it.offSol, 0, it.N, 0, it.N,
-                                   it.kl, it.ku, true, true, true, it.apply_scale != 0, it.scale, lane);
-            };
+        }
+        if constexpr (pair_ahead(R)) {
             double2 pf[2][R / 2];
-            const int64_t q = un.pair0 + wave;
             if (q < un.pair1) load_pair_ahead<R>(pf, lane, geo(), 2 * q);
             stream_pairs<R, true>(tab, stg, lane, geo, q, un.pair1, nwaves, pf);
-            continue;
-        }
-        if (un.item != cur) {
-            build_table_lds<R>(jobs + un.item);
-            __syncthreads();   // the build's scratch (the stagings) is free again
-            zero_staging<R>(stg, lane);
-            __syncthreads();
-            cur = un.item;
-        }
-        for (int q = un.pair0 + wave; q < un.pair1; q += nwaves) {
-            const jw_pass64 g = make_pass64(reinterpret_cast<double*>(it.rhs), it.nsys, it.stride, it.offSol, 0,
-                                            it.N, 0, it.N, it.kl, it.ku, true, true, true, it.apply_scale != 0,
-                                            it.scale, lane);
-            jw_pair64<R, true>(tab, stg, lane, g, 2 * (int64_t)q);
+        } else {
+            for (int64_t p = q; p < un.pair1; p += nwaves) jw_pair64<R, true>(tab, stg, lane, geo(), 2 * p);
         }
     }
     queue_leave(counter);
@@ -2022,22 +2034,22 @@ __device__ __forceinline__ void store_pair_direct(int lane, const jw_pass64& g, 
 {
     constexpr int H = R / 2;
     const bool ok1 = sys0 + 1 < g.nsys;
-    double2* dst0 = reinterpret_cast<double2*>(g.rhs) + ((sys0 * g.stride + g.offSol) >> 1);
+    double* dst0 = g.rhs + sys0 * g.stride + g.offSol;
 #pragma unroll
     for (int s = 0; s < 2; s++) {
         if (s == 1 && !ok1) continue;
-        double2* dst = dst0 + s * (g.stride >> 1);
+        JW_GLOBAL jw_d2u* dst = (JW_GLOBAL jw_d2u*)(dst0 + s * g.stride);
         const double(&x)[R] = s == 0 ? x0 : x1;
 #pragma unroll
         for (int m = 0; m < H; m++) {
             const int c = lane * H + m;
             // cached stores: the H stores of a lane each fill part of 64 lines that the
             // sibling stores complete, and L2 merges them before the write-back
-            if (c >= g.ocl && c < g.och) dst[c] = make_double2(x[2 * m], x[2 * m + 1]);
+            if (c >= g.ocl && c < g.och) dst[c] = jw_d2u{x[2 * m], x[2 * m + 1]};
         }
     }
     if (g.out_edge_lo || g.out_edge_hi) {
-        double* base = g.rhs + sys0 * g.stride + g.offSol;
+        JW_GLOBAL double* base = as_global(g.rhs) + sys0 * g.stride + g.offSol;
 #pragma unroll
         for (int e = 0; e < 2; e++) {
             const bool on = e == 0 ? g.out_edge_lo : g.out_edge_hi;
@@ -2279,7 +2291,15 @@ const void* kernel_ptr(bool all3)
 
 const void* pick64(int R, bool all3 = true, bool build = false)
 {
-    if (build) return R == 16 ? kernel_ptr<16, true>(all3) : nullptr;
+    if (build) {
+        switch (R) {
+        case 2: return kernel_ptr<2, true>(all3);
+        case 4: return kernel_ptr<4, true>(all3);
+        case 8: return kernel_ptr<8, true>(all3);
+        case 16: return kernel_ptr<16, true>(all3);
+        default: return nullptr;
+        }
+    }
     switch (R) {
     case 32: return all3 ? reinterpret_cast<const void*>(&jw_main64g_kernel<32, true>)
                          : reinterpret_cast<const void*>(&jw_main64g_kernel<32, false>);
@@ -2363,22 +2383,23 @@ int bsplit_threads_rt(int R) { return R <= 4 ? 1024 : (R == 8 ? 768 : 512); }
 template <int R>
 const void* split_ptr(bool all3, int io)
 {
+    if constexpr (R > 2)
+        if (io == 0)
+            return all3 ? reinterpret_cast<const void*>(&jw_main64s_kernel<R, true, 0>)
+                        : reinterpret_cast<const void*>(&jw_main64s_kernel<R, false, 0>);
     if (io == 1)
         return all3 ? reinterpret_cast<const void*>(&jw_main64s_kernel<R, true, 1>)
                     : reinterpret_cast<const void*>(&jw_main64s_kernel<R, false, 1>);
-    if (io == 2)
-        return all3 ? reinterpret_cast<const void*>(&jw_main64s_kernel<R, true, 2>)
-                    : reinterpret_cast<const void*>(&jw_main64s_kernel<R, false, 2>);
-    return all3 ? reinterpret_cast<const void*>(&jw_main64s_kernel<R, true, 0>)
-                : reinterpret_cast<const void*>(&jw_main64s_kernel<R, false, 0>);
+    return all3 ? reinterpret_cast<const void*>(&jw_main64s_kernel<R, true, 2>)
+                : reinterpret_cast<const void*>(&jw_main64s_kernel<R, false, 2>);
 }
 
-// io: 0 plain step, 1 complex in and out (block layouts 4 and 7), 2 complex in
+// io: 0 plain step (R = 4, 8), 1 complex in and out (block layouts 4 and 7), 2 complex in
 // (layout 4), real systems out
-const void* pick_split(int R, bool all3, int io = 0)
+const void* pick_split(int R, bool all3, int io)
 {
     switch (R) {
-    case 2: return split_ptr<2>(all3, io);
+    case 2: return io ? split_ptr<2>(all3, io) : nullptr;
     case 4: return split_ptr<4>(all3, io);
     case 8: return split_ptr<8>(all3, io);
     default: return nullptr;
@@ -2414,6 +2435,7 @@ thread_local char g_err64[256];
 extern "C" {
 
 int64_t jwdev_table64_elems(int R) { return JW_TAB64_ELEMS(R); }
+int jwdev_main64b_waves(int R);
 
 /* waves per workgroup: as many as LDS (table + 2 systems of staging per wave)
  * and the kernel's launch bound allow */
@@ -2436,17 +2458,13 @@ int64_t jwdev_main64_lds_bytes(int R, int waves)
     return table_lds_bytes(R) + pair_stage_bytes(R) * waves;
 }
 
-/* 1 when the kernel of R rows per lane can build its table in LDS (jwdev_main64 with a source) */
-int jwdev_main64_builds(int R) { return pick64(R, true, true) != NULL; }
-
-/* workgroups per CU, the smallest of the variants (all recurrences or some, table built or copied) */
-int jwdev_main64_occupancy(int R, int waves)
+/* workgroups per CU, the smaller of the two variants (all recurrences / some) */
+static int main64_occupancy(int R, int waves, int lds, bool build)
 {
     int best = -1;
-    for (int v = 0; v < (jwdev_main64_builds(R) ? 4 : 2); v++) {
-        const void* f = pick64(R, v % 2 == 0, v >= 2);
+    for (int v = 0; v < 2; v++) {
+        const void* f = pick64(R, v == 0, build);
         if (!f) return 0;
-        const int lds = (int)jwdev_main64_lds_bytes(R, waves);
         if (hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess) return 0;
         int nb = 0;
         if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, f, 64 * waves, lds) != hipSuccess) return 0;
@@ -2455,22 +2473,65 @@ int jwdev_main64_occupancy(int R, int waves)
     return best;
 }
 
-int jwdev_main64(const jw_run_desc* r, const jw_source_desc* src, const void* matrices, int R, int waves, int grid,
-                 void* stream)
+int jwdev_main64_occupancy(int R, int waves)
 {
-    if (!r->rhs || (src ? !matrices : !r->table)) { snprintf(g_err64, sizeof(g_err64), "main64: no rhs or table"); return -1; }
-    /* the build's partition: 2 rows per thread of a full workgroup, its scratch in the stagings */
-    if (src && waves != jwdev_main64_waves(R)) { snprintf(g_err64, sizeof(g_err64), "main64: bad build shape"); return -1; }
-    const void* f = pick64(R, r->fwd && r->b1 && r->b2, src != NULL);
+    return main64_occupancy(R, waves, (int)jwdev_main64_lds_bytes(R, waves), false);
+}
+
+int jwdev_main64(const jw_run_desc* r, int R, int waves, int grid, void* stream)
+{
+    if (!r->rhs || !r->table) { snprintf(g_err64, sizeof(g_err64), "main64: no rhs or table"); return -1; }
+    const void* f = pick64(R, r->fwd && r->b1 && r->b2);
     if (!f) { snprintf(g_err64, sizeof(g_err64), "no 64-lane kernel for R=%d", R); return -1; }
     const size_t lds = (size_t)jwdev_main64_lds_bytes(R, waves);
     hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) return -2;
-    /* R = 32 takes the descriptor alone (a launch reads the arguments its kernel has) */
+    /* the source and matrices are read by the building variants only (R = 32 has no such arguments) */
     jw_source_desc none;
-    if (!src) memset(&none, 0, sizeof(none));
-    void* args[] = {const_cast<jw_run_desc*>(r), src ? const_cast<jw_source_desc*>(src) : &none, &matrices};
+    memset(&none, 0, sizeof(none));
+    const void* nomat = NULL;
+    void* args[] = {const_cast<jw_run_desc*>(r), &none, &nomat};
     e = hipLaunchKernel(f, dim3(grid), dim3(64 * waves), args, lds, reinterpret_cast<hipStream_t>(stream));
+    return e == hipSuccess ? 0 : -3;
+}
+
+/* the same with the table built in LDS (R <= 16; systems at any 8-byte address): wavefronts
+ * per workgroup (the launch bound), workgroups per CU, launch */
+static int64_t main64b_lds_bytes(int R)
+{
+    return (int64_t)JW_TAB64_ELEMS(R) * 8 + max_i64(512LL * R * jwdev_main64b_waves(R), (int64_t)prologue_lds_bytes(64 * R, 8));
+}
+
+int jwdev_main64b_waves(int R)
+{
+    switch (R) {
+    case 2: return max_threads<2>() / 64;
+    case 4: return max_threads<4>() / 64;
+    case 8: return max_threads<8>() / 64;
+    case 16: return max_threads<16>() / 64;
+    default: return 0;
+    }
+}
+
+int jwdev_main64b_occupancy(int R)
+{
+    const int w = jwdev_main64b_waves(R);
+    return w ? main64_occupancy(R, w, (int)main64b_lds_bytes(R), true) : 0;
+}
+
+int jwdev_main64b(const jw_run_desc* r, const jw_source_desc* src, const void* matrices, int R, int grid, void* stream)
+{
+    const void* f = pick64(R, r->fwd && r->b1 && r->b2, true);
+    if (!r->rhs || !matrices || !f || grid < 1) {
+        snprintf(g_err64, sizeof(g_err64), "main64b: no rhs or matrices, or no kernel for R=%d", R);
+        return -1;
+    }
+    const size_t lds = (size_t)main64b_lds_bytes(R);
+    hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    if (e != hipSuccess) return -2;
+    void* args[] = {const_cast<jw_run_desc*>(r), const_cast<jw_source_desc*>(src), &matrices};
+    e = hipLaunchKernel(f, dim3(grid), dim3(64 * jwdev_main64b_waves(R)), args, lds,
+                        reinterpret_cast<hipStream_t>(stream));
     return e == hipSuccess ? 0 : -3;
 }
 
@@ -2593,13 +2654,18 @@ int jwdev_batch64(const jw_batch_item* d_items, const jw_batch_unit* d_units, in
     return e == hipSuccess ? 0 : -3;
 }
 
-static const void* pick_batch64b(int R)
+static const void* pick_batch64b(int R, int waves)
 {
+    const bool full = waves == max_waves64(R);
     switch (R) {
-    case 2: return reinterpret_cast<const void*>(&jw_batch64b_kernel<2>);
-    case 4: return reinterpret_cast<const void*>(&jw_batch64b_kernel<4>);
-    case 8: return reinterpret_cast<const void*>(&jw_batch64b_kernel<8>);
-    case 16: return reinterpret_cast<const void*>(&jw_batch64b_kernel<16>);
+    case 2: return full ? reinterpret_cast<const void*>(&jw_batch64b_kernel<2, true>)
+                        : reinterpret_cast<const void*>(&jw_batch64b_kernel<2, false>);
+    case 4: return full ? reinterpret_cast<const void*>(&jw_batch64b_kernel<4, true>)
+                        : reinterpret_cast<const void*>(&jw_batch64b_kernel<4, false>);
+    case 8: return full ? reinterpret_cast<const void*>(&jw_batch64b_kernel<8, true>)
+                        : reinterpret_cast<const void*>(&jw_batch64b_kernel<8, false>);
+    case 16: return full ? reinterpret_cast<const void*>(&jw_batch64b_kernel<16, true>)
+                         : reinterpret_cast<const void*>(&jw_batch64b_kernel<16, false>);
     default: return nullptr;
     }
 }
@@ -2607,14 +2673,14 @@ static const void* pick_batch64b(int R)
 /* the table build needs >= 256 threads and 4 threads per 16 rows */
 static bool batch64b_shape_ok(int R, int waves)
 {
-    return pick_batch64b(R) && waves >= 4 && waves <= max_waves64(R) && 4 * 64 * waves >= 64 * R &&
+    return pick_batch64b(R, waves) && waves >= 4 && waves <= max_waves64(R) && 4 * 64 * waves >= 64 * R &&
            batch64b_lds_bytes(R, waves) <= kLdsBytesMax;
 }
 
 int jwdev_batch64b_occupancy(int R, int waves)
 {
     if (!batch64b_shape_ok(R, waves)) return 0;
-    const void* f = pick_batch64b(R);
+    const void* f = pick_batch64b(R, waves);
     const int lds = (int)batch64b_lds_bytes(R, waves);
     if (hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess) return 0;
     int nb = 0;
@@ -2629,7 +2695,7 @@ int jwdev_batch64b(const jw_batch_item* d_items, const jw_batch_unit* d_units, i
         snprintf(g_err64, sizeof(g_err64), "bad build-in-LDS batch launch (R=%d, waves=%d)", R, waves);
         return -1;
     }
-    const void* f = pick_batch64b(R);
+    const void* f = pick_batch64b(R, waves);
     const size_t lds = (size_t)batch64b_lds_bytes(R, waves);
     hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) return -2;
@@ -2746,7 +2812,7 @@ int jwdev_batch64s(const jw_batch_item* d_items, const jw_batch_unit* d_units, i
 /* compute / store split kernel (R <= 8): shape, occupancy, launch */
 int jwdev_main64s_shape(int R, int* ncomp, int* nstore)
 {
-    if (!pick_split(R, true)) return 0;
+    if (!pick_split(R, true, 2)) return 0;
     return split_shape(R, ncomp, nstore) ? 1 : 0;
 }
 
@@ -2766,6 +2832,7 @@ int jwdev_main64s_occupancy(int R)
     int best = -1;
     for (int v = 0; v < 6; v++) {
         const void* f = pick_split(R, (v & 1) == 0, v >> 1);
+        if (!f) continue;
         const int lds = (int)jwdev_main64s_lds_bytes(R, c);
         if (hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess) return 0;
         int nb = 0;
@@ -2782,6 +2849,7 @@ int jwdev_main64s(const jw_run_desc* r, const jw_source_desc* src, const void* m
     int c = 0, st = 0;
     if (!jwdev_main64s_shape(R, &c, &st)) { snprintf(g_err64, sizeof(g_err64), "no split kernel for R=%d", R); return -1; }
     const void* f = pick_split(R, r->fwd && r->b1 && r->b2, (int)r->fused_io);
+    if (!f) { snprintf(g_err64, sizeof(g_err64), "no split kernel for R=%d, I/O %d", R, (int)r->fused_io); return -1; }
     const size_t lds = (size_t)jwdev_main64s_lds_bytes(R, c);
     hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) return -2;

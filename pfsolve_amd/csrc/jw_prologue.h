@@ -63,12 +63,15 @@ constexpr int kMaxRT = 8;     // rows per thread of the pivot scan: a build's ro
 // pivot scan alike), for the MAXJ / MAXRT bounds of a build whose size is known at compile time
 __host__ __device__ constexpr int pro_rows(int RL) { return RL <= 256 ? 1 : (RL + 255) / 256; }
 
-// LDS of prologue_body: 5 arrays of R*L elements (ld -> l -> l', ud -> h -> h', D, E, g)
-// five arrays of RL values; the last (g) is at least 16 values long, since the
-// pivot scan keeps its wavefront totals there before g is written
-__host__ __device__ inline size_t prologue_lds_bytes(int RL, size_t elt)
+// place of row r in prologue_body's LDS arrays (rows stay inside their 32)
+__host__ __device__ __forceinline__ int prologue_at(int r) { return r ^ ((r >> 3) & 31); }
+
+// LDS of prologue_body: four arrays of RL values (the last at least 32 long, since the pivot
+// scan keeps its wavefront totals there) and 24 values of the refinement.  1024 rows: 32 KiB,
+// so four batched builds fit a CU.
+__host__ __device__ constexpr size_t prologue_lds_bytes(int RL, size_t elt)
 {
-    return (4 * (size_t)RL + (RL > 16 ? (size_t)RL : 16)) * elt;
+    return (3 * (size_t)RL + (RL > 32 ? (size_t)RL : 32) + 24) * elt;
 }
 
 // The band coefficients v_{-2..2} of row r of the matvec (zero outside the matrix),
@@ -216,8 +219,28 @@ __device__ __forceinline__ int64_t source_pos(const jw_source_desc& d, int64_t r
 // No pivot hand-over between builds.
 struct NoPivotHooks {
     __device__ void wait_carry(int) const {}
-    template <typename T> __device__ void publish(int, const T*, int) const {}
+    template <typename T> __device__ void publish(int, const T*) const {}
 };
+// Nothing to issue behind the build's loads.
+struct NoAfterLoads {
+    __device__ void operator()() const {}
+};
+
+// DPP moves and readlane of either arithmetic type (lanes without a source receive 0)
+template <int CTRL, int ROWMASK = 0xf>
+__device__ __forceinline__ double lane_move(double v)
+{
+    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, ROWMASK, 0xf, true);
+    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, ROWMASK, 0xf, true);
+    return __hiloint2double(hi, lo);
+}
+template <int CTRL, int ROWMASK = 0xf>
+__device__ __forceinline__ dd lane_move(dd v)
+{
+    return dd_make(lane_move<CTRL, ROWMASK>(v.hi), lane_move<CTRL, ROWMASK>(v.lo));
+}
+__device__ __forceinline__ double lane_read(double v, int lane) { return readlane_d(v, lane); }
+__device__ __forceinline__ dd lane_read(dd v, int lane) { return dd_make(readlane_d(v.hi, lane), readlane_d(v.lo, lane)); }
 
 // One table build.  Local row r of the build is row rb + r of the system.  A build of a
 // long system's later rows (rb > 0) takes from `carry` the pivot of the row before its
@@ -228,14 +251,26 @@ struct NoPivotHooks {
 // tables of consecutive builds continue each other's scaled recurrences).
 // Hooks of a build that hands its pivots on (tridiagonal solves only): wait_carry(tid),
 // called by every thread just before the barrier after which carry[0] is first read, and
-// publish(tid, sg, RL), called by every thread once the g of every row is final in sg.
-// LANE_MAJOR: the rows of a format-2 build go lane-major over the threads (below).  MAXJ,
-// MAXRT: rows per thread at most in the row phases (RL <= MAXJ nthr) and in the pivot scan
-// (RL <= MAXRT NP); smaller bounds keep a small build's per-thread arrays in fewer registers.
-template <typename T, typename H = NoPivotHooks, bool LANE_MAJOR = false, int MAXJ = kProRows, int MAXRT = kMaxRT>
-__device__ __forceinline__ void prologue_body(const jw_source_desc& d, const void* mat, T* table, int L, int R, int format,
-                              unsigned char* smem_raw, int64_t rb = 0, const T* carry = nullptr, int nsub = 1,
-                              const H& hooks = H())
+// publish(tid, g), called by every thread once the g of every row is final (g: the last
+// row's, in LDS).  `after` is called once the build's own loads are issued (FP64): loads
+// issued there return behind them and overlap the build.
+// TP: T*, or a pointer to global memory stated as such.  MAXJ, MAXRT: rows per thread at most in the row phases (RL <= MAXJ nthr) and in the pivot
+// scan (RL <= MAXRT NP); smaller bounds keep a small build's per-thread arrays in fewer
+// registers.
+//
+// The build is a chain of short latencies (one workgroup, every launch of most kernels):
+// what it costs is instructions and memory round trips on one path, not bandwidth.  Hence
+// the row map below, cross-lane moves by DPP instead of ds_bpermute, one division per row
+// on the path of the pivots, and LDS arrays in a swizzled order (prologue_at: rows 1, 8 or 16
+// apart over the lanes meet at most two-way bank conflicts).  Steps before and
+// after this form, whole launches: 1024 systems of 64 rows 10.1 and 7.2 us, 8192 systems of
+// 256 rows (no pivots) 12.3 and 9.4, 16384 of 1000 rows 64.1 and 58.3, the tables of 1024
+// sets of 1024 - 513 rows in one launch 47 and 30.
+template <typename T, int FORMAT, typename H = NoPivotHooks, int MAXJ = kProRows, int MAXRT = kMaxRT,
+          typename F = NoAfterLoads, typename TP>
+__device__ __forceinline__ void prologue_body(const jw_source_desc& d, const void* mat, TP table, int L, int R,
+                                              unsigned char* smem_raw, int64_t rb = 0, const T* carry = nullptr,
+                                              int nsub = 1, const H& hooks = H(), const F& after = F())
 {
     using A = Ar<T>;
     const int RLs = R * L;                 // rows of one table
@@ -247,11 +282,12 @@ __device__ __forceinline__ void prologue_body(const jw_source_desc& d, const voi
         return k * tab_elems + tab_coef(p, rr % R, rr / R, c, R, L);
     };
     const bool has_carry = rb > 0 && carry != nullptr;
-    T* sl = reinterpret_cast<T*>(smem_raw);    // raw ld, then l, then (format 2) l'
-    T* sh = sl + RL;                           // raw ud, then h, then (format 2) h'
-    T* sD = sh + RL;
-    T* sE = sD + RL;
-    T* sg = sE + RL;
+    auto at = [](int r) -> int { return prologue_at(r); };
+    T* sl = reinterpret_cast<T*>(smem_raw);    // raw ld, then l (format 1) or l' (format 2)
+    T* sh = sl + RL;                           // raw ud, then h or h'
+    T* sE = sh + RL;                           // E (format 1) or 1 / D (format 2)
+    T* sg = sE + RL;                           // g = 1 / pivot, then E (format 2)
+    T* sx = sg + (RL > 32 ? RL : 32);          // the refinement's wavefront totals and flag
     const int tid = threadIdx.x;
     const int nthr = blockDim.x;
     const int64_t N = d.N;
@@ -260,24 +296,29 @@ __device__ __forceinline__ void prologue_body(const jw_source_desc& d, const voi
     const bool has_f = d.solve_kind == JW_SOLVE_LOWER || d.solve_kind == JW_SOLVE_TRI;
 
     // phase 1: raw solve coefficients per row (zeros outside the matrix) into LDS,
-    // band coefficients into registers (format 1: straight into the table); row
-    // row_of(j) of thread tid: tid + j nthr (consecutive threads read consecutive rows),
-    // or with LANE_MAJOR (format 2) lane t of wavefront w takes row t R + i of table k,
-    // (k, i) the (w + j nwaves)-th pair, so that a table store of the fold (a coefficient
-    // pair of row-in-lane i over the 64 lanes) writes 1 KiB of consecutive memory: without
-    // bank conflicts for a table in LDS, at the price of loads that stride R rows over the
-    // lanes.  Measured: faster for the split kernel's build (its matrices are read by every
-    // workgroup, from the L2), slower for a build that reads its own matrices from HBM
-    // (batch queue kernel 4, the long-system builds).  A row of RL or more: no row.
-    const int nwv = nthr >> 6;
-    const bool lane_major = LANE_MAJOR && format == 2;
+    // band coefficients into registers (format 1: straight into the table).  Row row_of(j)
+    // of thread tid; RL or more: no row.
+    // Format 1: consecutive threads take consecutive rows.  Format 2: a wavefront takes a
+    // tile of LT table lanes x NI rows-in-lane (LT NI = 64, NI = min(R, 8)), lane l the
+    // row of table lane l mod LT, row-in-lane l / LT.  Its rows are runs of NI consecutive
+    // ones (the natural-order band: few cache lines per load), and 8 neighbouring lanes
+    // write 128 consecutive bytes of the table (no bank conflicts in LDS, whole segments in
+    // memory).  Consecutive rows alone write 16-byte pieces 1 KiB apart, rows R apart alone
+    // read 64 lines per load: each cost the build over 1 us.
+    const int ni2 = FORMAT == 2 ? (R >= 8 ? 3 : (R == 4 ? 2 : 1)) : 0;   // log2 NI
     auto row_of = [&](int j) -> int {
-        if (!lane_major) return tid + j * nthr;
-        const int c = (tid >> 6) + nwv * j;
-        const int k = c / R;
-        return k * RLs + (tid & 63) * R + (c - k * R);
+        if (FORMAT != 2) return tid + j * nthr;
+        const int lt2 = 6 - ni2;
+        const int b = (tid >> 6) + (nthr >> 6) * j;                  // tile: R of them per table
+        const int k = R >= 16 ? b / R : b >> (ni2);                  // R == NI below 16
+        const int bb = b - k * R;
+        const int c = bb & ((1 << ni2) - 1), ib = bb >> ni2;
+        const int t = (c << lt2) + (tid & ((1 << lt2) - 1)), i = (ib << ni2) + ((tid & 63) >> lt2);
+        return k * RLs + t * R + i;
     };
-    T vb[MAXJ][5];
+    // no thread of the wavefront has a j-th row (wavefront-uniform)
+    auto none = [&](int j) -> bool { return FORMAT == 2 ? (tid >> 6) + (nthr >> 6) * j >= RL / 64 : j * nthr >= RL; };
+    T vb[MAXJ][5], Dr[MAXJ], Er[MAXJ];
     // FP64: every row's loads first (rows outside the matrix read row 0's positions and
     // are discarded), then the selects, products and LDS stores, so that a thread's rows
     // cost one round of memory latency.  Double-double loads and finishes row by row (the
@@ -287,10 +328,9 @@ __device__ __forceinline__ void prologue_body(const jw_source_desc& d, const voi
     if constexpr (PRE) {
 #pragma unroll
         for (int j = 0; j < MAXJ; j++) {
+            if (none(j)) continue;
             const int r = row_of(j);
             const int64_t gr = rb + r;
-            // no thread of the wavefront has a row here (wavefront-uniform)
-            if (!lane_major ? j * nthr >= RL : (tid >> 6) + nwv * j >= RL / 64) continue;
             const int64_t gq = (r < RL && gr < N) ? gr : 0;
             const int64_t P = source_pos(d, gq, N);
             sr[j][0] = has_f ? mem_load<T>(mat, d.ldS + P, mf) : A::zero();
@@ -300,53 +340,58 @@ __device__ __forceinline__ void prologue_body(const jw_source_desc& d, const voi
             row_band_load<T>(d, mat, gq, N, P, raw[j]);
         }
     }
-    // format 2 folds D and g of the rows next to the build into its first and last rows:
-    // a build of a long system's rows takes D_{rb-1} and D_{rb+RL} from the matrix
+    // format 2 folds D of the rows next to the build into its first and last rows: a build
+    // of a long system's rows takes D_{rb-1} and D_{rb+RL} from the matrix
     // (every thread reads them: one address each, workgroup-uniform conditions)
     T dprev = A::one(), dnext = A::one();
-    if (format == 2 && d.has_m) {
+    if (FORMAT == 2 && d.has_m) {
         if (rb >= 1 && rb - 1 < N) dprev = mem_load<T>(mat, d.mdM + source_pos(d, rb - 1, N), mf);
         if (rb + RL < N) dnext = mem_load<T>(mat, d.mdM + source_pos(d, rb + RL, N), mf);
     }
+    after();
 #pragma unroll
     for (int j = 0; j < MAXJ; j++) {
         const int r = row_of(j);
         const int64_t gr = rb + r;
-        T ldv = A::zero(), udv = A::zero(), Dv = A::zero(), Ev = A::zero();
+        T ldv = A::zero(), udv = A::zero();
+        Dr[j] = A::zero();
+        Er[j] = A::zero();
 #pragma unroll
         for (int k = 0; k < 5; k++) vb[j][k] = A::zero();
+        if (none(j)) continue;
         if (r < RL && gr < N) {
             if constexpr (PRE) {
                 row_band_finish<T>(d, gr, N, raw[j], vb[j]);
                 ldv = A::sel(gr >= 1, sr[j][0], A::zero());
                 udv = A::sel(gr + 1 < N, sr[j][1], A::zero());
-                Dv = sr[j][2];
-                Ev = A::sel(gr + 1 < N, sr[j][3], A::zero());
+                Dr[j] = sr[j][2];
+                Er[j] = A::sel(gr + 1 < N, sr[j][3], A::zero());
             } else {
                 const int64_t P = source_pos(d, gr, N);
                 // the solve diagonals' loads first (the band's products need its own
                 // loads), all at the row's position, zeroed by selects where the row has no
                 // entry
-                T ldr = A::zero(), udr = A::zero(), Dr = A::one(), Er = A::zero();
+                T ldr = A::zero(), udr = A::zero(), Dv = A::one(), Ev = A::zero();
                 if (has_f) ldr = mem_load<T>(mat, d.ldS + P, mf);
                 if (has_b1) udr = mem_load<T>(mat, d.udS + P, mf);
                 if (d.has_m) {
-                    Dr = mem_load<T>(mat, d.mdM + P, mf);
-                    Er = mem_load<T>(mat, d.udM + P, mf);
+                    Dv = mem_load<T>(mat, d.mdM + P, mf);
+                    Ev = mem_load<T>(mat, d.udM + P, mf);
                 }
                 row_band<T>(d, mat, gr, N, P, vb[j]);
                 ldv = A::sel(gr >= 1, ldr, A::zero());
                 udv = A::sel(gr + 1 < N, udr, A::zero());
-                Dv = Dr;
-                Ev = A::sel(gr + 1 < N, Er, A::zero());
+                Dr[j] = Dv;
+                Er[j] = A::sel(gr + 1 < N, Ev, A::zero());
             }
         }
         if (r < RL) {
-            sl[r] = ldv;
-            sh[r] = udv;
-            sD[r] = Dv;
-            sE[r] = Ev;
-            if (format == 1) {
+            sl[at(r)] = ldv;
+            sh[at(r)] = udv;
+            if constexpr (FORMAT == 1) {
+                sE[at(r)] = Er[j];
+                table[tab1(r, 4, 0)] = Dr[j];
+                table[tab1(r, 4, 1)] = Er[j];
                 table[tab1(r, 0, 0)] = vb[j][0];
                 table[tab1(r, 0, 1)] = vb[j][1];
                 table[tab1(r, 1, 0)] = vb[j][2];
@@ -355,36 +400,44 @@ __device__ __forceinline__ void prologue_body(const jw_source_desc& d, const voi
             }
         }
     }
+    if (tid == 0) sx[16] = A::zero();   // the refinement flag
     __syncthreads();
+    if (FORMAT == 2 && d.has_m) {
+        // 1 / D of the rows (zero past the matrix), for the neighbours' fold
+#pragma unroll
+        for (int j = 0; j < MAXJ; j++) {
+            if (none(j)) continue;
+            const int r = row_of(j);
+            if (r < RL) sE[at(r)] = rb + r < N ? A::div(A::one(), Dr[j]) : A::zero();
+        }
+    }
 
     // phase 2: factors of the unit-diagonal solve.  Pivots p_r = 1 - m_r / p_{r-1},
     // m_r = ld_r ud_{r-1}: the Moebius map p -> (p - m)/p is the 2x2 matrix
     // [[1,-m],[1,0]] on (num, den).  Thread t < NP composes the maps of its RT
-    // consecutive rows; an inclusive scan over those threads (Hillis-Steele in
-    // each wavefront, then the wavefront totals through LDS) gives every thread
-    // the map of all rows before its own, applied to (1,1) the pivot of the row
-    // before its first; each thread then runs the exact recurrence over its rows.
-    // NP depends on the build's rows only (256 up to 2048 rows, one wavefront more per
-    // further 512), so the rounding does not depend on the workgroup size (every kernel
-    // that builds a table gives the same table, bit for bit).
+    // consecutive rows; an inclusive scan over those threads (DPP inside each wavefront,
+    // then the wavefront totals through LDS) gives every thread the map of all rows before
+    // its own, applied to (1,1) the pivot of the row before its first; each thread then
+    // runs the exact recurrence over its rows.
+    // NP depends on the build's rows only (up to 256 threads for 2048 rows, one wavefront
+    // more per further 512), so the rounding does not depend on the workgroup size (every
+    // kernel that builds a table gives the same table, bit for bit).
     if (d.solve_kind == JW_SOLVE_TRI) {
         // participating threads (the workgroup has at least NP)
-        const int NP = RL <= 64 * 4 * kMaxRT ? 256 : (RL + 64 * kMaxRT - 1) / (64 * kMaxRT) * 64;
+        const int NP = RL <= 256 ? (RL + 63) / 64 * 64
+                                 : (RL <= 256 * kMaxRT ? 256 : (RL + 64 * kMaxRT - 1) / (64 * kMaxRT) * 64);
         // the wavefront totals live in g's array, which nothing reads or writes until the
-        // per-row pass below (a barrier keeps that pass after every read): no static LDS,
-        // so four 256-thread builds of 1024 rows fit one CU
+        // per-row pass below (a barrier keeps that pass after every read)
         T* s_tot = sg;
         const int RT = (RL + NP - 1) / NP;
         const int r0 = tid < NP ? tid * RT : RL;   // threads >= NP own no rows
         const int lane = tid & 63, wv = tid >> 6;
-        // the entries are rescaled by a power of two after every product (exact)
+        // the entries rescaled by a power of two (exact), so that no product over- or
+        // underflows: after at most four rows' maps or two scan steps
         auto normalize = [](T& a, T& b, T& c, T& e) {
-            double mx = fmax(fmax(fabs(A::hi(a)), fabs(A::hi(b))), fmax(fabs(A::hi(c)), fabs(A::hi(e))));
-            if (mx > 0.0) {
-                int ex;
-                frexp(mx, &ex);
-                a = A::ldexp_(a, -ex); b = A::ldexp_(b, -ex); c = A::ldexp_(c, -ex); e = A::ldexp_(e, -ex);
-            }
+            const double mx = fmax(fmax(fabs(A::hi(a)), fabs(A::hi(b))), fmax(fabs(A::hi(c)), fabs(A::hi(e))));
+            const int ex = -__builtin_amdgcn_frexp_exp(mx);
+            a = A::ldexp_(a, ex); b = A::ldexp_(b, ex); c = A::ldexp_(c, ex); e = A::ldexp_(e, ex);
         };
         // X <- X * P (P: the maps of earlier rows, applied first)
         auto compose = [&](T& a, T& b, T& c, T& e, T pa, T pb, T pc, T pe) {
@@ -393,37 +446,55 @@ __device__ __forceinline__ void prologue_body(const jw_source_desc& d, const voi
             T nc = A::madd(A::mul(c, pa), e, pc);
             T ne = A::madd(A::mul(c, pb), e, pe);
             a = na; b = nb; c = nc; e = ne;
-            normalize(a, b, c, e);
         };
-        T a = A::one(), b = A::zero(), c = A::zero(), e = A::one();
-        for (int i = 0; i < RT; i++) {
-            const int r = r0 + i;
-            if (r >= RL) break;
-            const int64_t gr = rb + r;
-            T m = A::zero();
-            if (gr >= 1 && gr < N) m = A::mul(sl[r], r >= 1 ? sh[r - 1] : (has_carry ? carry[1] : A::zero()));
-            T na = A::msub(a, m, c), nb = A::msub(b, m, e);
-            c = a;
-            e = b;
-            a = na;
-            b = nb;
-            normalize(a, b, c, e);
-        }
-        // ud of the row before this thread's first, read before any thread
-        // overwrites its ud with h (after the barrier below)
-        T udprev = (r0 >= 1 && r0 < RL) ? sh[r0 - 1] : ((r0 == 0 && has_carry) ? carry[1] : A::zero());
         // the wavefronts past the first NP threads own no rows: they skip the scan
         // (wave-uniform) and only keep the barriers
         const bool part = wv < NP / 64;
-        // inclusive scan inside the wavefront
+        // super-diagonal entry of the row before this thread's first
+        const T udp0 = (r0 >= 1 && r0 < RL) ? sh[at(r0 - 1)] : ((r0 == 0 && has_carry) ? carry[1] : A::zero());
+        T ldv[MAXRT], udv[MAXRT];
+        T a = A::one(), b = A::zero(), c = A::zero(), e = A::one();
         T xa = A::one(), xb = A::zero(), xc = A::zero(), xe = A::one();
         if (part) {
-            for (int k = 0; k < 6; k++) {
-                const int sft = 1 << k;
-                const int src = lane >= sft ? lane - sft : lane;
-                T pa = lane_fetch(a, src), pb = lane_fetch(b, src), pc = lane_fetch(c, src), pe = lane_fetch(e, src);
-                if (lane >= sft) compose(a, b, c, e, pa, pb, pc, pe);
+            T udp = udp0;
+#pragma unroll
+            for (int i = 0; i < MAXRT; i++) {
+                ldv[i] = A::zero();
+                udv[i] = A::zero();
+                const int r = r0 + i;
+                if (i >= RT || r >= RL) continue;
+                ldv[i] = sl[at(r)];
+                udv[i] = sh[at(r)];
+                // (rows outside the matrix and row 0 have no sub-diagonal: m = 0)
+                const T m = A::mul(ldv[i], udp);
+                udp = udv[i];
+                const T na = A::msub(a, m, c), nb = A::msub(b, m, e);
+                c = a;
+                e = b;
+                a = na;
+                b = nb;
+                if ((i & 3) == 3) normalize(a, b, c, e);
             }
+            normalize(a, b, c, e);
+            // inclusive scan inside the wavefront: Hillis-Steele inside 16-lane rows, then
+            // rows 1 and 3 take the ends of rows 0 and 2, rows 2 and 3 the end of row 1
+            const int tr = lane & 15;
+#define JW_SCAN_STEP(CTRL, MASK, ON)                                                                        \
+    do {                                                                                                    \
+        const T pa = lane_move<CTRL, MASK>(a), pb = lane_move<CTRL, MASK>(b);                               \
+        const T pc = lane_move<CTRL, MASK>(c), pe = lane_move<CTRL, MASK>(e);                               \
+        if (ON) compose(a, b, c, e, pa, pb, pc, pe);                                                        \
+    } while (0)
+            JW_SCAN_STEP(DPP_ROW_SHR(1), 0xf, tr >= 1);
+            JW_SCAN_STEP(DPP_ROW_SHR(2), 0xf, tr >= 2);
+            normalize(a, b, c, e);
+            JW_SCAN_STEP(DPP_ROW_SHR(4), 0xf, tr >= 4);
+            JW_SCAN_STEP(DPP_ROW_SHR(8), 0xf, tr >= 8);
+            normalize(a, b, c, e);
+            JW_SCAN_STEP(0x142 /* row_bcast15 */, 0xa, lane & 16);
+            JW_SCAN_STEP(0x143 /* row_bcast31 */, 0xc, lane & 32);
+            normalize(a, b, c, e);
+#undef JW_SCAN_STEP
             if (lane == 63) {
                 s_tot[4 * wv + 0] = a;
                 s_tot[4 * wv + 1] = b;
@@ -431,70 +502,61 @@ __device__ __forceinline__ void prologue_body(const jw_source_desc& d, const voi
                 s_tot[4 * wv + 3] = e;
             }
             // this thread's exclusive map within the wavefront (lane - 1's inclusive)
-            const int src = lane >= 1 ? lane - 1 : lane;
-            xa = lane_fetch(a, src);
-            xb = lane_fetch(b, src);
-            xc = lane_fetch(c, src);
-            xe = lane_fetch(e, src);
+            xa = lane_move<DPP_WAVE_SHR1>(a);
+            xb = lane_move<DPP_WAVE_SHR1>(b);
+            xc = lane_move<DPP_WAVE_SHR1>(c);
+            xe = lane_move<DPP_WAVE_SHR1>(e);
             if (lane == 0) {
                 xa = A::one(); xb = A::zero(); xc = A::zero(); xe = A::one();
             }
         }
         __syncthreads();   // the wavefront totals are in LDS
-        if (part) {
+        if (part && wv > 0) {
             // the maps of all earlier wavefronts, then the in-wavefront part on top (none of
             // it depends on a carry, so a build that waits for one has it ready)
-            T wa = A::one(), wb = A::zero(), wc = A::zero(), we = A::one();
-            for (int w = 0; w < wv; w++) {
+            T wa = s_tot[0], wb = s_tot[1], wc = s_tot[2], we = s_tot[3];
+            for (int w = 1; w < wv; w++) {
                 T ta = s_tot[4 * w + 0], tb = s_tot[4 * w + 1], tc = s_tot[4 * w + 2], te = s_tot[4 * w + 3];
                 compose(ta, tb, tc, te, wa, wb, wc, we);
                 wa = ta; wb = tb; wc = tc; we = te;
+                normalize(wa, wb, wc, we);
             }
             compose(xa, xb, xc, xe, wa, wb, wc, we);
+            normalize(xa, xb, xc, xe);
         }
         hooks.wait_carry(tid);
         __syncthreads();   // the carry is in LDS, the totals are read: g's array is free
-        T gprev = A::one();
+        // first pass over this thread's rows.  The prefix map applied to (1, 1) (the first
+        // row has no sub-diagonal, so any start works), or after a carry to (1, g_in), gives
+        // the pivot of the row before as num / den, so the first row's pivot is
+        // (num - m den) / num: its g and p by two independent divisions; the others by the
+        // exact recurrence p_r = 1 - ld_r ud_{r-1} g_{r-1},  g_r = 1 / p_r.
+        T pr[MAXRT];
         if (part) {
-            // g_{r-1} = 1 / p_{r-1} of the row before this thread's first: the prefix map
-            // applied to (1, 1) (the first row has no sub-diagonal, so any start works), or
-            // after a carry to (1, g_in), i.e. p = 1 / g_in
-            if (has_carry) {
-                const T gin = carry[0];
-                gprev = A::div(A::madd(xc, xe, gin), A::madd(xa, xb, gin));
-            } else if (r0 >= 1) {
-                gprev = A::div(A::add(xc, xe), A::add(xa, xb));
-            }
-        }
-        // first pass: the exact recurrence over this thread's rows from the scanned pivot;
-        // the rows' ld / ud stay in registers (nothing reads another thread's raw ld again)
-        T pr[MAXRT], ldv[MAXRT], udv[MAXRT];
-        const T udp0 = udprev;
-        if (part) {
+            const T gin = has_carry ? carry[0] : A::one();
+            const T num = A::madd(xa, xb, gin), den = A::madd(xc, xe, gin);
+            T gprev = A::one(), udprev = udp0;
 #pragma unroll
             for (int i = 0; i < MAXRT; i++) {
                 pr[i] = A::one();
-                ldv[i] = A::zero();
-                udv[i] = A::zero();
                 const int r = r0 + i;
                 if (i >= RT || r >= RL) continue;
-                ldv[i] = sl[r];
-                udv[i] = sh[r];
                 T g = A::zero();
                 if (rb + r < N) {
-                    // p_r = 1 - ld_r ud_{r-1} / p_{r-1},  g_r = 1/p_r
-                    const T l = (rb + r >= 1) ? A::mul(ldv[i], gprev) : A::zero();
-                    pr[i] = A::sub(A::one(), A::mul(l, udprev));
-                    g = A::div(A::one(), pr[i]);
+                    if (i == 0) {
+                        const T q = A::msub(num, A::mul(ldv[0], udprev), den);
+                        g = A::div(num, q);
+                        pr[0] = A::div(q, num);
+                    } else {
+                        pr[i] = A::msub(A::one(), A::mul(ldv[i], gprev), udprev);
+                        g = A::div(A::one(), pr[i]);
+                    }
                     gprev = g;
                 }
                 udprev = udv[i];
-                sg[r] = g;
+                sg[at(r)] = g;
             }
         }
-        // sh[0] becomes the refinement flag: its raw ud is in thread 0's registers by now,
-        // and the one other reader (the next thread's udprev) read it before the scan
-        if (tid == 0) sh[0] = A::zero();
         __syncthreads();   // every first-pass g is in sg
 
         // Refinement.  Near a parabolic fixed point of the pivot map (m_r -> 1/4, e.g. the
@@ -512,135 +574,123 @@ __device__ __forceinline__ void prologue_body(const jw_source_desc& d, const voi
         // and a function of the matrix alone, so every kernel still builds the same table).
         if (part && r0 >= 1 && rb + r0 < N) {
             const double tol = sizeof(T) == 8 ? 0x1p-51 : 0x1p-103;
-            const T rho0 = A::add(A::sub(pr[0], A::one()), A::mul(A::mul(ldv[0], udp0), sg[r0 - 1]));
-            if (!(fabs(A::hi(rho0)) <= tol * fabs(A::hi(pr[0])))) sh[0] = A::one();
+            const T rho0 = A::add(A::sub(pr[0], A::one()), A::mul(A::mul(ldv[0], udp0), sg[at(r0 - 1)]));
+            if (!(fabs(A::hi(rho0)) <= tol * fabs(A::hi(pr[0])))) sx[16] = A::one();
         }
         __syncthreads();
-        const bool refine = A::hi(sh[0]) != 0.0;
+        const bool refine = A::hi(sx[16]) != 0.0;
         // not refined: every first-pass g is final (in sg since the barrier before the
         // check), so the last one goes to the next build at once
-        if (!refine) hooks.publish(tid, sg, RL);
-        T rho[MAXRT], cc[MAXRT];
-        T sc = A::one(), ss = A::zero();      // this thread's map e -> sc e + ss
-        if (refine && part) {
-            T gm = (r0 >= 1 && r0 < RL) ? sg[r0 - 1] : ((r0 == 0 && has_carry) ? carry[0] : A::one());
-            udprev = udp0;
+        if (!refine) hooks.publish(tid, sg + at(RL - 1));
+        if (refine) {
+            T rho[MAXRT], cc[MAXRT];
+            T sc = A::one(), ss = A::zero();      // this thread's map e -> sc e + ss
+            if (part) {
+                T gm = (r0 >= 1 && r0 < RL) ? sg[at(r0 - 1)] : ((r0 == 0 && has_carry) ? carry[0] : A::one());
+                T udprev = udp0;
 #pragma unroll
-            for (int i = 0; i < MAXRT; i++) {
-                rho[i] = A::zero();
-                cc[i] = A::zero();
-                const int r = r0 + i;
-                if (i >= RT || rb + r >= N) continue;
-                const T m = (rb + r >= 1) ? A::mul(ldv[i], udprev) : A::zero();
-                const T mg = A::mul(m, gm);
-                rho[i] = A::add(A::sub(pr[i], A::one()), mg);
-                cc[i] = A::mul(mg, gm);
-                ss = A::madd(rho[i], cc[i], ss);
-                sc = A::mul(cc[i], sc);
-                gm = sg[r];
-                udprev = udv[i];
+                for (int i = 0; i < MAXRT; i++) {
+                    rho[i] = A::zero();
+                    cc[i] = A::zero();
+                    const int r = r0 + i;
+                    if (i >= RT || rb + r >= N) continue;
+                    const T m = (rb + r >= 1) ? A::mul(ldv[i], udprev) : A::zero();
+                    const T mg = A::mul(m, gm);
+                    rho[i] = A::add(A::sub(pr[i], A::one()), mg);
+                    cc[i] = A::mul(mg, gm);
+                    ss = A::madd(rho[i], cc[i], ss);
+                    sc = A::mul(cc[i], sc);
+                    gm = sg[at(r)];
+                    udprev = udv[i];
+                }
+                // inclusive scan of the maps inside the wavefront, wavefront totals to LDS
+                for (int k = 0; k < 6; k++) {
+                    const int sft = 1 << k;
+                    const int src = lane >= sft ? lane - sft : lane;
+                    const T pc = lane_fetch(sc, src), ps = lane_fetch(ss, src);
+                    if (lane >= sft) {
+                        ss = A::madd(ss, sc, ps);
+                        sc = A::mul(sc, pc);
+                    }
+                }
+                if (lane == 63) {
+                    sx[2 * wv] = sc;
+                    sx[2 * wv + 1] = ss;
+                }
+                const int src = lane >= 1 ? lane - 1 : lane;
+                const T xs = lane_fetch(ss, src), xk = lane_fetch(sc, src);
+                ss = lane == 0 ? A::zero() : xs;
+                sc = lane == 0 ? A::one() : xk;
             }
-            // inclusive scan of the maps inside the wavefront, wavefront totals to LDS
-            // (sl's first 8 values: every thread holds its raw ld in registers by now)
-            for (int k = 0; k < 6; k++) {
-                const int sft = 1 << k;
-                const int src = lane >= sft ? lane - sft : lane;
-                const T pc = lane_fetch(sc, src), ps = lane_fetch(ss, src);
-                if (lane >= sft) {
-                    ss = A::madd(ss, sc, ps);
-                    sc = A::mul(sc, pc);
+            __syncthreads();
+            if (part) {
+                // error entering this thread's first row: earlier wavefronts' maps, then this
+                // wavefront's exclusive part, applied to e = 0
+                T ein = A::zero();
+                for (int w = 0; w < wv; w++) ein = A::madd(sx[2 * w + 1], sx[2 * w], ein);
+                ein = A::madd(ss, sc, ein);
+#pragma unroll
+                for (int i = 0; i < MAXRT; i++) {
+                    const int r = r0 + i;
+                    if (i >= RT || rb + r >= N) continue;
+                    ein = A::madd(rho[i], cc[i], ein);
+                    // a correction that is not finite (no dominance, products out of range)
+                    // is not applied
+                    const double eh = A::hi(ein);
+                    const T p = (eh - eh == 0.0) ? A::sub(pr[i], ein) : pr[i];
+                    sg[at(r)] = A::div(A::one(), p);
                 }
             }
-            if (lane == 63) {
-                sl[2 * wv] = sc;
-                sl[2 * wv + 1] = ss;
-            }
-            const int src = lane >= 1 ? lane - 1 : lane;
-            const T xs = lane_fetch(ss, src), xc = lane_fetch(sc, src);
-            ss = lane == 0 ? A::zero() : xs;
-            sc = lane == 0 ? A::one() : xc;
-        }
-        if (refine) __syncthreads();
-        if (refine && part) {
-            // error entering this thread's first row: earlier wavefronts' maps, then this
-            // wavefront's exclusive part, applied to e = 0
-            T ein = A::zero();
-            for (int w = 0; w < wv; w++) ein = A::madd(sl[2 * w + 1], sl[2 * w], ein);
-            ein = A::madd(ss, sc, ein);
-#pragma unroll
-            for (int i = 0; i < MAXRT; i++) {
-                const int r = r0 + i;
-                if (i >= RT || rb + r >= N) continue;
-                ein = A::madd(rho[i], cc[i], ein);
-                // a correction that is not finite (no dominance, products out of range)
-                // is not applied
-                const double eh = A::hi(ein);
-                const T p = (eh - eh == 0.0) ? A::sub(pr[i], ein) : pr[i];
-                sg[r] = A::div(A::one(), p);
-            }
-        }
-        // refined: the corrected g of every row (and of the row before) is in sg; not
-        // refined: every thread has read the flag before thread 0 writes h_0 over it
-        __syncthreads();
-        if (refine) hooks.publish(tid, sg, RL);
-        if (part) {
-#pragma unroll
-            for (int i = 0; i < MAXRT; i++) {
-                const int r = r0 + i;
-                if (i >= RT || r >= RL) continue;
-                // l_r = ld_r g_{r-1},  h_r = ud_r g_r  (zero outside the matrix)
-                T l = A::zero(), h = A::zero();
-                if (rb + r < N) {
-                    if (rb + r >= 1) l = A::mul(ldv[i], r >= 1 ? sg[r - 1] : (has_carry ? carry[0] : A::zero()));
-                    h = A::mul(udv[i], sg[r]);
-                }
-                sl[r] = l;
-                sh[r] = h;
-            }
+            // the corrected g of every row is in sg
+            __syncthreads();
+            hooks.publish(tid, sg + at(RL - 1));
         }
     } else {
-        for (int r = tid; r < RL; r += nthr) {
-            const bool in = rb + r < N;
-            if (!(in && d.solve_kind == JW_SOLVE_LOWER)) sl[r] = A::zero();
-            sg[r] = in ? A::one() : A::zero();
-            if (!(in && d.solve_kind == JW_SOLVE_UPPER)) sh[r] = A::zero();
-        }
+        for (int r = tid; r < RL; r += nthr) sg[at(r)] = rb + r < N ? A::one() : A::zero();
+        __syncthreads();
     }
-    __syncthreads();
 
-    if (format == 2) {
-        // nsub tables of 64 R rows each, JW_TAB64_ELEMS(R) apart; in a build of a long
-        // system's rows the first row's l' and the last row's h' take a and D of the rows
-        // next to the build (g_{rb-1} from the carry of a tridiagonal solve, else 1)
+    if constexpr (FORMAT == 2) {
+        // nsub tables of 64 R rows each, JW_TAB64_ELEMS(R) apart, the scalings folded:
+        // with l_r = ld_r g_{r-1}, h_r = ud_r g_r and a_r = D_r g_r,
+        //   l'_r = a_r l_r / a_{r-1} = a_r ld_r / D_{r-1},  h'_r = D_r h_r / D_{r+1} = a_r ud_r / D_{r+1}
+        // (a build's first and last rows take D of the rows next to the build).  l', h' and
+        // E then replace ld, ud and g in LDS (a row reads only its own of those).
         const int64_t te2 = JW_TAB64_ELEMS(R);
-        const T aprev = A::mul(dprev, has_carry ? carry[0] : A::one());
-        // fold the scalings (row-parallel); l' and h' replace l and h in LDS (a row
-        // reads only its own l and h)
+        const T iprev = d.has_m && rb >= 1 ? A::div(A::one(), dprev) : A::one();
+        const T inext = d.has_m && rb + RL < N ? A::div(A::one(), dnext) : A::one();
 #pragma unroll
         for (int j = 0; j < MAXJ; j++) {
+            if (none(j)) continue;
             const int r = row_of(j);
             if (r >= RL) continue;
-            const int kt = r / RLs, rr = r - kt * RLs;
+            const int kt = nsub > 1 ? r / RLs : 0, rr = r - kt * RLs;
             const int t = rr / R, i = rr % R;
-            const T ar = A::mul(sD[r], sg[r]);
+            const T ar = A::mul(Dr[j], sg[at(r)]);
             T cf[8];
 #pragma unroll
             for (int k = 0; k < 5; k++) cf[k] = A::mul(ar, vb[j][k]);
             T lp = A::zero(), hp = A::zero();
-            if (rb + r >= 1 && rb + r < N)
-                lp = A::div(A::mul(ar, sl[r]), r >= 1 ? A::mul(sD[r - 1], sg[r - 1]) : aprev);
-            if (rb + r + 1 < N) hp = A::div(A::mul(sD[r], sh[r]), r + 1 < RL ? sD[r + 1] : dnext);
+            if (rb + r >= 1 && rb + r < N) {
+                lp = A::mul(ar, sl[at(r)]);
+                if (d.has_m) lp = A::mul(lp, r >= 1 ? sE[at(r - 1)] : iprev);
+            }
+            if (rb + r + 1 < N) {
+                hp = A::mul(ar, sh[at(r)]);
+                if (d.has_m) hp = A::mul(hp, r + 1 < RL ? sE[at(r + 1)] : inext);
+            }
             cf[5] = lp;
             cf[6] = hp;
-            cf[7] = sE[r];
-            T* tk = table + kt * te2;
+            cf[7] = Er[j];
+            const TP tk = table + kt * te2;
 #pragma unroll
             for (int p = 0; p < 4; p++) {
                 tk[tab_coef64(p, i, t, R)] = cf[2 * p];
                 tk[tab_coef64(p, i, t, R) + 1] = cf[2 * p + 1];
             }
-            sl[r] = lp;
-            sh[r] = hp;
+            sl[at(r)] = lp;
+            sh[at(r)] = hp;
+            sg[at(r)] = Er[j];
         }
         __syncthreads();
         // scan multipliers: wavefront item (wave-uniform) takes recurrence j = item % 3
@@ -649,101 +699,120 @@ __device__ __forceinline__ void prologue_body(const jw_source_desc& d, const voi
         for (int item = tid >> 6; item < 3 * nsub; item += nthr >> 6) {
             const int kt = item / 3, j = item - 3 * kt;
             const int t = tid & 63;
-            T* const tabk = table + kt * te2;
-            const T* src = (j == 0 ? sl : (j == 1 ? sh : sE)) + kt * RLs;
+            const TP tabk = table + kt * te2;
+            const T* src = j == 0 ? sl : (j == 1 ? sh : sg);
             T v = A::one();
-            for (int i = 0; i < R; i++) v = A::mul(v, A::neg(src[t * R + i]));
+            for (int i = 0; i < R; i++) v = A::mul(v, A::neg(src[at(kt * RLs + t * R + i)]));
             // in-row Hillis-Steele: before step k the value covers the 2^k lanes a
             // shift of 2^k combines; after 4 steps, the row prefix (j = 0) or suffix
             const int tr = t & 15;
-            const int64_t SC = (int64_t)8 * R * 64;
-#pragma unroll
-            for (int k = 0; k < 4; k++) {
-                const int s = 1 << k;
-                tabk[SC + (int64_t)(j * 8 + k) * 64 + t] = v;
-                if (j == 0) {
-                    const T up = lane_fetch(v, tr >= s ? t - s : t);
-                    if (tr >= s) v = A::mul(v, up);
-                } else {
-                    const T dn = lane_fetch(v, tr + s <= 15 ? t + s : t);
-                    if (tr + s <= 15) v = A::mul(v, dn);
-                }
+            const TP m = tabk + (int64_t)8 * R * 64 + (int64_t)j * 8 * 64 + t;
+            if (j == 0) {
+                m[0] = v;
+                T u = lane_move<DPP_ROW_SHR(1)>(v);
+                if (tr >= 1) v = A::mul(v, u);
+                m[64] = v;
+                u = lane_move<DPP_ROW_SHR(2)>(v);
+                if (tr >= 2) v = A::mul(v, u);
+                m[128] = v;
+                u = lane_move<DPP_ROW_SHR(4)>(v);
+                if (tr >= 4) v = A::mul(v, u);
+                m[192] = v;
+                u = lane_move<DPP_ROW_SHR(8)>(v);
+                if (tr >= 8) v = A::mul(v, u);
+            } else {
+                m[0] = v;
+                T u = lane_move<DPP_ROW_SHL(1)>(v);
+                if (tr + 1 <= 15) v = A::mul(v, u);
+                m[64] = v;
+                u = lane_move<DPP_ROW_SHL(2)>(v);
+                if (tr + 2 <= 15) v = A::mul(v, u);
+                m[128] = v;
+                u = lane_move<DPP_ROW_SHL(4)>(v);
+                if (tr + 4 <= 15) v = A::mul(v, u);
+                m[192] = v;
+                u = lane_move<DPP_ROW_SHL(8)>(v);
+                if (tr + 8 <= 15) v = A::mul(v, u);
             }
             const int rw = t >> 4;
             if (j == 0) {
                 // forward cross-row combine in two broadcasts: rows 1,3 take the end of
                 // rows 0,2 (multiplier: row prefix), then rows 2,3 take lane 31, which
                 // row 3 reaches through all of row 2 (prefix of lane 47 times its own)
-                const T pre47 = lane_fetch(v, 47);
+                const T pre47 = lane_read(v, 47);
                 T m2 = A::zero();
                 if (rw == 2) m2 = v;
                 if (rw == 3) m2 = A::mul(pre47, v);
-                tabk[SC + (int64_t)4 * 64 + t] = v;
-                tabk[SC + (int64_t)5 * 64 + t] = m2;
-                tabk[SC + (int64_t)6 * 64 + t] = A::zero();
-                tabk[SC + (int64_t)7 * 64 + t] = A::zero();
+                m[256] = v;
+                m[320] = m2;
+                m[384] = A::zero();
+                m[448] = A::zero();
             } else {
                 // backward cross-row combine from the in-row results S_1..S_3 at the
                 // row starts (lanes 16, 32, 48): a lane of row r adds
                 //   suf_t * F_{r+1},  F_q = S_q + P_q F_{q+1},  P_q = suffix product of lane 16q,
                 // i.e. c_k,t * S_k with c_k,t = suf_t * prod_{r<q<k} P_q for k > r, else 0
-                const T P1 = lane_fetch(v, 16), P2 = lane_fetch(v, 32);
+                const T P1 = lane_read(v, 16), P2 = lane_read(v, 32);
                 T c1 = A::zero(), c2 = A::zero(), c3 = A::zero();
                 if (rw == 0) { c1 = v; c2 = A::mul(v, P1); c3 = A::mul(c2, P2); }
                 if (rw == 1) { c2 = v; c3 = A::mul(v, P2); }
                 if (rw == 2) c3 = v;
-                tabk[SC + (int64_t)(j * 8 + 4) * 64 + t] = c1;
-                tabk[SC + (int64_t)(j * 8 + 5) * 64 + t] = c2;
-                tabk[SC + (int64_t)(j * 8 + 6) * 64 + t] = c3;
-                tabk[SC + (int64_t)(j * 8 + 7) * 64 + t] = A::zero();
+                m[256] = c1;
+                m[320] = c2;
+                m[384] = c3;
+                m[448] = A::zero();
             }
         }
-        return;
-    }
-
-    // format 1: pairs (vm2,vm1) (v0,vp1) (vp2,l) (g,h) (D,E) + Hillis-Steele multipliers
-    // (the band pairs were written in phase 1)
-    for (int r = tid; r < RL; r += nthr) {
-        table[tab1(r, 2, 1)] = sl[r];
-        table[tab1(r, 3, 0)] = sg[r];
-        table[tab1(r, 3, 1)] = sh[r];
-        table[tab1(r, 4, 0)] = sD[r];
-        table[tab1(r, 4, 1)] = sE[r];
-    }
-    // scan multipliers: wavefront k (wave-uniform) takes table k
-    if ((tid >> 6) < nsub) {
-        const int kt = tid >> 6;
-        const int t = tid & 63;
-        T* const tabk = table + kt * tab_elems;
-        const int rbase = kt * RLs;
-        const bool active = t < L;
-        const int log2L = ilog2_rt(L);
-        T bf = A::one(), bb1 = A::one(), bb2 = A::one();
-        if (active) {
-            for (int i = 0; i < R; i++) {
-                const int r = rbase + t * R + i;
-                bf = A::mul(bf, A::neg(sl[r]));
-                bb1 = A::mul(bb1, A::neg(sh[r]));
-                bb2 = A::mul(bb2, A::neg(sE[r]));
-            }
+    } else {
+        // format 1: pairs (vm2,vm1) (v0,vp1) (vp2,l) (g,h) (D,E) + Hillis-Steele multipliers
+        // (the band and D, E pairs were written in phase 1)
+        for (int r = tid; r < RL; r += nthr) {
+            // l_r = ld_r g_{r-1},  h_r = ud_r g_r  (zero outside the matrix)
+            const T gm = r >= 1 ? sg[at(r - 1)] : (has_carry ? carry[0] : A::one());
+            const T l = rb + r < N ? A::mul(sl[at(r)], gm) : A::zero();
+            const T h = rb + r < N ? A::mul(sh[at(r)], sg[at(r)]) : A::zero();
+            sl[at(r)] = l;
+            sh[at(r)] = h;
+            table[tab1(r, 2, 1)] = l;
+            table[tab1(r, 3, 0)] = sg[at(r)];
+            table[tab1(r, 3, 1)] = h;
         }
-        for (int k = 0; k < log2L; k++) {
-            const int s = 1 << k;
+        __syncthreads();
+        // scan multipliers: wavefront k (wave-uniform) takes table k
+        if ((tid >> 6) < nsub) {
+            const int kt = tid >> 6;
+            const int t = tid & 63;
+            const TP tabk = table + kt * tab_elems;
+            const int rbase = kt * RLs;
+            const bool active = t < L;
+            const int log2L = ilog2_rt(L);
+            T bf = A::one(), bb1 = A::one(), bb2 = A::one();
             if (active) {
-                tabk[tab_scan(k, t, 0, R, L)] = bf;
-                tabk[tab_scan(k, t, 1, R, L)] = bb1;
-                tabk[tab_scan(k, t, 2, R, L)] = bb2;
-                tabk[tab_scan(k, t, 3, R, L)] = A::zero();
+                for (int i = 0; i < R; i++) {
+                    const int r = at(rbase + t * R + i);
+                    bf = A::mul(bf, A::neg(sl[r]));
+                    bb1 = A::mul(bb1, A::neg(sh[r]));
+                    bb2 = A::mul(bb2, A::neg(sE[r]));
+                }
             }
-            const int su = (t >= s) ? t - s : t;
-            const int sdn = (t + s < L) ? t + s : t;
-            T ubf = lane_fetch(bf, su);
-            T ub1 = lane_fetch(bb1, sdn);
-            T ub2 = lane_fetch(bb2, sdn);
-            if (active && t >= s) bf = A::mul(bf, ubf);
-            if (active && t + s < L) {
-                bb1 = A::mul(bb1, ub1);
-                bb2 = A::mul(bb2, ub2);
+            for (int k = 0; k < log2L; k++) {
+                const int s = 1 << k;
+                if (active) {
+                    tabk[tab_scan(k, t, 0, R, L)] = bf;
+                    tabk[tab_scan(k, t, 1, R, L)] = bb1;
+                    tabk[tab_scan(k, t, 2, R, L)] = bb2;
+                    tabk[tab_scan(k, t, 3, R, L)] = A::zero();
+                }
+                const int su = (t >= s) ? t - s : t;
+                const int sdn = (t + s < L) ? t + s : t;
+                T ubf = lane_fetch(bf, su);
+                T ub1 = lane_fetch(bb1, sdn);
+                T ub2 = lane_fetch(bb2, sdn);
+                if (active && t >= s) bf = A::mul(bf, ubf);
+                if (active && t + s < L) {
+                    bb1 = A::mul(bb1, ub1);
+                    bb2 = A::mul(bb2, ub2);
+                }
             }
         }
     }
@@ -778,10 +847,10 @@ struct ChainHooks {
         }
         carry[0] = ok ? gval[build - 1] : Ar<T>::one();
     }
-    __device__ void publish(int tid, const T* sg, int RL) const
+    __device__ void publish(int tid, const T* g) const
     {
         if (!chained || tid != 0) return;
-        gval[build] = sg[RL - 1];
+        gval[build] = *g;
         __hip_atomic_store(&flags[build], 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
     }
 };

@@ -238,6 +238,9 @@ static PfSolveResult plan_setup(PfSolveApplication* app, struct pfsolve_plan* p)
                 p->waves64 = jwdev_main64_waves(r64);
                 p->occupancy64 = p->waves64 ? jwdev_main64_occupancy(r64, p->waves64) : 0;
                 if (p->occupancy64 < 1) p->R64 = 0;
+                p->waves64b = jwdev_main64b_waves(r64);
+                p->occupancy64b = p->waves64b ? jwdev_main64b_occupancy(r64) : 0;
+                if (p->occupancy64b < 1) p->waves64b = 0;
             }
             if (p->R64) {
                 size_t b2 = (size_t)jwdev_table64_elems(p->R64) * 8;
@@ -614,6 +617,23 @@ static PfSolveResult append_long(PfSolveApplication* app, const jw_source_desc* 
     return PFSOLVE_SUCCESS;
 }
 
+/* Which of the kernels that build their table in LDS takes npass pairs, with cap_* wavefronts
+ * (pairs per sweep of the grid): the compute / store split, or the plain one, which has more
+ * wavefronts per CU (R = 4: 16 against 12, R = 8: 12 against 8) and stores from each.  R = 16
+ * and R = 2: the plain one (N = 64: 1024 systems 7.2 against 7.5 us, 8192 7.7 / 9.4, 131072
+ * 39.3 / 39.8; N = 128: 131072 47.2 / 53.9).  Otherwise the split, whose store acknowledgements
+ * hold nobody up (N = 256, 131072 systems: 88.4 against 91.5 us; N = 512: 184 / 192), but where
+ * the plain one saves a sweep of few (R = 4, up to three sweeps: N = 256, 8192 systems 10.5 /
+ * 12.9 us, 16384 14.6 / 16.1, 24576 20.5 / 22.2; R = 8, one sweep instead of two: N = 512, 6144
+ * systems 13.6 / 15.2; two instead of three measured the same). */
+static int use_build_kernel(const struct pfsolve_plan* p, int64_t npass, int64_t cap_split, int64_t cap_build)
+{
+    if (!p->waves64b) return 0;
+    if (!p->split64 || p->R64 == 2) return 1;
+    const int64_t sweeps_split = (npass + cap_split - 1) / cap_split, sweeps_build = (npass + cap_build - 1) / cap_build;
+    return sweeps_build < sweeps_split && sweeps_build <= (p->R64 == 4 ? 3 : 1);
+}
+
 static PfSolveResult append_impl(PfSolveApplication* app, const PfSolveLaunchParams* lp, uint64_t slot)
 {
     struct pfsolve_plan* p = app->localFFTPlan;
@@ -662,30 +682,36 @@ static PfSolveResult append_impl(PfSolveApplication* app, const PfSolveLaunchPar
         if (p->long_only) return append_long(app, &src, &run, s, table);
         const uintptr_t base = (uintptr_t)run.rhs;
         run.vec2 = p->precision == JW_PREC_F64 && (base % 16) == 0 && (run.stride % 2) == 0 && (run.offSol % 2) == 0;
-        const int in_lds = p->split64 || jwdev_main64_builds(p->R64);
+        const int in_lds = p->split64 || p->waves64b;
         if (p->R64 && (run.vec2 || (in_lds && base % 8 == 0)) && cfg->kernelVariant != 1) {
-            /* wave-per-system kernel: table format 2, built by every workgroup in LDS (N <=
+            /* wave-per-system kernels: table format 2, built by every workgroup in LDS (N <=
              * 1024) or by a launch before.  The kernels that build in LDS load and store
              * global memory from registers and take systems at any 8-byte address (30000
              * systems of 333 rows, packed: 41.4 us a step, 61.8 us on the general kernel and
              * its table launch); the other stages by LDS DMA, 16-byte aligned */
             if (nsys <= 0) return PFSOLVE_SUCCESS;
-            if (!in_lds && jwdev_prologue(&src, cfg->buffer[0], table, 64, p->R64, p->precision, 2, s) != 0)
-                return PFSOLVE_ERROR_FAILED_TO_LAUNCH_KERNEL;
             /* wavefront passes: pairs of systems, single systems for R = 32 */
             const int64_t npass = p->R64 == 32 ? nsys : (nsys + 1) / 2;
-            const int per_wg = p->split64 ? p->split64 : p->waves64;
+            const int64_t cap_split = (int64_t)p->cu_count * p->occupancy_split * p->split64;
+            const int64_t cap_build = (int64_t)p->cu_count * p->occupancy64b * p->waves64b;
+            const int build = use_build_kernel(p, npass, cap_split, cap_build);
+            if (!in_lds && jwdev_prologue(&src, cfg->buffer[0], table, 64, p->R64, p->precision, 2, s) != 0)
+                return PFSOLVE_ERROR_FAILED_TO_LAUNCH_KERNEL;
+            const int per_wg = build ? p->waves64b : (p->split64 ? p->split64 : p->waves64);
             int64_t need = (npass + per_wg - 1) / per_wg;
-            int64_t grid = (int64_t)p->cu_count * (p->split64 ? p->occupancy_split : p->occupancy64);
+            int64_t grid = (int64_t)p->cu_count *
+                           (build ? p->occupancy64b : (p->split64 ? p->occupancy_split : p->occupancy64));
             if (grid > need) grid = need;
             if (grid < 1) grid = 1;
             if (p->ev_start && hipEventRecord(p->ev_start, s) != hipSuccess) return PFSOLVE_ERROR_FAILED_TO_EVENT_RECORD;
-            if (p->split64) {
+            if (build) {
+                if (jwdev_main64b(&run, &src, cfg->buffer[0], p->R64, (int)grid, s) != 0)
+                    return PFSOLVE_ERROR_FAILED_TO_LAUNCH_KERNEL;
+            } else if (p->split64) {
                 run.wait_polls = p->wait_polls;
                 if (jwdev_main64s(&run, &src, cfg->buffer[0], p->R64, (int)grid, p->d_err, s) != 0)
                     return PFSOLVE_ERROR_FAILED_TO_LAUNCH_KERNEL;
-            } else if (jwdev_main64(&run, in_lds ? &src : NULL, in_lds ? cfg->buffer[0] : NULL, p->R64, p->waves64,
-                                    (int)grid, s) != 0) {
+            } else if (jwdev_main64(&run, p->R64, p->waves64, (int)grid, s) != 0) {
                 return PFSOLVE_ERROR_FAILED_TO_LAUNCH_KERNEL;
             }
             if (p->ev_stop && hipEventRecord(p->ev_stop, s) != hipSuccess) return PFSOLVE_ERROR_FAILED_TO_EVENT_RECORD;
