@@ -7,10 +7,12 @@
  * per N, PfSolve/pfSolve_AppManagement/pfSolve_RunApp.h:80-159 per plan).
  * Here one step is:
  *   1. jw_prologue_batch_kernel: one workgroup per set writes the set's
- *      coefficient table (format 2) and zeroes the queue counters (only the
- *      counters when every row class builds its tables in LDS);
+ *      coefficient table (format 2) and zeroes the queue counters (nothing when
+ *      every row class builds its tables in LDS);
  *   2. per row class (R rows per lane, N <= 64 R): one persistent launch of a
  *      queue kernel over that class's work units.
+ * An untuned class whose units hold whole sets builds its tables in LDS during a run
+ * (group_run_kernel) as long as the caller never asks for resident tables.
  * Work units are (set, range of system pairs), listed largest N first, so
  * the long units start early and the short ones fill the tail.
  */
@@ -36,6 +38,7 @@ struct pfsolve_batch {
     jw_prologue_job* d_jobs;          /* every set's table build, indexed by set */
     jw_prologue_job* d_gjobs;         /* the builds of the sets whose tables go to global memory */
     int64_t n_gjobs;
+    int64_t n_rjobs;                  /* the first n_rjobs of them: needed by a run that builds the others in LDS */
     jw_batch_item* d_items;
     jw_batch_unit* d_units;           /* units of all launch groups, back to back */
     int* d_counters;                  /* per launch group a queue (next unit, workgroups left; the
@@ -43,6 +46,12 @@ struct pfsolve_batch {
     /* launch groups: sets run with R_eff = 2 << g rows per lane */
     int64_t unit_first[NCLS], unit_count[NCLS];
     int group_waves[NCLS], group_grid[NCLS], group_kernel[NCLS];
+    /* what a run launches while no resident tables are wanted: kernel 4 where run_lds[g], the
+     * group's kernel otherwise */
+    int run_lds[NCLS], run_waves[NCLS], run_grid[NCLS];
+    /* resident tables: the caller has prepared or solved (a run then writes them too), and
+     * the tables in memory are those of the last prepare or run */
+    int want_tables, tables_ready;
     int wait_polls;                   /* bound of the split kernel's waits (0: default) */
     int64_t total_units, total_systems;
     pfsolve_batch_tuning tuning;
@@ -221,18 +230,27 @@ static int group_waves_default(int g)
     return jwdev_main64_waves(2 << g);
 }
 
-/* kernel of launch group g: 1 = load, compute and store in every wavefront
- * (input through an LDS staging), 2 = compute / store split (R <= 16), 3 = direct
- * I/O (R <= 16: LDS holds the table only, loads one pass ahead, stores from
- * registers, up to 8 wavefronts on one table), 4 = kernel 1 with each set's table
- * built in the workgroup's LDS when its set changes (R <= 16, >= 4 wavefronts; no
- * table build launch, no table through HBM).  Default: the split where it is
- * measured faster (R <= 8: 5.35 against 4.94 TB/s at N = 512); at R = 16 the
- * staged kernels reach the same rate with the 4-5 wavefronts LDS leaves them, and
- * direct I/O measured slower (harmonic batch, solve only: 256-295 us against
- * 213-227 us: a lane's 16-byte accesses 128 bytes apart reach memory less well than
- * the staged, contiguous ones), so it is a tuner candidate only. */
-static int group_kernel_default(int g) { return g == 0 ? 1 : (g <= 2 ? 2 : 1); }
+/* kernel of launch group g: 1 = load, compute and store in every wavefront, 2 = compute /
+ * store split (R <= 16), 3 = direct I/O (R <= 16: LDS holds the table only, loads one pass
+ * ahead, stores from registers, up to 8 wavefronts on one table), 4 = kernel 1 with each set's
+ * table built in the workgroup's LDS when its set changes (R <= 16, >= 4 wavefronts; no table
+ * build launch, no table through HBM).  Default 1: solves on prepared tables, kernel 1 against
+ * 2 and 3: 512 sets of 512 - 257 rows, 64 systems each, 50.4, 58.6 and 68.6 us; 40 sets of 512
+ * rows, 1024 systems, 64.6 and 78.0; 256 sets of 256 - 129 rows 24.8 and 26.8; 512 sets of
+ * 128 - 65 rows 30.2 and 35.1; 1024 sets of 1024 - 513 rows 175, 196 and 252. */
+#define GROUP_KERNEL_DEFAULT 1
+
+/* Default 4 for a run that no resident tables are wanted from, where each set's table is then
+ * built about once: at most two units per set, and for R <= 8 at most two sets per CU.  Run on
+ * kernel 4 / table launch and kernel 1: 1024 sets of 1024 - 513 rows 196 / 215 us, 300 such
+ * sets 86 / 94, 512 sets of 512 - 257 rows 58 / 61, 200 of them with 8 systems 22 / 28, but
+ * 1024 sets of 512 - 257 rows with 32 systems 72 / 69 and 40 sets of 1024 systems 83 / 73.  R = 2:
+ * only without sets of N <= 64, whose sub-wavefront groups kernel 4 does not have. */
+static int run_in_lds(int g, int64_t units, int64_t sets, int64_t min_n, int cu_count)
+{
+    if (g > 3 || units > 2 * sets) return 0;
+    return g == 3 || (sets <= 2 * (int64_t)cu_count && !(g == 0 && min_n <= 64));
+}
 
 /* systems per wavefront pass of the R = 2 class on queue kernel 1 when not tuned: four
  * 16-lane groups for sets with N <= 32, two 32-lane groups for N <= 64 (measured on small-N
@@ -254,13 +272,16 @@ static int cmp_n_desc(const void* a, const void* c)
     return x->idx < y->idx ? -1 : (x->idx > y->idx);
 }
 
-/* passes per queue unit of set s (`pairs` passes in all): the tuned size, else `defup` when
- * set (and smaller than the set), else the whole set */
+/* passes per queue unit of set s (`pairs` passes in all): the tuned size, else equal units of
+ * about `defup` when set (and smaller than the set), else the whole set */
 static int64_t unit_passes(const pfsolve_batch* b, int64_t s, int64_t pairs, int64_t defup)
 {
     const int64_t tuned = b->tuning.unit_pairs[b->cls[s]];
     if (tuned > 0) return tuned;
-    if (defup > 0 && defup < pairs) return defup;
+    if (defup > 0 && defup < pairs) {
+        const int64_t n = pairs / defup;
+        return (pairs + n - 1) / n;
+    }
     return pairs > 0 ? pairs : 1;
 }
 
@@ -277,17 +298,23 @@ static PfSolveResult build_queue(pfsolve_batch* b, jw_batch_unit** out_units)
     for (int64_t i = 0; i < S; i++) order[i] = keys[i].idx;
     free(keys);
     /* untuned unit size: whole sets, unless a group has fewer sets than 4 units per CU; then
-     * units of at least 16 passes that give each CU about 4 of them */
-    int64_t nsets_g[NCLS] = {0}, passes_g[NCLS] = {0}, defup[NCLS] = {0};
+     * units that give each CU about 4 of them, but at least two passes per wavefront (four at
+     * R = 2): a unit costs a table copy and a pipeline start (512 sets of 512 - 257 rows, 32
+     * pairs each, solve: 47.6 us whole, 50.4 us in units of 16; 64 sets of 128 - 65 rows, 512
+     * pairs: 35.7 us in units of 64, 40.4 in units of 32) */
+    int64_t nsets_g[NCLS] = {0}, passes_g[NCLS] = {0}, defup[NCLS] = {0}, min_n[NCLS] = {0};
     for (int64_t s = 0; s < S; s++) {
-        nsets_g[eff_group(b, s)]++;
-        passes_g[eff_group(b, s)] += set_passes(b, s);
+        const int g = eff_group(b, s);
+        nsets_g[g]++;
+        passes_g[g] += set_passes(b, s);
+        if (min_n[g] == 0 || b->sets[s].N < min_n[g]) min_n[g] = b->sets[s].N;
     }
     for (int g = 0; g < NCLS; g++) {
         const int64_t target = 4 * (int64_t)(b->cu_count > 0 ? b->cu_count : 1);
         if (nsets_g[g] < target) {
+            const int64_t least = (g == 0 ? 4 : 2) * (int64_t)group_waves_default(g);
             defup[g] = (passes_g[g] + target - 1) / target;
-            if (defup[g] < 16) defup[g] = 16;
+            if (defup[g] < least) defup[g] = least;
         }
     }
     /* count units per group */
@@ -339,7 +366,9 @@ static PfSolveResult build_queue(pfsolve_batch* b, jw_batch_unit** out_units)
             if (b->tuning.grid_per_cu[c] > gpc) gpc = b->tuning.grid_per_cu[c];
             if (b->tuning.kernel[c] > k) k = b->tuning.kernel[c];
         }
-        if (!group_kernel_ok(g, k)) k = group_kernel_default(g);
+        b->run_lds[g] = 0;
+        const int untuned = k == 0;
+        if (!group_kernel_ok(g, k)) k = GROUP_KERNEL_DEFAULT;
         int occ = 0;
         if (k == 4) {
             /* the table build needs at least 4 wavefronts */
@@ -368,6 +397,15 @@ static PfSolveResult build_queue(pfsolve_batch* b, jw_batch_unit** out_units)
         b->group_waves[g] = w;
         b->group_grid[g] = (int)(grid > 0 ? grid : 1);
         b->group_kernel[g] = k;
+        if (untuned && run_in_lds(g, b->unit_count[g], nsets_g[g], min_n[g], b->cu_count)) {
+            const int rw = group_waves_default(g);
+            const int ro = jwdev_batch64b_occupancy(2 << g, rw);
+            int64_t rg = (int64_t)b->cu_count * ro;
+            if (rg > b->unit_count[g]) rg = b->unit_count[g];
+            b->run_lds[g] = ro >= 1;
+            b->run_waves[g] = rw;
+            b->run_grid[g] = (int)rg;
+        }
     }
     return PFSOLVE_SUCCESS;
 }
@@ -396,9 +434,17 @@ static PfSolveResult upload_queue(pfsolve_batch* b)
         jobs[s].matrices = b->sets[s].matrices;
         jobs[s].table = (char*)b->tables + b->table_off[s];
         jobs[s].R = 2 << eff_group(b, s);
-        if (b->group_kernel[eff_group(b, s)] == 4) continue;
-        gjobs[b->n_gjobs++] = jobs[s];
-        if (64 * jobs[s].R > b->max_RL) b->max_RL = 64 * jobs[s].R;
+    }
+    /* first the sets whose tables every run needs in memory, then those that only resident
+     * tables (prepare) need */
+    for (int lds = 0; lds < 2; lds++) {
+        for (int64_t s = 0; s < b->nsets; s++) {
+            const int g = eff_group(b, s);
+            if (b->group_kernel[g] == 4 || b->run_lds[g] != lds) continue;
+            gjobs[b->n_gjobs++] = jobs[s];
+            if (64 * jobs[s].R > b->max_RL) b->max_RL = 64 * jobs[s].R;
+        }
+        if (lds == 0) b->n_rjobs = b->n_gjobs;
     }
     e = hipMemcpy(b->d_jobs, jobs, sizeof(jw_prologue_job) * (size_t)b->nsets, hipMemcpyHostToDevice);
     if (e == hipSuccess && b->n_gjobs > 0)
@@ -408,6 +454,7 @@ static PfSolveResult upload_queue(pfsolve_batch* b)
     if (e != hipSuccess) return PFSOLVE_ERROR_FAILED_TO_COPY;
     if (b->graph_exec) { hipGraphExecDestroy(b->graph_exec); b->graph_exec = NULL; }
     if (b->graph) { hipGraphDestroy(b->graph); b->graph = NULL; }
+    b->tables_ready = 0;   /* the tables' places and forms may have changed */
     return PFSOLVE_SUCCESS;
 }
 
@@ -537,55 +584,82 @@ PfSolveResult pfsolve_batch_set_tuning(pfsolve_batch* b, const pfsolve_batch_tun
     return upload_queue(b);
 }
 
-/* the tables that live in global memory (that launch also clears the queues).  With none,
- * nothing is launched: every queue kernel leaves its queue empty when it ends, so a step
- * whose row classes all build their tables in LDS is one launch per class. */
-static int run_prologue(pfsolve_batch* b, hipStream_t stream)
+/* the first njobs of the tables that live in global memory (that launch also clears the
+ * queues).  With none, nothing is launched: every queue kernel leaves its queue empty when it
+ * ends, so a step whose row classes all build their tables in LDS is one launch per class. */
+static int run_prologue(pfsolve_batch* b, int64_t njobs, hipStream_t stream)
 {
-    if (b->n_gjobs > 0)
-        return jwdev_prologue_batch(b->d_gjobs, (int)b->n_gjobs, b->max_RL, b->d_counters, 2 * NCLS, stream);
+    if (njobs > 0) return jwdev_prologue_batch(b->d_gjobs, (int)njobs, b->max_RL, b->d_counters, 2 * NCLS, stream);
     return 0;
 }
 
-static PfSolveResult launch_step(pfsolve_batch* b, const jw_batch_item* d_items, hipStream_t stream, int only_group,
-                                 int with_prologue)
+/* the queue launches; lds: on kernel 4 where a run may build in LDS */
+static PfSolveResult launch_queues(pfsolve_batch* b, const jw_batch_item* d_items, hipStream_t stream, int only_group,
+                                   int lds)
 {
-    if (with_prologue && run_prologue(b, stream) != 0) return PFSOLVE_ERROR_FAILED_TO_LAUNCH_KERNEL;
     for (int g = 0; g < NCLS; g++) {
         if (!b->unit_count[g] || (only_group >= 0 && g != only_group)) continue;
-        const int k = b->group_kernel[g];
-        const int rc = k == 4 ? jwdev_batch64b(d_items, b->d_units + b->unit_first[g], (int)b->unit_count[g],
-                                               b->d_counters + 2 * g, 2 << g, b->group_waves[g], b->group_grid[g],
-                                               b->d_jobs, stream)
-                       : k == 2 ? jwdev_batch64s(d_items, b->d_units + b->unit_first[g], (int)b->unit_count[g],
-                                               b->d_counters + 2 * g, 2 << g, b->group_waves[g], b->group_grid[g],
-                                               b->d_counters + 2 * NCLS, b->wait_polls, stream)
-                       : k == 3 ? jwdev_batch64d(d_items, b->d_units + b->unit_first[g], (int)b->unit_count[g],
-                                                 b->d_counters + 2 * g, 2 << g, b->group_waves[g], b->group_grid[g], stream)
-                                : jwdev_batch64(d_items, b->d_units + b->unit_first[g], (int)b->unit_count[g],
-                                                b->d_counters + 2 * g, 2 << g, b->group_waves[g], b->group_grid[g],
-                                                spw_effective(b), stream);
+        const int in_lds = lds && b->run_lds[g];
+        const int k = in_lds ? 4 : b->group_kernel[g];
+        const int w = in_lds ? b->run_waves[g] : b->group_waves[g];
+        const int grid = in_lds ? b->run_grid[g] : b->group_grid[g];
+        const jw_batch_unit* units = b->d_units + b->unit_first[g];
+        const int n = (int)b->unit_count[g];
+        int* queue = b->d_counters + 2 * g;
+        const int rc = k == 4   ? jwdev_batch64b(d_items, units, n, queue, 2 << g, w, grid, b->d_jobs, stream)
+                       : k == 2 ? jwdev_batch64s(d_items, units, n, queue, 2 << g, w, grid, b->d_counters + 2 * NCLS,
+                                                 b->wait_polls, stream)
+                       : k == 3 ? jwdev_batch64d(d_items, units, n, queue, 2 << g, w, grid, stream)
+                                : jwdev_batch64(d_items, units, n, queue, 2 << g, w, grid, spw_effective(b), stream);
         if (rc != 0) return PFSOLVE_ERROR_FAILED_TO_LAUNCH_KERNEL;
     }
     return PFSOLVE_SUCCESS;
 }
 
+/* a step that leaves every table in memory, or (with_prologue 0) uses the tables there */
+static PfSolveResult launch_step(pfsolve_batch* b, const jw_batch_item* d_items, hipStream_t stream, int only_group,
+                                 int with_prologue)
+{
+    if (with_prologue && run_prologue(b, b->n_gjobs, stream) != 0) return PFSOLVE_ERROR_FAILED_TO_LAUNCH_KERNEL;
+    return launch_queues(b, d_items, stream, only_group, 0);
+}
+
+/* A run writes the tables (run = prepare + solve) when resident tables are wanted, and when
+ * it is recorded (a replay cannot tell what was called since); otherwise the classes with
+ * run_lds build theirs in LDS and leave none behind, which tables_ready = 0 tells a later
+ * solve. */
 PfSolveResult pfsolve_batch_run(pfsolve_batch* b, hipStream_t stream)
 {
     if (!b) return PFSOLVE_ERROR_PLAN_NOT_INITIALIZED;
-    return launch_step(b, b->d_items, stream, -1, 1);
+    int recorded = 0;
+    if (stream) {
+        hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+        recorded = hipStreamIsCapturing(stream, &st) != hipSuccess || st != hipStreamCaptureStatusNone;
+    }
+    if (recorded) return launch_step(b, b->d_items, stream, -1, 1);
+    if (b->want_tables) {
+        b->tables_ready = 1;
+        return launch_step(b, b->d_items, stream, -1, 1);
+    }
+    b->tables_ready = 0;
+    if (run_prologue(b, b->n_rjobs, stream) != 0) return PFSOLVE_ERROR_FAILED_TO_LAUNCH_KERNEL;
+    return launch_queues(b, b->d_items, stream, -1, 1);
 }
 
 PfSolveResult pfsolve_batch_prepare(pfsolve_batch* b, hipStream_t stream)
 {
     if (!b) return PFSOLVE_ERROR_PLAN_NOT_INITIALIZED;
-    return run_prologue(b, stream) == 0 ? PFSOLVE_SUCCESS : PFSOLVE_ERROR_FAILED_TO_LAUNCH_KERNEL;
+    b->want_tables = 1;
+    b->tables_ready = 1;
+    return run_prologue(b, b->n_gjobs, stream) == 0 ? PFSOLVE_SUCCESS : PFSOLVE_ERROR_FAILED_TO_LAUNCH_KERNEL;
 }
 
+/* after runs that left no tables for some classes, those build them in LDS once more */
 PfSolveResult pfsolve_batch_solve(pfsolve_batch* b, hipStream_t stream)
 {
     if (!b) return PFSOLVE_ERROR_PLAN_NOT_INITIALIZED;
-    return launch_step(b, b->d_items, stream, -1, 0);
+    b->want_tables = 1;
+    return launch_queues(b, b->d_items, stream, -1, !b->tables_ready);
 }
 
 PfSolveResult pfsolve_batch_run_plain(pfsolve_batch* b, hipStream_t stream)
@@ -706,7 +780,7 @@ PfSolveResult pfsolve_batch_get_info(const pfsolve_batch* b, pfsolve_batch_info*
     info->algorithmic_bytes = alg;
     /* per step: the table build launch (when some class reads tables from global memory)
      * and one queue launch per class */
-    int launches = b->n_gjobs > 0 ? 1 : 0;
+    int launches = (b->want_tables ? b->n_gjobs : b->n_rjobs) > 0 ? 1 : 0;
     for (int g = 0; g < NCLS; g++)
         if (b->unit_count[g]) { info->classes_used |= 1 << g; launches++; }
     info->launches = launches;
@@ -728,7 +802,7 @@ static int time_group(pfsolve_batch* b, const jw_batch_item* d_items, hipStream_
     for (int k = 0; rc == 0 && k < repeats; k++) {
         /* the whole step (the global tables' build, then the queue launches), or with
          * solve_only the queue launches alone on tables built beforehand */
-        if (solve_only && run_prologue(b, stream) != 0) { rc = -1; break; }
+        if (solve_only && run_prologue(b, b->n_gjobs, stream) != 0) { rc = -1; break; }
         hipEventRecord(e0, stream);
         if (launch_step(b, d_items, stream, g, !solve_only) != PFSOLVE_SUCCESS) { rc = -1; break; }
         hipEventRecord(e1, stream);
