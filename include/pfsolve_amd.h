@@ -127,7 +127,8 @@ typedef struct pfsolve_batch_tuning {
     int32_t rows_per_lane_shift[PFSOLVE_BATCH_CLASSES]; /* 1: sets of this class run with 2R rows
                                                            per lane (half the lanes, one scan level
                                                            fewer), when 2R <= 16 */
-    /* unit_pairs counts systems, not pairs, for the R = 32 class (one system per pass) */
+    /* unit_pairs counts systems, not pairs, for the R = 32 class, whose workgroup shape is fixed
+       (waves has no effect there) */
     int32_t kernel[PFSOLVE_BATCH_CLASSES];      /* 0: default, 1: every wavefront loads, computes and
                                                    stores its pairs, 2: compute / store split
                                                    (R <= 16; `waves` counts the computing

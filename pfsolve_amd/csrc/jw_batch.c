@@ -184,7 +184,7 @@ static int eff_group(const pfsolve_batch* b, int64_t s)
     return c + (c < NSHIFT && b->tuning.rows_per_lane_shift[c] ? 1 : 0);
 }
 
-/* wavefront passes of a set: pairs of systems, or systems for R = 32 */
+/* unit lengths of a set: pairs of systems, or systems for R = 32 */
 static int64_t set_passes(const pfsolve_batch* b, int64_t s)
 {
     return eff_group(b, s) == NCLS - 1 ? b->sets[s].nsys : (b->sets[s].nsys + 1) / 2;
@@ -386,7 +386,7 @@ static PfSolveResult build_queue(pfsolve_batch* b, jw_batch_unit** out_units)
             occ = jwdev_batch64s_occupancy(2 << g, w);
         } else {
             const int wmax = group_waves_default(g);
-            if (w <= 0 || w > wmax) w = wmax;
+            if (w <= 0 || w > wmax || g == NCLS - 1) w = wmax;   /* R = 32: one shape */
             if (w < 1) return PFSOLVE_ERROR_UNSUPPORTED_FFT_LENGTH;
             occ = jwdev_batch64_occupancy(2 << g, w);
         }
@@ -696,8 +696,8 @@ PfSolveResult pfsolve_batch_run_plain(pfsolve_batch* b, hipStream_t stream)
         const int waves = jwdev_main64_waves(R);
         const int occ = jwdev_main64_occupancy(R, waves);
         if (waves < 1 || occ < 1) return PFSOLVE_ERROR_UNSUPPORTED_FFT_LENGTH;
-        const int64_t npass = R == 32 ? st->nsys : (st->nsys + 1) / 2;
-        int64_t grid = (npass + waves - 1) / waves;
+        const int64_t npass = (st->nsys + 1) / 2, per_wg = jwdev_main64_pairs(R, waves);
+        int64_t grid = (npass + per_wg - 1) / per_wg;
         if (grid > (int64_t)b->cu_count * occ) grid = (int64_t)b->cu_count * occ;
         if (jwdev_main64(&run, R, waves, (int)grid, stream) != 0) return PFSOLVE_ERROR_FAILED_TO_LAUNCH_KERNEL;
     }
@@ -878,8 +878,8 @@ PfSolveResult pfsolve_batch_tune_mode(pfsolve_batch* b, hipStream_t stream, int 
                     if (k == 1) {
                         const int wmax = group_waves_default(g);
                         wl[0] = wmax;
-                        wl[1] = (wmax + 1) / 2;
-                        wl[2] = (wmax + 3) / 4;
+                        wl[1] = g == NCLS - 1 ? 0 : (wmax + 1) / 2;
+                        wl[2] = g == NCLS - 1 ? 0 : (wmax + 3) / 4;
                     } else if (k == 3) {
                         wl[0] = 8;
                         wl[1] = 4;

@@ -188,10 +188,11 @@ int jwdev_prologue_batch(const jw_prologue_job* d_jobs, int njobs, int max_RL, i
 /* wave-per-system FP64 kernel (table format 2, 64 lanes, R in {2,4,8,16}) */
 int64_t jwdev_table64_elems(int R);
 int jwdev_main64_waves(int R);
+int jwdev_main64_pairs(int R, int waves);   /* pairs of systems per workgroup and pass */
 int64_t jwdev_main64_lds_bytes(int R, int waves);
 int jwdev_main64_occupancy(int R, int waves);
 int jwdev_main64(const jw_run_desc* r, int R, int waves, int grid, void* stream);
-/* the same with the table built in each workgroup's LDS (R <= 16; systems at any 8-byte address) */
+/* the same with the table built by each workgroup (systems at any 8-byte address) */
 int jwdev_main64b_waves(int R);
 int jwdev_main64b_occupancy(int R);
 int jwdev_main64b(const jw_run_desc* r, const jw_source_desc* src, const void* matrices, int R, int grid, void* stream);

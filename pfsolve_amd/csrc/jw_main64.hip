@@ -1178,189 +1178,378 @@ __global__ __launch_bounds__(max_threads<kLong64R>()) void jw_long64_front_kerne
 }
 
 // ---------------------------------------------------------------------------
-// Long systems (R = 32 rows per lane, N <= 2048): one system per wavefront pass.
-// The 140 KiB table stays in global memory (every wavefront of the grid reads
-// it, so it is served from L2) and coefficients are streamed row by row instead
-// of held in registers; LDS holds the 16 KiB staging of each wavefront.
+// 1024 < N <= 2048: a group of four wavefronts owns a pair of systems, 512 rows (R = 8 per
+// lane) each; a workgroup is two groups.  The 8 coefficients of a lane's 8 rows do not
+// change from pair to pair and stay in its registers (128 VGPRs), so no pass reads a table:
+// LDS holds the scan multipliers (48 KiB) and a staging of 4 KiB per wavefront.  (The whole
+// table, 128 KiB, leaves no LDS for stagings; streamed through the L2 by one wavefront per
+// system it set the pace: 8192 systems of 2000 rows 142 us, 56 us
+// this way.)
+// What crosses wavefronts goes through LDS: the two rows on each side for the matvec, and
+// per recurrence each wavefront's end value for a zero carry; a wavefront's carry follows
+// from those of the wavefronts before it (matrix-only factors), and enters a lane's rows
+// by one more multiplier, the product over the lanes before it.  Four barriers per pass; the
+// arithmetic takes a third of the time the pass's memory traffic does.
+// Tables in memory (batches, the plain per-set form) are the format-2 tables of 32 rows per
+// lane, whose coefficients are read once per matrix set.
 // ---------------------------------------------------------------------------
-// table reads through a buffer resource: one VGPR lane offset, the row offset in
-// an SGPR, no 64-bit address per coefficient
-typedef double jw_d2v __attribute__((ext_vector_type(2)));
-__device__ __forceinline__ double2 tb2(__amdgpu_buffer_rsrc_t r, int voff, int soff)
+constexpr int kWideW = 4;                       // wavefronts per group
+constexpr int kWideR = 8;                       // rows per lane
+constexpr int kWideRows = 64 * kWideR;          // rows per wavefront
+constexpr int kWideThreads = 512;
+constexpr int kWideGroups = kWideThreads / 64 / kWideW;
+// LDS while solving: stagings, multipliers of the 4 wavefront places (3 recurrences x 8 x
+// 64), exchange; while building: the build's scratch and two 512-row coefficient slots
+constexpr int kWideMult = kWideGroups * kWideW * kWideRows * 8;
+constexpr int kWideExch = kWideMult + kWideW * 24 * 64 * 8;
+constexpr int kWideExchDoubles = kWideGroups * kWideW * (2 * 4 + 3 * 2) + 3 * kWideW;
+constexpr int kWideSlots = (int)((prologue_lds_bytes(kWideW * kWideRows, 8) + 1023) / 1024 * 1024);
+constexpr int kWideLds = kWideSlots + 2 * kWideRows * 64 > kWideExch + kWideExchDoubles * 8
+                             ? kWideSlots + 2 * kWideRows * 64 : kWideExch + kWideExchDoubles * 8;
+
+// the coefficients of a lane's rows: (v_-2, v_-1), (v_0, v_1), (v_2, l'), (h', E)
+struct wide_coef {
+    double2 p[4][kWideR];
+};
+
+// from a format-2 table of 32 rows per lane in global memory: row w 512 + 8 lane + k of the
+// system is row-in-lane 8 (lane mod 4) + k of table lane 16 w + lane / 4
+__device__ __forceinline__ void wide_load_table(wide_coef& c, const void* table, int w, int lane)
 {
-    const jw_d2v d = __builtin_bit_cast(jw_d2v, __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, 0));
-    return make_double2(d.x, d.y);
-}
-__device__ __forceinline__ double tb1(__amdgpu_buffer_rsrc_t r, int voff, int soff)
-{
-    return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(r, voff, soff, 0));
+    const double* tab = reinterpret_cast<const double*>(table);
+#pragma unroll
+    for (int p = 0; p < 4; p++)
+#pragma unroll
+        for (int k = 0; k < kWideR; k++) {
+            const int e = tab_coef64(p, 8 * (lane & 3) + k, 16 * w + (lane >> 2), 32);
+            c.p[p][k] = load_chunk(tab + e);
+        }
 }
 
-template <int R, bool ALL3>
-__device__ __forceinline__ void compute_single(__amdgpu_buffer_rsrc_t tr, int lane, const jw_pass64& g,
-                                               double (&x)[R])
-{
-    constexpr int SC = 8 * R * 64 * 8;        // byte offset of the scan multipliers
-    const int lp = lane * 16;                 // a lane's coefficient pair within a row block
-    const int ls = lane * 8;                  // a lane's scan multiplier
-    // coefficient pair p of row-in-lane i: byte offset ((p R + i) 64 + lane) 16
+// a build's rows (FORMAT 3 of prologue_body on 8 wavefronts: the j-th row of every thread
+// belongs to wavefront place j) through two LDS slots into the registers of their owners
+struct wide_sink {
+    double* slots;
+    wide_coef& c;
+    int w, lane;
+    __device__ __forceinline__ void operator()(int j, int i, int t, const double (&cf)[8]) const
     {
-        double m1 = 0.0, m2 = 0.0, p1 = 0.0, p2 = 0.0;
-        if (g.kl >= 1) m1 = dpp_d<DPP_WAVE_SHR1>(x[R - 1]);
-        if (g.kl >= 2) m2 = dpp_d<DPP_WAVE_SHR1>(x[R - 2]);
-        if (g.ku >= 1) p1 = dpp_d<DPP_WAVE_SHL1>(x[0]);
-        if (g.ku >= 2) p2 = dpp_d<DPP_WAVE_SHL1>(x[1]);
+        double* s = slots + (j & 1) * (kWideRows * 8);
 #pragma unroll
-        for (int i = 0; i < R; i++) {
-            const double2 c0 = tb2(tr, lp, (0 * R + i) * 1024);
-            const double2 c1 = tb2(tr, lp, (1 * R + i) * 1024);
-            const double vp2 = tb1(tr, lp, (2 * R + i) * 1024);
-            const double xi = x[i];
-            const double n1 = (i + 1 < R) ? x[(i + 1) % R] : p1;
-            const double n2 = (i + 2 < R) ? x[(i + 2) % R] : ((i + 2 == R) ? p1 : p2);
-            double u = c1.x * xi;
-            u = __builtin_fma(c0.y, m1, u);
-            u = __builtin_fma(c0.x, m2, u);
-            u = __builtin_fma(c1.y, n1, u);
-            u = __builtin_fma(vp2, n2, u);
-            m2 = m1;
-            m1 = xi;
-            x[i] = u;
+        for (int p = 0; p < 4; p++)
+            *reinterpret_cast<double2*>(s + tab_coef64(p, i, t, kWideR)) = make_double2(cf[2 * p], cf[2 * p + 1]);
+    }
+    __device__ __forceinline__ void done(int j) const
+    {
+        // a slot is written again two rows on, behind the next barrier
+        __syncthreads();
+        if (w != j) return;
+        const double* s = slots + (j & 1) * (kWideRows * 8);
+#pragma unroll
+        for (int p = 0; p < 4; p++)
+#pragma unroll
+            for (int k = 0; k < kWideR; k++)
+                c.p[p][k] = *reinterpret_cast<const double2*>(s + tab_coef64(p, k, lane, kWideR));
+    }
+};
+
+// scan multipliers of wavefront place w from its coefficients, by group 0: as the format-2
+// build's (jw_prologue.h) over the wavefront's 64 lanes, with the carry's multiplier (the
+// product over the lanes before, or behind) in place 7 and the whole wavefront's product in tot
+__device__ __forceinline__ void wide_multipliers(const wide_coef& c, double* mult, double* tot, int w, int t)
+{
+    const int tr = t & 15, rw = t >> 4;
+#pragma unroll
+    for (int j = 0; j < 3; j++) {
+        double v = 1.0;
+#pragma unroll
+        for (int k = 0; k < kWideR; k++)
+            v *= -(j == 0 ? c.p[2][k].y : (j == 1 ? c.p[3][k].x : c.p[3][k].y));
+        double* m = mult + (w * 24 + j * 8) * 64 + t;
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            const int s = 1 << k;
+            m[64 * k] = v;
+            const bool from = j == 0 ? tr >= s : tr + s <= 15;
+            double u;
+            switch (k) {
+            case 0: u = j == 0 ? dpp_d<DPP_ROW_SHR(1)>(v) : dpp_d<DPP_ROW_SHL(1)>(v); break;
+            case 1: u = j == 0 ? dpp_d<DPP_ROW_SHR(2)>(v) : dpp_d<DPP_ROW_SHL(2)>(v); break;
+            case 2: u = j == 0 ? dpp_d<DPP_ROW_SHR(4)>(v) : dpp_d<DPP_ROW_SHL(4)>(v); break;
+            default: u = j == 0 ? dpp_d<DPP_ROW_SHR(8)>(v) : dpp_d<DPP_ROW_SHL(8)>(v); break;
+            }
+            if (from) v *= u;
+        }
+        if (j == 0) {
+            const double T0 = readlane_d(v, 15), T1 = readlane_d(v, 31), T2 = readlane_d(v, 47), T3 = readlane_d(v, 63);
+            m[64 * 4] = v;
+            m[64 * 5] = rw == 2 ? v : (rw == 3 ? T2 * v : 0.0);
+            const double before = dpp_d<DPP_ROW_SHR(1)>(v);   // in every lane; a row's first takes 1
+            const double rows = rw == 0 ? 1.0 : (rw == 1 ? T0 : (rw == 2 ? T0 * T1 : T0 * T1 * T2));
+            m[64 * 7] = (tr == 0 ? 1.0 : before) * rows;
+            if (t == 0) tot[w] = T0 * T1 * T2 * T3;
+        } else {
+            const double T0 = readlane_d(v, 0), T1 = readlane_d(v, 16), T2 = readlane_d(v, 32), T3 = readlane_d(v, 48);
+            m[64 * 4] = rw == 0 ? v : 0.0;
+            m[64 * 5] = rw == 0 ? v * T1 : (rw == 1 ? v : 0.0);
+            m[64 * 6] = rw == 0 ? v * T1 * T2 : (rw == 1 ? v * T2 : (rw == 2 ? v : 0.0));
+            const double behind = dpp_d<DPP_ROW_SHL(1)>(v);
+            const double rows = rw == 3 ? 1.0 : (rw == 2 ? T3 : (rw == 1 ? T2 * T3 : T1 * T2 * T3));
+            m[64 * 7] = (tr == 15 ? 1.0 : behind) * rows;
+            if (t == 0) tot[j * kWideW + w] = T0 * T1 * T2 * T3;
         }
     }
+}
+
+// the step on a pair, in registers; every wavefront of the workgroup calls it (barriers)
+template <bool ALL3>
+__device__ __forceinline__ void wide_compute(const wide_coef& c, const double* mult, double* exch, int grp, int w,
+                                             int lane, const jw_pass64& g, double (&x0)[kWideR], double (&x1)[kWideR])
+{
+    constexpr int R = kWideR;
+    double* rows = exch + (grp * kWideW + w) * 8;   // first two and last two rows of both systems
+    double* ends = exch + kWideGroups * kWideW * 8;                     // per recurrence, group, place, system
+    const double* tot = ends + 3 * kWideGroups * kWideW * 2;
+    if (lane == 0) {
+        rows[0] = x0[0]; rows[1] = x0[1];
+        rows[4] = x1[0]; rows[5] = x1[1];
+    }
+    if (lane == 63) {
+        rows[2] = x0[R - 2]; rows[3] = x0[R - 1];
+        rows[6] = x1[R - 2]; rows[7] = x1[R - 1];
+    }
+    __syncthreads();
+    {
+        double m1a = 0.0, m2a = 0.0, p1a = 0.0, p2a = 0.0;
+        double m1b = 0.0, m2b = 0.0, p1b = 0.0, p2b = 0.0;
+        const bool lo = lane == 0 && w > 0, hi = lane == 63 && w + 1 < kWideW;
+        if (g.kl >= 1) {
+            m1a = dpp_d<DPP_WAVE_SHR1>(x0[R - 1]);
+            m1b = dpp_d<DPP_WAVE_SHR1>(x1[R - 1]);
+            if (lo) { m1a = rows[-8 + 3]; m1b = rows[-8 + 7]; }
+        }
+        if (g.kl >= 2) {
+            m2a = dpp_d<DPP_WAVE_SHR1>(x0[R - 2]);
+            m2b = dpp_d<DPP_WAVE_SHR1>(x1[R - 2]);
+            if (lo) { m2a = rows[-8 + 2]; m2b = rows[-8 + 6]; }
+        }
+        if (g.ku >= 1) {
+            p1a = dpp_d<DPP_WAVE_SHL1>(x0[0]);
+            p1b = dpp_d<DPP_WAVE_SHL1>(x1[0]);
+            if (hi) { p1a = rows[8]; p1b = rows[8 + 4]; }
+        }
+        if (g.ku >= 2) {
+            p2a = dpp_d<DPP_WAVE_SHL1>(x0[1]);
+            p2b = dpp_d<DPP_WAVE_SHL1>(x1[1]);
+            if (hi) { p2a = rows[8 + 1]; p2b = rows[8 + 5]; }
+        }
+#pragma unroll
+        for (int i = 0; i < R; i++) {
+            const double ia = x0[i], ib = x1[i];
+            const double n1a = (i + 1 < R) ? x0[(i + 1) % R] : p1a;
+            const double n1b = (i + 1 < R) ? x1[(i + 1) % R] : p1b;
+            const double n2a = (i + 2 < R) ? x0[(i + 2) % R] : ((i + 2 == R) ? p1a : p2a);
+            const double n2b = (i + 2 < R) ? x1[(i + 2) % R] : ((i + 2 == R) ? p1b : p2b);
+            double ua = c.p[1][i].x * ia, ub = c.p[1][i].x * ib;
+            ua = __builtin_fma(c.p[0][i].y, m1a, ua);
+            ub = __builtin_fma(c.p[0][i].y, m1b, ub);
+            ua = __builtin_fma(c.p[0][i].x, m2a, ua);
+            ub = __builtin_fma(c.p[0][i].x, m2b, ub);
+            ua = __builtin_fma(c.p[1][i].y, n1a, ua);
+            ub = __builtin_fma(c.p[1][i].y, n1b, ub);
+            ua = __builtin_fma(c.p[2][i].x, n2a, ua);
+            ub = __builtin_fma(c.p[2][i].x, n2b, ub);
+            m2a = m1a;
+            m2b = m1b;
+            m1a = ia;
+            m1b = ib;
+            x0[i] = ua;
+            x1[i] = ub;
+        }
+    }
+    // forward recurrence
     if (ALL3 || g.fwd) {
-        double a = x[0];
+        const double* m = mult + (w * 24) * 64 + lane;
+        double* e = ends + (grp * kWideW) * 2;
+        double a = x0[0], b = x1[0];
 #pragma unroll
-        for (int i = 1; i < R; i++) a = __builtin_fma(-tb1(tr, lp + 8, (2 * R + i) * 1024), a, x[i]);
-        a = __builtin_fma(tb1(tr, ls, SC + 0 * 512), dpp_d<DPP_ROW_SHR(1)>(a), a);
-        a = __builtin_fma(tb1(tr, ls, SC + 1 * 512), dpp_d<DPP_ROW_SHR(2)>(a), a);
-        a = __builtin_fma(tb1(tr, ls, SC + 2 * 512), dpp_d<DPP_ROW_SHR(4)>(a), a);
-        a = __builtin_fma(tb1(tr, ls, SC + 3 * 512), dpp_d<DPP_ROW_SHR(8)>(a), a);
-        a = __builtin_fma(tb1(tr, ls, SC + 4 * 512), dpp_rm<DPP_ROW_BCAST15, 0xa>(a), a);
-        a = __builtin_fma(tb1(tr, ls, SC + 5 * 512), dpp_rm<DPP_ROW_BCAST31, 0xc>(a), a);
-        double w = dpp_d<DPP_WAVE_SHR1>(a);
+        for (int i = 1; i < R; i++) {
+            a = __builtin_fma(-c.p[2][i].y, a, x0[i]);
+            b = __builtin_fma(-c.p[2][i].y, b, x1[i]);
+        }
+        a = __builtin_fma(m[0], dpp_d<DPP_ROW_SHR(1)>(a), a);
+        b = __builtin_fma(m[0], dpp_d<DPP_ROW_SHR(1)>(b), b);
+        a = __builtin_fma(m[64], dpp_d<DPP_ROW_SHR(2)>(a), a);
+        b = __builtin_fma(m[64], dpp_d<DPP_ROW_SHR(2)>(b), b);
+        a = __builtin_fma(m[128], dpp_d<DPP_ROW_SHR(4)>(a), a);
+        b = __builtin_fma(m[128], dpp_d<DPP_ROW_SHR(4)>(b), b);
+        a = __builtin_fma(m[192], dpp_d<DPP_ROW_SHR(8)>(a), a);
+        b = __builtin_fma(m[192], dpp_d<DPP_ROW_SHR(8)>(b), b);
+        a = __builtin_fma(m[256], dpp_rm<DPP_ROW_BCAST15, 0xa>(a), a);
+        b = __builtin_fma(m[256], dpp_rm<DPP_ROW_BCAST15, 0xa>(b), b);
+        a = __builtin_fma(m[320], dpp_rm<DPP_ROW_BCAST31, 0xc>(a), a);
+        b = __builtin_fma(m[320], dpp_rm<DPP_ROW_BCAST31, 0xc>(b), b);
+        if (lane == 63) *reinterpret_cast<double2*>(e + 2 * w) = make_double2(a, b);
+        double wa = dpp_d<DPP_WAVE_SHR1>(a), wb = dpp_d<DPP_WAVE_SHR1>(b);
+        const double pt = m[448];
+        __syncthreads();
+        // W' entering the wavefront
+        double ca = 0.0, cb = 0.0;
+        for (int k = 0; k < w; k++) {
+            const double2 s = *reinterpret_cast<const double2*>(e + 2 * k);
+            ca = __builtin_fma(tot[k], ca, s.x);
+            cb = __builtin_fma(tot[k], cb, s.y);
+        }
+        wa = __builtin_fma(pt, ca, wa);
+        wb = __builtin_fma(pt, cb, wb);
 #pragma unroll
         for (int i = 0; i < R; i++) {
-            w = __builtin_fma(-tb1(tr, lp + 8, (2 * R + i) * 1024), w, x[i]);
-            x[i] = w;
+            wa = __builtin_fma(-c.p[2][i].y, wa, x0[i]);
+            wb = __builtin_fma(-c.p[2][i].y, wb, x1[i]);
+            x0[i] = wa;
+            x1[i] = wb;
         }
     }
+    // backward recurrences
 #pragma unroll
     for (int stage = 0; stage < 2; stage++) {
         if (!ALL3 && stage == 0 && !g.b1) continue;
         if (!ALL3 && stage == 1 && !g.b2) continue;
-        const int j = 1 + stage;
-        double a = x[R - 1];
+        const double* m = mult + (w * 24 + 8 * (1 + stage)) * 64 + lane;
+        double* e = ends + ((1 + stage) * kWideGroups + grp) * kWideW * 2;
+        auto h = [&](int i) -> double { return stage == 0 ? c.p[3][i].x : c.p[3][i].y; };
+        double a = x0[R - 1], b = x1[R - 1];
 #pragma unroll
-        for (int i = R - 2; i >= 0; i--) a = __builtin_fma(-tb1(tr, lp + 8 * stage, (3 * R + i) * 1024), a, x[i]);
-        a = __builtin_fma(tb1(tr, ls, SC + (j * 8 + 0) * 512), dpp_d<DPP_ROW_SHL(1)>(a), a);
-        a = __builtin_fma(tb1(tr, ls, SC + (j * 8 + 1) * 512), dpp_d<DPP_ROW_SHL(2)>(a), a);
-        a = __builtin_fma(tb1(tr, ls, SC + (j * 8 + 2) * 512), dpp_d<DPP_ROW_SHL(4)>(a), a);
-        a = __builtin_fma(tb1(tr, ls, SC + (j * 8 + 3) * 512), dpp_d<DPP_ROW_SHL(8)>(a), a);
-        {
-            const double s1 = readlane_d(a, 16), s2 = readlane_d(a, 32), s3 = readlane_d(a, 48);
-            a = __builtin_fma(tb1(tr, ls, SC + (j * 8 + 4) * 512), s1, a);
-            a = __builtin_fma(tb1(tr, ls, SC + (j * 8 + 5) * 512), s2, a);
-            a = __builtin_fma(tb1(tr, ls, SC + (j * 8 + 6) * 512), s3, a);
+        for (int i = R - 2; i >= 0; i--) {
+            a = __builtin_fma(-h(i), a, x0[i]);
+            b = __builtin_fma(-h(i), b, x1[i]);
         }
-        double z = dpp_d<DPP_WAVE_SHL1>(a);
+        a = __builtin_fma(m[0], dpp_d<DPP_ROW_SHL(1)>(a), a);
+        b = __builtin_fma(m[0], dpp_d<DPP_ROW_SHL(1)>(b), b);
+        a = __builtin_fma(m[64], dpp_d<DPP_ROW_SHL(2)>(a), a);
+        b = __builtin_fma(m[64], dpp_d<DPP_ROW_SHL(2)>(b), b);
+        a = __builtin_fma(m[128], dpp_d<DPP_ROW_SHL(4)>(a), a);
+        b = __builtin_fma(m[128], dpp_d<DPP_ROW_SHL(4)>(b), b);
+        a = __builtin_fma(m[192], dpp_d<DPP_ROW_SHL(8)>(a), a);
+        b = __builtin_fma(m[192], dpp_d<DPP_ROW_SHL(8)>(b), b);
+        {
+            const double a1 = readlane_d(a, 16), a2 = readlane_d(a, 32), a3 = readlane_d(a, 48);
+            const double b1 = readlane_d(b, 16), b2 = readlane_d(b, 32), b3 = readlane_d(b, 48);
+            a = __builtin_fma(m[256], a1, a);
+            b = __builtin_fma(m[256], b1, b);
+            a = __builtin_fma(m[320], a2, a);
+            b = __builtin_fma(m[320], b2, b);
+            a = __builtin_fma(m[384], a3, a);
+            b = __builtin_fma(m[384], b3, b);
+        }
+        if (lane == 0) *reinterpret_cast<double2*>(e + 2 * w) = make_double2(a, b);
+        double za = dpp_d<DPP_WAVE_SHL1>(a), zb = dpp_d<DPP_WAVE_SHL1>(b);
+        const double pt = m[448];
+        __syncthreads();
+        // Z' (or y) entering the wavefront from the one behind it
+        double ca = 0.0, cb = 0.0;
+        for (int k = kWideW - 1; k > w; k--) {
+            const double2 s = *reinterpret_cast<const double2*>(e + 2 * k);
+            ca = __builtin_fma(tot[(1 + stage) * kWideW + k], ca, s.x);
+            cb = __builtin_fma(tot[(1 + stage) * kWideW + k], cb, s.y);
+        }
+        za = __builtin_fma(pt, ca, za);
+        zb = __builtin_fma(pt, cb, zb);
 #pragma unroll
         for (int i = R - 1; i >= 0; i--) {
-            z = __builtin_fma(-tb1(tr, lp + 8 * stage, (3 * R + i) * 1024), z, x[i]);
-            x[i] = z;
+            za = __builtin_fma(-h(i), za, x0[i]);
+            zb = __builtin_fma(-h(i), zb, x1[i]);
+            x0[i] = za;
+            x1[i] = zb;
         }
     }
-    if (g.apply_scale) x[0] *= g.row0_scale;
+    if (g.apply_scale) {
+        x0[0] *= g.row0_scale;
+        x1[0] *= g.row0_scale;
+    }
 }
 
-// one system per pass: stg holds 64 R / 2 chunks (the first system region of a pair staging)
-template <int R, bool ALL3>
-__device__ __forceinline__ void jw_single64(__amdgpu_buffer_rsrc_t tab, double2* stg, int lane, const jw_pass64& g,
-                                            int64_t sys)
+// pass geometry of wavefront place w: its 512 rows of the system as a system of their own
+__device__ __forceinline__ jw_pass64 wide_pass(double* rhs, int64_t nsys, int64_t stride, int64_t offSol, int64_t N,
+                                               int64_t in_lo, int64_t in_hi, int64_t out_lo, int64_t out_hi, int kl,
+                                               int ku, bool fwd, bool b1, bool b2, bool apply_scale, double scale,
+                                               int w, int lane)
 {
-    constexpr int H = R / 2;
-    const double* src = g.rhs + sys * g.stride + g.offSol;
-#pragma unroll
-    for (int k = 0; k < H; k++) {
-        const int c = swz<H>(64 * k + lane);
-        if (c >= g.icl && c < g.ich)
-            __builtin_amdgcn_global_load_lds(src + 2 * c, (__attribute__((address_space(3))) void*)(stg + 64 * k),
-                                             16, 0, 0);
-    }
-    __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0): the DMA writes have landed in LDS
-    compiler_fence();
-    double x[R];
-#pragma unroll
-    for (int m = 0; m < H; m++) {
-        const double2 v = stg[swz<H>(lane * H + m)];
-        x[2 * m] = v.x;
-        x[2 * m + 1] = v.y;
-    }
-#pragma unroll
-    for (int e = 0; e < 2; e++) {
-        const bool on = e == 0 ? g.in_edge_lo : g.in_edge_hi;
-        const int r = e == 0 ? g.in_lo : g.in_hi - 1;
-        if (on && lane == r / R) {
-            const double v = as_global(src)[r];
-#pragma unroll
-            for (int k = 0; k < R; k++)
-                if (k == r % R) x[k] = v;
-        }
-    }
-    compute_single<R, ALL3>(tab, lane, g, x);
-    compiler_fence();
-#pragma unroll
-    for (int m = 0; m < H; m++) stg[swz<H>(lane * H + m)] = make_double2(x[2 * m], x[2 * m + 1]);
-    compiler_fence();
-    double2 v[H];
-#pragma unroll
-    for (int k = 0; k < H; k++) v[k] = stg[swz<H>(64 * k + lane)];
-#pragma unroll
-    for (int k = 0; k < H; k++) asm volatile("" : "+v"(v[k].x), "+v"(v[k].y));
-    double* dst = g.rhs + sys * g.stride + g.offSol;
-#pragma unroll
-    for (int k = 0; k < H; k++) {
-        const int c = 64 * k + lane;
-        if (c >= g.ocl && c < g.och) store_stream(dst + 2 * c, v[k]);
-    }
-#pragma unroll
-    for (int e = 0; e < 2; e++) {
-        const bool on = e == 0 ? g.out_edge_lo : g.out_edge_hi;
-        const int r = e == 0 ? g.out_lo : g.out_hi - 1;
-        if (on && lane == 0) {
-            const double2 w = stg[swz<H>(r >> 1)];
-            as_global(g.rhs)[sys * g.stride + g.offSol + r] = (r & 1) ? w.y : w.x;
-        }
-    }
-#pragma unroll
-    for (int k = 0; k < H; k++) {
-        const int c = swz<H>(64 * k + lane);
-        if (!(c >= g.icl && c < g.ich)) stg[64 * k + lane] = make_double2(0.0, 0.0);
-    }
-    __builtin_amdgcn_s_waitcnt(0xC07F);   // lgkmcnt(0): LDS traffic done before the next DMA lands
-    compiler_fence();
+    const int64_t rb = (int64_t)w * kWideRows;
+    int64_t n = N - rb;
+    n = n < 0 ? 0 : (n > kWideRows ? kWideRows : n);
+    auto clip = [&](int64_t v) -> int {
+        const int64_t u = v - rb;
+        return (int)(u < 0 ? 0 : (u > n ? n : u));
+    };
+    const int il = clip(in_lo), ih = clip(in_hi), ol = clip(out_lo), oh = clip(out_hi);
+    return make_pass64(rhs, nsys, stride, offSol + rb, il, ih > il ? ih : il, ol, oh > ol ? oh : ol, kl, ku, fwd, b1, b2,
+                       apply_scale && w == 0, scale, lane);
 }
 
-template <int R, bool ALL3>
-__global__ __launch_bounds__(256) void jw_main64g_kernel(jw_run_desc d)
+// pairs p0 + 2 s + group for s = 0, step, ... (systems first + 2 pair, below the geometry's
+// nsys), one per group and pass, for a workgroup whose wavefronts hold their coefficients;
+// pf: the first pass's rows
+template <bool ALL3, class Geo>
+__device__ __forceinline__ void wide_stream(const wide_coef& c, unsigned char* smem, int grp, int w, int lane,
+                                            const Geo& geo, int64_t first, int64_t p, int64_t p1, int64_t step,
+                                            double2 (&pf)[2][kWideR / 2])
+{
+    constexpr int R = kWideR;
+    const double* mult = reinterpret_cast<const double*>(smem + kWideMult);
+    double* exch = reinterpret_cast<double*>(smem + kWideExch);
+    double2* stg = reinterpret_cast<double2*>(smem) + (size_t)(grp * kWideW + w) * 32 * R;
+    // every wavefront makes every pass (barriers)
+    for (; p < p1; p += step) {
+        jw_pass64 g = geo();
+        const int64_t q = p + grp, sys0 = first + 2 * q;
+        const bool on = q < p1;
+        // a group past the last pair goes through the pass on what its registers hold and
+        // reads and stores nothing
+        g.in_edge_lo = g.in_edge_lo && on;
+        g.in_edge_hi = g.in_edge_hi && on;
+        double x0[R], x1[R];
+        unpack_ahead<R>(pf, stg, lane, g, sys0, x0, x1);
+        const int64_t qn = q + step;
+        if (qn < p1) load_pair_ahead<R>(pf, lane, g, first + 2 * qn);
+        wide_compute<ALL3>(c, mult, exch, grp, w, lane, g, x0, x1);
+        if (on) {
+            store_system<R>(stg, lane, g, sys0, x0);
+            if (sys0 + 1 < g.nsys) store_system<R>(stg, lane, g, sys0 + 1, x1);
+        }
+    }
+}
+
+template <bool ALL3, bool BUILD>
+__global__ __launch_bounds__(kWideThreads) void jw_wide64_kernel(jw_run_desc d, jw_source_desc src, const void* mat)
 {
     extern __shared__ __align__(16) unsigned char smem[];
-    // word 3 of the buffer resource: the gfx9 raw-buffer default (data format 32)
-    const __amdgpu_buffer_rsrc_t tab = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(d.table), 0,
-                                                                         JW_TAB64_ELEMS(R) * 8, 0x00020000);
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int nwaves = blockDim.x >> 6;
-    double2* stg = reinterpret_cast<double2*>(smem) + (size_t)wave * 32 * R;
-#pragma unroll
-    for (int k = 0; k < R / 2; k++) stg[64 * k + lane] = make_double2(0.0, 0.0);
-    __syncthreads();
-    for (int64_t q = (int64_t)blockIdx.x * nwaves + wave; q < d.nsys; q += (int64_t)gridDim.x * nwaves) {
-        const jw_pass64 g = make_pass64(reinterpret_cast<double*>(d.rhs), d.nsys, d.stride, d.offSol,
-                                        (int)d.in_lo, (int)d.in_hi, (int)d.out_lo, (int)d.out_hi, d.kl, d.ku,
-                                        d.fwd, d.b1, d.b2, d.apply_scale, d.scale_hi, lane);
-        jw_single64<R, ALL3>(tab, stg, lane, g, q);
+    const int grp = wave / kWideW, w = wave % kWideW;
+    const int64_t npass = (d.nsys + 1) >> 1, step = (int64_t)gridDim.x * kWideGroups;
+    const int64_t p = (int64_t)blockIdx.x * kWideGroups;
+    auto geo = [&] {
+        return wide_pass(reinterpret_cast<double*>(d.rhs), d.nsys, d.stride, d.offSol, d.N, d.in_lo, d.in_hi, d.out_lo,
+                         d.out_hi, d.kl, d.ku, d.fwd, d.b1, d.b2, d.apply_scale, d.scale_hi, w, lane);
+    };
+    double2 pf[2][kWideR / 2] = {};
+    auto first = [&] { if (p + grp < npass) load_pair_ahead<kWideR>(pf, lane, geo(), 2 * (p + grp)); };
+    wide_coef c;
+    if constexpr (BUILD) {
+        const wide_sink sink{reinterpret_cast<double*>(smem + kWideSlots), c, w, lane};
+        prologue_body<double, 3, NoPivotHooks, kWideW, kMaxRT>(src, mat, static_cast<double*>(nullptr), 64, kWideR, smem,
+                                                               0, nullptr, kWideW, NoPivotHooks(), first, sink);
+    } else {
+        wide_load_table(c, d.table, w, lane);
+        first();
     }
+    __syncthreads();   // the build's LDS is free
+    if (grp == 0)
+        wide_multipliers(c, reinterpret_cast<double*>(smem + kWideMult),
+                         reinterpret_cast<double*>(smem + kWideExch) + kWideGroups * kWideW * (8 + 3 * 2), w, lane);
+    __syncthreads();
+    wide_stream<ALL3>(c, smem, grp, w, lane, geo, 0, p, npass, step, pf);
 }
 
 // ---------------------------------------------------------------------------
@@ -2116,40 +2305,44 @@ __global__ __launch_bounds__(kBatchDirectThreads) void jw_batch64d_kernel(const 
     queue_leave(counter);
 }
 
-// The same queue for long systems (R = 32): one system per wavefront pass, table
-// read through a buffer resource; the unit ranges count systems, not pairs.
-__global__ __launch_bounds__(256) void jw_batch64g_kernel(const jw_batch_item* items, const jw_batch_unit* units,
-                                                          int nunits, int* counter, int /* systems per pass: 1 */)
+// The same queue for 1024 < N <= 2048: two pairs of systems per pass of a workgroup, the
+// coefficients in its registers (above); the unit ranges count systems, not pairs.
+__global__ __launch_bounds__(kWideThreads) void jw_batch64w_kernel(const jw_batch_item* items, const jw_batch_unit* units,
+                                                                   int nunits, int* counter, int /* systems per pass */)
 {
-    constexpr int R = 32;
     extern __shared__ __align__(16) unsigned char smem[];
     __shared__ int s_unit;
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int nwaves = blockDim.x >> 6;
-    double2* stg = reinterpret_cast<double2*>(smem) + (size_t)wave * 32 * R;
+    const int grp = wave / kWideW, w = wave % kWideW;
     int cur = -1;
+    wide_coef c;
     for (;;) {
-        __syncthreads();
+        __syncthreads();   // the previous unit is finished: s_unit and the multipliers may change
         if (threadIdx.x == 0) s_unit = atomicAdd(counter, 1);
         __syncthreads();
         const int u = __builtin_amdgcn_readfirstlane(s_unit);
         if (u >= nunits) break;
         const jw_batch_unit un = units[u];
         const jw_batch_item& it = items[un.item];
+        const int64_t sys_end = it.nsys < un.pair1 ? it.nsys : un.pair1;
+        const int64_t npass = (sys_end - un.pair0 + 1) >> 1;
+        auto geo = [&] {
+            return wide_pass(reinterpret_cast<double*>(it.rhs), sys_end, it.stride, it.offSol, it.N, 0, it.N, 0, it.N,
+                             it.kl, it.ku, true, true, true, it.apply_scale != 0, it.scale, w, lane);
+        };
+        double2 pf[2][kWideR / 2] = {};
+        if (grp < npass) load_pair_ahead<kWideR>(pf, lane, geo(), un.pair0 + 2 * grp);
         if (un.item != cur) {
-#pragma unroll
-            for (int k = 0; k < R / 2; k++) stg[64 * k + lane] = make_double2(0.0, 0.0);
+            wide_load_table(c, it.table, w, lane);
+            if (grp == 0)
+                wide_multipliers(c, reinterpret_cast<double*>(smem + kWideMult),
+                                 reinterpret_cast<double*>(smem + kWideExch) + kWideGroups * kWideW * (8 + 3 * 2), w,
+                                 lane);
+            __syncthreads();
             cur = un.item;
         }
-        const __amdgpu_buffer_rsrc_t tab = __builtin_amdgcn_make_buffer_rsrc(
-            const_cast<void*>(it.table), 0, JW_TAB64_ELEMS(R) * 8, 0x00020000);
-        for (int q = un.pair0 + wave; q < un.pair1; q += nwaves) {
-            const jw_pass64 g = make_pass64(reinterpret_cast<double*>(it.rhs), it.nsys, it.stride, it.offSol, 0,
-                                            it.N, 0, it.N, it.kl, it.ku, true, true, true, it.apply_scale != 0,
-                                            it.scale, lane);
-            jw_single64<R, true>(tab, stg, lane, g, q);
-        }
+        wide_stream<true>(c, smem, grp, w, lane, geo, un.pair0, 0, npass, kWideGroups, pf);
     }
     queue_leave(counter);
 }
@@ -2297,12 +2490,14 @@ const void* pick64(int R, bool all3 = true, bool build = false)
         case 4: return kernel_ptr<4, true>(all3);
         case 8: return kernel_ptr<8, true>(all3);
         case 16: return kernel_ptr<16, true>(all3);
+        case 32: return all3 ? reinterpret_cast<const void*>(&jw_wide64_kernel<true, true>)
+                             : reinterpret_cast<const void*>(&jw_wide64_kernel<false, true>);
         default: return nullptr;
         }
     }
     switch (R) {
-    case 32: return all3 ? reinterpret_cast<const void*>(&jw_main64g_kernel<32, true>)
-                         : reinterpret_cast<const void*>(&jw_main64g_kernel<32, false>);
+    case 32: return all3 ? reinterpret_cast<const void*>(&jw_wide64_kernel<true, false>)
+                         : reinterpret_cast<const void*>(&jw_wide64_kernel<false, false>);
     case 2: return kernel_ptr<2>(all3);
     case 4: return kernel_ptr<4>(all3);
     case 8: return kernel_ptr<8>(all3);
@@ -2358,7 +2553,7 @@ const void* batch_ptr()
 const void* pick_batch64(int R)
 {
     switch (R) {
-    case 32: return reinterpret_cast<const void*>(&jw_batch64g_kernel);
+    case 32: return reinterpret_cast<const void*>(&jw_batch64w_kernel);
     case 2: return batch_ptr<2>();
     case 4: return batch_ptr<4>();
     case 8: return batch_ptr<8>();
@@ -2426,7 +2621,7 @@ bool split_shape(int R, int* ncomp, int* nstore)
     return true;
 }
 
-int max_waves64(int R) { return R <= 4 ? 16 : R == 8 ? 12 : (R == 16 ? 8 : 4); }
+int max_waves64(int R) { return R <= 4 ? 16 : (R == 8 ? 12 : 8); }
 
 thread_local char g_err64[256];
 
@@ -2439,14 +2634,11 @@ int jwdev_main64b_waves(int R);
 
 /* waves per workgroup: as many as LDS (table + 2 systems of staging per wave)
  * and the kernel's launch bound allow */
-/* LDS copy of the table: R <= 16 (R = 32 reads it from global memory) */
-static int64_t table_lds_bytes(int R) { return R <= 16 ? jwdev_table64_elems(R) * 8 : 0; }
-
 int jwdev_main64_waves(int R)
 {
     if (!pick64(R)) return 0;
-    if (R == 32) return 4;
-    const int64_t table = table_lds_bytes(R);
+    if (R == 32) return kWideThreads / 64;   /* the kernel's shape is fixed */
+    const int64_t table = JW_TAB64_ELEMS(R) * 8;
     int w = (int)((kLdsBytesMax - table) / pair_stage_bytes(R));
     if (w > max_waves64(R)) w = max_waves64(R);
     return w < 1 ? 0 : w;
@@ -2454,9 +2646,12 @@ int jwdev_main64_waves(int R)
 
 int64_t jwdev_main64_lds_bytes(int R, int waves)
 {
-    if (R == 32) return 64LL * R * 8 * waves;   /* one system per wavefront */
-    return table_lds_bytes(R) + pair_stage_bytes(R) * waves;
+    if (R == 32) return kWideLds;
+    return JW_TAB64_ELEMS(R) * 8 + pair_stage_bytes(R) * waves;
 }
+
+/* pairs of systems per workgroup and pass */
+int jwdev_main64_pairs(int R, int waves) { return R == 32 ? kWideGroups : waves; }
 
 /* workgroups per CU, the smaller of the two variants (all recurrences / some) */
 static int main64_occupancy(int R, int waves, int lds, bool build)
@@ -2486,7 +2681,7 @@ int jwdev_main64(const jw_run_desc* r, int R, int waves, int grid, void* stream)
     const size_t lds = (size_t)jwdev_main64_lds_bytes(R, waves);
     hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) return -2;
-    /* the source and matrices are read by the building variants only (R = 32 has no such arguments) */
+    /* the source and matrices are read by the building variants only */
     jw_source_desc none;
     memset(&none, 0, sizeof(none));
     const void* nomat = NULL;
@@ -2495,10 +2690,11 @@ int jwdev_main64(const jw_run_desc* r, int R, int waves, int grid, void* stream)
     return e == hipSuccess ? 0 : -3;
 }
 
-/* the same with the table built in LDS (R <= 16; systems at any 8-byte address): wavefronts
+/* the same with the table built in the kernel (systems at any 8-byte address): wavefronts
  * per workgroup (the launch bound), workgroups per CU, launch */
 static int64_t main64b_lds_bytes(int R)
 {
+    if (R == 32) return kWideLds;
     return (int64_t)JW_TAB64_ELEMS(R) * 8 + max_i64(512LL * R * jwdev_main64b_waves(R), (int64_t)prologue_lds_bytes(64 * R, 8));
 }
 
@@ -2509,6 +2705,7 @@ int jwdev_main64b_waves(int R)
     case 4: return max_threads<4>() / 64;
     case 8: return max_threads<8>() / 64;
     case 16: return max_threads<16>() / 64;
+    case 32: return kWideThreads / 64;
     default: return 0;
     }
 }
@@ -2629,7 +2826,7 @@ int jwdev_chain64(const jw_run_desc* r, const jw_chain_jobs* jobs, int up, int g
 int jwdev_batch64_occupancy(int R, int waves)
 {
     const void* f = pick_batch64(R);
-    if (!f || waves < 1 || waves > max_waves64(R)) return 0;
+    if (!f || waves < 1 || waves > max_waves64(R) || (R == 32 && waves != max_waves64(R))) return 0;
     const int lds = (int)jwdev_main64_lds_bytes(R, waves);
     if (lds > kLdsBytesMax) return 0;
     if (hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess) return 0;
@@ -2643,7 +2840,10 @@ int jwdev_batch64(const jw_batch_item* d_items, const jw_batch_unit* d_units, in
 {
     const void* f = pick_batch64(R);
     if (!f) { snprintf(g_err64, sizeof(g_err64), "no batch kernel for R=%d", R); return -1; }
-    if (waves < 1 || waves > max_waves64(R) || grid < 1) { snprintf(g_err64, sizeof(g_err64), "bad batch launch"); return -1; }
+    if (waves < 1 || waves > max_waves64(R) || (R == 32 && waves != max_waves64(R)) || grid < 1) {
+        snprintf(g_err64, sizeof(g_err64), "bad batch launch");
+        return -1;
+    }
     const size_t lds = (size_t)jwdev_main64_lds_bytes(R, waves);
     if (lds > (size_t)kLdsBytesMax) { snprintf(g_err64, sizeof(g_err64), "batch LDS %zu too large", lds); return -1; }
     hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);

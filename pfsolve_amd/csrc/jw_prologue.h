@@ -226,6 +226,12 @@ struct NoAfterLoads {
     __device__ void operator()() const {}
 };
 
+// Takes the folded coefficients of a build that writes no table (FORMAT 3).
+struct NoSink {
+    template <typename T> __device__ void operator()(int, int, int, const T (&)[8]) const {}
+    __device__ void done(int) const {}
+};
+
 // DPP moves and readlane of either arithmetic type (lanes without a source receive 0)
 template <int CTRL, int ROWMASK = 0xf>
 __device__ __forceinline__ double lane_move(double v)
@@ -254,7 +260,10 @@ __device__ __forceinline__ dd lane_read(dd v, int lane) { return dd_make(readlan
 // publish(tid, g), called by every thread once the g of every row is final (g: the last
 // row's, in LDS).  `after` is called once the build's own loads are issued (FP64): loads
 // issued there return behind them and overlap the build.
-// TP: T*, or a pointer to global memory stated as such.  MAXJ, MAXRT: rows per thread at most in the row phases (RL <= MAXJ nthr) and in the pivot
+// TP: T*, or a pointer to global memory stated as such.  FORMAT 3 folds as format 2, but
+// hands row-in-lane i, lane t of the thread's j-th row to sink(j, i, t, coefficients) and
+// calls sink.done(j) after each j (every thread does); it forms no scan multipliers and
+// writes no table.  MAXJ, MAXRT: rows per thread at most in the row phases (RL <= MAXJ nthr) and in the pivot
 // scan (RL <= MAXRT NP); smaller bounds keep a small build's per-thread arrays in fewer
 // registers.
 //
@@ -267,11 +276,13 @@ __device__ __forceinline__ dd lane_read(dd v, int lane) { return dd_make(readlan
 // 256 rows (no pivots) 12.3 and 9.4, 16384 of 1000 rows 64.1 and 58.3, the tables of 1024
 // sets of 1024 - 513 rows in one launch 47 and 30.
 template <typename T, int FORMAT, typename H = NoPivotHooks, int MAXJ = kProRows, int MAXRT = kMaxRT,
-          typename F = NoAfterLoads, typename TP>
+          typename F = NoAfterLoads, typename TP, typename S = NoSink>
 __device__ __forceinline__ void prologue_body(const jw_source_desc& d, const void* mat, TP table, int L, int R,
                                               unsigned char* smem_raw, int64_t rb = 0, const T* carry = nullptr,
-                                              int nsub = 1, const H& hooks = H(), const F& after = F())
+                                              int nsub = 1, const H& hooks = H(), const F& after = F(),
+                                              const S& sink = S())
 {
+    constexpr bool FOLD = FORMAT != 1;
     using A = Ar<T>;
     const int RLs = R * L;                 // rows of one table
     const int RL = RLs * nsub;             // rows of this build
@@ -305,9 +316,9 @@ __device__ __forceinline__ void prologue_body(const jw_source_desc& d, const voi
     // write 128 consecutive bytes of the table (no bank conflicts in LDS, whole segments in
     // memory).  Consecutive rows alone write 16-byte pieces 1 KiB apart, rows R apart alone
     // read 64 lines per load: each cost the build over 1 us.
-    const int ni2 = FORMAT == 2 ? (R >= 8 ? 3 : (R == 4 ? 2 : 1)) : 0;   // log2 NI
+    const int ni2 = FOLD ? (R >= 8 ? 3 : (R == 4 ? 2 : 1)) : 0;   // log2 NI
     auto row_of = [&](int j) -> int {
-        if (FORMAT != 2) return tid + j * nthr;
+        if (!FOLD) return tid + j * nthr;
         const int lt2 = 6 - ni2;
         const int b = (tid >> 6) + (nthr >> 6) * j;                  // tile: R of them per table
         const int k = R >= 16 ? b / R : b >> (ni2);                  // R == NI below 16
@@ -317,7 +328,7 @@ __device__ __forceinline__ void prologue_body(const jw_source_desc& d, const voi
         return k * RLs + t * R + i;
     };
     // no thread of the wavefront has a j-th row (wavefront-uniform)
-    auto none = [&](int j) -> bool { return FORMAT == 2 ? (tid >> 6) + (nthr >> 6) * j >= RL / 64 : j * nthr >= RL; };
+    auto none = [&](int j) -> bool { return FOLD ? (tid >> 6) + (nthr >> 6) * j >= RL / 64 : j * nthr >= RL; };
     T vb[MAXJ][5], Dr[MAXJ], Er[MAXJ];
     // FP64: every row's loads first (rows outside the matrix read row 0's positions and
     // are discarded), then the selects, products and LDS stores, so that a thread's rows
@@ -344,7 +355,7 @@ __device__ __forceinline__ void prologue_body(const jw_source_desc& d, const voi
     // of a long system's rows takes D_{rb-1} and D_{rb+RL} from the matrix
     // (every thread reads them: one address each, workgroup-uniform conditions)
     T dprev = A::one(), dnext = A::one();
-    if (FORMAT == 2 && d.has_m) {
+    if (FOLD && d.has_m) {
         if (rb >= 1 && rb - 1 < N) dprev = mem_load<T>(mat, d.mdM + source_pos(d, rb - 1, N), mf);
         if (rb + RL < N) dnext = mem_load<T>(mat, d.mdM + source_pos(d, rb + RL, N), mf);
     }
@@ -402,7 +413,7 @@ __device__ __forceinline__ void prologue_body(const jw_source_desc& d, const voi
     }
     if (tid == 0) sx[16] = A::zero();   // the refinement flag
     __syncthreads();
-    if (FORMAT == 2 && d.has_m) {
+    if (FOLD && d.has_m) {
         // 1 / D of the rows (zero past the matrix), for the neighbours' fold
 #pragma unroll
         for (int j = 0; j < MAXJ; j++) {
@@ -650,7 +661,7 @@ __device__ __forceinline__ void prologue_body(const jw_source_desc& d, const voi
         __syncthreads();
     }
 
-    if constexpr (FORMAT == 2) {
+    if constexpr (FOLD) {
         // nsub tables of 64 R rows each, JW_TAB64_ELEMS(R) apart, the scalings folded:
         // with l_r = ld_r g_{r-1}, h_r = ud_r g_r and a_r = D_r g_r,
         //   l'_r = a_r l_r / a_{r-1} = a_r ld_r / D_{r-1},  h'_r = D_r h_r / D_{r+1} = a_r ud_r / D_{r+1}
@@ -661,37 +672,43 @@ __device__ __forceinline__ void prologue_body(const jw_source_desc& d, const voi
         const T inext = d.has_m && rb + RL < N ? A::div(A::one(), dnext) : A::one();
 #pragma unroll
         for (int j = 0; j < MAXJ; j++) {
-            if (none(j)) continue;
-            const int r = row_of(j);
-            if (r >= RL) continue;
-            const int kt = nsub > 1 ? r / RLs : 0, rr = r - kt * RLs;
-            const int t = rr / R, i = rr % R;
-            const T ar = A::mul(Dr[j], sg[at(r)]);
-            T cf[8];
+            const int r = none(j) ? RL : row_of(j);
+            if (r < RL) {
+                const int kt = nsub > 1 ? r / RLs : 0, rr = r - kt * RLs;
+                const int t = rr / R, i = rr % R;
+                const T ar = A::mul(Dr[j], sg[at(r)]);
+                T cf[8];
 #pragma unroll
-            for (int k = 0; k < 5; k++) cf[k] = A::mul(ar, vb[j][k]);
-            T lp = A::zero(), hp = A::zero();
-            if (rb + r >= 1 && rb + r < N) {
-                lp = A::mul(ar, sl[at(r)]);
-                if (d.has_m) lp = A::mul(lp, r >= 1 ? sE[at(r - 1)] : iprev);
-            }
-            if (rb + r + 1 < N) {
-                hp = A::mul(ar, sh[at(r)]);
-                if (d.has_m) hp = A::mul(hp, r + 1 < RL ? sE[at(r + 1)] : inext);
-            }
-            cf[5] = lp;
-            cf[6] = hp;
-            cf[7] = Er[j];
-            const TP tk = table + kt * te2;
+                for (int k = 0; k < 5; k++) cf[k] = A::mul(ar, vb[j][k]);
+                T lp = A::zero(), hp = A::zero();
+                if (rb + r >= 1 && rb + r < N) {
+                    lp = A::mul(ar, sl[at(r)]);
+                    if (d.has_m) lp = A::mul(lp, r >= 1 ? sE[at(r - 1)] : iprev);
+                }
+                if (rb + r + 1 < N) {
+                    hp = A::mul(ar, sh[at(r)]);
+                    if (d.has_m) hp = A::mul(hp, r + 1 < RL ? sE[at(r + 1)] : inext);
+                }
+                cf[5] = lp;
+                cf[6] = hp;
+                cf[7] = Er[j];
+                if constexpr (FORMAT == 3) {
+                    sink(j, i, t, cf);
+                } else {
+                    const TP tk = table + kt * te2;
 #pragma unroll
-            for (int p = 0; p < 4; p++) {
-                tk[tab_coef64(p, i, t, R)] = cf[2 * p];
-                tk[tab_coef64(p, i, t, R) + 1] = cf[2 * p + 1];
+                    for (int p = 0; p < 4; p++) {
+                        tk[tab_coef64(p, i, t, R)] = cf[2 * p];
+                        tk[tab_coef64(p, i, t, R) + 1] = cf[2 * p + 1];
+                    }
+                    sl[at(r)] = lp;
+                    sh[at(r)] = hp;
+                    sg[at(r)] = Er[j];
+                }
             }
-            sl[at(r)] = lp;
-            sh[at(r)] = hp;
-            sg[at(r)] = Er[j];
+            if constexpr (FORMAT == 3) sink.done(j);
         }
+        if constexpr (FORMAT == 3) return;
         __syncthreads();
         // scan multipliers: wavefront item (wave-uniform) takes recurrence j = item % 3
         // (0: forward through l', 1: backward through h', 2: backward through E) of

@@ -682,22 +682,24 @@ static PfSolveResult append_impl(PfSolveApplication* app, const PfSolveLaunchPar
         if (p->long_only) return append_long(app, &src, &run, s, table);
         const uintptr_t base = (uintptr_t)run.rhs;
         run.vec2 = p->precision == JW_PREC_F64 && (base % 16) == 0 && (run.stride % 2) == 0 && (run.offSol % 2) == 0;
-        const int in_lds = p->split64 || p->waves64b;
+        /* (the allocation-free entry point, whose area is capped, refuses unaligned systems of
+         * N > 1024 as the chunk path it would take does) */
+        const int in_lds = p->split64 || (p->waves64b && (run.vec2 || !(p->R64 == 32 && p->area_cap)));
         if (p->R64 && (run.vec2 || (in_lds && base % 8 == 0)) && cfg->kernelVariant != 1) {
-            /* wave-per-system kernels: table format 2, built by every workgroup in LDS (N <=
-             * 1024) or by a launch before.  The kernels that build in LDS load and store
+            /* wave-per-system kernels: table format 2, built by every workgroup, or by a
+             * launch before where that variant is not available.  The kernels that build load and store
              * global memory from registers and take systems at any 8-byte address (30000
              * systems of 333 rows, packed: 41.4 us a step, 61.8 us on the general kernel and
              * its table launch); the other stages by LDS DMA, 16-byte aligned */
             if (nsys <= 0) return PFSOLVE_SUCCESS;
-            /* wavefront passes: pairs of systems, single systems for R = 32 */
-            const int64_t npass = p->R64 == 32 ? nsys : (nsys + 1) / 2;
+            const int64_t npass = (nsys + 1) / 2;   /* pairs of systems */
             const int64_t cap_split = (int64_t)p->cu_count * p->occupancy_split * p->split64;
             const int64_t cap_build = (int64_t)p->cu_count * p->occupancy64b * p->waves64b;
             const int build = use_build_kernel(p, npass, cap_split, cap_build);
-            if (!in_lds && jwdev_prologue(&src, cfg->buffer[0], table, 64, p->R64, p->precision, 2, s) != 0)
+            if (!build && !p->split64 && jwdev_prologue(&src, cfg->buffer[0], table, 64, p->R64, p->precision, 2, s) != 0)
                 return PFSOLVE_ERROR_FAILED_TO_LAUNCH_KERNEL;
-            const int per_wg = build ? p->waves64b : (p->split64 ? p->split64 : p->waves64);
+            const int per_wg = build ? jwdev_main64_pairs(p->R64, p->waves64b)
+                                     : (p->split64 ? p->split64 : jwdev_main64_pairs(p->R64, p->waves64));
             int64_t need = (npass + per_wg - 1) / per_wg;
             int64_t grid = (int64_t)p->cu_count *
                            (build ? p->occupancy64b : (p->split64 ? p->occupancy_split : p->occupancy64));

@@ -22,7 +22,7 @@ def fused(N, perm, seed):
 
 
 @pytest.mark.parametrize("pad,off", [(0, 0), (1, 0), (2, 1), (3, 5)])
-@pytest.mark.parametrize("N", [1, 2, 3, 63, 64, 65, 127, 128, 129, 255, 257, 333, 511, 512, 513, 777, 1023, 1024])
+@pytest.mark.parametrize("N", [1, 2, 3, 63, 64, 65, 127, 128, 129, 255, 257, 333, 511, 512, 513, 777, 1023, 1024, 1025, 1535, 1537, 1999, 2047, 2048])
 def test_unaligned_fused_step(N, pad, off):
     B = 7
     stride = N + pad
