@@ -301,7 +301,11 @@ static PfSolveResult build_queue(pfsolve_batch* b, jw_batch_unit** out_units)
      * units that give each CU about 4 of them, but at least two passes per wavefront (four at
      * R = 2): a unit costs a table copy and a pipeline start (512 sets of 512 - 257 rows, 32
      * pairs each, solve: 47.6 us whole, 50.4 us in units of 16; 64 sets of 128 - 65 rows, 512
-     * pairs: 35.7 us in units of 64, 40.4 in units of 32) */
+     * pairs: 35.7 us in units of 64, 40.4 in units of 32).  R = 32 (counted in systems; one
+     * workgroup per CU, its table in registers): about one unit per CU for fewer sets than
+     * CUs (128 sets of 2048 rows, 64 systems each, solve: 65 us in units of 32, 72 in 16, 87
+     * whole), from there on up to 8, of at least 32 systems (300 sets: 153 us in units of 32,
+     * 173 in 12, 175 whole) */
     int64_t nsets_g[NCLS] = {0}, passes_g[NCLS] = {0}, defup[NCLS] = {0}, min_n[NCLS] = {0};
     for (int64_t s = 0; s < S; s++) {
         const int g = eff_group(b, s);
@@ -310,9 +314,12 @@ static PfSolveResult build_queue(pfsolve_batch* b, jw_batch_unit** out_units)
         if (min_n[g] == 0 || b->sets[s].N < min_n[g]) min_n[g] = b->sets[s].N;
     }
     for (int g = 0; g < NCLS; g++) {
-        const int64_t target = 4 * (int64_t)(b->cu_count > 0 ? b->cu_count : 1);
-        if (nsets_g[g] < target) {
-            const int64_t least = (g == 0 ? 4 : 2) * (int64_t)group_waves_default(g);
+        const int64_t cus = b->cu_count > 0 ? b->cu_count : 1;
+        const int wide = g == NCLS - 1, few = nsets_g[g] < cus;
+        const int64_t target = (wide ? (few ? 1 : 8) : 4) * cus;
+        if (nsets_g[g] < 4 * cus) {
+            const int64_t least =
+                wide ? (few ? 4 : 32) : (g == 0 ? 4 : 2) * (int64_t)group_waves_default(g);
             defup[g] = (passes_g[g] + target - 1) / target;
             if (defup[g] < least) defup[g] = least;
         }

@@ -65,6 +65,41 @@ __device__ __forceinline__ void store_stream(double* p, double2 v)
     __builtin_nontemporal_store(t, (JW_GLOBAL jw_d2u*)p);
 }
 
+// A system's chunks [lo, hi) through a buffer resource: accesses outside read zeros and store
+// nothing, without a branch around each.  vmcnt counts loads and stores in order, and only
+// straight-line stores let the compiler wait for a pass's loads alone; with branches it waits
+// for the stores behind them too, that is for the last pass's write acknowledgements: 256
+// sets of 2000 rows, 64 systems each, 172 -> 129 us; 300 sets of 1024 rows, 74 -> 70; one
+// plan of 30000 systems of 1024 rows, 104 -> 99.  The plain kernel for 1024 < N <= 2048 is
+// no faster for it (1500 rows: 133 us by branches, 138 so) and neither are the chained steps
+// up to 512 rows (115.2, 116.9); those keep the branches.  Offsets are whole chunks, so no
+// access straddles the end.
+struct chunk_range {
+    __amdgpu_buffer_rsrc_t rsrc;
+    int lo;
+    __device__ __forceinline__ int offset(int c) const { return c >= lo ? c * 16 : 0x40000000; }
+};
+__device__ __forceinline__ chunk_range make_chunks(const double* system, int lo, int hi, bool on)
+{
+    // word 3 of the resource: the gfx9 raw-buffer default (data format 32)
+    return chunk_range{__builtin_amdgcn_make_buffer_rsrc(const_cast<double*>(system), 0, on ? hi * 16 : 0, 0x00020000),
+                       lo};
+}
+__device__ __forceinline__ double2 load_chunk(const chunk_range& r, int c)
+{
+    typedef double d2v __attribute__((ext_vector_type(2)));
+    const d2v t = __builtin_bit_cast(d2v, __builtin_amdgcn_raw_buffer_load_b128(r.rsrc, r.offset(c), 0, 0));
+    return make_double2(t.x, t.y);
+}
+// (nontemporal: the store_stream above)
+__device__ __forceinline__ void store_chunk(const chunk_range& r, int c, double2 v)
+{
+    typedef double d2v __attribute__((ext_vector_type(2)));
+    typedef uint32_t u4v __attribute__((ext_vector_type(4)));
+    const d2v t = {v.x, v.y};
+    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4v, t), r.rsrc, r.offset(c), 0, 2);
+}
+
 // keeps the scheduler from hoisting one phase's table loads into the previous
 // phase, which would raise register pressure past the launch bound
 __device__ __forceinline__ void phase_barrier() { __builtin_amdgcn_sched_barrier(0); }
@@ -207,7 +242,7 @@ __device__ __forceinline__ void dma_pair(double2* stg, int lane, const jw_pass64
     }
 }
 
-template <int R>
+template <int R, bool LOOP = false>
 __device__ __forceinline__ void read_edges(int lane, const jw_pass64& g, int64_t sys0, double (&x0)[R], double (&x1)[R]);
 
 // blocked read-back of the landed input (lane t: rows t R .. t R + R-1), odd range
@@ -231,8 +266,9 @@ __device__ __forceinline__ void read_pair(const double2* stg, int lane, const jw
 }
 
 // the odd ends of the input keep-range (rows whose 16-byte chunk is only half
-// inside), read from global memory by their owning lane
-template <int R>
+// inside), read from global memory by their owning lane.  LOOP: waited for behind the branch,
+// the wait would be every pass's, for all its loads and stores; so it is inside
+template <int R, bool LOOP>
 __device__ __forceinline__ void read_edges(int lane, const jw_pass64& g, int64_t sys0, double (&x0)[R], double (&x1)[R])
 {
     const bool ok1 = sys0 + 1 < g.nsys;
@@ -243,8 +279,9 @@ __device__ __forceinline__ void read_edges(int lane, const jw_pass64& g, int64_t
             const bool on = e == 0 ? g.in_edge_lo : g.in_edge_hi;
             const int r = e == 0 ? g.in_lo : g.in_hi - 1;
             if (on && lane == r / R) {
-                const double v0 = src0[r];
-                const double v1 = ok1 ? src0[g.stride + r] : 0.0;
+                double v0 = src0[r];
+                double v1 = ok1 ? src0[g.stride + r] : 0.0;
+                if constexpr (LOOP) asm volatile("" : "+v"(v0), "+v"(v1));
 #pragma unroll
                 for (int k = 0; k < R; k++)
                     if (k == r % R) {
@@ -694,26 +731,31 @@ __device__ __forceinline__ void unpack_pair(const double2 (&pf)[2][R / 2], int l
 // comes from the L2 8 times (1024 sets of 1024 to 513 rows, solve: 251 us direct, 187 us
 // contiguous; chained steps of 1000 rows, K = 4: 76 and 67 us).  At R <= 8 the chained steps
 // measured the same or up to 4 % faster direct.
-template <int R>
+template <int R, bool BUF = true>
 __device__ __forceinline__ void load_pair_ahead(double2 (&pf)[2][R / 2], int lane, const jw_pass64& g, int64_t sys0)
 {
     constexpr int H = R / 2;
-    const bool ok1 = sys0 + 1 < g.nsys;
     const double* src0 = g.rhs + sys0 * g.stride + g.offSol;
 #pragma unroll
     for (int s = 0; s < 2; s++) {
         const double* src = src0 + s * g.stride;
+        const bool ok = s == 0 || sys0 + 1 < g.nsys;
+        const chunk_range r = make_chunks(src, g.icl, g.ich, ok);
 #pragma unroll
         for (int k = 0; k < H; k++) {
             const int c = 64 * k + lane;
-            double2 v = make_double2(0.0, 0.0);
-            if (c >= g.icl && c < g.ich && (s == 0 || ok1)) v = load_chunk(src + 2 * c);
-            pf[s][k] = v;
+            if constexpr (BUF) {
+                pf[s][k] = load_chunk(r, c);
+            } else {
+                double2 v = make_double2(0.0, 0.0);
+                if (c >= g.icl && c < g.ich && ok) v = load_chunk(src + 2 * c);
+                pf[s][k] = v;
+            }
         }
     }
 }
 
-template <int R>
+template <int R, bool LOOP = true>
 __device__ __forceinline__ void unpack_ahead(const double2 (&pf)[2][R / 2], double2* stg, int lane, const jw_pass64& g,
                                              int64_t sys0, double (&x0)[R], double (&x1)[R])
 {
@@ -732,14 +774,24 @@ __device__ __forceinline__ void unpack_ahead(const double2 (&pf)[2][R / 2], doub
             x[2 * m + 1] = v.y;
         }
     }
-    read_edges<R>(lane, g, sys0, x0, x1);
+    read_edges<R, LOOP>(lane, g, sys0, x0, x1);
+}
+
+// the first pair's loads end here, so that the pass loop's wait counts only what a pass issues
+template <int R>
+__device__ __forceinline__ void hold_pair(double2 (&pf)[2][R / 2])
+{
+#pragma unroll
+    for (int s = 0; s < 2; s++)
+#pragma unroll
+        for (int k = 0; k < R / 2; k++) asm volatile("" : "+v"(pf[s][k].x), "+v"(pf[s][k].y));
 }
 
 // one system's results through a staging of 32 R chunks to contiguous 16-byte stores of
 // the output keep-range; odd range ends by their owning lanes
-template <int R>
+template <int R, bool BUF = true>
 __device__ __forceinline__ void store_system(double2* stg, int lane, const jw_pass64& g, int64_t sys,
-                                             const double (&x)[R])
+                                             const double (&x)[R], bool on)
 {
     constexpr int H = R / 2;
     compiler_fence();   // the staging's previous reads are issued (LDS keeps their order)
@@ -752,13 +804,30 @@ __device__ __forceinline__ void store_system(double2* stg, int lane, const jw_pa
 #pragma unroll
     for (int k = 0; k < H; k++) asm volatile("" : "+v"(v[k].x), "+v"(v[k].y));
     double* dst = g.rhs + sys * g.stride + g.offSol;
+    const chunk_range out = make_chunks(dst, g.ocl, g.och, on);
 #pragma unroll
     for (int k = 0; k < H; k++) {
         const int c = 64 * k + lane;
-        if (c >= g.ocl && c < g.och) store_stream(dst + 2 * c, v[k]);
+        if constexpr (BUF) store_chunk(out, c, v[k]);
+        else if (c >= g.ocl && c < g.och) store_stream(dst + 2 * c, v[k]);
     }
+    if (BUF && !on) return;
     if (g.out_edge_lo && lane == g.out_lo / R) as_global(dst)[g.out_lo] = pick_row<R>(x, g.out_lo % R);
     if (g.out_edge_hi && lane == (g.out_hi - 1) / R) as_global(dst)[g.out_hi - 1] = pick_row<R>(x, (g.out_hi - 1) % R);
+}
+
+// the results of systems sys0 and sys0 + 1 (on: sys0 is one)
+template <int R, bool BUF>
+__device__ __forceinline__ void store_pair(double2* stg, int lane, const jw_pass64& g, int64_t sys0,
+                                           const double (&x0)[R], const double (&x1)[R], bool on)
+{
+    if constexpr (BUF) {
+        store_system<R, true>(stg, lane, g, sys0, x0, on);
+        store_system<R, true>(stg, lane, g, sys0 + 1, x1, on && sys0 + 1 < g.nsys);
+    } else if (on) {
+        store_system<R, false>(stg, lane, g, sys0, x0, true);
+        if (sys0 + 1 < g.nsys) store_system<R, false>(stg, lane, g, sys0 + 1, x1, true);
+    }
 }
 
 // Pairs q, q + step, ... below q1 through one wavefront: each pair's rows were loaded into
@@ -769,6 +838,7 @@ template <int R, bool ALL3, class Geo>
 __device__ __forceinline__ void stream_pairs(const double* tab, double2* stg, int lane, const Geo& geo, int64_t q,
                                              int64_t q1, int64_t step, double2 (&pf)[2][R / 2])
 {
+    hold_pair<R>(pf);
     while (q < q1) {
         const jw_pass64 g = geo();
         double x0[R], x1[R];
@@ -776,8 +846,7 @@ __device__ __forceinline__ void stream_pairs(const double* tab, double2* stg, in
         const int64_t qn = q + step;
         if (qn < q1) load_pair_ahead<R>(pf, lane, g, 2 * qn);
         compute_pair<R, ALL3>(tab, lane, g, x0, x1);
-        store_system<R>(stg, lane, g, 2 * q, x0);
-        if (2 * q + 1 < g.nsys) store_system<R>(stg, lane, g, 2 * q + 1, x1);
+        store_pair<R, true>(stg, lane, g, 2 * q, x0, x1, true);
         q = qn;
     }
 }
@@ -1490,7 +1559,7 @@ __device__ __forceinline__ jw_pass64 wide_pass(double* rhs, int64_t nsys, int64_
 // pairs p0 + 2 s + group for s = 0, step, ... (systems first + 2 pair, below the geometry's
 // nsys), one per group and pass, for a workgroup whose wavefronts hold their coefficients;
 // pf: the first pass's rows
-template <bool ALL3, class Geo>
+template <bool ALL3, bool BUF, class Geo>
 __device__ __forceinline__ void wide_stream(const wide_coef& c, unsigned char* smem, int grp, int w, int lane,
                                             const Geo& geo, int64_t first, int64_t p, int64_t p1, int64_t step,
                                             double2 (&pf)[2][kWideR / 2])
@@ -1499,6 +1568,7 @@ __device__ __forceinline__ void wide_stream(const wide_coef& c, unsigned char* s
     const double* mult = reinterpret_cast<const double*>(smem + kWideMult);
     double* exch = reinterpret_cast<double*>(smem + kWideExch);
     double2* stg = reinterpret_cast<double2*>(smem) + (size_t)(grp * kWideW + w) * 32 * R;
+    if constexpr (BUF) hold_pair<R>(pf);
     // every wavefront makes every pass (barriers)
     for (; p < p1; p += step) {
         jw_pass64 g = geo();
@@ -1509,14 +1579,11 @@ __device__ __forceinline__ void wide_stream(const wide_coef& c, unsigned char* s
         g.in_edge_lo = g.in_edge_lo && on;
         g.in_edge_hi = g.in_edge_hi && on;
         double x0[R], x1[R];
-        unpack_ahead<R>(pf, stg, lane, g, sys0, x0, x1);
+        unpack_ahead<R, BUF>(pf, stg, lane, g, sys0, x0, x1);
         const int64_t qn = q + step;
-        if (qn < p1) load_pair_ahead<R>(pf, lane, g, first + 2 * qn);
+        if (qn < p1) load_pair_ahead<R, BUF>(pf, lane, g, first + 2 * qn);
         wide_compute<ALL3>(c, mult, exch, grp, w, lane, g, x0, x1);
-        if (on) {
-            store_system<R>(stg, lane, g, sys0, x0);
-            if (sys0 + 1 < g.nsys) store_system<R>(stg, lane, g, sys0 + 1, x1);
-        }
+        store_pair<R, BUF>(stg, lane, g, sys0, x0, x1, on);
     }
 }
 
@@ -1534,7 +1601,7 @@ __global__ __launch_bounds__(kWideThreads) void jw_wide64_kernel(jw_run_desc d, 
                          d.out_hi, d.kl, d.ku, d.fwd, d.b1, d.b2, d.apply_scale, d.scale_hi, w, lane);
     };
     double2 pf[2][kWideR / 2] = {};
-    auto first = [&] { if (p + grp < npass) load_pair_ahead<kWideR>(pf, lane, geo(), 2 * (p + grp)); };
+    auto first = [&] { if (p + grp < npass) load_pair_ahead<kWideR, false>(pf, lane, geo(), 2 * (p + grp)); };
     wide_coef c;
     if constexpr (BUILD) {
         const wide_sink sink{reinterpret_cast<double*>(smem + kWideSlots), c, w, lane};
@@ -1549,7 +1616,7 @@ __global__ __launch_bounds__(kWideThreads) void jw_wide64_kernel(jw_run_desc d, 
         wide_multipliers(c, reinterpret_cast<double*>(smem + kWideMult),
                          reinterpret_cast<double*>(smem + kWideExch) + kWideGroups * kWideW * (8 + 3 * 2), w, lane);
     __syncthreads();
-    wide_stream<ALL3>(c, smem, grp, w, lane, geo, 0, p, npass, step, pf);
+    wide_stream<ALL3, false>(c, smem, grp, w, lane, geo, 0, p, npass, step, pf);
 }
 
 // ---------------------------------------------------------------------------
@@ -1746,6 +1813,7 @@ __global__ __launch_bounds__(64 * chain_max_waves(R)) void jw_chain64_kernel(jw_
     if (solve)
         for (int k = wave; k < kl; k += nwaves) chain_multipliers<R, UP>(ltab + k * TE, lane);
     __syncthreads();
+    if constexpr (pair_ahead(R)) hold_pair<R>(pf);
     while (q < npass) {
         double x0[R], x1[R];
         if constexpr (pair_ahead(R)) unpack_ahead<R>(pf, stg, lane, g, 2 * q, x0, x1);
@@ -1756,8 +1824,7 @@ __global__ __launch_bounds__(64 * chain_max_waves(R)) void jw_chain64_kernel(jw_
             chain_pair<R, UP>(ltab + k * TE, lane, d.band, solve, g.apply_scale, g.row0_scale, x0, x1);
         for (int k = kl; k < K; k++)
             chain_pair<R, UP>(gtab + (int64_t)k * TE, lane, d.band, solve, g.apply_scale, g.row0_scale, x0, x1);
-        store_system<R>(stg, lane, g, 2 * q, x0);
-        if (2 * q + 1 < d.nsys) store_system<R>(stg, lane, g, 2 * q + 1, x1);
+        store_pair<R, pair_ahead(R)>(stg, lane, g, 2 * q, x0, x1, true);
         q = qn;
     }
 }
@@ -2342,7 +2409,7 @@ __global__ __launch_bounds__(kWideThreads) void jw_batch64w_kernel(const jw_batc
             __syncthreads();
             cur = un.item;
         }
-        wide_stream<true>(c, smem, grp, w, lane, geo, un.pair0, 0, npass, kWideGroups, pf);
+        wide_stream<true, true>(c, smem, grp, w, lane, geo, un.pair0, 0, npass, kWideGroups, pf);
     }
     queue_leave(counter);
 }
