@@ -213,7 +213,10 @@ void pfsolve_batch_destroy(pfsolve_batch* b);
  * output rhs_out, systems contiguous) whose fused-step matrices (the jw_type
  * 14 / 1014 layout, host memory, unchanged during the run) are identified by
  * matrix_key.  Requests are admitted in arrival order while device memory (one
- * arena of hbm_budget bytes for bundles in flight and resident matrices) and
+ * arena of hbm_budget bytes, or of what all requests need if that is less, for
+ * bundles in flight and resident matrices; a slot's descriptors and new matrices on
+ * their way take at most 4 MiB and 1/64 of the budget more, plus 1.5 KiB per request
+ * of a launch) and
  * max_inflight allow; matrices and their coefficient table stay resident per key
  * (any number of keys) until the arena needs their room: keys with no request in
  * flight are then evicted least recently used first.  Every admitted request
@@ -223,7 +226,8 @@ void pfsolve_batch_destroy(pfsolve_batch* b);
  * are still on the device; finished launches are found from their events.
  * realtime = 1 admits a request no earlier than its arrival_s (seconds from the
  * start, wall clock); realtime = 0 treats every request as arrived at the start.
- * Host buffers should be pinned for the copies to overlap.  A request that cannot
+ * Host buffers should be pinned (one coherent allocation each): a kernel then moves
+ * the bundles of a launch together; others are copied one by one.  A request that cannot
  * fit the budget even alone is rejected (status PFSOLVE_ERROR_FAILED_TO_ALLOCATE),
  * as is a key reused with another N (PFSOLVE_ERROR_UNSUPPORTED_FFT_LENGTH) or with
  * another band (KL, KU), matrix offsets or storage order (PFSOLVE_ERROR_UNSUPPORTED_RADIX).  A launch that fails ends its requests with

@@ -65,6 +65,71 @@ __global__ __launch_bounds__(NT, NT == 256 ? 4 : 2) void jw_prologue_batch_kerne
 }
 
 // ------------------------------------------------------------------------
+// packed bundles between mapped host memory and padded device memory
+// ------------------------------------------------------------------------
+// Bound by the host link (57 GB/s; both directions at once share it here).  The runtime's
+// copies reach that rate too, but one bundle after another with gaps of 15 to 100 us between
+// them, row by row where a system's stride is padded (odd N).  Here all bundles of a launch
+// are one flat queue of tiles, a wavefront's instruction one contiguous KiB of the host's
+// side, and each thread has 8 loads of 16 bytes in flight, 32 KiB per workgroup: 24 MB take
+// 409 us alone.  16 workgroups cover the link's latency; 64 are no faster, and the reads they
+// queue hold up whatever else crosses the link (200 small requests: 5.5 ms against 5.7).  48
+// requests of up to 2048 rows, 140 MB each way: 9.1 ms by copies, 5.7 ms so (two times 2.46
+// ms for the bytes alone).
+constexpr int kMoveThreads = 256, kMoveLoads = 8, kMoveTile = 2 * kMoveLoads * kMoveThreads;
+constexpr int kMoveGroups = 16;
+
+template <bool IN>
+__global__ __launch_bounds__(kMoveThreads) void jw_move_kernel(const jw_move_job* jobs, int njobs, int64_t ntiles)
+{
+    typedef double d2u __attribute__((ext_vector_type(2), aligned(8)));
+    for (int64_t t = blockIdx.x; t < ntiles; t += gridDim.x) {
+        int lo = 0, hi = njobs;   // the last job whose first tile is not behind t
+        while (hi - lo > 1) {
+            const int mid = (lo + hi) >> 1;
+            if (jobs[mid].first_tile <= t) lo = mid;
+            else hi = mid;
+        }
+        const jw_move_job job = jobs[lo];
+        const int64_t e0 = (t - job.first_tile) * kMoveTile, left = job.nsys * job.N - e0;
+        const uint32_t n = left < kMoveTile ? (uint32_t)left : (uint32_t)kMoveTile;
+        const int64_t row0 = e0 / job.N;
+        const uint32_t N = (uint32_t)job.N, col0 = (uint32_t)(e0 - row0 * job.N);
+        JW_GLOBAL double* host = as_global(reinterpret_cast<double*>(job.host)) + e0;
+        JW_GLOBAL double* dev = as_global(reinterpret_cast<double*>(job.dev)) + row0 * job.stride;
+        // element p of the tile on the device's side
+        auto at = [&](uint32_t p) -> JW_GLOBAL double* {
+            const uint32_t c = col0 + p, r = c / N;
+            return dev + (int64_t)r * job.stride + (c - r * N);
+        };
+        d2u v[kMoveLoads];
+#pragma unroll
+        for (int k = 0; k < kMoveLoads; k++) {
+            const uint32_t p = 2 * (k * kMoveThreads + threadIdx.x);
+            v[k] = d2u{0.0, 0.0};
+            if constexpr (IN) {
+                if (p + 1 < n) v[k] = __builtin_nontemporal_load((JW_GLOBAL d2u*)(host + p));
+                else if (p < n) v[k].x = host[p];
+            } else {
+                if (p < n) v[k].x = *at(p);
+                if (p + 1 < n) v[k].y = *at(p + 1);
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < kMoveLoads; k++) {
+            const uint32_t p = 2 * (k * kMoveThreads + threadIdx.x);
+            if constexpr (IN) {
+                if (p < n) *at(p) = v[k].x;
+                if (p + 1 < n) *at(p + 1) = v[k].y;
+            } else {
+                if (p + 1 < n) __builtin_nontemporal_store(v[k], (JW_GLOBAL d2u*)(host + p));
+                else if (p < n) host[p] = v[k].x;
+            }
+        }
+    }
+}
+
+// ------------------------------------------------------------------------
 // main kernel
 // ------------------------------------------------------------------------
 template <typename T> struct Pair { T a, b; };
@@ -573,6 +638,20 @@ int jwdev_prologue_batch(const jw_prologue_job* d_jobs, int njobs, int max_RL, i
     if (el != hipSuccess) { set_err("prologue batch launch", el); return -1; }
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) { set_err("prologue batch launch", e); return -1; }
+    return 0;
+}
+
+int jwdev_move_tile(void) { return kMoveTile; }
+
+int jwdev_move(const jw_move_job* d_jobs, int njobs, int64_t ntiles, int to_device, void* stream)
+{
+    if (njobs < 1 || ntiles < 1) return 0;
+    const int grid = ntiles < kMoveGroups ? (int)ntiles : kMoveGroups;
+    hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+    if (to_device) hipLaunchKernelGGL(jw_move_kernel<true>, dim3(grid), dim3(kMoveThreads), 0, s, d_jobs, njobs, ntiles);
+    else hipLaunchKernelGGL(jw_move_kernel<false>, dim3(grid), dim3(kMoveThreads), 0, s, d_jobs, njobs, ntiles);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) { set_err("move launch", e); return -1; }
     return 0;
 }
 

@@ -207,6 +207,17 @@ int jwdev_main64s(const jw_run_desc* r, const jw_source_desc* src, const void* m
 /* persistent uneven-batch kernel over a unit queue; *d_counter must be 0 at launch */
 int jwdev_batch64_occupancy(int R, int waves);
 int jwdev_zero_counters(int* d_counters, int n, void* stream);
+/* Packed bundles in mapped host memory (nsys systems of N rows, back to back) to or from
+ * device memory (rows `stride` apart), by a kernel; tiles of jwdev_move_tile() elements. */
+typedef struct jw_move_job {
+    void* host;               /* the device's address of the bundle */
+    void* dev;
+    int64_t nsys, stride;
+    int64_t first_tile;       /* tiles of the jobs before this one */
+    int64_t N;
+} jw_move_job;
+int jwdev_move_tile(void);
+int jwdev_move(const jw_move_job* d_jobs, int njobs, int64_t ntiles, int to_device, void* stream);
 /* spw (R = 2 only): systems per wavefront pass, 2 (pairs), 4 (two 32-lane groups for sets
  * with N <= 64) or 8 (four 16-lane groups for N <= 32, two groups for 32 < N <= 64) */
 int jwdev_batch64(const jw_batch_item* d_items, const jw_batch_unit* d_units, int nunits, int* d_counter, int R,

@@ -13,9 +13,10 @@
  *   - merges every admitted, not yet launched request into one launch on the
  *     next free stream slot: the matrices of keys new to the device (copied and
  *     turned into their coefficient table on that stream; later launches on other
- *     streams wait for that event), host->device copies of the bundles, one
- *     persistent queue kernel per row class over all bundles of the launch (the
- *     kernels of the uneven-size batch), device->host copies, an event;
+ *     streams wait for that event), the bundles to the device (by one kernel those in
+ *     mapped host memory, by copies the others), one persistent queue kernel per row
+ *     class over all bundles of the launch (the kernels of the uneven-size batch), the
+ *     results back in the same way, an event;
  *   - finds finished launches by their events (blocking on the oldest one when
  *     nothing else can be done before the next arrival); a finished launch returns
  *     its memory, pins and slot, so requests that arrived meanwhile are admitted
@@ -291,7 +292,8 @@ typedef struct resident {
     jw_source_desc src;       /* where the table build finds them (offsets in the block) */
     void* table;
     hipEvent_t ready;         /* table written (recorded on the stream of the launch that wrote it) */
-    int written;              /* the table build is enqueued (ready recorded) */
+    int written;              /* 1: the table build is enqueued (ready recorded); -1: it will be, by
+                                 the launch being put together */
     int pins;                 /* admitted, unfinished requests using the key */
     int prev, next;           /* LRU links (pool indices, -1 none) */
     int live;
@@ -451,16 +453,71 @@ typedef struct slot {
     int nreqs;
     int* wrote;               /* keys whose table this launch writes */
     int nwrote;
-    jw_batch_item* h_items;   /* pinned */
-    jw_batch_unit* h_units;   /* pinned */
-    jw_batch_item* d_items;
-    jw_batch_unit* d_units;
+    hipEvent_t loaded;        /* the launch's bundles are on the device (jwdev_move) */
+    char* h_desc;             /* pinned: what a launch sends along (desc_layout) */
+    char* d_desc;
     int* d_counters;
 } slot;
+
+/* What a launch sends along, one block (offsets in bytes): its items, table builds and
+ * moves, the matrices of new keys (as far as kStageBytes goes) and the work units */
+typedef struct desc_layout { int64_t items, jobs, in, out, mats, units, end; } desc_layout;
+enum { kStageBytes = 4 << 20 };
+
+static int64_t aligned(int64_t bytes) { return (bytes + ALIGN - 1) / ALIGN * ALIGN; }
+
+static desc_layout desc_of(int64_t nb, int64_t mat_bytes, int64_t nunits)
+{
+    desc_layout l;
+    l.items = 0;
+    l.jobs = l.items + aligned(nb * (int64_t)sizeof(jw_batch_item));
+    l.in = l.jobs + aligned(nb * (int64_t)sizeof(jw_prologue_job));
+    l.out = l.in + aligned(nb * (int64_t)sizeof(jw_move_job));
+    l.mats = l.out + aligned(nb * (int64_t)sizeof(jw_move_job));
+    l.units = l.mats + aligned(mat_bytes);
+    l.end = l.units + aligned(nunits * (int64_t)sizeof(jw_batch_unit));
+    return l;
+}
+
+/* host memory, which the host may read (device and managed matrices are copied instead) */
+static int host_readable(const void* p)
+{
+    hipPointerAttribute_t a;
+    const int known = hipPointerGetAttributes(&a, p) == hipSuccess;
+    (void)hipGetLastError();
+    return !known || a.type == hipMemoryTypeHost || a.type == hipMemoryTypeUnregistered;
+}
+
+/* The device's address of [p, p + bytes) if the current device may read and write it from
+ * a kernel: one allocation (or registration) of mapped, coherent host memory of this device,
+ * whole doubles.  Anything else (pageable, managed, non-coherent or device memory) is NULL:
+ * the copies of the runtime take those. */
+static void* mapped_host(const serve_dev* d, const void* p, size_t bytes)
+{
+    if (d->dry || bytes == 0 || ((uintptr_t)p & 7)) return NULL;
+    hipPointerAttribute_t a, b;
+    hipDeviceptr_t base = 0;
+    size_t size = 0;
+    unsigned flags = 0;
+    int dev = -1;
+    void* at = NULL;
+    if (hipGetDevice(&dev) == hipSuccess && hipPointerGetAttributes(&a, p) == hipSuccess &&
+        a.type == hipMemoryTypeHost && a.device == dev && a.devicePointer &&
+        hipPointerGetAttributes(&b, (const char*)p + bytes - 1) == hipSuccess && b.type == hipMemoryTypeHost &&
+        b.device == dev && (char*)b.devicePointer == (char*)a.devicePointer + bytes - 1 &&
+        hipHostGetFlags(&flags, (void*)p) == hipSuccess && !(flags & hipHostMallocNonCoherent) &&
+        hipMemGetAddressRange(&base, &size, (hipDeviceptr_t)a.devicePointer) == hipSuccess &&
+        (char*)a.devicePointer >= (char*)base &&
+        (size_t)((char*)a.devicePointer - (char*)base) + bytes <= size)
+        at = a.devicePointer;
+    (void)hipGetLastError();   /* an unknown pointer is no error of a later launch */
+    return at;
+}
 
 typedef struct reqstate {
     int64_t off, bytes;       /* device block of the bundle, -1 when not admitted */
     int64_t stride;
+    void* host_out;           /* the results leave through jwdev_move (mapped host memory) */
     int key;                  /* pool index of the request's key while pinned, else -1 */
     int state;                /* 0 waiting, 1 admitted, 2 launched, 3 done, 4 rejected, 5 failed */
 } reqstate;
@@ -505,12 +562,53 @@ static void fused_source(const pfsolve_serve_request* q, jw_source_desc* src)
     src->permuted = !q->naturalOrder && q->N > 64;
 }
 
+/* a request's bundle as a job of jwdev_move; the tiles up to its end */
+static int64_t add_move(jw_move_job* j, void* host, void* dev, const pfsolve_serve_request* q, int64_t stride,
+                        int64_t first_tile)
+{
+    const int64_t tile = jwdev_move_tile();
+    j->host = host;
+    j->dev = dev;
+    j->nsys = q->nsys;
+    j->stride = stride;
+    j->first_tile = first_tile;
+    j->N = q->N;
+    return first_tile + (q->nsys * q->N + tile - 1) / tile;
+}
+
 typedef struct serve_run {
     serve_dev dev;
     arena A;
     keycache K;
     int nkeys_peak;
 } serve_run;
+
+/* bytes of a key's block: the matrices (padded), then the table */
+static int64_t key_bytes(const pfsolve_serve_request* q)
+{
+    return aligned(matrix_extent(q) * 8) + jwdev_table64_elems(2 << row_class(q->N)) * 8;
+}
+
+/* The arena: the budget, or less if every request and its key fit side by side (then no
+ * block ever waits for another, so nothing a request sees depends on the size).  A budget
+ * that the device does not have is refused either way.  Allocating and freeing 2 GiB for a
+ * call that uses 0.15 cost 0.3 ms and, now and then, 50 ms. */
+static int64_t arena_bytes(const serve_dev* d, const pfsolve_serve_config* cfg, const pfsolve_serve_request* reqs,
+                           int64_t nreq)
+{
+    int64_t need = 0;
+    for (int64_t i = 0; i < nreq; i++) {
+        const int64_t row = (reqs[i].N + (reqs[i].N & 1)) * 8;
+        const int64_t key = key_bytes(&reqs[i]);
+        if (reqs[i].nsys > cfg->hbm_budget / row || key < 0 || key > cfg->hbm_budget) return cfg->hbm_budget;
+        need += aligned(reqs[i].nsys * row) + aligned(key);
+        if (need >= cfg->hbm_budget) return cfg->hbm_budget;
+    }
+    size_t have = 0, total = 0;
+    if (!d->dry && (hipMemGetInfo(&have, &total) != hipSuccess || have < (size_t)cfg->hbm_budget))
+        return cfg->hbm_budget;
+    return need;
+}
 
 /* frees the key's block (its launches are all finished: it has no pins) */
 static void evict(serve_run* S, int v)
@@ -534,6 +632,21 @@ static int64_t alloc_evicting(serve_run* S, int64_t len)
         if (v < 0) return -1;
         evict(S, v);
     }
+}
+
+/* a slot's stream and buffers; opened when a launch first needs the slot (a stream and its
+ * end cost 0.15 ms) */
+static int slot_open(slot* x, const serve_dev* dev, int maxb, int64_t desc_bytes)
+{
+    x->reqs = (int64_t*)malloc(sizeof(int64_t) * (size_t)maxb);
+    x->wrote = (int*)malloc(sizeof(int) * (size_t)maxb);
+    if (!x->reqs || !x->wrote || dev_stream(dev, &x->stream) != 0 || dev_event(dev, &x->done) != 0 ||
+        dev_event(dev, &x->loaded) != 0 || dev_host_alloc(dev, (void**)&x->h_desc, (size_t)desc_bytes) != 0 ||
+        dev_alloc(dev, (void**)&x->d_desc, (size_t)desc_bytes) != 0 ||
+        dev_alloc(dev, (void**)&x->d_counters, sizeof(int) * 2 * NCLS) != 0)
+        return -1;
+    /* the slot's queues start empty (each queue kernel leaves them so) */
+    return dev->dry ? 0 : jwdev_zero_counters(x->d_counters, 2 * NCLS, x->stream);
 }
 
 PfSolveResult pfsolve_serve(const pfsolve_serve_config* cfg, pfsolve_serve_request* reqs, int64_t nreq,
@@ -569,30 +682,15 @@ PfSolveResult pfsolve_serve(const pfsolve_serve_config* cfg, pfsolve_serve_reque
     double* lat = (double*)malloc(sizeof(double) * (size_t)nreq);
     const int maxb = cfg->max_batch;
     /* units per launch: a request's passes are cut into at most kUnitsPerReq units */
-    const int64_t max_units = (int64_t)maxb * kUnitsPerReq;
+    int64_t stage = 0;
+    for (int64_t i = 0; i < nreq && stage < kStageBytes; i++) stage += aligned(matrix_extent(&reqs[i]) * 8);
+    if (stage > kStageBytes || stage < 0) stage = kStageBytes;
+    if (stage > cfg->hbm_budget / 64) stage = cfg->hbm_budget / 64;
+    const int64_t desc_bytes = desc_of(maxb, stage, (int64_t)maxb * kUnitsPerReq).end;
     if (!SL || !st || !pending || !lat) { res = PFSOLVE_ERROR_MALLOC_FAILED; goto out; }
-    if (arena_init(&S.A, dev, cfg->hbm_budget) != 0) { res = PFSOLVE_ERROR_FAILED_TO_ALLOCATE; goto out; }
+    if (arena_init(&S.A, dev, arena_bytes(dev, cfg, reqs, nreq)) != 0) { res = PFSOLVE_ERROR_FAILED_TO_ALLOCATE; goto out; }
     if (kc_init(&S.K, 1024) != 0) { res = PFSOLVE_ERROR_MALLOC_FAILED; goto out; }
-    for (int s = 0; s < cfg->streams; s++) {
-        slot* x = &SL[s];
-        if (dev_stream(dev, &x->stream) != 0 || dev_event(dev, &x->done) != 0 ||
-            dev_host_alloc(dev, (void**)&x->h_items, sizeof(jw_batch_item) * (size_t)maxb) != 0 ||
-            dev_host_alloc(dev, (void**)&x->h_units, sizeof(jw_batch_unit) * (size_t)max_units) != 0 ||
-            dev_alloc(dev, (void**)&x->d_items, sizeof(jw_batch_item) * (size_t)maxb) != 0 ||
-            dev_alloc(dev, (void**)&x->d_units, sizeof(jw_batch_unit) * (size_t)max_units) != 0 ||
-            dev_alloc(dev, (void**)&x->d_counters, sizeof(int) * 2 * NCLS) != 0) {
-            res = PFSOLVE_ERROR_FAILED_TO_ALLOCATE;
-            goto out;
-        }
-        /* the slot's queues start empty (each queue kernel leaves them so) */
-        if (!dev->dry && jwdev_zero_counters(x->d_counters, 2 * NCLS, x->stream) != 0) {
-            res = PFSOLVE_ERROR_FAILED_TO_LAUNCH_KERNEL;
-            goto out;
-        }
-        x->reqs = (int64_t*)malloc(sizeof(int64_t) * (size_t)maxb);
-        x->wrote = (int*)malloc(sizeof(int) * (size_t)maxb);
-        if (!x->reqs || !x->wrote) { res = PFSOLVE_ERROR_MALLOC_FAILED; goto out; }
-    }
+    if (slot_open(&SL[0], dev, maxb, desc_bytes) != 0) { res = PFSOLVE_ERROR_FAILED_TO_ALLOCATE; goto out; }
     for (int64_t i = 0; i < nreq; i++) {
         st[i].off = -1;
         st[i].key = -1;
@@ -614,6 +712,7 @@ PfSolveResult pfsolve_serve(const pfsolve_serve_config* cfg, pfsolve_serve_reque
     const double t0 = now_s();
     int64_t next = 0, npend = 0, ndone = 0, inflight = 0, launches = 0, launched_reqs = 0, failed = 0;
     int64_t integrity = 0;
+    int loading = -1;         /* slot of the newest launch with bundles moved by a kernel */
     double last_progress = now_s();
     while (ndone < nreq) {
         int progress = 0;
@@ -627,8 +726,8 @@ PfSolveResult pfsolve_serve(const pfsolve_serve_config* cfg, pfsolve_serve_reque
             r->bytes = q->nsys * r->stride * 8;
             int v = kc_find(&S.K, q->matrix_key);
             const int R = 2 << row_class(q->N);
-            const int64_t mbytes = (matrix_extent(q) * 8 + ALIGN - 1) / ALIGN * ALIGN;
-            const int64_t kbytes = mbytes + jwdev_table64_elems(R) * 8;
+            const int64_t mbytes = aligned(matrix_extent(q) * 8);
+            const int64_t kbytes = key_bytes(q);
             int status = PFSOLVE_SUCCESS;
             jw_source_desc qs;
             fused_source(q, &qs);
@@ -717,6 +816,10 @@ PfSolveResult pfsolve_serve(const pfsolve_serve_config* cfg, pfsolve_serve_reque
                 if (!SL[i].busy) { s = i; break; }
             if (s >= 0) {
                 slot* x = &SL[s];
+                if (!x->reqs && slot_open(x, dev, maxb, desc_bytes) != 0) {
+                    res = PFSOLVE_ERROR_FAILED_TO_ALLOCATE;
+                    goto out;
+                }
                 const int nb = npend < maxb ? (int)npend : maxb;
                 x->nreqs = nb;
                 x->nwrote = 0;
@@ -728,27 +831,49 @@ PfSolveResult pfsolve_serve(const pfsolve_serve_config* cfg, pfsolve_serve_reque
                 for (int i = 0; i < nb; i++) st[x->reqs[i]].state = 2;
                 int err = 0;
                 int64_t nunits = 0;
+                desc_layout L = desc_of(nb, 0, 0);
+                jw_batch_item* items = (jw_batch_item*)(x->h_desc + L.items);
+                jw_prologue_job* jobs = (jw_prologue_job*)(x->h_desc + L.jobs);
+                jw_move_job* in = (jw_move_job*)(x->h_desc + L.in);
+                jw_move_job* out = (jw_move_job*)(x->h_desc + L.out);
+                int64_t staged = 0;
+                int nin = 0, nout = 0;
+                int64_t in_tiles = 0, out_tiles = 0;
+                /* the table builds: N <= 1024 from the front, above from the back (a launch
+                 * each: a build's shape, and so its rounding, depends on its own N alone) */
+                int nlow = 0, nhigh = 0, rl_low = 0;
                 int64_t cls_first[NCLS], cls_n[NCLS];
                 for (int c = 0; c < NCLS; c++) cls_n[c] = 0;
-                /* keys new to the device: matrices copied and the table written on this
-                 * stream; keys written by an earlier launch: wait for that event */
+                /* keys new to the device: matrices sent along or copied, the table to be written
+                 * on this stream; keys written by an earlier launch: wait for that event */
                 for (int i = 0; i < nb && !err; i++) {
                     resident* k = &S.K.pool[st[x->reqs[i]].key];
                     if (!k->written) {
-                        if (dev_copy(dev, S.A.base + k->off, k->host_mat, (size_t)k->mat_bytes, x->stream) != 0 ||
-                            (!k->ready && dev_event(dev, &k->ready) != 0)) {
+                        const void* mats = S.A.base + k->off;
+                        if (!dev->dry && staged + aligned(k->mat_bytes) <= stage && host_readable(k->host_mat)) {
+                            memcpy(x->h_desc + L.mats + staged, k->host_mat, (size_t)k->mat_bytes);
+                            mats = x->d_desc + L.mats + staged;
+                            staged += aligned(k->mat_bytes);
+                        } else if (dev_copy(dev, S.A.base + k->off, k->host_mat, (size_t)k->mat_bytes,
+                                            x->stream) != 0) {
                             err = PFSOLVE_ERROR_FAILED_TO_COPY;
                             break;
                         }
-                        if (!dev->dry &&
-                            jwdev_prologue(&k->src, S.A.base + k->off, k->table, 64, k->R, JW_PREC_F64, 2, x->stream) != 0) {
-                            err = PFSOLVE_ERROR_FAILED_TO_LAUNCH_KERNEL;
+                        if (!k->ready && dev_event(dev, &k->ready) != 0) {
+                            err = PFSOLVE_ERROR_FAILED_TO_COPY;
                             break;
                         }
-                        if (dev_record(dev, k->ready, x->stream) != 0) { err = PFSOLVE_ERROR_FAILED_TO_EVENT_RECORD; break; }
-                        k->written = 1;
+                        const int low = k->R <= 16;
+                        jw_prologue_job* j = low ? &jobs[nlow++] : &jobs[nb - 1 - nhigh++];
+                        memset(j, 0, sizeof(*j));
+                        j->src = k->src;
+                        j->matrices = mats;
+                        j->table = k->table;
+                        j->R = k->R;
+                        if (low && 64 * k->R > rl_low) rl_low = 64 * k->R;
+                        k->written = -1;
                         x->wrote[x->nwrote++] = st[x->reqs[i]].key;
-                    } else if (dev_wait(dev, x->stream, k->ready) != 0) {
+                    } else if (k->written > 0 && dev_wait(dev, x->stream, k->ready) != 0) {
                         err = PFSOLVE_ERROR_FAILED_TO_LAUNCH_KERNEL;
                     }
                 }
@@ -757,14 +882,21 @@ PfSolveResult pfsolve_serve(const pfsolve_serve_config* cfg, pfsolve_serve_reque
                     const int64_t qi = x->reqs[i];
                     pfsolve_serve_request* q = &reqs[qi];
                     reqstate* r = &st[qi];
-                    if (q->nsys > 0 && dev_copy_rows(dev, S.A.base + r->off, (size_t)(r->stride * 8), q->rhs_in,
-                                                     (size_t)(q->N * 8), (size_t)(q->N * 8), (size_t)q->nsys,
-                                                     x->stream) != 0) {
+                    void* host = mapped_host(dev, q->rhs_in, (size_t)(q->nsys * q->N * 8));
+                    if (host) {
+                        in_tiles = add_move(&in[nin++], host, S.A.base + r->off, q, r->stride, in_tiles);
+                    } else if (q->nsys > 0 &&
+                               dev_copy_rows(dev, S.A.base + r->off, (size_t)(r->stride * 8), q->rhs_in,
+                                             (size_t)(q->N * 8), (size_t)(q->N * 8), (size_t)q->nsys,
+                                             x->stream) != 0) {
                         err = PFSOLVE_ERROR_FAILED_TO_COPY;
                         break;
                     }
+                    r->host_out = mapped_host(dev, q->rhs_out, (size_t)(q->nsys * q->N * 8));
+                    if (r->host_out)
+                        out_tiles = add_move(&out[nout++], r->host_out, S.A.base + r->off, q, r->stride, out_tiles);
                     const resident* k = &S.K.pool[r->key];
-                    jw_batch_item* it = &x->h_items[i];
+                    jw_batch_item* it = &items[i];
                     memset(it, 0, sizeof(*it));
                     it->rhs = S.A.base + r->off;
                     it->table = k->table;
@@ -778,6 +910,8 @@ PfSolveResult pfsolve_serve(const pfsolve_serve_config* cfg, pfsolve_serve_reque
                     it->scale = q->scaleC;
                 }
                 /* work units per row class, largest N first within a class */
+                L = desc_of(nb, staged, 0);
+                jw_batch_unit* units = (jw_batch_unit*)(x->h_desc + L.units);
                 for (int c = NCLS - 1; c >= 0 && !err; c--) {
                     cls_first[c] = nunits;
                     for (int i = 0; i < nb; i++) {
@@ -788,7 +922,7 @@ PfSolveResult pfsolve_serve(const pfsolve_serve_config* cfg, pfsolve_serve_reque
                         int64_t up = (passes + kUnitsPerReq - 1) / kUnitsPerReq;
                         if (up < 8) up = 8;
                         for (int64_t p = 0; p < passes; p += up) {
-                            jw_batch_unit* u = &x->h_units[nunits++];
+                            jw_batch_unit* u = &units[nunits++];
                             u->item = i;
                             u->pair0 = (int32_t)p;
                             u->pair1 = (int32_t)(p + up < passes ? p + up : passes);
@@ -799,26 +933,51 @@ PfSolveResult pfsolve_serve(const pfsolve_serve_config* cfg, pfsolve_serve_reque
                 /* a launch failure injected from the host: the kernels of this launch */
                 if (!err && cfg->fail_launch == launches) err = PFSOLVE_ERROR_FAILED_TO_LAUNCH_KERNEL;
                 if (!err && !dev->dry) {
-                    /* the queues are empty: zeroed at set-up, left empty by every queue kernel */
-                    if (dev_copy(dev, x->d_items, x->h_items, sizeof(jw_batch_item) * (size_t)nb, x->stream) != 0 ||
-                        (nunits > 0 &&
-                         dev_copy(dev, x->d_units, x->h_units, sizeof(jw_batch_unit) * (size_t)nunits, x->stream) != 0))
+                    L = desc_of(nb, staged, nunits);
+                    const jw_prologue_job* d_jobs = (const jw_prologue_job*)(x->d_desc + L.jobs);
+                    if (dev_copy(dev, x->d_desc, x->h_desc, (size_t)L.end, x->stream) != 0 ||
+                        jwdev_prologue_batch(d_jobs, nlow, rl_low, NULL, 0, x->stream) != 0 ||
+                        jwdev_prologue_batch(d_jobs + nb - nhigh, nhigh, 64 * 32, NULL, 0, x->stream) != 0)
                         err = PFSOLVE_ERROR_FAILED_TO_LAUNCH_KERNEL;
+                }
+                for (int w = 0; w < x->nwrote && !err; w++) {
+                    resident* k = &S.K.pool[x->wrote[w]];
+                    if (dev_record(dev, k->ready, x->stream) != 0) err = PFSOLVE_ERROR_FAILED_TO_EVENT_RECORD;
+                    k->written = 1;
+                }
+                if (!err && nin > 0) {
+                    /* The launches' bundles go to the device one launch after another: side by
+                     * side they would share the link and all arrive last. */
+                    if (loading >= 0 && loading != s && SL[loading].busy &&
+                        dev_wait(dev, x->stream, SL[loading].loaded) != 0)
+                        err = PFSOLVE_ERROR_FAILED_TO_LAUNCH_KERNEL;
+                    else if (jwdev_move((const jw_move_job*)(x->d_desc + L.in), nin, in_tiles, 1, x->stream) != 0)
+                        err = PFSOLVE_ERROR_FAILED_TO_LAUNCH_KERNEL;
+                    else if (dev_record(dev, x->loaded, x->stream) != 0)
+                        err = PFSOLVE_ERROR_FAILED_TO_EVENT_RECORD;
+                    loading = s;
+                }
+                if (!err && !dev->dry) {
+                    const jw_batch_item* d_items = (const jw_batch_item*)(x->d_desc + L.items);
+                    const jw_batch_unit* d_units = (const jw_batch_unit*)(x->d_desc + L.units);
+                    /* the queues are empty: zeroed at set-up, left empty by every queue kernel */
                     for (int c = 0; c < NCLS && !err; c++) {
                         if (!cls_n[c]) continue;
                         int64_t grid = cls_n[c] < grid_max[c] ? cls_n[c] : grid_max[c];
                         /* R = 2: sub-wavefront groups for requests with N <= 64 (8 systems
                          * per wavefront pass for N <= 32, 4 for N <= 64) */
-                        if (jwdev_batch64(x->d_items, x->d_units + cls_first[c], (int)cls_n[c], x->d_counters + 2 * c,
+                        if (jwdev_batch64(d_items, d_units + cls_first[c], (int)cls_n[c], x->d_counters + 2 * c,
                                           2 << c, waves[c], (int)grid, 8, x->stream) != 0)
                             err = PFSOLVE_ERROR_FAILED_TO_LAUNCH_KERNEL;
                     }
                 }
+                if (!err && jwdev_move((const jw_move_job*)(x->d_desc + L.out), nout, out_tiles, 0, x->stream) != 0)
+                    err = PFSOLVE_ERROR_FAILED_TO_LAUNCH_KERNEL;
                 for (int i = 0; i < nb && !err; i++) {
                     const int64_t qi = x->reqs[i];
                     pfsolve_serve_request* q = &reqs[qi];
                     reqstate* r = &st[qi];
-                    if (q->nsys > 0 && dev_copy_rows(dev, q->rhs_out, (size_t)(q->N * 8), S.A.base + r->off,
+                    if (q->nsys > 0 && !r->host_out && dev_copy_rows(dev, q->rhs_out, (size_t)(q->N * 8), S.A.base + r->off,
                                                      (size_t)(r->stride * 8), (size_t)(q->N * 8), (size_t)q->nsys,
                                                      x->stream) != 0)
                         err = PFSOLVE_ERROR_FAILED_TO_COPY;
@@ -951,10 +1110,9 @@ out:
             slot* x = &SL[s];
             dev_event_free(dev, x->done);
             dev_stream_free(dev, x->stream);
-            dev_host_free(dev, x->h_items);
-            dev_host_free(dev, x->h_units);
-            dev_free(dev, x->d_items);
-            dev_free(dev, x->d_units);
+            dev_event_free(dev, x->loaded);
+            dev_host_free(dev, x->h_desc);
+            dev_free(dev, x->d_desc);
             dev_free(dev, x->d_counters);
             free(x->reqs);
             free(x->wrote);
