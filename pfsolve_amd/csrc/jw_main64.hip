@@ -1085,55 +1085,126 @@ __global__ __launch_bounds__(max_threads<kLong64R>()) void jw_long64_kernel(jw_l
 
 // The front of a long FP64 step in one launch: the chunks' table builds, then COEF and
 // REDUCE of the first slice of systems behind them.  Workgroups take tickets in start
-// order.  The first nbuild build the tables, NSUB chunks each (pivots handed from build to
-// build), mark the build's tables written (tflags) and leave.  The others drain a queue
+// order.  The first nbuild build the tables, NSUB chunks each (the pivots' way through them:
+// below), mark the build's tables written (tflags) and leave.  The others drain a queue
 // of units in chunk order (unit 0 of a chunk: COEF on two wavefronts; unit j > 0: REDUCE of
-// pairs [(j-1) P, j P), two passes per wavefront), waiting for each chunk's tables before
+// pairs [(j-1) P, j P)), waiting for each chunk's tables before
 // staging them, so that the reduction runs while later tables are still being built.  A
 // worker's ticket comes after every build's, so every build it waits for has started, and
 // builds wait only for earlier builds: the launch drains whatever the residency.  All
 // waits are bounded (the device error flag is raised when one runs out).
 // sync: [0] ticket, [1] queue counter, [kLong64Tflags + b] build b's tables written;
-// slots: build b's last pivot (below); both set by jw_long64_clear_kernel before the launch.
-constexpr int kLong64Nsub = 6;   // chunks per table build (3072 rows: 384 threads in the pivot scan)
+// lines: the builds' maps and pivots (below); both set by jw_long64_clear_kernel before the launch.
+constexpr int kLong64Nsub = 4;   // chunks per table build: 2, 3, 4 and 6 measured 87, 88, 89
+                                 // and 93 us (100000 rows, 64 systems), 309, 275, 260 and
+                                 // 246 us (10^6 rows, 8 systems: 490 builds' maps at 4)
 constexpr int kLong64PairsPerUnit = 2 * (max_threads<kLong64R>() / 64);
+constexpr int kLong64UnitsPerWorker = 2;
 constexpr int kLong64Tflags = 32;   // the table flags start one 128-byte line after the counters
 
-// Pivot hand-over between the builds through one 64-bit slot per build that holds the bits
-// of the build's last pivot, all ones (a NaN pattern never published: a NaN pivot is
-// published as the canonical NaN) until then.  The value carries its own readiness, so
-// relaxed atomics suffice (the next build needs nothing else the previous one wrote): one
-// store and the polls that see it, no flag, no release or acquire.  The wait is bounded:
-// when it runs out the device error flag is raised and the build goes on with a unit pivot.
+// The pivots' way through the builds.  Every build publishes the map of its rows; a build
+// composes the maps of all builds before it (one wavefront, 64 at a time) for the pivot that
+// enters it, runs its rows, publishes its last pivot and checks its first one against the
+// last of the build before, as a build's threads check theirs.  If that holds for it and for
+// every build before it, its pivots stand.  If not (near a parabolic fixed point the scanned
+// products lose accuracy) it takes the final last pivot of the build before and makes its
+// pass again, refined where needed: from the first such build on, one build after another.
+// So the builds wait for three hand-overs, not for one per build before them: 100000 rows,
+// 2 systems 159 -> 111 us, 64 systems 128 -> 87, 512 systems 319 -> 312; 8 systems of 10^6
+// rows 1290 -> 257.  Where the scanned pivots do not hold (ld_r ud_{r-1} within 1e-7 of 1/4
+// everywhere, 64 systems of 100000 rows) the extra hand-overs cost 202 -> 227.
+// A word of a build's line holds all ones (a NaN pattern never published: a NaN is
+// published as the canonical one) until it is written; it carries its own readiness, so
+// relaxed atomics suffice, no flag, no release or acquire.  The waits are bounded: when one
+// runs out the device error flag is raised and the build goes on with a one, so the grid
+// always drains.
 constexpr unsigned long long kPivotEmpty = ~0ull;
+constexpr int kPivotLine = 8;   // words per build: the map (4), then
+enum { kPivotFirst = 4, kPivotState = 5, kPivotFinal = 6 };   // last pivot, whether it holds, and finally
 
-struct SlotHooks {
-    double* carry;                  // LDS: carry[0] = g entering the build
-    unsigned long long* slots;
+struct AheadHooks {
+    static constexpr bool kAhead = true;
+    double* carry;                  // LDS: carry[0] = g entering the build, carry[2]: settle's answer
+    unsigned long long* lines;
     int* err;
     int64_t build;
-    int chained;
-    __device__ void wait_carry(int tid) const
+    __device__ void put(int64_t b, int word, double v) const
     {
-        if (!chained || build == 0 || tid != 0) return;
+        const unsigned long long u = v != v ? 0x7FF8000000000000ull : (unsigned long long)__double_as_longlong(v);
+        __hip_atomic_store(&lines[b * kPivotLine + word], u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    __device__ double get(int64_t b, int word) const
+    {
         int polls = 0;
         unsigned long long v;
-        while ((v = __hip_atomic_load(&slots[build - 1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) == kPivotEmpty) {
+        while ((v = __hip_atomic_load(&lines[b * kPivotLine + word], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) ==
+               kPivotEmpty) {
             if (++polls > kLongMaxPolls) {
                 __hip_atomic_store(err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                v = (unsigned long long)__double_as_longlong(1.0);
-                break;
+                return 1.0;
             }
             __builtin_amdgcn_s_sleep(1);
         }
-        carry[0] = __longlong_as_double((long long)v);
+        return __longlong_as_double((long long)v);
+    }
+    __device__ void publish_map(double a, double b, double c, double e) const
+    {
+        put(build, 0, a);
+        put(build, 1, b);
+        put(build, 2, c);
+        put(build, 3, e);
+    }
+    // (wavefront 0; the pivot before row 0 may be any, the first row has no sub-diagonal)
+    __device__ void wait_carry(int tid) const
+    {
+        if (build == 0 || tid >= 64) return;
+        double ta = 1.0, tb = 0.0, tc = 0.0, te = 1.0;
+        for (int64_t b0 = 0; b0 < build; b0 += 64) {
+            double a = 1.0, b = 0.0, c = 0.0, e = 1.0;
+            if (b0 + tid < build) {
+                a = get(b0 + tid, 0);
+                b = get(b0 + tid, 1);
+                c = get(b0 + tid, 2);
+                e = get(b0 + tid, 3);
+            }
+            moebius_scan(a, b, c, e, tid);
+            a = readlane_d(a, 63);
+            b = readlane_d(b, 63);
+            c = readlane_d(c, 63);
+            e = readlane_d(e, 63);
+            moebius_compose(a, b, c, e, ta, tb, tc, te);
+            moebius_normalize(a, b, c, e);
+            ta = a; tb = b; tc = c; te = e;
+        }
+        // g = 1 / p of p = (ta + tb) / (tc + te)
+        if (tid == 0) carry[0] = (tc + te) / (ta + tb);
+    }
+    __device__ bool settle(int tid, bool refine, const double* gl, double p, double m) const
+    {
+        if (tid < 64) {
+            if (tid == 0) {
+                put(build, kPivotFirst, *gl);
+                bool bad = refine;
+                if (build > 0) {
+                    const double rho = (p - 1.0) + m * get(build - 1, kPivotFirst);
+                    bad = bad || !(fabs(rho) <= pivot_tol<double>() * fabs(p));
+                }
+                put(build, kPivotState, bad ? 1.0 : 0.0);
+            }
+            bool bad = false;
+            for (int64_t b = tid; b <= build; b += 64) bad = bad || get(b, kPivotState) != 0.0;
+            const bool again = __ballot(bad) != 0;
+            if (tid == 0) {
+                if (again && build > 0) carry[0] = get(build - 1, kPivotFinal);
+                carry[2] = again ? 1.0 : 0.0;
+            }
+        }
+        __syncthreads();
+        return carry[2] != 0.0;
     }
     __device__ void publish(int tid, const double* gl) const
     {
-        if (!chained || tid != 0) return;
-        const double g = *gl;
-        const unsigned long long v = g != g ? 0x7FF8000000000000ull : (unsigned long long)__double_as_longlong(g);
-        __hip_atomic_store(&slots[build], v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (tid == 0) put(build, kPivotFinal, *gl);
     }
 };
 
@@ -1154,14 +1225,13 @@ __device__ __forceinline__ void wait_table(int* flag, int* err)
 template <bool ALL3>
 __global__ __launch_bounds__(max_threads<kLong64R>()) void jw_long64_front_kernel(jw_source_desc src, const void* mat,
                                                                                  jw_long_desc d, int* sync,
-                                                                                 unsigned long long* slots, int* err,
-                                                                                 int nbuild, int chained)
+                                                                                 unsigned long long* lines, int* err,
+                                                                                 int nbuild, int chained, int P)
 {
     constexpr int R = kLong64R;
     constexpr int C = 64 * R;
     constexpr int SR = kLong64Nsub * C;
     constexpr int NTAB = JW_TAB64_ELEMS(R);
-    constexpr int P = kLong64PairsPerUnit;
     extern __shared__ __align__(16) unsigned char smem[];
     __shared__ int s_id;
     int* queue = sync + 1;
@@ -1178,8 +1248,8 @@ __global__ __launch_bounds__(max_threads<kLong64R>()) void jw_long64_front_kerne
         double* carry = reinterpret_cast<double*>(smem + prologue_lds_bytes(SR, sizeof(double)));
         if (chained && threadIdx.x == 0)
             carry[1] = rb > 0 ? mem_load<double>(mat, src.udS + source_pos(src, rb - 1, src.N), src.mem_f64) : 0.0;
-        const SlotHooks hooks{carry, slots, err, tk, chained};
-        prologue_body<double, 2, SlotHooks>(src, mat, table + (int64_t)tk * kLong64Nsub * NTAB, 64, R, smem, rb,
+        const AheadHooks hooks{carry, lines, err, tk};
+        prologue_body<double, 2, AheadHooks>(src, mat, table + (int64_t)tk * kLong64Nsub * NTAB, 64, R, smem, rb,
                                             chained ? carry : nullptr, kLong64Nsub, hooks);
         // every wavefront waits for its own table stores (written into the L2), then one
         // agent-scope release by thread 0 writes the L2 back and sets the flag (one L2
@@ -2599,10 +2669,10 @@ const void* pick_long64_front(bool all3)
 }
 
 // zeroes the counters and table flags, empties the pivot slots
-__global__ void jw_long64_clear_kernel(int* p, int n, unsigned long long* slots, int nslots)
+__global__ void jw_long64_clear_kernel(int* p, int n, unsigned long long* lines, int nwords)
 {
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) p[i] = 0;
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < nslots; i += gridDim.x * blockDim.x) slots[i] = kPivotEmpty;
+    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < nwords; i += gridDim.x * blockDim.x) lines[i] = kPivotEmpty;
 }
 
 // clears the work-queue counters (a kernel, so that it can sit in a captured graph)
@@ -3129,6 +3199,12 @@ int jwdev_main64s(const jw_run_desc* r, const jw_source_desc* src, const void* m
  * wavefronts per CU (the chunk's table and a staging of 2 x 512 rows per wavefront) */
 int jwdev_long64_nsub(void) { return kLong64Nsub; }
 
+int64_t jwdev_long64_table_bytes(int64_t N)
+{
+    const int64_t nbuild = (N + (int64_t)kLong64Nsub * 64 * kLong64R - 1) / ((int64_t)kLong64Nsub * 64 * kLong64R);
+    return nbuild * (kLong64Nsub * JW_TAB64_ELEMS(kLong64R) + kPivotLine) * 8;
+}
+
 int64_t jwdev_long64_lds_bytes(void)
 {
     return (int64_t)JW_TAB64_ELEMS(kLong64R) * 8 + 2LL * 64 * kLong64R * 8 * kLong64Waves;
@@ -3152,13 +3228,13 @@ int jwdev_long64_occupancy(void)
 
 /* the front of a step (jw_long64_front_kernel): the table builds of every chunk, COEF and
  * REDUCE of the slice in d (its first systems) in one launch, after a fill kernel that
- * zeroes the 32 + nbuild ints of sync and empties the nbuild 8-byte pivot slots at gval */
-int jwdev_long64_front(const jw_source_desc* src, const void* matrices, const jw_long_desc* d, int* sync, void* gval,
-                       int* err, int cu_count, int occupancy, void* stream)
+ * zeroes the 32 + nbuild ints of sync and empties the builds' pivot lines behind the tables */
+int jwdev_long64_front(const jw_source_desc* src, const void* matrices, const jw_long_desc* d, int* sync, int* err,
+                       int cu_count, int occupancy, void* stream)
 {
     const int C = 64 * kLong64R;
     const int64_t SR = (int64_t)kLong64Nsub * C;
-    if (!matrices || !d->table || !d->red || !d->run.rhs || !sync || !gval || !err) {
+    if (!matrices || !d->table || !d->red || !d->run.rhs || !sync || !err) {
         jwdev_set_error("long64 front: no matrices, table, reduced data, rhs or hand-over scratch");
         return -1;
     }
@@ -3174,16 +3250,26 @@ int jwdev_long64_front(const jw_source_desc* src, const void* matrices, const jw
         return -1;
     }
     const int64_t ppc = (d->run.nsys + 1) / 2;
-    const int64_t units = (int64_t)d->nchunks * (1 + (ppc + kLong64PairsPerUnit - 1) / kLong64PairsPerUnit);
+    /* pairs per unit: about two units a worker, in whole rounds of its wavefronts, since a unit
+     * of another chunk costs a table copy (512 systems of 100000 rows, units of 24 pairs: 330
+     * us, two units a worker: 320; one: 338, for the workers that get a second) */
+    const int64_t workers = (int64_t)cu_count * occupancy;
+    int64_t P = ((int64_t)d->nchunks * ppc + kLong64UnitsPerWorker * workers - 1) / (kLong64UnitsPerWorker * workers);
+    P = (P + kLong64Waves - 1) / kLong64Waves * kLong64Waves;
+    if (P < kLong64PairsPerUnit) P = kLong64PairsPerUnit;
+    if (P > ppc) P = ppc;
+    const int64_t units = (int64_t)d->nchunks * (1 + (ppc + P - 1) / P);
     if (units > (1LL << 30)) {
         jwdev_set_error("long64 front: too many work units");
         return -1;
     }
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
     const int nclear = (int)(kLong64Tflags + nbuild);
-    unsigned long long* slots = reinterpret_cast<unsigned long long*>(gval);
-    hipLaunchKernelGGL(jw_long64_clear_kernel, dim3((unsigned)((nclear + 255) / 256)), dim3(256), 0, s, sync, nclear,
-                       slots, (int)nbuild);
+    unsigned long long* lines = reinterpret_cast<unsigned long long*>(
+        reinterpret_cast<double*>(const_cast<void*>(d->table)) + nbuild * kLong64Nsub * JW_TAB64_ELEMS(kLong64R));
+    const int nwords = (int)nbuild * kPivotLine;
+    hipLaunchKernelGGL(jw_long64_clear_kernel, dim3((unsigned)((nwords + 32 + 255) / 256)), dim3(256), 0, s, sync,
+                       nclear, lines, nwords);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) {
         jwdev_set_error("long64 front: clear launch failed");
@@ -3191,7 +3277,7 @@ int jwdev_long64_front(const jw_source_desc* src, const void* matrices, const jw
     }
     const void* f = pick_long64_front(d->run.fwd && d->run.b1 && d->run.b2);
     const size_t lds = (size_t)jwdev_long64_lds_bytes();
-    if (prologue_lds_bytes((int)SR, sizeof(double)) + 2 * sizeof(double) > lds) {
+    if (prologue_lds_bytes((int)SR, sizeof(double)) + 3 * sizeof(double) > lds) {
         jwdev_set_error("long64 front: table build does not fit");
         return -1;
     }
@@ -3206,8 +3292,8 @@ int jwdev_long64_front(const jw_source_desc* src, const void* matrices, const jw
     const void* mat = matrices;
     jw_long_desc dd = *d;
     int nb = (int)nbuild;
-    int chained = src->solve_kind == JW_SOLVE_TRI;
-    void* args[] = {&sd, (void*)&mat, &dd, &sync, &slots, &err, &nb, &chained};
+    int chained = src->solve_kind == JW_SOLVE_TRI, pu = (int)P;
+    void* args[] = {&sd, (void*)&mat, &dd, &sync, &lines, &err, &nb, &chained, &pu};
     e = hipLaunchKernel(f, dim3((unsigned)grid), dim3(64 * kLong64Waves), args, lds, s);
     if (e != hipSuccess) {
         jwdev_set_error("long64 front: launch failed");

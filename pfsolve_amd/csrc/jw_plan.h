@@ -55,7 +55,8 @@ struct pfsolve_plan {
     int64_t long_nc, long_ntab, long_tab_elems, long_red_sys;
     size_t long_tab_off, long_red_off;
     /* pivot hand-over between table builds: ticket and per-build flags (ints), then the
-     * per-build last pivots from long_gval_off */
+     * per-build last pivots from long_gval_off (chunk kernel; the pair path keeps its builds'
+     * maps and pivots behind its tables) */
     size_t long_sync_off, long_gval_off;
     /* bytes of a slot's area the paths other than chunks use (the chunk fallback of FP64
      * 1025-2048 rows adds its tables after them), and the area actually provided (0: the

@@ -218,6 +218,7 @@ __device__ __forceinline__ int64_t source_pos(const jw_source_desc& d, int64_t r
 
 // No pivot hand-over between builds.
 struct NoPivotHooks {
+    static constexpr bool kAhead = false;
     __device__ void wait_carry(int) const {}
     template <typename T> __device__ void publish(int, const T*) const {}
 };
@@ -248,6 +249,54 @@ __device__ __forceinline__ dd lane_move(dd v)
 __device__ __forceinline__ double lane_read(double v, int lane) { return readlane_d(v, lane); }
 __device__ __forceinline__ dd lane_read(dd v, int lane) { return dd_make(readlane_d(v.hi, lane), readlane_d(v.lo, lane)); }
 
+// The pivot map p -> (a p + b) / (c p + e) of consecutive rows, up to a factor.
+// moebius_normalize rescales its entries by a power of two (exact), so that no product over-
+// or underflows: after at most four rows' maps or two scan steps.
+template <typename T>
+__device__ __forceinline__ void moebius_normalize(T& a, T& b, T& c, T& e)
+{
+    using A = Ar<T>;
+    const double mx = fmax(fmax(fabs(A::hi(a)), fabs(A::hi(b))), fmax(fabs(A::hi(c)), fabs(A::hi(e))));
+    const int ex = -__builtin_amdgcn_frexp_exp(mx);
+    a = A::ldexp_(a, ex); b = A::ldexp_(b, ex); c = A::ldexp_(c, ex); e = A::ldexp_(e, ex);
+}
+// X <- X * P (P: the maps of earlier rows, applied first)
+template <typename T>
+__device__ __forceinline__ void moebius_compose(T& a, T& b, T& c, T& e, T pa, T pb, T pc, T pe)
+{
+    using A = Ar<T>;
+    T na = A::madd(A::mul(a, pa), b, pc);
+    T nb = A::madd(A::mul(a, pb), b, pe);
+    T nc = A::madd(A::mul(c, pa), e, pc);
+    T ne = A::madd(A::mul(c, pb), e, pe);
+    a = na; b = nb; c = nc; e = ne;
+}
+// inclusive scan over the wavefront (lower lanes applied first): Hillis-Steele inside 16-lane
+// rows, then rows 1 and 3 take the ends of rows 0 and 2, rows 2 and 3 the end of row 1
+template <typename T>
+__device__ __forceinline__ void moebius_scan(T& a, T& b, T& c, T& e, int lane)
+{
+    const int tr = lane & 15;
+#define JW_SCAN_STEP(CTRL, MASK, ON)                                                                        \
+    do {                                                                                                    \
+        const T pa = lane_move<CTRL, MASK>(a), pb = lane_move<CTRL, MASK>(b);                               \
+        const T pc = lane_move<CTRL, MASK>(c), pe = lane_move<CTRL, MASK>(e);                               \
+        if (ON) moebius_compose(a, b, c, e, pa, pb, pc, pe);                                                \
+    } while (0)
+    JW_SCAN_STEP(DPP_ROW_SHR(1), 0xf, tr >= 1);
+    JW_SCAN_STEP(DPP_ROW_SHR(2), 0xf, tr >= 2);
+    moebius_normalize(a, b, c, e);
+    JW_SCAN_STEP(DPP_ROW_SHR(4), 0xf, tr >= 4);
+    JW_SCAN_STEP(DPP_ROW_SHR(8), 0xf, tr >= 8);
+    moebius_normalize(a, b, c, e);
+    JW_SCAN_STEP(0x142 /* row_bcast15 */, 0xa, lane & 16);
+    JW_SCAN_STEP(0x143 /* row_bcast31 */, 0xc, lane & 32);
+    moebius_normalize(a, b, c, e);
+#undef JW_SCAN_STEP
+}
+// residual bound of a scanned pivot that needs no refinement, relative: a few ulps
+template <typename T> constexpr double pivot_tol() { return sizeof(T) == 8 ? 0x1p-51 : 0x1p-103; }
+
 // One table build.  Local row r of the build is row rb + r of the system.  A build of a
 // long system's later rows (rb > 0) takes from `carry` the pivot of the row before its
 // first (carry[0] = g_{rb-1}) and that row's raw super-diagonal entry (carry[1] =
@@ -258,7 +307,12 @@ __device__ __forceinline__ dd lane_read(dd v, int lane) { return dd_make(readlan
 // Hooks of a build that hands its pivots on (tridiagonal solves only): wait_carry(tid),
 // called by every thread just before the barrier after which carry[0] is first read, and
 // publish(tid, g), called by every thread once the g of every row is final (g: the last
-// row's, in LDS).  `after` is called once the build's own loads are issued (FP64): loads
+// row's, in LDS).  With kAhead the carry need not be final: publish_map(a, b, c, e) gives
+// the map of the build's rows (one thread, before wait_carry), and settle(tid, refine, g, p,
+// m), called by every thread after the first pass (refine: that pass needs the refinement,
+// g: its last row's, p, m: the thread's first pivot and map entry), returns whether the pass
+// is to be made again (workgroup-uniform, carry[0] then final; it has a barrier).  `after` is
+// called once the build's own loads are issued (FP64): loads
 // issued there return behind them and overlap the build.
 // TP: T*, or a pointer to global memory stated as such.  FORMAT 3 folds as format 2, but
 // hands row-in-lane i, lane t of the thread's j-th row to sink(j, i, t, coefficients) and
@@ -443,21 +497,6 @@ __device__ __forceinline__ void prologue_body(const jw_source_desc& d, const voi
         const int RT = (RL + NP - 1) / NP;
         const int r0 = tid < NP ? tid * RT : RL;   // threads >= NP own no rows
         const int lane = tid & 63, wv = tid >> 6;
-        // the entries rescaled by a power of two (exact), so that no product over- or
-        // underflows: after at most four rows' maps or two scan steps
-        auto normalize = [](T& a, T& b, T& c, T& e) {
-            const double mx = fmax(fmax(fabs(A::hi(a)), fabs(A::hi(b))), fmax(fabs(A::hi(c)), fabs(A::hi(e))));
-            const int ex = -__builtin_amdgcn_frexp_exp(mx);
-            a = A::ldexp_(a, ex); b = A::ldexp_(b, ex); c = A::ldexp_(c, ex); e = A::ldexp_(e, ex);
-        };
-        // X <- X * P (P: the maps of earlier rows, applied first)
-        auto compose = [&](T& a, T& b, T& c, T& e, T pa, T pb, T pc, T pe) {
-            T na = A::madd(A::mul(a, pa), b, pc);
-            T nb = A::madd(A::mul(a, pb), b, pe);
-            T nc = A::madd(A::mul(c, pa), e, pc);
-            T ne = A::madd(A::mul(c, pb), e, pe);
-            a = na; b = nb; c = nc; e = ne;
-        };
         // the wavefronts past the first NP threads own no rows: they skip the scan
         // (wave-uniform) and only keep the barriers
         const bool part = wv < NP / 64;
@@ -484,28 +523,10 @@ __device__ __forceinline__ void prologue_body(const jw_source_desc& d, const voi
                 e = b;
                 a = na;
                 b = nb;
-                if ((i & 3) == 3) normalize(a, b, c, e);
+                if ((i & 3) == 3) moebius_normalize(a, b, c, e);
             }
-            normalize(a, b, c, e);
-            // inclusive scan inside the wavefront: Hillis-Steele inside 16-lane rows, then
-            // rows 1 and 3 take the ends of rows 0 and 2, rows 2 and 3 the end of row 1
-            const int tr = lane & 15;
-#define JW_SCAN_STEP(CTRL, MASK, ON)                                                                        \
-    do {                                                                                                    \
-        const T pa = lane_move<CTRL, MASK>(a), pb = lane_move<CTRL, MASK>(b);                               \
-        const T pc = lane_move<CTRL, MASK>(c), pe = lane_move<CTRL, MASK>(e);                               \
-        if (ON) compose(a, b, c, e, pa, pb, pc, pe);                                                        \
-    } while (0)
-            JW_SCAN_STEP(DPP_ROW_SHR(1), 0xf, tr >= 1);
-            JW_SCAN_STEP(DPP_ROW_SHR(2), 0xf, tr >= 2);
-            normalize(a, b, c, e);
-            JW_SCAN_STEP(DPP_ROW_SHR(4), 0xf, tr >= 4);
-            JW_SCAN_STEP(DPP_ROW_SHR(8), 0xf, tr >= 8);
-            normalize(a, b, c, e);
-            JW_SCAN_STEP(0x142 /* row_bcast15 */, 0xa, lane & 16);
-            JW_SCAN_STEP(0x143 /* row_bcast31 */, 0xc, lane & 32);
-            normalize(a, b, c, e);
-#undef JW_SCAN_STEP
+            moebius_normalize(a, b, c, e);
+            moebius_scan(a, b, c, e, lane);
             if (lane == 63) {
                 s_tot[4 * wv + 0] = a;
                 s_tot[4 * wv + 1] = b;
@@ -522,18 +543,28 @@ __device__ __forceinline__ void prologue_body(const jw_source_desc& d, const voi
             }
         }
         __syncthreads();   // the wavefront totals are in LDS
+        if constexpr (H::kAhead) {
+            // the map of all the build's rows, for the builds behind it
+            if (tid == NP - 1) {
+                for (int w = wv - 1; w >= 0; w--) {
+                    moebius_compose(a, b, c, e, s_tot[4 * w + 0], s_tot[4 * w + 1], s_tot[4 * w + 2], s_tot[4 * w + 3]);
+                    moebius_normalize(a, b, c, e);
+                }
+                hooks.publish_map(a, b, c, e);
+            }
+        }
         if (part && wv > 0) {
             // the maps of all earlier wavefronts, then the in-wavefront part on top (none of
             // it depends on a carry, so a build that waits for one has it ready)
             T wa = s_tot[0], wb = s_tot[1], wc = s_tot[2], we = s_tot[3];
             for (int w = 1; w < wv; w++) {
                 T ta = s_tot[4 * w + 0], tb = s_tot[4 * w + 1], tc = s_tot[4 * w + 2], te = s_tot[4 * w + 3];
-                compose(ta, tb, tc, te, wa, wb, wc, we);
+                moebius_compose(ta, tb, tc, te, wa, wb, wc, we);
                 wa = ta; wb = tb; wc = tc; we = te;
-                normalize(wa, wb, wc, we);
+                moebius_normalize(wa, wb, wc, we);
             }
-            compose(xa, xb, xc, xe, wa, wb, wc, we);
-            normalize(xa, xb, xc, xe);
+            moebius_compose(xa, xb, xc, xe, wa, wb, wc, we);
+            moebius_normalize(xa, xb, xc, xe);
         }
         hooks.wait_carry(tid);
         __syncthreads();   // the carry is in LDS, the totals are read: g's array is free
@@ -543,7 +574,8 @@ __device__ __forceinline__ void prologue_body(const jw_source_desc& d, const voi
         // (num - m den) / num: its g and p by two independent divisions; the others by the
         // exact recurrence p_r = 1 - ld_r ud_{r-1} g_{r-1},  g_r = 1 / p_r.
         T pr[MAXRT];
-        if (part) {
+        auto first_pass = [&] {
+            if (!part) return;
             const T gin = has_carry ? carry[0] : A::one();
             const T num = A::madd(xa, xb, gin), den = A::madd(xc, xe, gin);
             T gprev = A::one(), udprev = udp0;
@@ -567,7 +599,8 @@ __device__ __forceinline__ void prologue_body(const jw_source_desc& d, const voi
                 udprev = udv[i];
                 sg[at(r)] = g;
             }
-        }
+        };
+        first_pass();
         __syncthreads();   // every first-pass g is in sg
 
         // Refinement.  Near a parabolic fixed point of the pivot map (m_r -> 1/4, e.g. the
@@ -583,13 +616,26 @@ __device__ __forceinline__ void prologue_body(const jw_source_desc& d, const voi
         // row.  The refinement runs only when some first-row residual exceeds a few ulps
         // (the flag is raised by any thread, read by all: the choice is workgroup-uniform
         // and a function of the matrix alone, so every kernel still builds the same table).
-        if (part && r0 >= 1 && rb + r0 < N) {
-            const double tol = sizeof(T) == 8 ? 0x1p-51 : 0x1p-103;
+        auto check = [&] {
+            if (!part || r0 < 1 || rb + r0 >= N) return;
             const T rho0 = A::add(A::sub(pr[0], A::one()), A::mul(A::mul(ldv[0], udp0), sg[at(r0 - 1)]));
-            if (!(fabs(A::hi(rho0)) <= tol * fabs(A::hi(pr[0])))) sx[16] = A::one();
-        }
+            if (!(fabs(A::hi(rho0)) <= pivot_tol<T>() * fabs(A::hi(pr[0])))) sx[16] = A::one();
+        };
+        check();
         __syncthreads();
-        const bool refine = A::hi(sx[16]) != 0.0;
+        bool refine = A::hi(sx[16]) != 0.0;
+        if constexpr (H::kAhead) {
+            // a carry taken from the earlier builds' maps: when it does not hold (settle), the
+            // pass is made again from the pivot that the build before ends with
+            if (hooks.settle(tid, refine, sg + at(RL - 1), pr[0], A::mul(ldv[0], udp0))) {
+                if (tid == 0) sx[16] = A::zero();
+                first_pass();
+                __syncthreads();
+                check();
+                __syncthreads();
+                refine = A::hi(sx[16]) != 0.0;
+            }
+        }
         // not refined: every first-pass g is final (in sg since the barrier before the
         // check), so the last one goes to the next build at once
         if (!refine) hooks.publish(tid, sg + at(RL - 1));
@@ -843,6 +889,7 @@ constexpr int kLongMaxPolls = 1 << 22;
 
 template <typename T>
 struct ChainHooks {
+    static constexpr bool kAhead = false;
     T* carry;        // LDS: carry[0] = g entering the build
     int* flags;      // per build: 1 once its last pivot is in gval
     T* gval;         // per build: g of its last row

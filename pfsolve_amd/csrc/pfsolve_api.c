@@ -140,8 +140,7 @@ static PfSolveResult long_setup(PfSolveApplication* app, struct pfsolve_plan* p)
     /* the pair path's format-2 tables (builds of jwdev_long64_nsub chunks) in the same space */
     size_t tab_bytes = (size_t)p->long_ntab * p->long_tab_elems * elt;
     if (kp == JW_PREC_F64) {
-        const int64_t b64 = rows * jwdev_long64_nsub();
-        const size_t t64 = (size_t)((p->N + b64 - 1) / b64 * jwdev_long64_nsub()) * jwdev_table64_elems(8) * elt;
+        const size_t t64 = (size_t)jwdev_long64_table_bytes(p->N);
         if (t64 > tab_bytes) tab_bytes = t64;
     }
     p->long_red_off = p->long_tab_off + (tab_bytes + 255) / 256 * 256;
@@ -578,7 +577,7 @@ static PfSolveResult append_long(PfSolveApplication* app, const jw_source_desc* 
             d.run.offSol = run->offSol + s0 * run->stride;
             d.mode = JW_LONG_REDUCE;
             if (s0 == 0) {
-                if (jwdev_long64_front(src, cfg->buffer[0], &d, sync, gval, p->d_err, p->cu_count, p->long64_occ, s) != 0)
+                if (jwdev_long64_front(src, cfg->buffer[0], &d, sync, p->d_err, p->cu_count, p->long64_occ, s) != 0)
                     return PFSOLVE_ERROR_FAILED_TO_LAUNCH_KERNEL;
             } else if (jwdev_long64(&d, p->cu_count, p->long64_occ, s) != 0) {
                 return PFSOLVE_ERROR_FAILED_TO_LAUNCH_KERNEL;
