@@ -4,10 +4,12 @@
 // in XXII layout, or two consecutive real systems); lane t owns rows
 // t*R .. t*R+R-1 of both.  Per pair:
 //   1. input: the 16-byte chunks (row pairs) inside the input keep-range; the
-//      compute / store split kernel loads a lane's own chunks straight into
-//      registers one pass ahead, the pair and batch kernels DMA them global ->
-//      LDS (global_load_lds_dwordx4, 64 lanes per instruction on one contiguous
-//      KiB, XOR-swizzled slots so the blocked read-back is bank-conflict free);
+//      compute / store split kernel and the chained steps load a lane's own chunks
+//      straight into registers one pass ahead, the others contiguous chunks (64
+//      lanes per instruction on one KiB) that LDS turns into a lane's rows: loaded
+//      into registers one pass ahead, or by LDS DMA at the pass's start (queue
+//      kernel 1 at R <= 8, long systems; XOR-swizzled slots so the blocked
+//      read-back is bank-conflict free);
 //      an odd range end is read by its owning lane alone;
 //   2. banded matvec u' = a.(V x) with neighbour rows by DPP wave shifts;
 //   3. three first-order recurrences (forward W, backward Z, backward y),
@@ -19,9 +21,10 @@
 //      stored with 16-byte nontemporal stores (rows outside the output
 //      keep-range untouched; an odd range end is written by its owning lane).
 // Coefficients (8 per row, scalings folded) and scan multipliers come from the
-// per-matrix-set table (format 2): built by each workgroup of the split kernel
-// in its LDS, written by jw_prologue_kernel / jw_prologue_batch_kernel for the
-// other kernels and staged once per workgroup (or per work unit) in LDS.
+// per-matrix-set table (format 2): built by each workgroup in its LDS (plans), or
+// written by jw_prologue_kernel / jw_prologue_batch_kernel and staged once per
+// workgroup or work unit in LDS (batches, serving, the plain per-set form).
+// Systems of 1025 to 2048 rows: four wavefronts hold a pair (jw_wide64_kernel).
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 #include <stdio.h>
@@ -937,42 +940,50 @@ __device__ __forceinline__ void long64_pass(const double* tab, double2* stg, int
         e.cz[s] = 0.0;
         e.cy[s] = 0.0;
     }
-    if constexpr (MODE != JW_LONG_COEF) dma_pair<R>(stg, lane, g, sys0);
-    // the edges, loaded while the DMA is in flight
+    // The edges, loaded while the DMA is in flight: lane 0 and lane 63 take them.  Every lane
+    // loads (an address in bounds where it needs nothing) and selects afterwards: with a branch
+    // around each load the compiler waited for it there, four round trips one after another
+    // in FINISH.  With the stores below moved behind the arithmetic: 512 systems of 100000
+    // rows 322 -> 300 us, 1000 of 20000 rows 138 -> 130.
+    double l1[2], l2[2], ca[2], cb[2];
+    bool k1[2], k2[2];
+    if constexpr (MODE == JW_LONG_COEF) {
 #pragma unroll
-    for (int s = 0; s < 2; s++) {
-        const int64_t sys = sys0 + s;
-        if constexpr (MODE == JW_LONG_COEF) {
+        for (int s = 0; s < 2; s++) {
             // unit carries, zero right-hand sides: system 0 takes w, 1 takes z, 2 takes y
+            const int64_t sys = sys0 + s;
             if (lane == 0 && sys == 0) e.cw[s] = 1.0;
             if (lane == 63 && sys == 1) e.cz[s] = 1.0;
             if (lane == 63 && sys == 2) e.cy[s] = 1.0;
-        } else if (sys < g.nsys) {
-            const int64_t base = sys * rd.stride + rd.offSol;
-            if (rd.band) {
-                if constexpr (MODE == JW_LONG_REDUCE) {
-                    // rows next to the chunk, before any chunk is written: lane 0 rows rb-1,
-                    // rb-2, lane 63 rows rb+C, rb+C+1 (inside the input keep-range)
-                    const int64_t g1 = lane == 0 ? rb - 1 : rb + C;
-                    const int64_t g2 = lane == 0 ? rb - 2 : rb + C + 1;
-                    const bool edge = lane == 0 || lane == 63;
-                    if (edge && g1 >= rd.in_lo && g1 < rd.in_hi) e.h1[s] = rhs[base + g1];
-                    if (edge && g2 >= rd.in_lo && g2 < rd.in_hi) e.h2[s] = rhs[base + g2];
-                } else {
-                    // the same rows as REDUCE read them (the step runs in place)
-                    const bool lo = lane == 0 && c > 0, hi = lane == 63 && c + 1 < d.nchunks;
-                    if (lo || hi) {
-                        e.h1[s] = red[lo ? long_at(d, 6, c - 1, sys) : long_at(d, 3, c + 1, sys)];
-                        e.h2[s] = red[lo ? long_at(d, 5, c - 1, sys) : long_at(d, 4, c + 1, sys)];
-                    }
-                }
-            }
-            if constexpr (MODE == JW_LONG_FINISH) {
-                if (lane == 0) e.cw[s] = red[long_at(d, 7, c, sys)];
-                if (lane == 63) {
-                    e.cz[s] = red[long_at(d, 8, c, sys)];
-                    e.cy[s] = red[long_at(d, 9, c, sys)];
-                }
+        }
+    } else {
+        dma_pair<R>(stg, lane, g, sys0);
+        const bool first = lane == 0, last = lane == 63;
+#pragma unroll
+        for (int s = 0; s < 2; s++) {
+            const bool have = sys0 + s < g.nsys;
+            const int64_t sys = have ? sys0 + s : sys0;
+            if constexpr (MODE == JW_LONG_REDUCE) {
+                // rows next to the chunk, before any chunk is written: lane 0 rows rb-1,
+                // rb-2, lane 63 rows rb+C, rb+C+1 (inside the input keep-range)
+                const int64_t g1 = first ? rb - 1 : rb + C;
+                const int64_t g2 = first ? rb - 2 : rb + C + 1;
+                const bool edge = have && rd.band && (first || last);
+                k1[s] = edge && g1 >= rd.in_lo && g1 < rd.in_hi;
+                k2[s] = edge && g2 >= rd.in_lo && g2 < rd.in_hi;
+                const JW_GLOBAL double* x = as_global(rhs) + sys * rd.stride + rd.offSol;
+                l1[s] = x[k1[s] ? g1 : rb];
+                l2[s] = x[k2[s] ? g2 : rb];
+            } else {
+                // the same rows as REDUCE read them (the step runs in place), and the carries
+                k1[s] = k2[s] = have && rd.band && ((first && c > 0) || (last && c + 1 < d.nchunks));
+                const JW_GLOBAL double* r = as_global(red);
+                l1[s] = r[k1[s] ? (first ? long_at(d, 6, c - 1, sys) : long_at(d, 3, c + 1, sys))
+                                : long_at(d, 7, c, sys)];
+                l2[s] = r[k1[s] ? (first ? long_at(d, 5, c - 1, sys) : long_at(d, 4, c + 1, sys))
+                                : long_at(d, 7, c, sys)];
+                ca[s] = r[long_at(d, last ? 8 : 7, c, sys)];
+                cb[s] = r[long_at(d, 9, c, sys)];
             }
         }
     }
@@ -986,23 +997,28 @@ __device__ __forceinline__ void long64_pass(const double* tab, double2* stg, int
     } else {
         __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0): the DMA writes have landed in LDS
         compiler_fence();
-        read_pair<R>(stg, lane, g, sys0, x0, x1);
-    }
-    if constexpr (MODE == JW_LONG_REDUCE) {
-        // the rows the neighbouring chunks' banded matvec needs, as read
 #pragma unroll
         for (int s = 0; s < 2; s++) {
-            const int64_t sys = sys0 + s;
-            if (sys >= g.nsys) continue;
-            if (lane == 0) {
-                red[long_at(d, 3, c, sys)] = s == 0 ? x0[0] : x1[0];
-                red[long_at(d, 4, c, sys)] = s == 0 ? x0[1] : x1[1];
-            }
-            if (lane == 63) {
-                red[long_at(d, 5, c, sys)] = s == 0 ? x0[R - 2] : x1[R - 2];
-                red[long_at(d, 6, c, sys)] = s == 0 ? x0[R - 1] : x1[R - 1];
+            const bool have = sys0 + s < g.nsys;
+            e.h1[s] = k1[s] ? l1[s] : 0.0;
+            e.h2[s] = k2[s] ? l2[s] : 0.0;
+            if constexpr (MODE == JW_LONG_FINISH) {
+                e.cw[s] = have && lane == 0 ? ca[s] : 0.0;
+                e.cz[s] = have && lane == 63 ? ca[s] : 0.0;
+                e.cy[s] = have && lane == 63 ? cb[s] : 0.0;
             }
         }
+        read_pair<R>(stg, lane, g, sys0, x0, x1);
+    }
+    // REDUCE: the rows the neighbouring chunks' banded matvec needs, as read (lane 0: the
+    // first two, lane 63: the last two), stored with the boundary values: stored here, their
+    // acknowledgements were waited for before the arithmetic
+    double n0[2], n1[2];
+    if constexpr (MODE == JW_LONG_REDUCE) {
+        n0[0] = lane == 0 ? x0[0] : x0[R - 2];
+        n1[0] = lane == 0 ? x0[1] : x0[R - 1];
+        n0[1] = lane == 0 ? x1[0] : x1[R - 2];
+        n1[1] = lane == 0 ? x1[1] : x1[R - 1];
     }
     compute_pair<R, ALL3, 1, true>(tab, lane, g, x0, x1, &e);
     if constexpr (MODE == JW_LONG_FINISH) {
@@ -1025,12 +1041,11 @@ __device__ __forceinline__ void long64_pass(const double* tab, double2* stg, int
                     coef[9 * c + 3 * sys + 1] = e.zf[s];
                     coef[9 * c + 3 * sys + 2] = y0;
                 }
-            } else {
-                if (lane == 63) red[long_at(d, 0, c, sys)] = e.wl[s];
-                if (lane == 0) {
-                    red[long_at(d, 1, c, sys)] = e.zf[s];
-                    red[long_at(d, 2, c, sys)] = y0;
-                }
+            } else if (lane == 0 || lane == 63) {
+                red[long_at(d, lane == 0 ? 3 : 5, c, sys)] = n0[s];
+                red[long_at(d, lane == 0 ? 4 : 6, c, sys)] = n1[s];
+                red[long_at(d, lane == 0 ? 1 : 0, c, sys)] = lane == 0 ? e.zf[s] : e.wl[s];
+                if (lane == 0) red[long_at(d, 2, c, sys)] = y0;
             }
         }
     }
