@@ -135,7 +135,7 @@ constexpr int max_threads()
 // How the pair kernels (plain, batch queue kernels 1 and 4) move right-hand sides.  R = 16:
 // contiguous loads into registers one pass ahead and a staging of one system (8 KiB), so
 // that 8 wavefronts fit beside the 76 KiB table and no wavefront waits for its own loads;
-// 16384 systems of 1000 rows: 64 us per step, 74.5 us when R = 16 staged pairs by LDS DMA
+// 16384 systems of 1000 rows: 57 us per step, 74.5 us when R = 16 staged pairs by LDS DMA
 // (16 KiB each: 5 wavefronts, which waited for their loads) behind a table build launch.
 // Smaller R: LDS DMA into a staging of two systems at the pass's start, where 12 and more
 // wavefronts hide it (512 sets of 512 to 257 rows, solve: 51.5 us, 54.3 us one pass ahead).
