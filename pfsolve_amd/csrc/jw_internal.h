@@ -269,7 +269,6 @@ int jwdev_long_reduced(const jw_long_desc* d, int precision, void* stream);
 /* long FP64 systems whose rows are 16-byte aligned: the chunk modes on the pair machinery
  * (format-2 tables of JW_TAB64_ELEMS(8) elements per chunk, built by jwdev_long_prologue
  * when given that table size); a persistent grid of cu_count * occupancy workgroups at most */
-int jwdev_long64_nsub(void);   /* chunks per table build */
 int64_t jwdev_long64_table_bytes(int64_t N);   /* the tables, then a pivot line per build */
 int64_t jwdev_long64_lds_bytes(void);
 int jwdev_long64_occupancy(void);

@@ -3212,8 +3212,6 @@ int jwdev_main64s(const jw_run_desc* r, const jw_source_desc* src, const void* m
 
 /* Long FP64 systems (16-byte aligned) on the pair machinery: one workgroup of 12
  * wavefronts per CU (the chunk's table and a staging of 2 x 512 rows per wavefront) */
-int jwdev_long64_nsub(void) { return kLong64Nsub; }
-
 int64_t jwdev_long64_table_bytes(int64_t N)
 {
     const int64_t nbuild = (N + (int64_t)kLong64Nsub * 64 * kLong64R - 1) / ((int64_t)kLong64Nsub * 64 * kLong64R);

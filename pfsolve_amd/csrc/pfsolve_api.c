@@ -137,7 +137,7 @@ static PfSolveResult long_setup(PfSolveApplication* app, struct pfsolve_plan* p)
     cap = (cap + 1) / 2 * 2;
     p->long_red_sys = cap;
     p->long_tab_off = (p->table_bytes + 255) / 256 * 256;
-    /* the pair path's format-2 tables (builds of jwdev_long64_nsub chunks) in the same space */
+    /* the pair path's format-2 tables and pivot lines in the same space */
     size_t tab_bytes = (size_t)p->long_ntab * p->long_tab_elems * elt;
     if (kp == JW_PREC_F64) {
         const size_t t64 = (size_t)jwdev_long64_table_bytes(p->N);
