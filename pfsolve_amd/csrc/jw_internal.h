@@ -135,6 +135,27 @@ typedef struct jw_long_desc {
     int32_t nchunks, mode;
 } jw_long_desc;
 
+#ifdef __HIPCC__
+#define JW_HD __host__ __device__
+#else
+#define JW_HD
+#endif
+/* The row next to the chunk of C rows from row rb that a lane of REDUCE reads for the banded
+ * matvec: k = 0 the nearest, 1 the second; lane 0 before the chunk, lane 63 behind it.  -1
+ * where there is none to read: every other lane, and rows outside the input keep-range. */
+static inline JW_HD int64_t jw_long_edge_row(int64_t rb, int64_t C, int lane, int k, int64_t in_lo, int64_t in_hi)
+{
+    if (lane != 0 && lane != 63) return -1;
+    const int64_t row = lane == 0 ? rb - 1 - k : rb + C + k;
+    return row >= in_lo && row < in_hi ? row : -1;
+}
+/* A row that may be read in its place, for a keep-range that is not empty: the chunk's first
+ * one if it is in the range, else the range's nearest (the buffer need not hold any other). */
+static inline JW_HD int64_t jw_long_idle_row(int64_t rb, int64_t in_lo, int64_t in_hi)
+{
+    return rb < in_lo ? in_lo : (rb < in_hi ? rb : in_hi - 1);
+}
+
 /* One matrix set for the batched prologue (FP64, table format 2; one workgroup each). */
 typedef struct jw_prologue_job {
     jw_source_desc src;

@@ -941,10 +941,10 @@ __device__ __forceinline__ void long64_pass(const double* tab, double2* stg, int
         e.cy[s] = 0.0;
     }
     // The edges, loaded while the DMA is in flight: lane 0 and lane 63 take them.  Every lane
-    // loads (an address in bounds where it needs nothing) and selects afterwards: with a branch
-    // around each load the compiler waited for it there, four round trips one after another
-    // in FINISH.  With the stores below moved behind the arithmetic: 512 systems of 100000
-    // rows 322 -> 300 us, 1000 of 20000 rows 138 -> 130.
+    // loads (where it needs nothing, from inside the keep-range: the buffer need not hold a
+    // system's other rows) and selects afterwards: with a branch around each load the compiler
+    // waited for it there, four round trips one after another in FINISH.  With the stores below moved behind the arithmetic: 512 systems of 100000
+    // rows 332 -> 318 us, 1000 of 20000 rows 138 -> 130.
     double l1[2], l2[2], ca[2], cb[2];
     bool k1[2], k2[2];
     if constexpr (MODE == JW_LONG_COEF) {
@@ -964,16 +964,21 @@ __device__ __forceinline__ void long64_pass(const double* tab, double2* stg, int
             const bool have = sys0 + s < g.nsys;
             const int64_t sys = have ? sys0 + s : sys0;
             if constexpr (MODE == JW_LONG_REDUCE) {
-                // rows next to the chunk, before any chunk is written: lane 0 rows rb-1,
-                // rb-2, lane 63 rows rb+C, rb+C+1 (inside the input keep-range)
-                const int64_t g1 = first ? rb - 1 : rb + C;
-                const int64_t g2 = first ? rb - 2 : rb + C + 1;
-                const bool edge = have && rd.band && (first || last);
-                k1[s] = edge && g1 >= rd.in_lo && g1 < rd.in_hi;
-                k2[s] = edge && g2 >= rd.in_lo && g2 < rd.in_hi;
-                const JW_GLOBAL double* x = as_global(rhs) + sys * rd.stride + rd.offSol;
-                l1[s] = x[k1[s] ? g1 : rb];
-                l2[s] = x[k2[s] ? g2 : rb];
+                // rows next to the chunk, before any chunk is written, as offsets from a row that
+                // may be read (the same for the wavefront; an empty keep-range has none: the
+                // reduced data stand in)
+                const bool rows = rd.in_lo < rd.in_hi, edge = have && rd.band;
+                const int64_t idle = rows ? jw_long_idle_row(rb, rd.in_lo, rd.in_hi) : 0;
+                const JW_GLOBAL double* x =
+                    rows ? as_global(rhs) + sys * rd.stride + rd.offSol + idle : as_global(red);
+                const int64_t b1 = jw_long_edge_row(rb, C, 0, 0, rd.in_lo, rd.in_hi);
+                const int64_t b2 = jw_long_edge_row(rb, C, 0, 1, rd.in_lo, rd.in_hi);
+                const int64_t a1 = jw_long_edge_row(rb, C, 63, 0, rd.in_lo, rd.in_hi);
+                const int64_t a2 = jw_long_edge_row(rb, C, 63, 1, rd.in_lo, rd.in_hi);
+                k1[s] = edge && ((first && b1 >= 0) || (last && a1 >= 0));
+                k2[s] = edge && ((first && b2 >= 0) || (last && a2 >= 0));
+                l1[s] = x[k1[s] ? (first ? (int)(b1 - idle) : (int)(a1 - idle)) : 0];
+                l2[s] = x[k2[s] ? (first ? (int)(b2 - idle) : (int)(a2 - idle)) : 0];
             } else {
                 // the same rows as REDUCE read them (the step runs in place), and the carries
                 k1[s] = k2[s] = have && rd.band && ((first && c > 0) || (last && c + 1 < d.nchunks));
