@@ -1347,7 +1347,8 @@ __global__ __launch_bounds__(max_threads<kLong64R>()) void jw_long64_front_kerne
 // What crosses wavefronts goes through LDS: the two rows on each side for the matvec, and
 // per recurrence each wavefront's end value for a zero carry; a wavefront's carry follows
 // from those of the wavefronts before it (matrix-only factors), and enters a lane's rows
-// by one more multiplier, the product over the lanes before it.  Four barriers per pass; the
+// by one more multiplier, the product over the lanes before it.  A barrier per exchange, four
+// per pass with all three recurrences, two with one or none; the
 // arithmetic takes a third of the time the pass's memory traffic does.
 // Tables in memory (batches, the plain per-set form) are the format-2 tables of 32 rows per
 // lane, whose coefficients are read once per matrix set.
@@ -1626,6 +1627,9 @@ __device__ __forceinline__ void wide_compute(const wide_coef& c, const double* m
         x0[0] *= g.row0_scale;
         x1[0] *= g.row0_scale;
     }
+    // A recurrence's barrier comes after every wavefront has read its neighbours' rows; a
+    // product alone has none, and the next pass must not write rows still to be read
+    if (!ALL3 && !g.fwd && !g.b1 && !g.b2) __syncthreads();
 }
 
 // pass geometry of wavefront place w: its 512 rows of the system as a system of their own
