@@ -168,8 +168,7 @@ PfSolveResult pfsolve_batch_run(pfsolve_batch* b, hipStream_t stream);
  * matrices (except for row classes on queue kernel 4, whose solve builds them in
  * LDS); solve applies the resident tables to the right-hand sides.  A
  * caller whose matrices do not change between steps prepares once and then
- * only solves.  (Until the first prepare or solve, a run may build tables in LDS
- * and leave none in memory; a solve that finds none builds them from the matrices.) */
+ * only solves. */
 PfSolveResult pfsolve_batch_prepare(pfsolve_batch* b, hipStream_t stream);
 PfSolveResult pfsolve_batch_solve(pfsolve_batch* b, hipStream_t stream);
 PfSolveResult pfsolve_batch_run_plain(pfsolve_batch* b, hipStream_t stream);

@@ -11,8 +11,8 @@
  *      every row class builds its tables in LDS);
  *   2. per row class (R rows per lane, N <= 64 R): one persistent launch of a
  *      queue kernel over that class's work units.
- * An untuned class whose units hold whole sets builds its tables in LDS during a run
- * (group_run_kernel) as long as the caller never asks for resident tables.
+ * An untuned class whose units hold about whole sets builds its tables in LDS during a run
+ * (run_in_lds) and writes them out from there.
  * Work units are (set, range of system pairs), listed largest N first, so
  * the long units start early and the short ones fill the tail.
  */
@@ -38,7 +38,7 @@ struct pfsolve_batch {
     jw_prologue_job* d_jobs;          /* every set's table build, indexed by set */
     jw_prologue_job* d_gjobs;         /* the builds of the sets whose tables go to global memory */
     int64_t n_gjobs;
-    int64_t n_rjobs;                  /* the first n_rjobs of them: needed by a run that builds the others in LDS */
+    int64_t n_rjobs;                  /* the first n_rjobs of them: those a run does not build in LDS */
     jw_batch_item* d_items;
     jw_batch_unit* d_units;           /* units of all launch groups, back to back */
     int* d_counters;                  /* per launch group a queue (next unit, workgroups left; the
@@ -46,12 +46,9 @@ struct pfsolve_batch {
     /* launch groups: sets run with R_eff = 2 << g rows per lane */
     int64_t unit_first[NCLS], unit_count[NCLS];
     int group_waves[NCLS], group_grid[NCLS], group_kernel[NCLS];
-    /* what a run launches while no resident tables are wanted: kernel 4 where run_lds[g], the
-     * group's kernel otherwise */
+    /* what a run launches: kernel 4, which writes the tables it builds, where run_lds[g], the
+     * group's kernel on tables built before otherwise */
     int run_lds[NCLS], run_waves[NCLS], run_grid[NCLS];
-    /* resident tables: the caller has prepared or solved (a run then writes them too), and
-     * the tables in memory are those of the last prepare or run */
-    int want_tables, tables_ready;
     int wait_polls;                   /* bound of the split kernel's waits (0: default) */
     int64_t total_units, total_systems;
     pfsolve_batch_tuning tuning;
@@ -442,8 +439,8 @@ static PfSolveResult upload_queue(pfsolve_batch* b)
         jobs[s].table = (char*)b->tables + b->table_off[s];
         jobs[s].R = 2 << eff_group(b, s);
     }
-    /* first the sets whose tables every run needs in memory, then those that only resident
-     * tables (prepare) need */
+    /* first the sets whose tables a run needs built before its queues, then those it builds
+     * in LDS (built by the launch for prepare alone) */
     for (int lds = 0; lds < 2; lds++) {
         for (int64_t s = 0; s < b->nsets; s++) {
             const int g = eff_group(b, s);
@@ -461,7 +458,6 @@ static PfSolveResult upload_queue(pfsolve_batch* b)
     if (e != hipSuccess) return PFSOLVE_ERROR_FAILED_TO_COPY;
     if (b->graph_exec) { hipGraphExecDestroy(b->graph_exec); b->graph_exec = NULL; }
     if (b->graph) { hipGraphDestroy(b->graph); b->graph = NULL; }
-    b->tables_ready = 0;   /* the tables' places and forms may have changed */
     return PFSOLVE_SUCCESS;
 }
 
@@ -600,7 +596,7 @@ static int run_prologue(pfsolve_batch* b, int64_t njobs, hipStream_t stream)
     return 0;
 }
 
-/* the queue launches; lds: on kernel 4 where a run may build in LDS */
+/* the queue launches; lds: on kernel 4 where a run builds in LDS (and writes the tables) */
 static PfSolveResult launch_queues(pfsolve_batch* b, const jw_batch_item* d_items, hipStream_t stream, int only_group,
                                    int lds)
 {
@@ -613,7 +609,7 @@ static PfSolveResult launch_queues(pfsolve_batch* b, const jw_batch_item* d_item
         const jw_batch_unit* units = b->d_units + b->unit_first[g];
         const int n = (int)b->unit_count[g];
         int* queue = b->d_counters + 2 * g;
-        const int rc = k == 4   ? jwdev_batch64b(d_items, units, n, queue, 2 << g, w, grid, b->d_jobs, stream)
+        const int rc = k == 4   ? jwdev_batch64b(d_items, units, n, queue, 2 << g, w, grid, b->d_jobs, in_lds, stream)
                        : k == 2 ? jwdev_batch64s(d_items, units, n, queue, 2 << g, w, grid, b->d_counters + 2 * NCLS,
                                                  b->wait_polls, stream)
                        : k == 3 ? jwdev_batch64d(d_items, units, n, queue, 2 << g, w, grid, stream)
@@ -627,46 +623,26 @@ static PfSolveResult launch_queues(pfsolve_batch* b, const jw_batch_item* d_item
 static PfSolveResult launch_step(pfsolve_batch* b, const jw_batch_item* d_items, hipStream_t stream, int only_group,
                                  int with_prologue)
 {
-    if (with_prologue && run_prologue(b, b->n_gjobs, stream) != 0) return PFSOLVE_ERROR_FAILED_TO_LAUNCH_KERNEL;
-    return launch_queues(b, d_items, stream, only_group, 0);
+    if (with_prologue && run_prologue(b, b->n_rjobs, stream) != 0) return PFSOLVE_ERROR_FAILED_TO_LAUNCH_KERNEL;
+    return launch_queues(b, d_items, stream, only_group, with_prologue);
 }
 
-/* A run writes the tables (run = prepare + solve) when resident tables are wanted, and when
- * it is recorded (a replay cannot tell what was called since); otherwise the classes with
- * run_lds build theirs in LDS and leave none behind, which tables_ready = 0 tells a later
- * solve. */
 PfSolveResult pfsolve_batch_run(pfsolve_batch* b, hipStream_t stream)
 {
     if (!b) return PFSOLVE_ERROR_PLAN_NOT_INITIALIZED;
-    int recorded = 0;
-    if (stream) {
-        hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-        recorded = hipStreamIsCapturing(stream, &st) != hipSuccess || st != hipStreamCaptureStatusNone;
-    }
-    if (recorded) return launch_step(b, b->d_items, stream, -1, 1);
-    if (b->want_tables) {
-        b->tables_ready = 1;
-        return launch_step(b, b->d_items, stream, -1, 1);
-    }
-    b->tables_ready = 0;
-    if (run_prologue(b, b->n_rjobs, stream) != 0) return PFSOLVE_ERROR_FAILED_TO_LAUNCH_KERNEL;
-    return launch_queues(b, b->d_items, stream, -1, 1);
+    return launch_step(b, b->d_items, stream, -1, 1);
 }
 
 PfSolveResult pfsolve_batch_prepare(pfsolve_batch* b, hipStream_t stream)
 {
     if (!b) return PFSOLVE_ERROR_PLAN_NOT_INITIALIZED;
-    b->want_tables = 1;
-    b->tables_ready = 1;
     return run_prologue(b, b->n_gjobs, stream) == 0 ? PFSOLVE_SUCCESS : PFSOLVE_ERROR_FAILED_TO_LAUNCH_KERNEL;
 }
 
-/* after runs that left no tables for some classes, those build them in LDS once more */
 PfSolveResult pfsolve_batch_solve(pfsolve_batch* b, hipStream_t stream)
 {
     if (!b) return PFSOLVE_ERROR_PLAN_NOT_INITIALIZED;
-    b->want_tables = 1;
-    return launch_queues(b, b->d_items, stream, -1, !b->tables_ready);
+    return launch_step(b, b->d_items, stream, -1, 0);
 }
 
 PfSolveResult pfsolve_batch_run_plain(pfsolve_batch* b, hipStream_t stream)
@@ -785,9 +761,9 @@ PfSolveResult pfsolve_batch_get_info(const pfsolve_batch* b, pfsolve_batch_info*
     int64_t alg = 0;
     for (int64_t s = 0; s < b->nsets; s++) alg += 16 * b->sets[s].N * b->sets[s].nsys + 80 * b->sets[s].N;
     info->algorithmic_bytes = alg;
-    /* per step: the table build launch (when some class reads tables from global memory)
-     * and one queue launch per class */
-    int launches = (b->want_tables ? b->n_gjobs : b->n_rjobs) > 0 ? 1 : 0;
+    /* per run: the table build launch (when some class does not build in LDS) and one queue
+     * launch per class */
+    int launches = b->n_rjobs > 0 ? 1 : 0;
     for (int g = 0; g < NCLS; g++)
         if (b->unit_count[g]) { info->classes_used |= 1 << g; launches++; }
     info->launches = launches;

@@ -250,10 +250,10 @@ int jwdev_batch64d(const jw_batch_item* d_items, const jw_batch_unit* d_units, i
                    int waves, int grid, void* stream);
 /* the same queue with each set's table built in the workgroup's LDS from the matrices
  * of d_jobs[item] when the workgroup's set changes (R <= 16, waves >= 4): no table build
- * launch and no table in global memory */
+ * launch.  keep: the table of each set with a unit is also written to d_jobs[item].table */
 int jwdev_batch64b_occupancy(int R, int waves);
 int jwdev_batch64b(const jw_batch_item* d_items, const jw_batch_unit* d_units, int nunits, int* d_counter, int R,
-                   int waves, int grid, const jw_prologue_job* d_jobs, void* stream);
+                   int waves, int grid, const jw_prologue_job* d_jobs, int keep, void* stream);
 /* the same queue with the compute / store split (R <= 16): `ncomp` compute
  * wavefronts (0: default); *d_err is raised if a bounded wait ran out (after
  * `wait_polls` polls: 0 the default, negative none) */

@@ -2325,7 +2325,8 @@ __device__ __noinline__ void build_table_lds(const jw_prologue_job* job)
 template <int R, bool FULL>
 __global__ __launch_bounds__(max_threads<R>()) void jw_batch64b_kernel(const jw_batch_item* items,
                                                                        const jw_batch_unit* units, int nunits,
-                                                                       int* counter, const jw_prologue_job* jobs)
+                                                                       int* counter, const jw_prologue_job* jobs,
+                                                                       int keep)
 {
     extern __shared__ __align__(16) unsigned char smem[];
     constexpr int NTAB = JW_TAB64_ELEMS(R);
@@ -2364,11 +2365,20 @@ __global__ __launch_bounds__(max_threads<R>()) void jw_batch64b_kernel(const jw_
                 __syncthreads();
             }
         }
+        // the set's first unit writes the table for later solves (behind the first pairs' loads)
+        auto write_table = [&] {
+            if (!keep || un.pair0 != 0) return;
+            double* out = reinterpret_cast<double*>(jobs[un.item].table);
+            for (int i = 2 * threadIdx.x; i < NTAB; i += 2 * blockDim.x)
+                store_stream(out + i, *reinterpret_cast<const double2*>(tab + i));
+        };
         if constexpr (pair_ahead(R)) {
             double2 pf[2][R / 2];
             if (q < un.pair1) load_pair_ahead<R>(pf, lane, geo(), 2 * q);
+            write_table();
             stream_pairs<R, true>(tab, stg, lane, geo, q, un.pair1, nwaves, pf);
         } else {
+            write_table();
             for (int64_t p = q; p < un.pair1; p += nwaves) jw_pair64<R, true>(tab, stg, lane, geo(), 2 * p);
         }
     }
@@ -3050,7 +3060,7 @@ int jwdev_batch64b_occupancy(int R, int waves)
 }
 
 int jwdev_batch64b(const jw_batch_item* d_items, const jw_batch_unit* d_units, int nunits, int* d_counter, int R,
-                   int waves, int grid, const jw_prologue_job* d_jobs, void* stream)
+                   int waves, int grid, const jw_prologue_job* d_jobs, int keep, void* stream)
 {
     if (!batch64b_shape_ok(R, waves) || grid < 1 || !d_jobs) {
         snprintf(g_err64, sizeof(g_err64), "bad build-in-LDS batch launch (R=%d, waves=%d)", R, waves);
@@ -3061,7 +3071,7 @@ int jwdev_batch64b(const jw_batch_item* d_items, const jw_batch_unit* d_units, i
     hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) return -2;
     void* args[] = {const_cast<jw_batch_item**>(&d_items), const_cast<jw_batch_unit**>(&d_units), &nunits,
-                    &d_counter, const_cast<jw_prologue_job**>(&d_jobs)};
+                    &d_counter, const_cast<jw_prologue_job**>(&d_jobs), &keep};
     e = hipLaunchKernel(f, dim3(grid), dim3(64 * waves), args, lds, reinterpret_cast<hipStream_t>(stream));
     return e == hipSuccess ? 0 : -3;
 }
