@@ -237,16 +237,21 @@ static int group_waves_default(int g)
  * 128 - 65 rows 30.2 and 35.1; 1024 sets of 1024 - 513 rows 175, 196 and 252. */
 #define GROUP_KERNEL_DEFAULT 1
 
-/* Default 4 for a run that no resident tables are wanted from, where each set's table is then
- * built about once: at most two units per set, and for R <= 8 at most two sets per CU.  Run on
- * kernel 4 / table launch and kernel 1: 1024 sets of 1024 - 513 rows 196 / 215 us, 300 such
- * sets 86 / 94, 512 sets of 512 - 257 rows 58 / 61, 200 of them with 8 systems 22 / 28, but
- * 1024 sets of 512 - 257 rows with 32 systems 72 / 69 and 40 sets of 1024 systems 83 / 73.  R = 2:
- * only without sets of N <= 64, whose sub-wavefront groups kernel 4 does not have. */
-static int run_in_lds(int g, int64_t units, int64_t sets, int64_t min_n, int cu_count)
+/* Default 4 for a run whose tables are then built about once each: at most two units per set.
+ * R = 16: any number of sets (runs on kernel 4 / a table launch and kernel 1, in us: 100 sets of
+ * 1024 - 513 rows with 2, 16, 64 systems each 19 / 26, 26 / 32, 36 / 43; 1024 sets 67 / 66,
+ * 89 / 97, 205 / 214; 4096 sets with 2, 4, 8, 16 systems 240 / 249, 267 / 260, 301 / 296,
+ * 351 / 377).  R <= 8, where the tables a run writes weigh more: all units
+ * at once, one per CU (200 sets of 512 - 257 rows with 2, 64 systems 20 / 24, 34.2 / 34.4;
+ * 100 sets of 100 systems, two units each, 31 / 32, but 200 such sets 52 / 48), or two whole sets
+ * of few systems per CU (512 sets with 2, 8, 32, 64 systems 32 / 35, 36 / 37, 48 / 47, 64 / 61;
+ * 512 sets of 256 - 129 rows with 8, 64 systems 31 / 33, 44 / 43; 256 sets of 128 - 65 rows with
+ * 300 systems, two units each, 49 / 47).  R = 2: only without sets of N <= 64, whose
+ * sub-wavefront groups kernel 4 does not have. */
+static int run_in_lds(int g, int64_t units, int64_t sets, int64_t passes, int64_t min_n, int cu_count)
 {
-    if (g > 3 || units > 2 * sets) return 0;
-    return g == 3 || (sets <= 2 * (int64_t)cu_count && !(g == 0 && min_n <= 64));
+    if (g > 3 || units > 2 * sets || (g == 0 && min_n <= 64)) return 0;
+    return g == 3 || units <= cu_count || (units <= sets && sets <= 2 * (int64_t)cu_count && passes <= 8 * sets);
 }
 
 /* systems per wavefront pass of the R = 2 class on queue kernel 1 when not tuned: four
@@ -401,7 +406,7 @@ static PfSolveResult build_queue(pfsolve_batch* b, jw_batch_unit** out_units)
         b->group_waves[g] = w;
         b->group_grid[g] = (int)(grid > 0 ? grid : 1);
         b->group_kernel[g] = k;
-        if (untuned && run_in_lds(g, b->unit_count[g], nsets_g[g], min_n[g], b->cu_count)) {
+        if (untuned && run_in_lds(g, b->unit_count[g], nsets_g[g], passes_g[g], min_n[g], b->cu_count)) {
             const int rw = group_waves_default(g);
             const int ro = jwdev_batch64b_occupancy(2 << g, rw);
             int64_t rg = (int64_t)b->cu_count * ro;
