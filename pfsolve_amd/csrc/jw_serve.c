@@ -634,6 +634,20 @@ static int64_t alloc_evicting(serve_run* S, int64_t len)
     }
 }
 
+/* gives back what an open slot, or one that could not be opened, holds */
+static void slot_close(slot* x, const serve_dev* dev)
+{
+    dev_event_free(dev, x->done);
+    dev_stream_free(dev, x->stream);
+    dev_event_free(dev, x->loaded);
+    dev_host_free(dev, x->h_desc);
+    dev_free(dev, x->d_desc);
+    dev_free(dev, x->d_counters);
+    free(x->reqs);
+    free(x->wrote);
+    memset(x, 0, sizeof(*x));
+}
+
 /* a slot's stream and buffers; opened when a launch first needs the slot (a stream and its
  * end cost 0.15 ms) */
 static int slot_open(slot* x, const serve_dev* dev, int maxb, int64_t desc_bytes)
@@ -712,6 +726,7 @@ PfSolveResult pfsolve_serve(const pfsolve_serve_config* cfg, pfsolve_serve_reque
     const double t0 = now_s();
     int64_t next = 0, npend = 0, ndone = 0, inflight = 0, launches = 0, launched_reqs = 0, failed = 0;
     int64_t integrity = 0;
+    int nslots = cfg->streams;   /* slots that may be used */
     int loading = -1;         /* slot of the newest launch with bundles moved by a kernel */
     double last_progress = now_s();
     while (ndone < nreq) {
@@ -812,14 +827,17 @@ PfSolveResult pfsolve_serve(const pfsolve_serve_config* cfg, pfsolve_serve_reque
         /* 2. one launch of the pending requests on a free stream slot */
         if (npend > 0) {
             int s = -1;
-            for (int i = 0; i < cfg->streams; i++)
+            for (int i = 0; i < nslots; i++)
                 if (!SL[i].busy) { s = i; break; }
+            if (s >= 0 && !SL[s].reqs && slot_open(&SL[s], dev, maxb, desc_bytes) != 0) {
+                /* no memory for one more: the slots before it, all busy, carry on without */
+                slot_close(&SL[s], dev);
+                if (!dev->dry) (void)hipGetLastError();   /* no error of a later launch */
+                nslots = s;
+                s = -1;
+            }
             if (s >= 0) {
                 slot* x = &SL[s];
-                if (!x->reqs && slot_open(x, dev, maxb, desc_bytes) != 0) {
-                    res = PFSOLVE_ERROR_FAILED_TO_ALLOCATE;
-                    goto out;
-                }
                 const int nb = npend < maxb ? (int)npend : maxb;
                 x->nreqs = nb;
                 x->nwrote = 0;
@@ -1106,17 +1124,7 @@ out:
             slot* x = &SL[s];
             if (x->stream) dev_stream_sync(dev, x->stream);
         }
-        for (int s = 0; s < cfg->streams; s++) {
-            slot* x = &SL[s];
-            dev_event_free(dev, x->done);
-            dev_stream_free(dev, x->stream);
-            dev_event_free(dev, x->loaded);
-            dev_host_free(dev, x->h_desc);
-            dev_free(dev, x->d_desc);
-            dev_free(dev, x->d_counters);
-            free(x->reqs);
-            free(x->wrote);
-        }
+        for (int s = 0; s < cfg->streams; s++) slot_close(&SL[s], dev);
     }
     for (int v = 0; v < S.K.npool; v++)
         if (S.K.pool && S.K.pool[v].live) dev_event_free(dev, S.K.pool[v].ready);
