@@ -350,7 +350,7 @@ __device__ __forceinline__ void prologue_body(const jw_source_desc& d, const voi
     auto at = [](int r) -> int { return prologue_at(r); };
     T* sl = reinterpret_cast<T*>(smem_raw);    // raw ld, then l (format 1) or l' (format 2)
     T* sh = sl + RL;                           // raw ud, then h or h'
-    T* sE = sh + RL;                           // E (format 1) or 1 / D (format 2)
+    T* sE = sh + RL;                           // E (format 1) or D (format 2)
     T* sg = sE + RL;                           // g = 1 / pivot, then E (format 2)
     T* sx = sg + (RL > 32 ? RL : 32);          // the refinement's wavefront totals and flag
     const int tid = threadIdx.x;
@@ -453,6 +453,7 @@ __device__ __forceinline__ void prologue_body(const jw_source_desc& d, const voi
         if (r < RL) {
             sl[at(r)] = ldv;
             sh[at(r)] = udv;
+            if (FOLD && d.has_m) sE[at(r)] = Dr[j];
             if constexpr (FORMAT == 1) {
                 sE[at(r)] = Er[j];
                 table[tab1(r, 4, 0)] = Dr[j];
@@ -467,16 +468,6 @@ __device__ __forceinline__ void prologue_body(const jw_source_desc& d, const voi
     }
     if (tid == 0) sx[16] = A::zero();   // the refinement flag
     __syncthreads();
-    if (FOLD && d.has_m) {
-        // 1 / D of the rows (zero past the matrix), for the neighbours' fold
-#pragma unroll
-        for (int j = 0; j < MAXJ; j++) {
-            if (none(j)) continue;
-            const int r = row_of(j);
-            if (r < RL) sE[at(r)] = rb + r < N ? A::div(A::one(), Dr[j]) : A::zero();
-        }
-    }
-
     // phase 2: factors of the unit-diagonal solve.  Pivots p_r = 1 - m_r / p_{r-1},
     // m_r = ld_r ud_{r-1}: the Moebius map p -> (p - m)/p is the 2x2 matrix
     // [[1,-m],[1,0]] on (num, den).  Thread t < NP composes the maps of its RT
@@ -714,8 +705,6 @@ __device__ __forceinline__ void prologue_body(const jw_source_desc& d, const voi
         // (a build's first and last rows take D of the rows next to the build).  l', h' and
         // E then replace ld, ud and g in LDS (a row reads only its own of those).
         const int64_t te2 = JW_TAB64_ELEMS(R);
-        const T iprev = d.has_m && rb >= 1 ? A::div(A::one(), dprev) : A::one();
-        const T inext = d.has_m && rb + RL < N ? A::div(A::one(), dnext) : A::one();
 #pragma unroll
         for (int j = 0; j < MAXJ; j++) {
             const int r = none(j) ? RL : row_of(j);
@@ -729,11 +718,11 @@ __device__ __forceinline__ void prologue_body(const jw_source_desc& d, const voi
                 T lp = A::zero(), hp = A::zero();
                 if (rb + r >= 1 && rb + r < N) {
                     lp = A::mul(ar, sl[at(r)]);
-                    if (d.has_m) lp = A::mul(lp, r >= 1 ? sE[at(r - 1)] : iprev);
+                    if (d.has_m) lp = A::div(lp, r >= 1 ? sE[at(r - 1)] : dprev);
                 }
                 if (rb + r + 1 < N) {
                     hp = A::mul(ar, sh[at(r)]);
-                    if (d.has_m) hp = A::mul(hp, r + 1 < RL ? sE[at(r + 1)] : inext);
+                    if (d.has_m) hp = A::div(hp, r + 1 < RL ? sE[at(r + 1)] : dnext);
                 }
                 cf[5] = lp;
                 cf[6] = hp;
