@@ -251,7 +251,9 @@ __device__ __forceinline__ dd lane_read(dd v, int lane) { return dd_make(readlan
 
 // The pivot map p -> (a p + b) / (c p + e) of consecutive rows, up to a factor.
 // moebius_normalize rescales its entries by a power of two (exact), so that no product over-
-// or underflows: after at most four rows' maps or two scan steps.
+// or underflows: after at most two rows (whose entries are linear in each m; four rows' hold
+// m_r m_{r+2}, beyond range from |m| = 1e154 on) and after every product of two maps (a row
+// with |m| = 1e120 has entries of that ratio, whose products of four underflow).
 template <typename T>
 __device__ __forceinline__ void moebius_normalize(T& a, T& b, T& c, T& e)
 {
@@ -282,16 +284,14 @@ __device__ __forceinline__ void moebius_scan(T& a, T& b, T& c, T& e, int lane)
         const T pa = lane_move<CTRL, MASK>(a), pb = lane_move<CTRL, MASK>(b);                               \
         const T pc = lane_move<CTRL, MASK>(c), pe = lane_move<CTRL, MASK>(e);                               \
         if (ON) moebius_compose(a, b, c, e, pa, pb, pc, pe);                                                \
+        moebius_normalize(a, b, c, e);                                                                      \
     } while (0)
     JW_SCAN_STEP(DPP_ROW_SHR(1), 0xf, tr >= 1);
     JW_SCAN_STEP(DPP_ROW_SHR(2), 0xf, tr >= 2);
-    moebius_normalize(a, b, c, e);
     JW_SCAN_STEP(DPP_ROW_SHR(4), 0xf, tr >= 4);
     JW_SCAN_STEP(DPP_ROW_SHR(8), 0xf, tr >= 8);
-    moebius_normalize(a, b, c, e);
     JW_SCAN_STEP(0x142 /* row_bcast15 */, 0xa, lane & 16);
     JW_SCAN_STEP(0x143 /* row_bcast31 */, 0xc, lane & 32);
-    moebius_normalize(a, b, c, e);
 #undef JW_SCAN_STEP
 }
 // residual bound of a scanned pivot that needs no refinement, relative: a few ulps
@@ -514,9 +514,10 @@ __device__ __forceinline__ void prologue_body(const jw_source_desc& d, const voi
                 e = b;
                 a = na;
                 b = nb;
-                if ((i & 3) == 3) moebius_normalize(a, b, c, e);
+                if ((i & 1) == 1) moebius_normalize(a, b, c, e);
             }
-            moebius_normalize(a, b, c, e);
+            // (a row alone goes into the scan's first product as it is, which is two rows then)
+            if (MAXRT > 2 && RT > 1 && (RT & 1)) moebius_normalize(a, b, c, e);
             moebius_scan(a, b, c, e, lane);
             if (lane == 63) {
                 s_tot[4 * wv + 0] = a;
