@@ -681,9 +681,10 @@ static PfSolveResult append_impl(PfSolveApplication* app, const PfSolveLaunchPar
         if (p->long_only) return append_long(app, &src, &run, s, table);
         const uintptr_t base = (uintptr_t)run.rhs;
         run.vec2 = p->precision == JW_PREC_F64 && (base % 16) == 0 && (run.stride % 2) == 0 && (run.offSol % 2) == 0;
-        /* (the allocation-free entry point, whose area is capped, refuses unaligned systems of
-         * N > 1024 as the chunk path it would take does) */
-        const int in_lds = p->split64 || (p->waves64b && (run.vec2 || !(p->R64 == 32 && p->area_cap)));
+        /* unaligned systems of N > 1024 are taken where the chunk path takes them: not with
+         * kernelVariant 2, nor by the allocation-free entry point, whose area has no room for it */
+        const int chunks = p->long_R && !(p->area_cap && p->table_bytes > p->area_cap);
+        const int in_lds = p->split64 || (p->waves64b && (run.vec2 || p->R64 < 32 || chunks));
         if (p->R64 && (run.vec2 || (in_lds && base % 8 == 0)) && cfg->kernelVariant != 1) {
             /* wave-per-system kernels: table format 2, built by every workgroup, or by a
              * launch before where that variant is not available.  The kernels that build load and store
