@@ -297,6 +297,71 @@ __device__ __forceinline__ void read_edges(int lane, const jw_pass64& g, int64_t
 
 }
 
+// The banded matvec of a lane's rows: coef(p, i) is row i's coefficient pair (v_-2, v_-1),
+// (v_0, v_1), (v_2, .) for p = 0, 1, 2, m and p the rows on either side of the lane's.  All five
+// products are formed, with zeros where the band is narrower, so a NaN or infinity reaches the
+// rows on both sides (and through zero scan multipliers some more).  EXACT (a single operator, one
+// neighbour at most): rows outside the band count as zeros, and it spreads to the rows that depend
+// on it only.  Systems at odd addresses take that form, since the general kernel (their other one)
+// spreads it no further than a row or two; the fused step spreads it to every row in any case, and
+// the aligned single operators never had it: the selects cost 8192 systems of 256 rows 9.5 -> 9.9 us.
+struct band_side {
+    double a1, a2, b1, b2;   // nearest and second row, of both systems
+};
+template <int R, bool EXACT, bool FENCE, class Coef>
+__device__ __forceinline__ void band_rows(const Coef& coef, const jw_pass64& g, band_side m, band_side p,
+                                          double (&x0)[R], double (&x1)[R])
+{
+#pragma unroll
+    for (int i = 0; i < R; i++) {
+        const double2 c0 = coef(0, i), c1 = coef(1, i);
+        const double ia = x0[i], ib = x1[i];
+        double n1a = (i + 1 < R) ? x0[(i + 1) % R] : p.a1;
+        double n1b = (i + 1 < R) ? x1[(i + 1) % R] : p.b1;
+        double ua = c1.x * ia, ub = c1.x * ib;
+        if (EXACT) {
+            m.a1 = g.kl ? m.a1 : 0.0;
+            m.b1 = g.kl ? m.b1 : 0.0;
+            n1a = g.ku ? n1a : 0.0;
+            n1b = g.ku ? n1b : 0.0;
+        }
+        ua = __builtin_fma(c0.y, m.a1, ua);
+        ub = __builtin_fma(c0.y, m.b1, ub);
+        if (!EXACT) {
+            ua = __builtin_fma(c0.x, m.a2, ua);
+            ub = __builtin_fma(c0.x, m.b2, ub);
+        }
+        ua = __builtin_fma(c1.y, n1a, ua);
+        ub = __builtin_fma(c1.y, n1b, ub);
+        if (!EXACT) {
+            const double vp2 = coef(2, i).x;
+            ua = __builtin_fma(vp2, (i + 2 < R) ? x0[(i + 2) % R] : ((i + 2 == R) ? p.a1 : p.a2), ua);
+            ub = __builtin_fma(vp2, (i + 2 < R) ? x1[(i + 2) % R] : ((i + 2 == R) ? p.b1 : p.b2), ub);
+            m.a2 = m.a1;
+            m.b2 = m.b1;
+        }
+        m.a1 = ia;
+        m.b1 = ib;
+        x0[i] = ua;
+        x1[i] = ub;
+        if (FENCE && (i & 3) == 3) phase_barrier();
+    }
+}
+// the form of the kernels that build their table: all three recurrences, some, or some on
+// systems at odd addresses
+enum { kAllThree = 0, kSome = 1, kSomeExact = 2 };
+int solve_form(const jw_run_desc& r)
+{
+    return r.fwd && r.b1 && r.b2 ? kAllThree : (r.vec2 || r.kl > 1 || r.ku > 1 || r.fused_io ? kSome : kSomeExact);
+}
+
+// adds c s; where not `on` c is 0, and EXACT does not look at s
+template <bool EXACT>
+__device__ __forceinline__ double add_from(double c, double s, bool on, double a)
+{
+    return __builtin_fma(c, !EXACT || on ? s : 0.0, a);
+}
+
 // banded matvec, the three recurrences and row-0 scaleC, in registers.
 // ALL3: all three recurrences present (the fused step), decided at compile time.
 // G > 1 (R = 2 only): sub-wavefront groups.  The 64 lanes form G groups of LG = 64 / G
@@ -319,7 +384,7 @@ struct jw_edge64 {
     double wl[2], zf[2];
 };
 
-template <int R, bool ALL3, int G = 1, bool EDGE = false>
+template <int R, bool ALL3, int G = 1, bool EDGE = false, bool EXACT = false>
 __device__ __forceinline__ void compute_pair(const double* tab, int lane, const jw_pass64& g, double (&x0)[R],
                                              double (&x1)[R], jw_edge64* e = nullptr)
 {
@@ -350,33 +415,11 @@ __device__ __forceinline__ void compute_pair(const double* tab, int lane, const 
                 if (g.ku >= 2) { p2a = e->h2[0]; p2b = e->h2[1]; }
             }
         }
-#pragma unroll
-        for (int i = 0; i < R; i++) {
-            const double2 c0 = *reinterpret_cast<const double2*>(tab + tab_coef64(0, i, tl, R));
-            const double2 c1 = *reinterpret_cast<const double2*>(tab + tab_coef64(1, i, tl, R));
-            const double vp2 = tab[tab_coef64(2, i, tl, R)];
-            const double ia = x0[i], ib = x1[i];
-            const double n1a = (i + 1 < R) ? x0[(i + 1) % R] : p1a;
-            const double n1b = (i + 1 < R) ? x1[(i + 1) % R] : p1b;
-            const double n2a = (i + 2 < R) ? x0[(i + 2) % R] : ((i + 2 == R) ? p1a : p2a);
-            const double n2b = (i + 2 < R) ? x1[(i + 2) % R] : ((i + 2 == R) ? p1b : p2b);
-            double ua = c1.x * ia, ub = c1.x * ib;
-            ua = __builtin_fma(c0.y, m1a, ua);
-            ub = __builtin_fma(c0.y, m1b, ub);
-            ua = __builtin_fma(c0.x, m2a, ua);
-            ub = __builtin_fma(c0.x, m2b, ub);
-            ua = __builtin_fma(c1.y, n1a, ua);
-            ub = __builtin_fma(c1.y, n1b, ub);
-            ua = __builtin_fma(vp2, n2a, ua);
-            ub = __builtin_fma(vp2, n2b, ub);
-            m2a = m1a;
-            m2b = m1b;
-            m1a = ia;
-            m1b = ib;
-            x0[i] = ua;
-            x1[i] = ub;
-            if (R >= 16 && (i & 3) == 3) phase_barrier();
-        }
+        auto coef = [&](int p, int i) -> double2 {
+            const double* c = tab + tab_coef64(p, i, tl, R);
+            return p == 2 ? make_double2(*c, 0.0) : *reinterpret_cast<const double2*>(c);
+        };
+        band_rows<R, EXACT, (R >= 16)>(coef, g, band_side{m1a, m2a, m1b, m2b}, band_side{p1a, p2a, p1b, p2b}, x0, x1);
     }
     if (R >= 16) phase_barrier();
 
@@ -485,12 +528,12 @@ __device__ __forceinline__ void compute_pair(const double* tab, int lane, const 
             const double c3 = tab[SC + (j * 8 + 6) * 64 + lane];
             const double a1 = readlane_d(a, 16), a2 = readlane_d(a, 32), a3 = readlane_d(a, 48);
             const double b1 = readlane_d(b, 16), b2 = readlane_d(b, 32), b3 = readlane_d(b, 48);
-            a = __builtin_fma(c1, a1, a);
-            b = __builtin_fma(c1, b1, b);
-            a = __builtin_fma(c2, a2, a);
-            b = __builtin_fma(c2, b2, b);
-            a = __builtin_fma(c3, a3, a);
-            b = __builtin_fma(c3, b3, b);
+            a = add_from<EXACT>(c1, a1, lane < 16, a);
+            b = add_from<EXACT>(c1, b1, lane < 16, b);
+            a = add_from<EXACT>(c2, a2, lane < 32, a);
+            b = add_from<EXACT>(c2, b2, lane < 32, b);
+            a = add_from<EXACT>(c3, a3, lane < 48, a);
+            b = add_from<EXACT>(c3, b3, lane < 48, b);
         } else if (G == 2) {
             // the group's second row start: lane 16 of group 0, lane 48 of group 1
             const double c1 = tab[SC + (j * 8 + 4) * 64 + tl];
@@ -837,7 +880,7 @@ __device__ __forceinline__ void store_pair(double2* stg, int lane, const jw_pass
 // registers a pass ahead (pf holds the first pair's on entry), results leave through a
 // staging of one system.  geo() gives the pass geometry, rebuilt every pass from the kernel
 // arguments, so that nothing derived from them stays live in registers across the loop.
-template <int R, bool ALL3, class Geo>
+template <int R, bool ALL3, bool EXACT = false, class Geo>
 __device__ __forceinline__ void stream_pairs(const double* tab, double2* stg, int lane, const Geo& geo, int64_t q,
                                              int64_t q1, int64_t step, double2 (&pf)[2][R / 2])
 {
@@ -848,7 +891,7 @@ __device__ __forceinline__ void stream_pairs(const double* tab, double2* stg, in
         unpack_ahead<R>(pf, stg, lane, g, 2 * q, x0, x1);
         const int64_t qn = q + step;
         if (qn < q1) load_pair_ahead<R>(pf, lane, g, 2 * qn);
-        compute_pair<R, ALL3>(tab, lane, g, x0, x1);
+        compute_pair<R, ALL3, 1, false, EXACT>(tab, lane, g, x0, x1);
         store_pair<R, true>(stg, lane, g, 2 * q, x0, x1, true);
         q = qn;
     }
@@ -864,7 +907,7 @@ __device__ __forceinline__ void copy_table_lds(unsigned char* smem, const void* 
 
 // BUILD: the table is built in LDS from the caller's matrices (the stagings as scratch)
 // and pairs are loaded ahead at every R; otherwise it is copied from global memory.
-template <int R, bool ALL3, bool BUILD>
+template <int R, bool ALL3, bool BUILD, bool EXACT = false>
 __global__ __launch_bounds__(max_threads<R>()) void jw_main64_kernel(jw_run_desc d, jw_source_desc src, const void* mat)
 {
     constexpr int NTAB = JW_TAB64_ELEMS(R);
@@ -895,7 +938,7 @@ __global__ __launch_bounds__(max_threads<R>()) void jw_main64_kernel(jw_run_desc
             copy_table_lds<NTAB>(smem, d.table, wave, nwaves, lane);
         }
         __syncthreads();
-        stream_pairs<R, ALL3>(tab, stg, lane, geo, q, npass, step, pf);
+        stream_pairs<R, ALL3, EXACT>(tab, stg, lane, geo, q, npass, step, pf);
     } else {
         copy_table_lds<NTAB>(smem, d.table, wave, nwaves, lane);
         zero_staging<R>(stg, lane);
@@ -1462,7 +1505,7 @@ __device__ __forceinline__ void wide_multipliers(const wide_coef& c, double* mul
 }
 
 // the step on a pair, in registers; every wavefront of the workgroup calls it (barriers)
-template <bool ALL3>
+template <bool ALL3, bool EXACT>
 __device__ __forceinline__ void wide_compute(const wide_coef& c, const double* mult, double* exch, int grp, int w,
                                              int lane, const jw_pass64& g, double (&x0)[kWideR], double (&x1)[kWideR])
 {
@@ -1503,29 +1546,8 @@ __device__ __forceinline__ void wide_compute(const wide_coef& c, const double* m
             p2b = dpp_d<DPP_WAVE_SHL1>(x1[1]);
             if (hi) { p2a = rows[8 + 1]; p2b = rows[8 + 5]; }
         }
-#pragma unroll
-        for (int i = 0; i < R; i++) {
-            const double ia = x0[i], ib = x1[i];
-            const double n1a = (i + 1 < R) ? x0[(i + 1) % R] : p1a;
-            const double n1b = (i + 1 < R) ? x1[(i + 1) % R] : p1b;
-            const double n2a = (i + 2 < R) ? x0[(i + 2) % R] : ((i + 2 == R) ? p1a : p2a);
-            const double n2b = (i + 2 < R) ? x1[(i + 2) % R] : ((i + 2 == R) ? p1b : p2b);
-            double ua = c.p[1][i].x * ia, ub = c.p[1][i].x * ib;
-            ua = __builtin_fma(c.p[0][i].y, m1a, ua);
-            ub = __builtin_fma(c.p[0][i].y, m1b, ub);
-            ua = __builtin_fma(c.p[0][i].x, m2a, ua);
-            ub = __builtin_fma(c.p[0][i].x, m2b, ub);
-            ua = __builtin_fma(c.p[1][i].y, n1a, ua);
-            ub = __builtin_fma(c.p[1][i].y, n1b, ub);
-            ua = __builtin_fma(c.p[2][i].x, n2a, ua);
-            ub = __builtin_fma(c.p[2][i].x, n2b, ub);
-            m2a = m1a;
-            m2b = m1b;
-            m1a = ia;
-            m1b = ib;
-            x0[i] = ua;
-            x1[i] = ub;
-        }
+        auto coef = [&](int p, int i) -> double2 { return c.p[p][i]; };
+        band_rows<R, EXACT, false>(coef, g, band_side{m1a, m2a, m1b, m2b}, band_side{p1a, p2a, p1b, p2b}, x0, x1);
     }
     // forward recurrence
     if (ALL3 || g.fwd) {
@@ -1595,12 +1617,12 @@ __device__ __forceinline__ void wide_compute(const wide_coef& c, const double* m
         {
             const double a1 = readlane_d(a, 16), a2 = readlane_d(a, 32), a3 = readlane_d(a, 48);
             const double b1 = readlane_d(b, 16), b2 = readlane_d(b, 32), b3 = readlane_d(b, 48);
-            a = __builtin_fma(m[256], a1, a);
-            b = __builtin_fma(m[256], b1, b);
-            a = __builtin_fma(m[320], a2, a);
-            b = __builtin_fma(m[320], b2, b);
-            a = __builtin_fma(m[384], a3, a);
-            b = __builtin_fma(m[384], b3, b);
+            a = add_from<EXACT>(m[256], a1, lane < 16, a);
+            b = add_from<EXACT>(m[256], b1, lane < 16, b);
+            a = add_from<EXACT>(m[320], a2, lane < 32, a);
+            b = add_from<EXACT>(m[320], b2, lane < 32, b);
+            a = add_from<EXACT>(m[384], a3, lane < 48, a);
+            b = add_from<EXACT>(m[384], b3, lane < 48, b);
         }
         if (lane == 0) *reinterpret_cast<double2*>(e + 2 * w) = make_double2(a, b);
         double za = dpp_d<DPP_WAVE_SHL1>(a), zb = dpp_d<DPP_WAVE_SHL1>(b);
@@ -1653,7 +1675,7 @@ __device__ __forceinline__ jw_pass64 wide_pass(double* rhs, int64_t nsys, int64_
 // pairs p0 + 2 s + group for s = 0, step, ... (systems first + 2 pair, below the geometry's
 // nsys), one per group and pass, for a workgroup whose wavefronts hold their coefficients;
 // pf: the first pass's rows
-template <bool ALL3, bool BUF, class Geo>
+template <bool ALL3, bool BUF, bool EXACT = false, class Geo>
 __device__ __forceinline__ void wide_stream(const wide_coef& c, unsigned char* smem, int grp, int w, int lane,
                                             const Geo& geo, int64_t first, int64_t p, int64_t p1, int64_t step,
                                             double2 (&pf)[2][kWideR / 2])
@@ -1676,12 +1698,12 @@ __device__ __forceinline__ void wide_stream(const wide_coef& c, unsigned char* s
         unpack_ahead<R, BUF>(pf, stg, lane, g, sys0, x0, x1);
         const int64_t qn = q + step;
         if (qn < p1) load_pair_ahead<R, BUF>(pf, lane, g, first + 2 * qn);
-        wide_compute<ALL3>(c, mult, exch, grp, w, lane, g, x0, x1);
+        wide_compute<ALL3, EXACT>(c, mult, exch, grp, w, lane, g, x0, x1);
         store_pair<R, BUF>(stg, lane, g, sys0, x0, x1, on);
     }
 }
 
-template <bool ALL3, bool BUILD>
+template <bool ALL3, bool BUILD, bool EXACT = false>
 __global__ __launch_bounds__(kWideThreads) void jw_wide64_kernel(jw_run_desc d, jw_source_desc src, const void* mat)
 {
     extern __shared__ __align__(16) unsigned char smem[];
@@ -1710,7 +1732,7 @@ __global__ __launch_bounds__(kWideThreads) void jw_wide64_kernel(jw_run_desc d, 
         wide_multipliers(c, reinterpret_cast<double*>(smem + kWideMult),
                          reinterpret_cast<double*>(smem + kWideExch) + kWideGroups * kWideW * (8 + 3 * 2), w, lane);
     __syncthreads();
-    wide_stream<ALL3, false>(c, smem, grp, w, lane, geo, 0, p, npass, step, pf);
+    wide_stream<ALL3, false, EXACT>(c, smem, grp, w, lane, geo, 0, p, npass, step, pf);
 }
 
 // ---------------------------------------------------------------------------
@@ -2077,7 +2099,7 @@ constexpr int split_threads()
     return R <= 4 ? 1024 : (R == 8 ? 768 : 320);
 }
 
-template <int R, bool ALL3, int IOMODE>
+template <int R, bool ALL3, int IOMODE, bool EXACT = false>
 __global__ __launch_bounds__(split_threads<R>())
 __attribute__((amdgpu_waves_per_eu(split_threads<R>() / 256, split_threads<R>() / 256))) void jw_main64s_kernel(jw_run_desc d, int ncomp, int* err,
                                                                         jw_source_desc src, const void* mat)
@@ -2149,7 +2171,7 @@ __attribute__((amdgpu_waves_per_eu(split_threads<R>() / 256, split_threads<R>() 
                 else load_pair_direct<R>(pf, lane, g, 2 * qn);
             }
             if (IOMODE != 0) scale_input<R>(x0, x1, lane, d, fin);
-            compute_pair<R, ALL3>(tab, lane, g, x0, x1);
+            compute_pair<R, ALL3, 1, false, EXACT>(tab, lane, g, x0, x1);
             if (!wait_flag(vfull + wave, 0, polls)) { ok = false; break; }
             write_blocked<R>(stg, lane, x0, x1);
             if (lane == 0) __hip_atomic_store(&s_pair[wave], (long long)q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
@@ -2646,26 +2668,15 @@ __global__ __launch_bounds__(bsplit_threads<R>()) void jw_batch64s_kernel(const 
     queue_leave(counter);
 }
 
-template <int R, bool BUILD = false>
+template <int R>
 const void* kernel_ptr(bool all3)
 {
-    return all3 ? reinterpret_cast<const void*>(&jw_main64_kernel<R, true, BUILD>)
-                : reinterpret_cast<const void*>(&jw_main64_kernel<R, false, BUILD>);
+    return all3 ? reinterpret_cast<const void*>(&jw_main64_kernel<R, true, false>)
+                : reinterpret_cast<const void*>(&jw_main64_kernel<R, false, false>);
 }
 
-const void* pick64(int R, bool all3 = true, bool build = false)
+const void* pick64(int R, bool all3 = true)
 {
-    if (build) {
-        switch (R) {
-        case 2: return kernel_ptr<2, true>(all3);
-        case 4: return kernel_ptr<4, true>(all3);
-        case 8: return kernel_ptr<8, true>(all3);
-        case 16: return kernel_ptr<16, true>(all3);
-        case 32: return all3 ? reinterpret_cast<const void*>(&jw_wide64_kernel<true, true>)
-                             : reinterpret_cast<const void*>(&jw_wide64_kernel<false, true>);
-        default: return nullptr;
-        }
-    }
     switch (R) {
     case 32: return all3 ? reinterpret_cast<const void*>(&jw_wide64_kernel<true, false>)
                          : reinterpret_cast<const void*>(&jw_wide64_kernel<false, false>);
@@ -2673,6 +2684,29 @@ const void* pick64(int R, bool all3 = true, bool build = false)
     case 4: return kernel_ptr<4>(all3);
     case 8: return kernel_ptr<8>(all3);
     case 16: return kernel_ptr<16>(all3);
+    default: return nullptr;
+    }
+}
+
+// the kernels that build their table, for a solve_form
+template <int R>
+const void* build_ptr(int form)
+{
+    return form == kAllThree ? reinterpret_cast<const void*>(&jw_main64_kernel<R, true, true>)
+           : form == kSome   ? reinterpret_cast<const void*>(&jw_main64_kernel<R, false, true>)
+                             : reinterpret_cast<const void*>(&jw_main64_kernel<R, false, true, true>);
+}
+
+const void* pick64b(int R, int form)
+{
+    switch (R) {
+    case 2: return build_ptr<2>(form);
+    case 4: return build_ptr<4>(form);
+    case 8: return build_ptr<8>(form);
+    case 16: return build_ptr<16>(form);
+    case 32: return form == kAllThree ? reinterpret_cast<const void*>(&jw_wide64_kernel<true, true>)
+                    : form == kSome   ? reinterpret_cast<const void*>(&jw_wide64_kernel<false, true>)
+                                      : reinterpret_cast<const void*>(&jw_wide64_kernel<false, true, true>);
     default: return nullptr;
     }
 }
@@ -2747,12 +2781,14 @@ const void* pick_batch64s(int R)
 int bsplit_threads_rt(int R) { return R <= 4 ? 1024 : (R == 8 ? 768 : 512); }
 
 template <int R>
-const void* split_ptr(bool all3, int io)
+const void* split_ptr(int form, int io)
 {
+    const bool all3 = form == kAllThree;
     if constexpr (R > 2)
         if (io == 0)
-            return all3 ? reinterpret_cast<const void*>(&jw_main64s_kernel<R, true, 0>)
-                        : reinterpret_cast<const void*>(&jw_main64s_kernel<R, false, 0>);
+            return all3            ? reinterpret_cast<const void*>(&jw_main64s_kernel<R, true, 0>)
+                   : form == kSome ? reinterpret_cast<const void*>(&jw_main64s_kernel<R, false, 0>)
+                                   : reinterpret_cast<const void*>(&jw_main64s_kernel<R, false, 0, true>);
     if (io == 1)
         return all3 ? reinterpret_cast<const void*>(&jw_main64s_kernel<R, true, 1>)
                     : reinterpret_cast<const void*>(&jw_main64s_kernel<R, false, 1>);
@@ -2760,14 +2796,14 @@ const void* split_ptr(bool all3, int io)
                 : reinterpret_cast<const void*>(&jw_main64s_kernel<R, false, 2>);
 }
 
-// io: 0 plain step (R = 4, 8), 1 complex in and out (block layouts 4 and 7), 2 complex in
-// (layout 4), real systems out
-const void* pick_split(int R, bool all3, int io)
+// io: 0 plain step (R = 4, 8; every form), 1 complex in and out (block layouts 4 and 7),
+// 2 complex in (layout 4), real systems out
+const void* pick_split(int R, int form, int io)
 {
     switch (R) {
-    case 2: return io ? split_ptr<2>(all3, io) : nullptr;
-    case 4: return split_ptr<4>(all3, io);
-    case 8: return split_ptr<8>(all3, io);
+    case 2: return io ? split_ptr<2>(form, io) : nullptr;
+    case 4: return split_ptr<4>(form, io);
+    case 8: return split_ptr<8>(form, io);
     default: return nullptr;
     }
 }
@@ -2824,29 +2860,30 @@ int64_t jwdev_main64_lds_bytes(int R, int waves)
 /* pairs of systems per workgroup and pass */
 int jwdev_main64_pairs(int R, int waves) { return R == 32 ? kWideGroups : waves; }
 
-/* workgroups per CU, the smaller of the two variants (all recurrences / some) */
-static int main64_occupancy(int R, int waves, int lds, bool build)
+/* workgroups per CU of a kernel (0: it cannot run) */
+static int occupancy_of(const void* f, int threads, int lds)
 {
-    int best = -1;
-    for (int v = 0; v < 2; v++) {
-        const void* f = pick64(R, v == 0, build);
-        if (!f) return 0;
-        if (hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess) return 0;
-        int nb = 0;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, f, 64 * waves, lds) != hipSuccess) return 0;
-        if (best < 0 || nb < best) best = nb;
-    }
-    return best;
+    int nb = 0;
+    if (!f || hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess ||
+        hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, f, threads, lds) != hipSuccess)
+        return 0;
+    return nb;
 }
 
+/* the smaller of the variants (all recurrences / some) */
 int jwdev_main64_occupancy(int R, int waves)
 {
-    return main64_occupancy(R, waves, (int)jwdev_main64_lds_bytes(R, waves), false);
+    const int lds = (int)jwdev_main64_lds_bytes(R, waves);
+    const int all = occupancy_of(pick64(R, true), 64 * waves, lds), some = occupancy_of(pick64(R, false), 64 * waves, lds);
+    return all < some ? all : some;
 }
 
 int jwdev_main64(const jw_run_desc* r, int R, int waves, int grid, void* stream)
 {
-    if (!r->rhs || !r->table) { snprintf(g_err64, sizeof(g_err64), "main64: no rhs or table"); return -1; }
+    if (!r->rhs || !r->table) {
+        snprintf(g_err64, sizeof(g_err64), "main64: no rhs or table");
+        return -1;
+    }
     const void* f = pick64(R, r->fwd && r->b1 && r->b2);
     if (!f) { snprintf(g_err64, sizeof(g_err64), "no 64-lane kernel for R=%d", R); return -1; }
     const size_t lds = (size_t)jwdev_main64_lds_bytes(R, waves);
@@ -2884,12 +2921,17 @@ int jwdev_main64b_waves(int R)
 int jwdev_main64b_occupancy(int R)
 {
     const int w = jwdev_main64b_waves(R);
-    return w ? main64_occupancy(R, w, (int)main64b_lds_bytes(R), true) : 0;
+    int best = 1 << 30;
+    for (int form = kAllThree; w && form <= kSomeExact; form++) {
+        const int nb = occupancy_of(pick64b(R, form), 64 * w, (int)main64b_lds_bytes(R));
+        if (nb < best) best = nb;
+    }
+    return w ? best : 0;
 }
 
 int jwdev_main64b(const jw_run_desc* r, const jw_source_desc* src, const void* matrices, int R, int grid, void* stream)
 {
-    const void* f = pick64(R, r->fwd && r->b1 && r->b2, true);
+    const void* f = pick64b(R, solve_form(*r));
     if (!r->rhs || !matrices || !f || grid < 1) {
         snprintf(g_err64, sizeof(g_err64), "main64b: no rhs or matrices, or no kernel for R=%d", R);
         return -1;
@@ -3183,7 +3225,7 @@ int jwdev_batch64s(const jw_batch_item* d_items, const jw_batch_unit* d_units, i
 /* compute / store split kernel (R <= 8): shape, occupancy, launch */
 int jwdev_main64s_shape(int R, int* ncomp, int* nstore)
 {
-    if (!pick_split(R, true, 2)) return 0;
+    if (!pick_split(R, kAllThree, 2)) return 0;
     return split_shape(R, ncomp, nstore) ? 1 : 0;
 }
 
@@ -3201,13 +3243,10 @@ int jwdev_main64s_occupancy(int R)
     int c = 0, st = 0;
     if (!jwdev_main64s_shape(R, &c, &st)) return 0;
     int best = -1;
-    for (int v = 0; v < 6; v++) {
-        const void* f = pick_split(R, (v & 1) == 0, v >> 1);
+    for (int v = 0; v < 9; v++) {
+        const void* f = pick_split(R, v % 3, v / 3);
         if (!f) continue;
-        const int lds = (int)jwdev_main64s_lds_bytes(R, c);
-        if (hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess) return 0;
-        int nb = 0;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, f, 64 * (c + st), lds) != hipSuccess) return 0;
+        const int nb = occupancy_of(f, 64 * (c + st), (int)jwdev_main64s_lds_bytes(R, c));
         if (best < 0 || nb < best) best = nb;
     }
     return best;
@@ -3216,10 +3255,13 @@ int jwdev_main64s_occupancy(int R)
 int jwdev_main64s(const jw_run_desc* r, const jw_source_desc* src, const void* matrices, int R, int grid, int* d_err,
                   void* stream)
 {
-    if (!r->rhs || !matrices || !d_err) { snprintf(g_err64, sizeof(g_err64), "main64s: no rhs, matrices or flag"); return -1; }
+    if (!r->rhs || !matrices || !d_err) {
+        snprintf(g_err64, sizeof(g_err64), "main64s: no rhs, matrices or flag");
+        return -1;
+    }
     int c = 0, st = 0;
     if (!jwdev_main64s_shape(R, &c, &st)) { snprintf(g_err64, sizeof(g_err64), "no split kernel for R=%d", R); return -1; }
-    const void* f = pick_split(R, r->fwd && r->b1 && r->b2, (int)r->fused_io);
+    const void* f = pick_split(R, solve_form(*r), (int)r->fused_io);
     if (!f) { snprintf(g_err64, sizeof(g_err64), "no split kernel for R=%d, I/O %d", R, (int)r->fused_io); return -1; }
     const size_t lds = (size_t)jwdev_main64s_lds_bytes(R, c);
     hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
