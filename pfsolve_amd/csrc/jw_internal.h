@@ -287,9 +287,9 @@ int jwdev_long_prologue(const jw_source_desc* src, const void* matrices, void* t
                         int precision, int* sync, void* gval, int* err, void* stream);
 int jwdev_long_chunks(const jw_long_desc* d, int precision, int grid_x, void* stream);
 int jwdev_long_reduced(const jw_long_desc* d, int precision, void* stream);
-/* long FP64 systems whose rows are 16-byte aligned: the chunk modes on the pair machinery
- * (format-2 tables of JW_TAB64_ELEMS(8) elements per chunk, built by jwdev_long_prologue
- * when given that table size); a persistent grid of cu_count * occupancy workgroups at most */
+/* long FP64 systems whose rows are 16-byte aligned: REDUCE and FINISH on the pair machinery
+ * (format-2 tables of JW_TAB64_ELEMS(8) elements per chunk, built by jwdev_long64_front, which
+ * also runs COEF); a persistent grid of cu_count * occupancy workgroups at most */
 int64_t jwdev_long64_table_bytes(int64_t N);   /* the tables, then a pivot line per build */
 int64_t jwdev_long64_lds_bytes(void);
 int jwdev_long64_occupancy(void);

@@ -1116,8 +1116,7 @@ __global__ __launch_bounds__(max_threads<kLong64R>()) void jw_long64_kernel(jw_l
     double2* stg = reinterpret_cast<double2*>(smem + NTAB * 8) + (size_t)wave * 64 * R;
     const jw_run_desc& rd = d.run;
     const int64_t nc = d.nchunks;
-    const int64_t nsys = MODE == JW_LONG_COEF ? 3 : rd.nsys;
-    const int64_t ppc = (nsys + 1) >> 1;
+    const int64_t ppc = (rd.nsys + 1) >> 1;
     const int64_t u0 = (int64_t)blockIdx.x * per_wg;
     const int64_t u1 = u0 + per_wg < nc * ppc ? u0 + per_wg : nc * ppc;
     for (int64_t c = u0 / ppc; c < nc && c * ppc < u1; c++) {
@@ -1138,7 +1137,7 @@ __global__ __launch_bounds__(max_threads<kLong64R>()) void jw_long64_kernel(jw_l
         const int64_t q0 = (u0 > c * ppc ? u0 : c * ppc) - c * ppc;
         const int64_t q1 = (u1 < (c + 1) * ppc ? u1 : (c + 1) * ppc) - c * ppc;
         for (int64_t q = q0 + wave; q < q1; q += nwaves) {
-            const jw_pass64 g = make_pass64(reinterpret_cast<double*>(rd.rhs), nsys, rd.stride, rd.offSol + rb, ilo,
+            const jw_pass64 g = make_pass64(reinterpret_cast<double*>(rd.rhs), rd.nsys, rd.stride, rd.offSol + rb, ilo,
                                             ihi, olo, ohi, rd.kl, rd.ku, rd.fwd, rd.b1, rd.b2,
                                             MODE == JW_LONG_FINISH && c == 0 && rd.apply_scale, rd.scale_hi, lane);
             long64_pass<MODE, ALL3>(tab, stg, lane, g, d, c, 2 * q);
@@ -2668,22 +2667,15 @@ __global__ __launch_bounds__(bsplit_threads<R>()) void jw_batch64s_kernel(const 
     queue_leave(counter);
 }
 
-template <int R>
-const void* kernel_ptr(bool all3)
-{
-    return all3 ? reinterpret_cast<const void*>(&jw_main64_kernel<R, true, false>)
-                : reinterpret_cast<const void*>(&jw_main64_kernel<R, false, false>);
-}
-
-const void* pick64(int R, bool all3 = true)
+// the kernels on tables in memory (the fused step)
+const void* pick64(int R)
 {
     switch (R) {
-    case 32: return all3 ? reinterpret_cast<const void*>(&jw_wide64_kernel<true, false>)
-                         : reinterpret_cast<const void*>(&jw_wide64_kernel<false, false>);
-    case 2: return kernel_ptr<2>(all3);
-    case 4: return kernel_ptr<4>(all3);
-    case 8: return kernel_ptr<8>(all3);
-    case 16: return kernel_ptr<16>(all3);
+    case 2: return reinterpret_cast<const void*>(&jw_main64_kernel<2, true, false>);
+    case 4: return reinterpret_cast<const void*>(&jw_main64_kernel<4, true, false>);
+    case 8: return reinterpret_cast<const void*>(&jw_main64_kernel<8, true, false>);
+    case 16: return reinterpret_cast<const void*>(&jw_main64_kernel<16, true, false>);
+    case 32: return reinterpret_cast<const void*>(&jw_wide64_kernel<true, false>);
     default: return nullptr;
     }
 }
@@ -2721,7 +2713,6 @@ const void* long64_ptr(bool all3)
 const void* pick_long64(int mode, bool all3)
 {
     switch (mode) {
-    case JW_LONG_COEF: return long64_ptr<JW_LONG_COEF>(all3);
     case JW_LONG_REDUCE: return long64_ptr<JW_LONG_REDUCE>(all3);
     case JW_LONG_FINISH: return long64_ptr<JW_LONG_FINISH>(all3);
     default: return nullptr;
@@ -2870,21 +2861,18 @@ static int occupancy_of(const void* f, int threads, int lds)
     return nb;
 }
 
-/* the smaller of the variants (all recurrences / some) */
 int jwdev_main64_occupancy(int R, int waves)
 {
-    const int lds = (int)jwdev_main64_lds_bytes(R, waves);
-    const int all = occupancy_of(pick64(R, true), 64 * waves, lds), some = occupancy_of(pick64(R, false), 64 * waves, lds);
-    return all < some ? all : some;
+    return occupancy_of(pick64(R), 64 * waves, (int)jwdev_main64_lds_bytes(R, waves));
 }
 
 int jwdev_main64(const jw_run_desc* r, int R, int waves, int grid, void* stream)
 {
-    if (!r->rhs || !r->table) {
-        snprintf(g_err64, sizeof(g_err64), "main64: no rhs or table");
+    if (!r->rhs || !r->table || solve_form(*r) != kAllThree) {
+        snprintf(g_err64, sizeof(g_err64), "main64: no rhs or table, or not a fused step");
         return -1;
     }
-    const void* f = pick64(R, r->fwd && r->b1 && r->b2);
+    const void* f = pick64(R);
     if (!f) { snprintf(g_err64, sizeof(g_err64), "no 64-lane kernel for R=%d", R); return -1; }
     const size_t lds = (size_t)jwdev_main64_lds_bytes(R, waves);
     hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
@@ -3287,7 +3275,7 @@ int64_t jwdev_long64_lds_bytes(void)
 int jwdev_long64_occupancy(void)
 {
     int best = -1;
-    for (int m = JW_LONG_COEF; m <= JW_LONG_FINISH + 1; m++) {
+    for (int m = JW_LONG_REDUCE; m <= JW_LONG_FINISH + 1; m++) {
         for (int v = 0; v < 2; v++) {
             const void* f = m <= JW_LONG_FINISH ? pick_long64(m, v == 0) : pick_long64_front(v == 0);
             const int lds = (int)jwdev_long64_lds_bytes();
@@ -3379,27 +3367,26 @@ int jwdev_long64_front(const jw_source_desc* src, const void* matrices, const jw
 int jwdev_long64(const jw_long_desc* d, int cu_count, int occupancy, void* stream)
 {
     const int C = 64 * kLong64R;
-    if (!d->table || !d->red || (d->mode != JW_LONG_COEF && !d->run.rhs)) {
+    if (!d->table || !d->red || !d->run.rhs) {
         jwdev_set_error("long64: no table, reduced data or rhs");
         return -1;
     }
-    if (d->mode < JW_LONG_COEF || d->mode > JW_LONG_FINISH || d->nchunks < 1 ||
+    if ((d->mode != JW_LONG_REDUCE && d->mode != JW_LONG_FINISH) || d->nchunks < 1 ||
         (int64_t)d->nchunks * C < d->run.N || d->tab_elems != JW_TAB64_ELEMS(kLong64R) || cu_count < 1 ||
         occupancy < 1) {
         jwdev_set_error("long64: bad mode, chunk count, table size or grid");
         return -1;
     }
-    if (d->mode != JW_LONG_COEF && d->run.nsys > d->red_sys) {
+    if (d->run.nsys > d->red_sys) {
         jwdev_set_error("long64: slice exceeds reduced data");
         return -1;
     }
     /* the DMA moves 16-byte row pairs: aligned systems only */
-    if (d->mode != JW_LONG_COEF &&
-        (((uintptr_t)d->run.rhs % 16) != 0 || (d->run.stride % 2) != 0 || (d->run.offSol % 2) != 0)) {
+    if (((uintptr_t)d->run.rhs % 16) != 0 || (d->run.stride % 2) != 0 || (d->run.offSol % 2) != 0) {
         jwdev_set_error("long64: systems not 16-byte aligned");
         return -1;
     }
-    const int64_t nsys = d->mode == JW_LONG_COEF ? 3 : d->run.nsys;
+    const int64_t nsys = d->run.nsys;
     if (nsys < 1) return 0;
     const int64_t total = (int64_t)d->nchunks * ((nsys + 1) / 2);
     int64_t grid = (int64_t)cu_count * occupancy;

@@ -23,11 +23,9 @@ struct pfsolve_plan {
     size_t table_bytes;
     size_t table_stride;      /* bytes between the slots' tables */
     int64_t lds_bytes;
-    /* wave-per-system FP64 path (table format 2): rows per lane (0 = not available),
-     * waves per workgroup and workgroups per CU */
+    /* wave-per-system FP64 path (the kernels that build their table in LDS): rows per lane
+     * (0 = not available), waves per workgroup and workgroups per CU */
     int R64, waves64, occupancy64;
-    /* the variant that builds its table in LDS (R64 <= 16; 0: not available) */
-    int waves64b, occupancy64b;
     /* compute / store split kernel for R64 <= 8 (0 = not used), its workgroups per
      * CU, and the device flag it raises when a bounded wait runs out */
     int split64, occupancy_split;

@@ -233,13 +233,9 @@ static PfSolveResult plan_setup(PfSolveApplication* app, struct pfsolve_plan* p)
             int r64 = 2;
             while (r64 * 64 < p->N) r64 *= 2;
             if (r64 <= 32) {
-                p->R64 = r64;
-                p->waves64 = jwdev_main64_waves(r64);
-                p->occupancy64 = p->waves64 ? jwdev_main64_occupancy(r64, p->waves64) : 0;
-                if (p->occupancy64 < 1) p->R64 = 0;
-                p->waves64b = jwdev_main64b_waves(r64);
-                p->occupancy64b = p->waves64b ? jwdev_main64b_occupancy(r64) : 0;
-                if (p->occupancy64b < 1) p->waves64b = 0;
+                p->waves64 = jwdev_main64b_waves(r64);
+                p->occupancy64 = p->waves64 ? jwdev_main64b_occupancy(r64) : 0;
+                if (p->occupancy64 >= 1) p->R64 = r64;
             }
             if (p->R64) {
                 size_t b2 = (size_t)jwdev_table64_elems(p->R64) * 8;
@@ -627,7 +623,6 @@ static PfSolveResult append_long(PfSolveApplication* app, const jw_source_desc* 
  * systems 13.6 / 15.2; two instead of three measured the same). */
 static int use_build_kernel(const struct pfsolve_plan* p, int64_t npass, int64_t cap_split, int64_t cap_build)
 {
-    if (!p->waves64b) return 0;
     if (!p->split64 || p->R64 == 2) return 1;
     const int64_t sweeps_split = (npass + cap_split - 1) / cap_split, sweeps_build = (npass + cap_build - 1) / cap_build;
     return sweeps_build < sweeps_split && sweeps_build <= (p->R64 == 4 ? 3 : 1);
@@ -684,37 +679,29 @@ static PfSolveResult append_impl(PfSolveApplication* app, const PfSolveLaunchPar
         /* unaligned systems of N > 1024 are taken where the chunk path takes them: not with
          * kernelVariant 2, nor by the allocation-free entry point, whose area has no room for it */
         const int chunks = p->long_R && !(p->area_cap && p->table_bytes > p->area_cap);
-        const int in_lds = p->split64 || (p->waves64b && (run.vec2 || p->R64 < 32 || chunks));
-        if (p->R64 && (run.vec2 || (in_lds && base % 8 == 0)) && cfg->kernelVariant != 1) {
-            /* wave-per-system kernels: table format 2, built by every workgroup, or by a
-             * launch before where that variant is not available.  The kernels that build load and store
-             * global memory from registers and take systems at any 8-byte address (30000
-             * systems of 333 rows, packed: 41.4 us a step, 61.8 us on the general kernel and
-             * its table launch); the other stages by LDS DMA, 16-byte aligned */
+        if (p->R64 && (run.vec2 || (base % 8 == 0 && (p->R64 < 32 || chunks))) && cfg->kernelVariant != 1) {
+            /* wave-per-system kernels: table format 2, built by every workgroup in its LDS.  They
+             * load and store global memory from registers and take systems at any 8-byte address
+             * (30000 systems of 333 rows, packed: 39 us a step, 62 us on the general kernel and
+             * its table launch) */
             if (nsys <= 0) return PFSOLVE_SUCCESS;
             const int64_t npass = (nsys + 1) / 2;   /* pairs of systems */
             const int64_t cap_split = (int64_t)p->cu_count * p->occupancy_split * p->split64;
-            const int64_t cap_build = (int64_t)p->cu_count * p->occupancy64b * p->waves64b;
+            const int64_t cap_build = (int64_t)p->cu_count * p->occupancy64 * p->waves64;
             const int build = use_build_kernel(p, npass, cap_split, cap_build);
-            if (!build && !p->split64 && jwdev_prologue(&src, cfg->buffer[0], table, 64, p->R64, p->precision, 2, s) != 0)
-                return PFSOLVE_ERROR_FAILED_TO_LAUNCH_KERNEL;
-            const int per_wg = build ? jwdev_main64_pairs(p->R64, p->waves64b)
-                                     : (p->split64 ? p->split64 : jwdev_main64_pairs(p->R64, p->waves64));
+            const int per_wg = build ? jwdev_main64_pairs(p->R64, p->waves64) : p->split64;
             int64_t need = (npass + per_wg - 1) / per_wg;
-            int64_t grid = (int64_t)p->cu_count *
-                           (build ? p->occupancy64b : (p->split64 ? p->occupancy_split : p->occupancy64));
+            int64_t grid = (int64_t)p->cu_count * (build ? p->occupancy64 : p->occupancy_split);
             if (grid > need) grid = need;
             if (grid < 1) grid = 1;
             if (p->ev_start && hipEventRecord(p->ev_start, s) != hipSuccess) return PFSOLVE_ERROR_FAILED_TO_EVENT_RECORD;
             if (build) {
                 if (jwdev_main64b(&run, &src, cfg->buffer[0], p->R64, (int)grid, s) != 0)
                     return PFSOLVE_ERROR_FAILED_TO_LAUNCH_KERNEL;
-            } else if (p->split64) {
+            } else {
                 run.wait_polls = p->wait_polls;
                 if (jwdev_main64s(&run, &src, cfg->buffer[0], p->R64, (int)grid, p->d_err, s) != 0)
                     return PFSOLVE_ERROR_FAILED_TO_LAUNCH_KERNEL;
-            } else if (jwdev_main64(&run, p->R64, p->waves64, (int)grid, s) != 0) {
-                return PFSOLVE_ERROR_FAILED_TO_LAUNCH_KERNEL;
             }
             if (p->ev_stop && hipEventRecord(p->ev_stop, s) != hipSuccess) return PFSOLVE_ERROR_FAILED_TO_EVENT_RECORD;
             return PFSOLVE_SUCCESS;
