@@ -891,7 +891,9 @@ struct ChainHooks {
         if (!chained || build == 0 || tid != 0) return;
         int polls = 0;
         bool ok = true;
-        while (__hip_atomic_load(&flags[build - 1], __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_AGENT) == 0) {
+        // relaxed polls, one acquire once the flag is seen: an acquire per poll invalidates caches
+        // under the builds that are not waiting
+        while (__hip_atomic_load(&flags[build - 1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0) {
             if (++polls > kLongMaxPolls) {
                 ok = false;
                 __hip_atomic_store(err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -899,6 +901,7 @@ struct ChainHooks {
             }
             __builtin_amdgcn_s_sleep(2);
         }
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
         carry[0] = ok ? gval[build - 1] : Ar<T>::one();
     }
     __device__ void publish(int tid, const T* g) const
