@@ -1823,18 +1823,84 @@ __device__ __forceinline__ void chain_multipliers(double* tab, int t)
     }
 }
 
+// A lane's part of an iteration's table: read where it is used from LDS, or from global memory
+// into registers as a whole (left to the compiler, in the kernel for tables in LDS, the loads came
+// one after another, 14 round trips through the L2 per iteration: N = 512, K = 16, 2000 systems
+// 46 us, 30 us this way)
+template <int R>
+struct chain_lds {
+    const double* tab;
+    int lane;
+    __device__ __forceinline__ double2 v(int i) const { return *reinterpret_cast<const double2*>(tab + (64 * i + lane) * 2); }
+    __device__ __forceinline__ double s(int i) const { return tab[128 * R + 64 * i + lane]; }
+    __device__ __forceinline__ double m(int k) const { return tab[192 * R + 64 * k + lane]; }
+    __device__ __forceinline__ void before_band() {}
+    __device__ __forceinline__ void before_solve() {}
+};
+template <int R>
+struct chain_regs {
+    const double* tab;
+    int lane;
+    double2 vv[R];
+    double ss[R], mm[7];
+    __device__ __forceinline__ double2 v(int i) const { return vv[i]; }
+    __device__ __forceinline__ double s(int i) const { return ss[i]; }
+    __device__ __forceinline__ double m(int k) const { return mm[k]; }
+    __device__ __forceinline__ void load_band()
+    {
+#pragma unroll
+        for (int i = 0; i < R; i++) vv[i] = load_chunk(tab + (64 * i + lane) * 2);
+    }
+    __device__ __forceinline__ void load_solve()
+    {
+        const JW_GLOBAL double* t = as_global(tab) + 128 * R + lane;
+#pragma unroll
+        for (int i = 0; i < R; i++) ss[i] = t[64 * i];
+#pragma unroll
+        for (int k = 0; k < 7; k++) mm[k] = t[64 * (R + k)];
+    }
+    // waits for the loads: none is put off to its use
+    __device__ __forceinline__ void hold_band()
+    {
+#pragma unroll
+        for (int i = 0; i < R; i++) asm volatile("" : "+v"(vv[i].x), "+v"(vv[i].y));
+    }
+    __device__ __forceinline__ void hold_solve()
+    {
+#pragma unroll
+        for (int i = 0; i < R; i++) asm volatile("" : "+v"(ss[i]));
+#pragma unroll
+        for (int k = 0; k < 7; k++) asm volatile("" : "+v"(mm[k]));
+    }
+    // R = 16: in two parts, for the registers
+    __device__ __forceinline__ void before_band()
+    {
+        load_band();
+        if (R < 16) load_solve();
+        hold_band();
+        if (R < 16) hold_solve();
+    }
+    __device__ __forceinline__ void before_solve()
+    {
+        if (R < 16) return;
+        load_solve();
+        hold_solve();
+    }
+};
+
 // one iteration on a pair in registers (the steps of compute_pair for these operators)
-template <int R, bool UP>
-__device__ __forceinline__ void chain_pair(const double* tab, int lane, bool band, bool solve, bool apply_scale,
-                                           double row0_scale, double (&x0)[R], double (&x1)[R])
+template <int R, bool UP, class Tab>
+__device__ __forceinline__ void chain_pair(Tab tab, bool band, bool solve, bool apply_scale, double row0_scale,
+                                           double (&x0)[R], double (&x1)[R])
 {
+    tab.before_band();
     if (band) {
         double na = UP ? dpp_d<DPP_WAVE_SHL1>(x0[0]) : dpp_d<DPP_WAVE_SHR1>(x0[R - 1]);
         double nb = UP ? dpp_d<DPP_WAVE_SHL1>(x1[0]) : dpp_d<DPP_WAVE_SHR1>(x1[R - 1]);
 #pragma unroll
         for (int k = 0; k < R; k++) {
             const int i = UP ? R - 1 - k : k;   // from the end whose neighbour came from the next lane
-            const double2 v = *reinterpret_cast<const double2*>(tab + (64 * i + lane) * 2);
+            const double2 v = tab.v(i);
             const double xa = x0[i], xb = x1[i];
             x0[i] = __builtin_fma(v.y, na, v.x * xa);
             x1[i] = __builtin_fma(v.y, nb, v.x * xb);
@@ -1843,10 +1909,10 @@ __device__ __forceinline__ void chain_pair(const double* tab, int lane, bool ban
         }
     }
     if (!solve) return;
+    tab.before_solve();
     double s[R];
 #pragma unroll
-    for (int i = 0; i < R; i++) s[i] = tab[128 * R + 64 * i + lane];
-    const double* m = tab + 192 * R + lane;
+    for (int i = 0; i < R; i++) s[i] = tab.s(i);
     // row order of the recurrence: forward (UP) or backward
     double a = x0[UP ? 0 : R - 1], b = x1[UP ? 0 : R - 1];
 #pragma unroll
@@ -1857,7 +1923,7 @@ __device__ __forceinline__ void chain_pair(const double* tab, int lane, bool ban
     }
 #pragma unroll
     for (int k = 0; k < 4; k++) {
-        const double f = m[64 * k];
+        const double f = tab.m(k);
         double sa, sb;
         switch (k) {
         case 0: sa = dpp_d<UP ? DPP_ROW_SHR(1) : DPP_ROW_SHL(1)>(a); sb = dpp_d<UP ? DPP_ROW_SHR(1) : DPP_ROW_SHL(1)>(b); break;
@@ -1869,7 +1935,7 @@ __device__ __forceinline__ void chain_pair(const double* tab, int lane, bool ban
         b = __builtin_fma(f, sb, b);
     }
     if (UP) {
-        const double f4 = m[64 * 4], f5 = m[64 * 5];
+        const double f4 = tab.m(4), f5 = tab.m(5);
         const double sa = dpp_rm<DPP_ROW_BCAST15, 0xa>(a), sb = dpp_rm<DPP_ROW_BCAST15, 0xa>(b);
         a = __builtin_fma(f4, sa, a);
         b = __builtin_fma(f4, sb, b);
@@ -1879,7 +1945,7 @@ __device__ __forceinline__ void chain_pair(const double* tab, int lane, bool ban
     } else {
         const double a1 = readlane_d(a, 16), a2 = readlane_d(a, 32), a3 = readlane_d(a, 48);
         const double b1 = readlane_d(b, 16), b2 = readlane_d(b, 32), b3 = readlane_d(b, 48);
-        const double c1 = m[64 * 4], c2 = m[64 * 5], c3 = m[64 * 6];
+        const double c1 = tab.m(4), c2 = tab.m(5), c3 = tab.m(6);
         a = __builtin_fma(c1, a1, a);
         b = __builtin_fma(c1, b1, b);
         a = __builtin_fma(c2, a2, a);
@@ -1905,10 +1971,11 @@ __device__ __forceinline__ void chain_pair(const double* tab, int lane, bool ban
 
 __host__ __device__ constexpr int chain_max_waves(int R) { return R <= 8 ? 16 : 8; }
 
-// LDS: the first kl tables, then one system's staging per wavefront; the tables of
-// iterations kl .. K-1 (if any) are in global memory
-template <int R, bool UP>
-__global__ __launch_bounds__(64 * chain_max_waves(R)) void jw_chain64_kernel(jw_run_desc d, jw_chain_jobs jobs, int kl)
+// LDS: the first kl tables, then one system's staging per wavefront.  GLOB: the tables of
+// iterations kl .. K-1 are in global memory (at most 8 wavefronts, for the registers)
+template <int R, bool UP, bool GLOB>
+__global__ __launch_bounds__(64 * (GLOB ? 8 : chain_max_waves(R))) void jw_chain64_kernel(jw_run_desc d,
+                                                                                        jw_chain_jobs jobs, int kl)
 {
     constexpr int TE = chain_tab_elems(R);
     extern __shared__ __align__(16) unsigned char smem[];
@@ -1946,9 +2013,15 @@ __global__ __launch_bounds__(64 * chain_max_waves(R)) void jw_chain64_kernel(jw_
         const int64_t qn = q + step;
         if (qn < npass) load(qn);
         for (int k = 0; k < kl; k++)
-            chain_pair<R, UP>(ltab + k * TE, lane, d.band, solve, g.apply_scale, g.row0_scale, x0, x1);
-        for (int k = kl; k < K; k++)
-            chain_pair<R, UP>(gtab + (int64_t)k * TE, lane, d.band, solve, g.apply_scale, g.row0_scale, x0, x1);
+            chain_pair<R, UP>(chain_lds<R>{ltab + k * TE, lane}, d.band, solve, g.apply_scale, g.row0_scale, x0, x1);
+        if constexpr (GLOB) {
+            for (int k = kl; k < K; k++) {
+                chain_regs<R> t;
+                t.tab = gtab + (int64_t)k * TE;
+                t.lane = lane;
+                chain_pair<R, UP>(t, d.band, solve, g.apply_scale, g.row0_scale, x0, x1);
+            }
+        }
         store_pair<R, pair_ahead(R)>(stg, lane, g, 2 * q, x0, x1, true);
         q = qn;
     }
@@ -2948,42 +3021,57 @@ int jwdev_main64b(const jw_run_desc* r, const jw_source_desc* src, const void* m
 
 namespace {
 template <int R, bool UP>
-const void* chain_ptr(bool tables)
+const void* chain_ptr(bool glob)
 {
-    return tables ? reinterpret_cast<const void*>(&jw_chain_tables_kernel<R, UP>)
-                  : reinterpret_cast<const void*>(&jw_chain64_kernel<R, UP>);
+    // (R <= 4: 16 tables fit)
+    if constexpr (R >= 8)
+        if (glob) return reinterpret_cast<const void*>(&jw_chain64_kernel<R, UP, true>);
+    return glob ? nullptr : reinterpret_cast<const void*>(&jw_chain64_kernel<R, UP, false>);
 }
 
-// the chain kernel, or the build of its global tables
-const void* pick_chain(int R, bool up, bool tables)
+// the chain kernel, with some of its tables in global memory or none
+const void* pick_chain(int R, bool up, bool glob)
 {
     switch (R) {
-    case 2: return up ? chain_ptr<2, true>(tables) : chain_ptr<2, false>(tables);
-    case 4: return up ? chain_ptr<4, true>(tables) : chain_ptr<4, false>(tables);
-    case 8: return up ? chain_ptr<8, true>(tables) : chain_ptr<8, false>(tables);
-    case 16: return up ? chain_ptr<16, true>(tables) : chain_ptr<16, false>(tables);
+    case 2: return up ? chain_ptr<2, true>(glob) : chain_ptr<2, false>(glob);
+    case 4: return up ? chain_ptr<4, true>(glob) : chain_ptr<4, false>(glob);
+    case 8: return up ? chain_ptr<8, true>(glob) : chain_ptr<8, false>(glob);
+    case 16: return up ? chain_ptr<16, true>(glob) : chain_ptr<16, false>(glob);
     default: return nullptr;
     }
+}
+
+// the build of the tables in global memory
+const void* pick_chain_tables(int R, bool up)
+{
+    if (R == 8)
+        return up ? reinterpret_cast<const void*>(&jw_chain_tables_kernel<8, true>)
+                  : reinterpret_cast<const void*>(&jw_chain_tables_kernel<8, false>);
+    if (R == 16)
+        return up ? reinterpret_cast<const void*>(&jw_chain_tables_kernel<16, true>)
+                  : reinterpret_cast<const void*>(&jw_chain_tables_kernel<16, false>);
+    return nullptr;
 }
 
 int64_t chain_stage_bytes(int R) { return 64LL * R * 8; }   // one system per wavefront
 
 // Tables in LDS and wavefronts per workgroup: every table with at least 4 stagings after
-// them (one wavefront per SIMD), else as many tables as leave room for 8 stagings (6 at
-// R = 16): N = 1000, K = 8, 16384 systems: 161 us with 4 of the 8 tables in LDS, 195 us with none.
+// them (one wavefront per SIMD), else as many tables as leave room for 8 stagings: N = 1000, K = 8,
+// 16384 systems: 109 us with none of the 8 tables in LDS, 93 with 3, 106 with 4 and 6 stagings;
+// N = 512, K = 12, 20000 systems: 104 with none of the 12, 86 with 4, 75 with 8.
 void chain_split(int R, int K, int* kl, int* waves)
 {
     const int64_t tab = (int64_t)chain_tab_elems(R) * 8;
     int64_t w = (kLdsBytesMax - K * tab) / chain_stage_bytes(R);
     *kl = K;
     if (w < 4) {
-        w = R == 16 ? 6 : 8;
+        w = 8;
         *kl = (int)((kLdsBytesMax - w * chain_stage_bytes(R)) / tab);
     }
     *waves = w > chain_max_waves(R) ? chain_max_waves(R) : (int)w;
 }
 
-size_t chain_lds(int R, int kl, int waves)
+size_t chain_lds_bytes(int R, int kl, int waves)
 {
     return (size_t)(kl * (int64_t)chain_tab_elems(R) * 8 + waves * chain_stage_bytes(R));
 }
@@ -2994,14 +3082,14 @@ extern "C" {
 /* wavefronts per workgroup, workgroups per CU of a chained step (0: not available) */
 int jwdev_chain64_shape(int R, int K, int* waves)
 {
-    if (!pick_chain(R, true, false) || K < 1) return 0;
+    if (!pick_chain(R, true, false) || K < 1 || K > JW_CHAIN_MAX) return 0;
     int kl = 0;
     chain_split(R, K, &kl, waves);
-    const int lds = (int)chain_lds(R, kl, *waves);
+    const int lds = (int)chain_lds_bytes(R, kl, *waves);
     int best = -1;
     for (int up = 0; up < 2; up++) {
-        const void* f = pick_chain(R, up, false);
-        if (hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess) return 0;
+        const void* f = pick_chain(R, up, kl < K);
+        if (!f || hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess) return 0;
         int nb = 0;
         if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, f, 64 * *waves, lds) != hipSuccess) return 0;
         if (best < 0 || nb < best) best = nb;
@@ -3017,18 +3105,21 @@ int jwdev_chain64(const jw_run_desc* r, const jw_chain_jobs* jobs, int up, int g
     }
     int kl = 0, waves = 0;
     chain_split(jobs->R, jobs->K, &kl, &waves);
-    if (kl < jobs->K && !jobs->table) { snprintf(g_err64, sizeof(g_err64), "chain64: no tables"); return -1; }
+    if (kl < jobs->K && (!jobs->table || !pick_chain_tables(jobs->R, up))) {
+        snprintf(g_err64, sizeof(g_err64), "chain64: no tables");
+        return -1;
+    }
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
     jw_run_desc rr = *r;
     jw_chain_jobs jj = *jobs;
     if (kl < jobs->K) {
         void* args[] = {&jj, &kl};
-        if (hipLaunchKernel(pick_chain(jobs->R, up, true), dim3(jobs->K - kl), dim3(64 * jobs->R), args, 0, s) !=
+        if (hipLaunchKernel(pick_chain_tables(jobs->R, up), dim3(jobs->K - kl), dim3(64 * jobs->R), args, 0, s) !=
             hipSuccess)
             return -3;
     }
-    const void* f = pick_chain(jobs->R, up, false);
-    const size_t lds = chain_lds(jobs->R, kl, waves);
+    const void* f = pick_chain(jobs->R, up, kl < jobs->K);
+    const size_t lds = chain_lds_bytes(jobs->R, kl, waves);
     hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) return -2;
     void* args[] = {&rr, &jj, &kl};
