@@ -731,7 +731,7 @@ def bench_chain(torch, pf, steps: int, warmup: int, N: int = 512, ncx: int = 655
                     f"Jones-Worland connection matrices of degree 2N, {ncx} complex systems (XXII), FP64",
         "value": ncx / (ms * 1e-3), "unit": "complex systems/s (K-step)", "ms_per_step": ms,
         "p50_ms": float(np.percentile(per, 50)), "p99_ms": float(np.percentile(per, 99)),
-        "kernel": f"jw_chain64_kernel<{plan_rows(N)}, true>", "kernel_ms": kms,
+        "kernel": f"jw_chain64_kernel<{plan_rows(N)}, true, false>", "kernel_ms": kms,
         "bytes_per_k_step": alg, "hbm_frac": alg / (kms * 1e-3) / HBM_PEAK,
         "unchained_ms_per_step": ms_un, "unchained_bytes_per_k_step": alg_un,
         "speedup_vs_unchained": ms_un / ms,

@@ -986,8 +986,9 @@ __device__ __forceinline__ void long64_pass(const double* tab, double2* stg, int
     // The edges, loaded while the DMA is in flight: lane 0 and lane 63 take them.  Every lane
     // loads (where it needs nothing, from inside the keep-range: the buffer need not hold a
     // system's other rows) and selects afterwards: with a branch around each load the compiler
-    // waited for it there, four round trips one after another in FINISH.  With the stores below moved behind the arithmetic: 512 systems of 100000
-    // rows 332 -> 318 us, 1000 of 20000 rows 138 -> 130.
+    // waited for it there, four round trips one after another in FINISH.  With the stores below
+    // moved behind the arithmetic: 512 systems of 100000 rows 332 -> 318 us, 1000 of 20000 rows
+    // 138 -> 130.
     double l1[2], l2[2], ca[2], cb[2];
     bool k1[2], k2[2];
     if constexpr (MODE == JW_LONG_COEF) {
